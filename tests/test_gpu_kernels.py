@@ -557,6 +557,53 @@ def test_product_of_few_rows(m, n, k, form):
         assert torch.equal(one[0], out[m - 1])
 
 
+# Sizes at which the product for prompts takes each of its tiles (one case each), rows and features that do not fill the last ones,
+# K of one turn and more, and K in pieces (the last four).
+@pytest.mark.parametrize("m,n,k", [(4001, 3584, 256), (2049, 3584, 768), (1000, 8224, 256), (513, 8224, 1280), (800, 3584, 768), (421, 8224, 256),
+                                   (129, 16, 256), (257, 48, 512), (129, 16, 768), (300, 4608, 2048), (300, 3584, 18944), (422, 3584, 9472)])
+def test_product_of_many_rows(m, n, k):
+    x, w = rand(m, k, seed=60, dtype=torch.bfloat16), rand(n, k, seed=61, scale=0.05, dtype=torch.bfloat16)
+    want = x.double() @ w.double().t()
+    # float32 sums: each of K additions rounds to 2^-24 of a sum that is at most that of the terms' sizes, and such errors mostly cancel
+    slack = 2.0 ** -22 * (x.double().abs() @ w.double().abs().t())
+    packed = K.pack_weight(w)
+    assert K.prompt_takes(m, n, k) and not K.prompt_takes(m, n, k + 64) and not K.prompt_takes(m, n + 8, k)
+    out = torch.full((m + 1, n), float("nan"), device=DEV)
+    K.prompt_store(x, packed, out[:m])
+    assert torch.isnan(out[m]).all() and ((out[:m].double() - want).abs() <= slack).all()
+    out16 = torch.full((m + 1, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    K.prompt_store(x, packed, out16[:m])
+    assert torch.isnan(out16[m].float()).all() and torch.equal(out16[:m], out[:m].to(torch.bfloat16))
+    left = K.prompt_store(x, packed, finish=False)
+    if isinstance(left, K.PartialSums):
+        assert torch.equal(sum(left.sums.unbind(0)), out[:m])
+    else:
+        assert torch.equal(left, out16[:m])
+    act = K.prompt_store(x, packed, gate=4)                 # max(z, 0)^2 of the rounded product
+    z = out16[:m].float().clamp(min=0)
+    assert torch.equal(act, (z * z).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("m,inter,k", [(1025, 18944, 512), (800, 4112, 512), (257, 18944, 256), (300, 4112, 512), (513, 8208, 768), (145, 18944, 512),
+                                       (129, 16, 256), (257, 48, 1280)])
+def test_gated_product_of_many_rows(m, inter, k):
+    x, w = rand(m, k, seed=62, dtype=torch.bfloat16), rand(2 * inter, k, seed=63, scale=0.05, dtype=torch.bfloat16)
+    packed = K.pack_weight(w, 2)
+    out = torch.full((m + 1, inter), float("nan"), dtype=torch.bfloat16, device=DEV)
+    K.prompt_gated(x, packed, out[:m])
+    g, u = (x.double() @ w.double().t()).chunk(2, 1)
+    want = torch.nn.functional.silu(g) * u
+    # gate and up are rounded to bfloat16 (2^-9 of each, or a whole step of 2^-8 where the float32 sum falls on the other side), then
+    # the result: the derivative of silu is at most silu / g + |silu|
+    bound = 2.0 ** -8 * (want.abs() * (2.5 + g.abs())) + 1e-4
+    assert torch.isnan(out[m].float()).all() and ((out[:m].double() - want).abs() <= bound).all()
+    # the other gates take the same sums: up itself where the gate is positive
+    K.prompt_gated(x, packed, out[:m], gate=1)
+    relu = g.clamp(min=0).to(torch.bfloat16).double() * u.to(torch.bfloat16).double()
+    # (the sums' own error, 2^-22 of the sum of their terms' sizes, is below 1e-4 at these K)
+    assert ((out[:m].double() - relu).abs() <= 3 * 2.0 ** -8 * relu.abs() + 1e-4 * (g.abs() + u.abs())).all()
+
+
 @pytest.mark.parametrize("m", [17, 32, 33, 64, 65, 100, 128])
 @pytest.mark.parametrize("n,k", [(100, 96), (3584, 3584), (1000, 18944), (4608, 1536), (48, 32), (65610, 64), (152064, 128), (264, 1056)])
 def test_product_of_17_to_128_rows(m, n, k):

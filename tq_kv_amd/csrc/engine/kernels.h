@@ -34,6 +34,11 @@ TQ_KERNEL(fused_qkv, cptr, cf32, int, float, cptr, int, cptr, cf32, cf32, int, c
 TQ_QUERY(int, mid_splits, int, int, int);
 TQ_KERNEL(mid_store, cptr, cptr, void*, int, int, int, int, void*, int, void*);
 TQ_KERNEL(mid_gated, cptr, cptr, void*, int, int, int, void*, void*);
+TQ_QUERY(int, prompt_takes, int, int, int, int);
+TQ_QUERY(int, prompt_splits, int, int, int);
+TQ_KERNEL(prompt_store, cptr, cptr, void*, int, int, int, int, void*, int, void*);
+TQ_KERNEL(prompt_store_act, cptr, cptr, void*, int, int, int, void*, int, float, float, void*);
+TQ_KERNEL(prompt_gated_act, cptr, cptr, void*, int, int, int, int, float, float, void*);
 TQ_KERNEL(rope_store, cptr, int, cptr, int, cf32, cf32, int, int, int, ci32, ci32, ci32, int, int, void*, void*, int, void*, int, int, int, int,
           int, void*);
 TQ_QUERY(int, rope_store_takes_sums, int, int, int, int, int, int);

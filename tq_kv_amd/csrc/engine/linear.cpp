@@ -25,6 +25,7 @@ int* policy_field(const std::string& name) {
     if (name == "packed") return &p.packed;
     if (name == "mid") return &p.mid;
     if (name == "keep_rows") return &p.keep_rows;
+    if (name == "prompt") return &p.prompt;
     if (name == "decode_mfma") return &p.decode_mfma;
     if (name == "prefill_mfma") return &p.prefill_mfma;
     return nullptr;
@@ -82,22 +83,35 @@ bool fusable(int64_t x_rows, const Weight& w, bool adds) {
     return p.fused && p.skinny && x_rows <= skinny_max_rows() && w.dtype == BF16 && w.k % 32 == 0 && (!adds || w.n % 4 == 0);
 }
 
-bool leaves_sums(int64_t x_rows, const Weight& w) {
+static bool mid_rows(int64_t x_rows, const Weight& w) {
     const Policy& p = policy();
     return p.mid && w.packed && w.dtype == BF16 && x_rows > skinny_max_rows() && x_rows <= mid_max_rows();
+}
+
+// whether the kernel for prompts takes a product of x_rows rows (its gated form reads the two parts' tiles for itself; the plain
+// one reads the tiles in a row, which is the features' order where every part is whole tiles)
+static bool prompt_rows(int64_t x_rows, const Weight& w, bool gated = false) {
+    if (!policy().prompt || !w.packed || w.dtype != BF16 || null_device() || x_rows <= mid_max_rows() || x_rows > INT32_MAX) return false;
+    if (gated ? w.parts != 2 : (w.n / w.parts) % 16 != 0) return false;
+    return K::prompt_takes.raw((int)x_rows, (int)w.n, (int)w.k, gated ? 1 : 0) != 0;
+}
+
+bool leaves_sums(int64_t x_rows, const Weight& w) {
+    if (mid_rows(x_rows, w)) return true;
+    return prompt_rows(x_rows, w) && K::prompt_splits.raw((int)x_rows, (int)w.n, (int)w.k) > 1;
 }
 
 void classify_step(StepContext& c, int64_t hidden) {
     const Policy& p = policy();
     c.fuse_small = p.fused && c.act_dtype == BF16 && c.all_decode && c.n_tokens <= skinny_max_rows() && hidden % 32 == 0;
-    c.fuse_mid = p.mid && c.act_dtype == BF16 && c.n_tokens > skinny_max_rows() && c.n_tokens <= mid_max_rows();
+    c.fuse_mid = p.mid && c.act_dtype == BF16 && c.n_tokens > skinny_max_rows();
 }
 
 static bool skinny_ok(const Tensor& x, const Weight& w) {
     return policy().skinny && x.dtype == BF16 && w.dtype == BF16 && x.shape[1] % 32 == 0 && x.shape[0] <= skinny_max_rows();
 }
 
-static bool mid_ok(const Tensor& x, const Weight& w) { return x.dtype == BF16 && leaves_sums(x.shape[0], w); }
+static bool mid_ok(const Tensor& x, const Weight& w) { return x.dtype == BF16 && mid_rows(x.shape[0], w); }
 
 // pointer and packed flag of a product's weight for the few-row kernels
 static const void* few_ptr(const Weight& w, int* packed) {
@@ -147,6 +161,23 @@ static Product k_mid_store(StepContext& c, const Tensor& x, const Weight& w, int
     return p;
 }
 
+// the product through the kernel for prompts; leave: its sums where it cuts K into pieces
+static Product k_prompt_store(StepContext& c, const Tensor& x, const Weight& w, int out_dtype, bool leave, Tensor* out) {
+    const int64_t m = x.shape[0];
+    const int splits = K::prompt_splits.raw((int)m, (int)w.n, (int)w.k);
+    Product p;
+    Tensor scratch;
+    if (splits > 1) scratch = c.alloc(F32, {splits, m, w.n});
+    p.is_sums = leave && splits > 1;
+    if (!p.is_sums) p.t = out ? *out : c.alloc(out_dtype, {m, w.n});
+    K::prompt_store(x.data, w.packed->t.data, p.t.data, out_dtype, (int)m, (int)w.n, (int)w.k, scratch.data, p.is_sums ? 0 : 1, c.stream);
+    if (p.is_sums) {
+        p.sums.sums = scratch;
+        p.sums.dtype = out_dtype;
+    }
+    return p;
+}
+
 static void k_mid_gated(StepContext& c, const Tensor& x, const Weight& w, Tensor& out, const Gate& gate) {
     const int64_t m = x.shape[0];
     const int splits = K::mid_splits.raw((int)w.n, (int)w.k, 1);
@@ -176,6 +207,7 @@ Product linear(StepContext& c, const Tensor& x, const Weight& w, const Tensor* b
             return p;
         }
         if (mid_ok(x, w)) return k_mid_store(c, x, w, out_dtype, leave_sums, out);
+        if (prompt_rows(m, w)) return k_prompt_store(c, x, w, out_dtype, leave_sums, out);
         if (!w.rows && m > mid_max_rows() && policy().library && !null_device() && w.n % 8 == 0) {
             // the rows were given up and this is a prompt: the rows come back for the length of this product (the weight
             // read and written once more, against reading it once per 128 rows of x)
@@ -213,7 +245,7 @@ Product linear(StepContext& c, const Tensor& x, const Weight& w, const Tensor* b
 bool takes_groups(int64_t x_rows, const Weight& w, int64_t group_rows) {
     if (w.dtype != BF16 || w.k % 32 || group_rows % 32 || null_device()) return false;
     if (policy().skinny && x_rows <= skinny_max_rows()) return true;
-    return leaves_sums(x_rows, w) && K::mid_takes_groups.raw((int)w.n, (int)w.k, (int)group_rows) != 0;
+    return mid_rows(x_rows, w) && K::mid_takes_groups.raw((int)w.n, (int)w.k, (int)group_rows) != 0;
 }
 
 Tensor linear_groups(StepContext& c, const Tensor& x, int64_t x_group_stride, const Weight& w, int64_t group_rows, int out_dtype) {
@@ -300,6 +332,10 @@ Tensor gated_linear(StepContext& c, const Tensor& x, const Weight& w, const Gate
     Tensor act = c.alloc(x.dtype, {m, inter});
     if (skinny_ok(x, w)) { k_fused_gated(c, x, nullptr, w, act, gate); return act; }
     if (mid_ok(x, w)) { k_mid_gated(c, x, w, act, gate); return act; }
+    if (x.dtype == BF16 && prompt_rows(m, w, true)) {
+        K::prompt_gated_act(x.data, w.packed->t.data, act.data, (int)m, (int)w.n, (int)w.k, gate.kind, gate.limit, gate.alpha, c.stream);
+        return act;
+    }
     if (!w.rows && !(m > mid_max_rows() && policy().library && !null_device() && w.n % 8 == 0)) {
         const int64_t step = mid_max_rows();
         for (int64_t r = 0; r < m; r += step) {
@@ -331,6 +367,14 @@ Tensor activated_linear(StepContext& c, const Tensor& x, const Weight& w, const 
         K::mid_store_act(x.data, w.packed->t.data, act.data, (int)m, (int)w.n, (int)w.k, scratch.data, gate.kind, gate.limit, gate.alpha, c.stream);
         return act;
     }
+    if (x.dtype == BF16 && prompt_rows(m, w)) {
+        Tensor act = c.alloc(BF16, {m, w.n});
+        const int splits = K::prompt_splits.raw((int)m, (int)w.n, (int)w.k);
+        Tensor scratch;
+        if (splits > 1) scratch = c.alloc(F32, {splits, m, w.n});
+        K::prompt_store_act(x.data, w.packed->t.data, act.data, (int)m, (int)w.n, (int)w.k, scratch.data, gate.kind, gate.limit, gate.alpha, c.stream);
+        return act;
+    }
     Tensor u = linear(c, x, w, nullptr, x.dtype).t;
     K::unary_act(u.data, u.data, u.dtype, (long long)u.numel(), gate.kind, gate.limit, gate.alpha, c.stream);
     return u;
@@ -356,7 +400,7 @@ static bool pieces_pay(const Weight& w) {
 void add_product(StepContext& c, Stream& stream, const Tensor& x, const Weight& w) {
     if (x.shape[0] > skinny_max_rows() || pieces_pay(w)) {
         const bool leave = stream.next_norm && stream.next_norm->takes_partial_sums();
-        Product p = k_mid_store(c, x, w, BF16, leave, nullptr);
+        Product p = x.shape[0] > mid_max_rows() ? k_prompt_store(c, x, w, BF16, leave, nullptr) : k_mid_store(c, x, w, BF16, leave, nullptr);
         stream.pending = p.is_sums ? Pending::of(p.sums) : Pending::of(p.t);
         stream.invalidate();
         return;

@@ -11,7 +11,9 @@
 //            copy of the weight, packed at loading time in the order its lanes take it.
 //   bfloat16, more rows up to what the kernel for mid-sized steps takes, where the weight has a packed copy
 //         -> the hand-written kernel that stages x in LDS and streams the packed weights
-//   bfloat16, more rows (prompts, large decoding batches)
+//   bfloat16, more rows (prompts, large decoding batches), where the weight has a packed copy and K is a multiple of 256
+//         -> the hand-written kernel that shares x in LDS and streams the packed weights (prompt_product.hip)
+//   bfloat16, more rows of other shapes, or without a packed copy
 //         -> the library GEMM (hipBLASLt), float32 accumulation; float32 output where logits are wanted
 #pragma once
 #include "parts.h"
@@ -24,9 +26,10 @@ namespace tq {
 // weights for the few-row kernels (twice the weight memory, about an eighth less time per
 // decoding step).  "keep_rows": off gives the rows up once a weight is packed (set it before
 // loading): a product of more rows than the own kernels take then gets the rows back from the
-// packed copy for its own length (or, with the library off, goes through the own kernels in pieces).
+// packed copy for its own length (or, with the library off, goes through the own kernels in pieces), unless the kernel for
+// prompts takes the packed copy itself.
 struct Policy {
-    int skinny = 1, library = 1, fused = 1, prune_last = 1, packed = 1, mid = 1, keep_rows = 1;
+    int skinny = 1, library = 1, fused = 1, prune_last = 1, packed = 1, mid = 1, keep_rows = 1, prompt = 1;
     int decode_mfma = 1, prefill_mfma = 1;
 };
 Policy& policy();
@@ -50,10 +53,11 @@ int mid_max_rows();
 // Whether the folded skinny kernels take a product of x_rows rows with this weight (adds: with
 // the result added to the stream).
 bool fusable(int64_t x_rows, const Weight& w, bool adds = false);
-// Whether a product of x_rows rows goes through the kernel for mid-sized steps, which can leave its sums to the next norm.
+// Whether a product of x_rows rows goes through a kernel that can leave its sums over pieces of K to the next norm: the one for
+// mid-sized steps, or the one for prompts where it cuts K.
 bool leaves_sums(int64_t x_rows, const Weight& w);
 // What kind of step this is for the parts' folding: small (norms and residual sums folded into
-// the products), mid (sums over pieces of K left to the next kernel), or neither.
+// the products), mid (sums over pieces of K may be left to the next kernel: any step of more rows), or neither.
 void classify_step(StepContext& c, int64_t hidden);
 
 struct Product {

@@ -227,7 +227,11 @@ void Model::tune_library(int64_t rows, hipStream_t stream) {
     for (const auto& b : blocks_) b->product_shapes(shapes);
     std::sort(shapes.begin(), shapes.end());
     shapes.erase(std::unique(shapes.begin(), shapes.end()), shapes.end());
-    for (const auto& nk : shapes) library_tune(rows, nk.first, nk.second, BF16, stream);
+    for (const auto& nk : shapes) {
+        // (the library is not asked for what the own kernel for prompts takes)
+        if (policy().prompt && policy().packed && K::prompt_takes.raw((int)std::min<int64_t>(rows, INT32_MAX), (int)nk.first, (int)nk.second, 0)) continue;
+        library_tune(rows, nk.first, nk.second, BF16, stream);
+    }
 }
 
 Json Model::describe() const {

@@ -117,6 +117,16 @@ int tqk_mid_store(const void* x, const void* w_packed, void* y, int y_dtype, int
 /* y[M, N/2] = silu(gate) * up, w = gate rows then up rows, packed in two parts */
 int tqk_mid_gated(const void* x, const void* w_packed, void* y, int M, int N, int K, void* scratch, void* stream);
 
+/* More rows than tqk_mid_max_rows (prompts): y[M,N] = x[M,K] w[N,K]^T, bfloat16, w packed (tqk_pack_weight; gated: in two parts), where
+ * tqk_prompt_takes.  K is cut into tqk_prompt_splits(M, N, K) pieces; where that is more than 1, scratch is float32 [pieces][M][N], and with
+ * finish == 0 the pieces' sums are left there and y is not written.  tqk_prompt_gated_act: y[M, N/2], never cut.
+ * tqk_prompt_store_act: bfloat16, an activation of the product (TQK_GATE_*). */
+int tqk_prompt_takes(int M, int N, int K, int gated);
+int tqk_prompt_splits(int M, int N, int K);
+int tqk_prompt_store(const void* x, const void* w_packed, void* y, int y_dtype, int M, int N, int K, void* scratch, int finish, void* stream);
+int tqk_prompt_store_act(const void* x, const void* w_packed, void* y, int M, int N, int K, void* scratch, int gate, float limit, float alpha, void* stream);
+int tqk_prompt_gated_act(const void* x, const void* w_packed, void* y, int M, int N, int K, int gate, float limit, float alpha, void* stream);
+
 /* For each token t and head: add bias, rotate q and k heads by the angle table row
  * tok_pos[t] (style 0: none, 1: halves (j, j+rot/2), 2: pairs (2j, 2j+1)), write q to
  * q_out [tokens, heads, head_dim] and, if write_kv, k and v into the pages of the

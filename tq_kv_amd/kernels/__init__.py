@@ -553,6 +553,45 @@ def mid_gated(x, weight_gate_up, out):
     return out
 
 
+def prompt_takes(m, n, k, gated=False):
+    """Whether prompt_store (prompt_gated: n counts both parts) takes a product of these sizes."""
+    return bool(library().tqk_prompt_takes(int(m), int(n), int(k), 1 if gated else 0))
+
+
+def prompt_store(x, weight, out=None, finish=True, gate=None, limit=0.0, alpha=1.0):
+    """out[M,N] = x weight^T (gate: that activation of it) for many rows of bfloat16; weight: a PackedWeight; out: bfloat16 or float32,
+    made here (bfloat16) if not given.  finish=False: as mid_store's."""
+    m, k = x.shape
+    if not isinstance(weight, PackedWeight):
+        raise KernelError("prompt_store: the weight must be packed (pack_weight)")
+    n = weight.shape[0]
+    w, _ = _weight(weight, "weight", n, k)
+    splits = int(library().tqk_prompt_splits(m, n, k))
+    scratch = torch.empty((splits, m, n), dtype=torch.float32, device=x.device) if splits > 1 else None
+    leave = not finish and scratch is not None
+    dtype = out.dtype if out is not None else torch.bfloat16
+    if out is None and not leave:
+        out = torch.empty((m, n), dtype=dtype, device=x.device)
+    xp, op, sp = _dev(x, "x", torch.bfloat16, (m, k)), _opt(None if leave else out, "out", None, (m, n)), _opt(scratch, "scratch")
+    if gate is not None:
+        _check(library().tqk_prompt_store_act(xp, w, op, m, n, k, sp, int(gate), ctypes.c_float(limit), ctypes.c_float(alpha), _stream()), "prompt_store")
+    else:
+        _check(library().tqk_prompt_store(xp, w, op, _code(dtype), m, n, k, sp, 0 if leave else 1, _stream()), "prompt_store")
+    return PartialSums(scratch, dtype) if leave else out
+
+
+def prompt_gated(x, weight_gate_up, out, gate=0, limit=0.0, alpha=1.0):
+    """out[M, I] = gate(x wg^T, x wu^T) for many rows; weight: a PackedWeight in 2 parts."""
+    m, inter = out.shape
+    k = x.shape[1]
+    if not isinstance(weight_gate_up, PackedWeight):
+        raise KernelError("prompt_gated: the weight must be packed (pack_weight with parts=2)")
+    w, _ = _weight(weight_gate_up, "weight", 2 * inter, k, parts=2)
+    _check(library().tqk_prompt_gated_act(_dev(x, "x", torch.bfloat16, (m, k)), w, _dev(out, "out", torch.bfloat16), m, 2 * inter, k, int(gate),
+                                          ctypes.c_float(limit), ctypes.c_float(alpha), _stream()), "prompt_gated")
+    return out
+
+
 def fused_residual_parts(n, k):
     """In how many pieces fused_residual gives the sums of squares for a weight [n, k]
     (never more than ceil(n / 16))."""

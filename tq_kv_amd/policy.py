@@ -1,19 +1,19 @@
 """Switches of the product and attention routines, for tests that compare one routine with
 another; nothing else reads these.  They live in the engine library (tqe_policy_set / _get):
 
-  skinny, mid, library   the hand-written products for few rows, for mid-sized steps, and the library's
+  skinny, mid, prompt, library   the hand-written products for few rows, for mid-sized steps and for prompts, and the library's
   fused                  norms and residual sums folded into the products of small decoding steps
   prune_last             the last run of the order computes the wanted rows only
   packed                 parts keep a second copy of their bfloat16 weights in the few-row kernels'
                          order (twice the weight memory, about an eighth less time per decoding step)
   keep_rows              off: the rows are given up once a weight is packed (set it before loading):
-                         half the weight memory again; a product of more than 128 rows (a prompt) gets the
-                         rows back from the packed copy for its own length
+                         half the weight memory again; a product of more than 128 rows (a prompt) that the kernel for
+                         prompts does not take gets the rows back from the packed copy for its own length
   decode_mfma, prefill_mfma   the two matrix-core attention kernels (off: the plain kernel)
 """
 from . import native
 
-NAMES = ("skinny", "library", "fused", "prune_last", "packed", "mid", "keep_rows", "decode_mfma", "prefill_mfma")
+NAMES = ("skinny", "library", "fused", "prune_last", "packed", "mid", "keep_rows", "decode_mfma", "prefill_mfma", "prompt")
 
 
 class _Policy:
