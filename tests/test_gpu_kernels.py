@@ -145,6 +145,23 @@ def test_gemm_generic_rows_do_not_depend_on_the_batch(rows, n, k, bias):
     assert torch.equal(few, full[41:41 + rows])
 
 
+@pytest.mark.parametrize("rows", [17, 64, 65, 300])
+@pytest.mark.parametrize("n,k", [(64, 32), (65, 1024), (130, 2052), (3584, 3584)])
+def test_float32_product_of_more_rows(rows, n, k):
+    """Through LDS, with and without the groups dealt out to several blocks: the bits of one row alone, and the error of float32 sums."""
+    x, w, b = rand(rows, k, seed=11), rand(n, k, seed=12), rand(n, seed=13)
+    out = torch.full((rows + 1, n), float("nan"), device=DEV)
+    K.gemm(x, w, b, out[:rows])
+    assert torch.isnan(out[rows]).all()
+    # every addition rounds to 2^-24 of a sum that is at most the sum of the terms' sizes; such errors mostly cancel
+    slack = 2.0 ** -21 * (x.double().abs() @ w.double().abs().t() + 1)
+    assert ((out[:rows].double() - (x.double() @ w.double().t() + b.double())).abs() <= slack).all()
+    for r in (0, rows - 1):
+        one = torch.empty(1, n, device=DEV)
+        K.gemm(x[r:r + 1].contiguous(), w, b, one)
+        assert torch.equal(one[0], out[r])
+
+
 def value_place(p):
     """Where position p of a page lies in a row of values: inside each 32 positions, the 4
     positions 4g..4g+3 of the first 16 are followed by 16+4g..16+4g+3 of the second 16."""
