@@ -324,6 +324,37 @@ def paged(k, v, page_ids, n_pages, dtype):
     return keys, values
 
 
+@pytest.mark.parametrize("d,nh,nkv", [(128, 28, 4), (128, 12, 2), (64, 40, 2), (32, 3, 1), (96, 4, 4), (256, 2, 1)])
+@pytest.mark.parametrize("n_sums,with_bias,window,n_parts", [(1, True, 0, 1), (7, True, 0, 2), (4, False, 70, 3), (5, True, 0, 8)])
+def test_decoding_attention_finishes_the_products_sums(d, nh, nkv, n_sums, with_bias, window, n_parts):
+    """Against the rotation's kernel followed by the attention alone: the outputs and what lies in the cache.  Positions at the edges of pages,
+    a row without earlier positions, heads in one group of 16 and in more, more partitions than pages."""
+    last = [0, 1, 63, 64, 127, 128, 300, 447]
+    n, width = len(last), 8
+    g = torch.Generator().manual_seed(70)
+    ids = torch.randperm(n * width, generator=g).tolist()
+    table = ints([[ids[i * width + j] if 64 * j <= p else -1 for j in range(width)] for i, p in enumerate(last)])
+    pos, total = ints(last), (nh + 2 * nkv) * d
+    sums = K.PartialSums(rand(n_sums, n, total, seed=71), torch.bfloat16)
+    bias = rand(total, seed=72, dtype=torch.bfloat16) if with_bias else None
+    c, s_ = plain.rope_tables(d, 1e4, 448)
+    cos, sin = c.to(DEV), s_.to(DEV)
+    cache = rand(n * width, nkv, 64, d, seed=73, dtype=torch.bfloat16), rand(n * width, nkv, d, 64, seed=74, dtype=torch.bfloat16)
+    keys, values = cache[0].clone(), cache[1].clone()
+    q = torch.empty(n, nh, d, dtype=torch.bfloat16, device=DEV)
+    K.rope_store(sums, bias, cos, sin, d, K.STYLE_HALVES, ints(range(n)), pos, table, keys, values, q, nh, nkv, d)
+    want = torch.empty(n, nh * d, dtype=torch.bfloat16, device=DEV)
+    K.attention_decode(q, keys, values, pos, table, window, d ** -0.5, want, n_parts=n_parts)
+    got = torch.full((n, nh * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    K.attention_decode(sums, cache[0], cache[1], pos, table, window, d ** -0.5, got, n_parts=n_parts, bias=bias, cos=cos, sin=sin)
+    # The values are the same bits.  In the rotation x0 c - x1 s the compiler joins a multiplication and the subtraction, not always the same
+    # one: a float32 result may differ by 2^-24 of its terms, and where it lies there bfloat16 rounds to the neighbour, a step of at
+    # most 2^-7.  A query or key that is such a step off moves a score by 2^-8 of one of d products, and an output by less than its own step.
+    assert torch.equal(cache[1], values)
+    for a, b in ((cache[0], keys), (got, want)):
+        assert ((a.float() - b.float()).abs() <= 2.0 ** -6 * b.float().abs() + 2.0 ** -9).all() and (a != b).float().mean() < 1e-2
+
+
 def attention_reference(q, k, v, pos, window, scale, cap=0.0):
     """q [T, nh, d] at absolute positions pos over k, v [nkv, S, d]: plain softmax attention (cap > 0: of cap tanh(score / cap))."""
     nh = q.shape[1]

@@ -42,10 +42,105 @@ union pack8 {
 
 #define AD_WAVES 4            // the most; blocks of 2 where the grid alone is more than the memory can serve at once
 
-template <int D, bool NT, int W>
+// The step's q, k and v as the sums over pieces of K that their product left (mid_product.hip), with what makes them queries and cache
+// entries: the work of tqk_rope_store_sums for one row.
+struct DecodeSums {
+    const float* sums;              // [n][rows][(heads + 2 kv heads) * head_dim]
+    int n;
+    size_t stride;
+    const bf16_t* bias;             // or null
+    const float *cos_table, *sin_table;         // [max_positions, head_dim / 2]
+    int max_positions;
+    bf16_t *keys, *values;          // the cache, to write
+};
+
+// Twice four values of the row, D / 2 apart, at their rounding to bfloat16 and the bias added: the pieces in their order, all of up to
+// eight under way together with the bias and the angles.
+template <int D>
+__device__ __forceinline__ void finished8(const DecodeSums& in, size_t at, size_t feature, float (&lo)[4], float (&hi)[4]) {
+    constexpr int BATCH = 8;
+    uint2 b_lo = make_uint2(0, 0), b_hi = b_lo;
+    if (in.bias) {
+        b_lo = *reinterpret_cast<const uint2*>(in.bias + feature);
+        b_hi = *reinterpret_cast<const uint2*>(in.bias + feature + D / 2);
+    }
+    floatx4_t a = {0.f, 0.f, 0.f, 0.f}, b = a;
+    for (int s = 0; s < in.n; s += BATCH) {
+        floatx4_t pa[BATCH], pb[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+            const float* src = in.sums + (size_t)min(s + u, in.n - 1) * in.stride + at;
+            pa[u] = *reinterpret_cast<const floatx4_t*>(src);
+            pb[u] = *reinterpret_cast<const floatx4_t*>(src + D / 2);
+        }
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+            const bool there = s + u < in.n;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { a[k] = there ? a[k] + pa[u][k] : a[k]; b[k] = there ? b[k] + pb[u][k] : b[k]; }
+        }
+    }
+    const float bias_lo[4] = {__uint_as_float(b_lo.x << 16), __uint_as_float(b_lo.x & 0xffff0000u), __uint_as_float(b_lo.y << 16), __uint_as_float(b_lo.y & 0xffff0000u)};
+    const float bias_hi[4] = {__uint_as_float(b_hi.x << 16), __uint_as_float(b_hi.x & 0xffff0000u), __uint_as_float(b_hi.y << 16), __uint_as_float(b_hi.y & 0xffff0000u)};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        lo[k] = to_float(from_float<bf16_t>(a[k]));
+        hi[k] = to_float(from_float<bf16_t>(b[k]));
+        if (in.bias) { lo[k] += bias_lo[k]; hi[k] += bias_hi[k]; }
+    }
+}
+
+// A block's part of that work: the queries of its heads (n_live of them from head0 on) into LDS, rows of D + 8; and where the block reads the
+// row's own position (owner), the position's key and value into the cache.  (Blocks that share a kv head and a page write the
+// same values; each reads its own writes, behind a barrier.)
+template <int D>
+__device__ __forceinline__ void finish_row(const DecodeSums& in, int seq, int pos, int page, bool owner, int head0, int n_live, int kvh, int n_heads,
+                                           int n_kv_heads, bf16_t* q_lds) {
+    constexpr int PER = D / 8;          // pieces of four and four values, half a head apart, that rotate with each other
+    const size_t row = (size_t)seq * (n_heads + 2 * n_kv_heads) * D;
+    const int jobs = (n_live + (owner ? 2 : 0)) * PER;
+    for (int job = threadIdx.x; job < jobs; job += blockDim.x) {
+        const int which = job / PER, i = (job % PER) * 4;
+        const int kind = which < n_live ? 0 : which - n_live + 1;
+        const size_t feature = (size_t)(kind == 0 ? head0 + which : n_heads + (kind - 1) * n_kv_heads + kvh) * D + i;
+        float lo[4], hi[4];
+        const size_t angle = (size_t)min(pos, in.max_positions - 1) * (D / 2) + i;
+        const float4 c4 = *reinterpret_cast<const float4*>(in.cos_table + angle), s4 = *reinterpret_cast<const float4*>(in.sin_table + angle);
+        finished8<D>(in, row + feature, feature, lo, hi);
+        if (kind != 2 && pos < in.max_positions) {
+            const float c[4] = {c4.x, c4.y, c4.z, c4.w}, sn[4] = {s4.x, s4.y, s4.z, s4.w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float x0 = lo[k], x1 = hi[k];
+                lo[k] = x0 * c[k] - x1 * sn[k];
+                hi[k] = x0 * sn[k] + x1 * c[k];
+            }
+        }
+        uint32_t l[4], h[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) { l[k] = float_to_bf16_bits(lo[k]); h[k] = float_to_bf16_bits(hi[k]); }
+        if (kind == 2) {
+            bf16_t* dst = in.values + ((size_t)page * n_kv_heads + kvh) * TQK_PAGE * D + value_place(pos % TQK_PAGE);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                dst[(size_t)(i + k) * TQK_PAGE].bits = (uint16_t)l[k];
+                dst[(size_t)(i + D / 2 + k) * TQK_PAGE].bits = (uint16_t)h[k];
+            }
+            continue;
+        }
+        bf16_t* dst = kind == 0 ? q_lds + which * (D + 8) : in.keys + (((size_t)page * n_kv_heads + kvh) * TQK_PAGE + pos % TQK_PAGE) * D;
+        *reinterpret_cast<uint2*>(dst + i) = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
+        *reinterpret_cast<uint2*>(dst + i + D / 2) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70);         // the writes have left for the memory that the block's loads come from
+    __syncthreads();
+}
+
+// SUMS: q, k and v come as `in` and are finished here (keys and values are then written, too, so nothing promises that they are not).
+template <int D, bool NT, int W, bool SUMS>
 __global__ __launch_bounds__(AD_WAVES * TQK_WAVE)
-void attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ keys,
-                             const bf16_t* __restrict__ values, const int32_t* __restrict__ tok_pos,
+void attention_decode_kernel(const DecodeSums in, const bf16_t* __restrict__ q, const bf16_t* keys,
+                             const bf16_t* values, const int32_t* __restrict__ tok_pos,
                              const int32_t* __restrict__ page_table, int table_width, int window, float scale,
                              int n_parts, int n_heads, int n_kv_heads, int q_blocks,
                              float* __restrict__ part_out, float* __restrict__ part_ml,
@@ -88,6 +183,16 @@ void attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restr
 #pragma unroll
     for (int i = 0; i < DB; ++i) o[i] = floatx4_t{0.f, 0.f, 0.f, 0.f};
 
+    __shared__ __attribute__((aligned(16))) bf16_t q_lds[SUMS ? 16 * (D + 8) : 8];
+    if constexpr (SUMS) {
+        const int first_page = lo / TQK_PAGE;
+        if (first_page + part <= last_page) {           // (the same for the block: one without pages has nothing to finish)
+            const int page = __builtin_amdgcn_readfirstlane(page_table[(size_t)seq * table_width + last_page]);
+            const bool owner = (last_page - first_page) % n_parts == part && page >= 0;
+            finish_row<D>(in, seq, pos, page, owner, kvh * n_rep + qb * 16, min(16, n_rep - qb * 16), kvh, n_heads, n_kv_heads, q_lds);
+        }
+    }
+
     if (start_page <= last_page) {
         pack8 zero;
         zero.q = make_uint4(0, 0, 0, 0);
@@ -96,7 +201,7 @@ void attention_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restr
         const bf16_t* qrow = q + ((size_t)seq * n_heads + head) * D + g * 8;
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
-            bq[kb] = head_live ? *reinterpret_cast<const bf16x8_t*>(qrow + kb * 32) : zero.v;
+            bq[kb] = head_live ? *reinterpret_cast<const bf16x8_t*>(SUMS ? q_lds + col * (D + 8) + g * 8 + kb * 32 : qrow + kb * 32) : zero.v;
 
         const int32_t* pages = page_table + (size_t)seq * table_width;
         const size_t page_stride = (size_t)n_kv_heads * TQK_PAGE * D;
@@ -317,11 +422,11 @@ extern "C" int tqk_attention_decode_supported(int head_dim) {
     return head_dim == 64 || head_dim == 128 || head_dim == 256 || head_dim == 32 || head_dim == 96;
 }
 
-extern "C" int tqk_attention_decode(const void* q, const void* keys, const void* values, const int32_t* tok_pos,
-                                    const int32_t* page_table, int table_width, int n_seqs, int n_pages, int window,
-                                    float scale, int n_parts, void* part_out, void* part_ml,
-                                    void* out, int n_heads, int n_kv_heads, int head_dim, void* stream) {
-    TQK_REQUIRE(q && keys && values && tok_pos && page_table && out, "tqk_attention_decode: null pointer");
+static int attention_decode(const DecodeSums& in, const void* q, const void* keys, const void* values, const int32_t* tok_pos,
+                            const int32_t* page_table, int table_width, int n_seqs, int n_pages, int window,
+                            float scale, int n_parts, void* part_out, void* part_ml,
+                            void* out, int n_heads, int n_kv_heads, int head_dim, void* stream) {
+    TQK_REQUIRE((q || in.sums) && keys && values && tok_pos && page_table && out, "tqk_attention_decode: null pointer");
     TQK_REQUIRE(n_parts == 1 || (part_out && part_ml), "tqk_attention_decode: more than one partition needs part_out and part_ml");
     TQK_REQUIRE(n_seqs >= 0 && n_heads > 0 && n_kv_heads > 0, "tqk_attention_decode: bad sizes");
     TQK_REQUIRE(n_heads % n_kv_heads == 0, "tqk_attention_decode: %d heads are not a multiple of %d kv heads", n_heads, n_kv_heads);
@@ -341,13 +446,14 @@ extern "C" int tqk_attention_decode(const void* q, const void* keys, const void*
     // Four waves a block; two where there are 512 blocks or more without partitions: then the memory has more
     // pages asked of it at once than it serves well (128 sequences x 4 kv heads of 2100 positions: 106 against 114 us).
     const bool two = n_parts == 1 && (long long)n_seqs * n_kv_heads * q_blocks >= 512;
-#define LAUNCH_W(DD, NT, W) attention_decode_kernel<DD, NT, W><<<grid, W * TQK_WAVE, 0, s>>>( \
-        (const bf16_t*)q, (const bf16_t*)keys, (const bf16_t*)values, tok_pos, page_table, table_width, window, scale, \
+#define LAUNCH_S(DD, NT, W, SUMS) attention_decode_kernel<DD, NT, W, SUMS><<<grid, W * TQK_WAVE, 0, s>>>( \
+        in, (const bf16_t*)q, (const bf16_t*)keys, (const bf16_t*)values, tok_pos, page_table, table_width, window, scale, \
         n_parts, n_heads, n_kv_heads, q_blocks, (float*)part_out, (float*)part_ml, (bf16_t*)out)
+#define LAUNCH_W(DD, NT, W) { if (in.sums) LAUNCH_S(DD, NT, W, true); else LAUNCH_S(DD, NT, W, false); }
     // A partition per page of the table: a block then has one page to read, and one wave does it (4 sequences of 2100
     // positions: 8.8 against 10.7 us with four waves on four pages each; one sequence 5.8 against 9.0).
     const bool one = n_parts > 1 && n_parts >= table_width;
-#define LAUNCH(DD) { if (one) { if (nt) LAUNCH_W(DD, true, 1); else LAUNCH_W(DD, false, 1); } else if (two) { if (nt) LAUNCH_W(DD, true, 2); else LAUNCH_W(DD, false, 2); } else { if (nt) LAUNCH_W(DD, true, 4); else LAUNCH_W(DD, false, 4); } }
+#define LAUNCH(DD) { if (one) { if (nt) LAUNCH_W(DD, true, 1) else LAUNCH_W(DD, false, 1) } else if (two) { if (nt) LAUNCH_W(DD, true, 2) else LAUNCH_W(DD, false, 2) } else { if (nt) LAUNCH_W(DD, true, 4) else LAUNCH_W(DD, false, 4) } }
     switch (head_dim) {
         case 32: LAUNCH(32); break;
         case 64: LAUNCH(64); break;
@@ -356,10 +462,38 @@ extern "C" int tqk_attention_decode(const void* q, const void* keys, const void*
         case 256: LAUNCH(256); break;
     }
 #undef LAUNCH_W
+#undef LAUNCH_S
 #undef LAUNCH
     if (tqk_check_launch("tqk_attention_decode")) return -1;
     if (n_parts == 1) return 0;
     attention_merge_kernel<<<n_seqs * n_heads, head_dim >= 128 ? 128 : 64, 0, s>>>(
         (const float*)part_out, (const float*)part_ml, n_parts, head_dim, (bf16_t*)out);
     return tqk_check_launch("tqk_attention_decode merge");
+}
+
+extern "C" int tqk_attention_decode(const void* q, const void* keys, const void* values, const int32_t* tok_pos,
+                                    const int32_t* page_table, int table_width, int n_seqs, int n_pages, int window,
+                                    float scale, int n_parts, void* part_out, void* part_ml,
+                                    void* out, int n_heads, int n_kv_heads, int head_dim, void* stream) {
+    const DecodeSums none = {};
+    TQK_REQUIRE(q, "tqk_attention_decode: null pointer");
+    return attention_decode(none, q, keys, values, tok_pos, page_table, table_width, n_seqs, n_pages, window, scale, n_parts, part_out, part_ml, out,
+                            n_heads, n_kv_heads, head_dim, stream);
+}
+
+/* The same with the step's q, k and v product given as its sums over n_sums pieces of K, float32 [n_sums][n_seqs][(heads + 2 kv heads) *
+ * head_dim]: bias (bfloat16 or null), rotation in halves over the whole head and the cache write happen here, as tqk_rope_store_sums
+ * does them (16-byte aligned operands), and keys and values are written at the rows' positions. */
+extern "C" int tqk_attention_decode_sums(const float* sums, int n_sums, const void* bias, const float* cos_table, const float* sin_table, int max_positions,
+                                         void* keys, void* values, const int32_t* tok_pos, const int32_t* page_table, int table_width, int n_seqs,
+                                         int n_pages, int window, float scale, int n_parts, void* part_out, void* part_ml,
+                                         void* out, int n_heads, int n_kv_heads, int head_dim, void* stream) {
+    TQK_REQUIRE(sums && n_sums > 0, "tqk_attention_decode_sums: no sums given");
+    TQK_REQUIRE(cos_table && sin_table && max_positions > 0, "tqk_attention_decode_sums: no angle tables");
+    TQK_REQUIRE(((((uintptr_t)sums) | ((uintptr_t)bias) | ((uintptr_t)cos_table) | ((uintptr_t)sin_table) | ((uintptr_t)keys)) & 15) == 0,
+                "tqk_attention_decode_sums: operands must be 16-byte aligned");
+    const DecodeSums in = {sums, n_sums, (size_t)n_seqs * (n_heads + 2 * n_kv_heads) * head_dim, (const bf16_t*)bias, cos_table, sin_table, max_positions,
+                           (bf16_t*)keys, (bf16_t*)values};
+    return attention_decode(in, nullptr, keys, values, tok_pos, page_table, table_width, n_seqs, n_pages, window, scale, n_parts, part_out, part_ml, out,
+                            n_heads, n_kv_heads, head_dim, stream);
 }

@@ -48,6 +48,8 @@ TQ_QUERY(int, attention_max_head_dim);
 TQ_KERNEL(attention, cptr, cptr, cptr, int, ci32, ci32, ci32, int, int, int, int, float, void*, int, int, int, int, void*);
 TQ_QUERY(int, attention_decode_supported, int);
 TQ_KERNEL(attention_decode, cptr, cptr, cptr, ci32, ci32, int, int, int, int, float, int, void*, void*, void*, int, int, int, void*);
+TQ_KERNEL(attention_decode_sums, cf32, int, cptr, cf32, cf32, int, void*, void*, ci32, ci32, int, int, int, int, float, int, void*, void*, void*, int, int,
+          int, void*);
 TQ_QUERY(int, attention_prefill_supported, int);
 TQ_QUERY(int, attention_prefill_tile, int, int, int, int);
 TQ_KERNEL(attention_prefill, cptr, cptr, cptr, ci32, ci32, int, int, int, ci32, ci32, ci32, int, int, ci32, ci32, int, float, void*, int, int,

@@ -515,7 +515,15 @@ public:
                          table.dev, table.width, entry.keys.data, entry.values.data, n_pages, q.data, (int)n, n_heads_, n_kv_heads_, head_dim_,
                          (int)hidden_, c.stream);
         } else {
-            qkv(c, x.x, entry, table, q);
+            Product sums = qkv(c, x.x, entry, table, q, !last_rows && finishes_sums(c, entry));
+            if (sums.is_sums) {
+                // (the product's sums, the biases, the rotation and the cache write are the attention kernel's)
+                Tensor y = c.alloc(dtype, {n, (int64_t)n_heads_ * value_dim_});
+                decode_kernel(c, q, &sums.sums, entry, c.dev.tok_pos, table.dev, table.width, y);
+                if (!stream) return linear(c, y, w_o_, b_o_ ? &b_o_->t : nullptr, dtype).t;
+                add_product(c, *stream, y, w_o_);
+                return Tensor();
+            }
         }
         const int64_t qd = (int64_t)n_heads_ * value_dim_;
         if (last_rows) {
@@ -668,8 +676,15 @@ private:
         return it->second;
     }
 
-    // product, then bias, position encoding and cache write in their own kernel
-    void qkv(StepContext& c, const Tensor& x, const CacheEntry& entry, const StepContext::Table& table, Tensor& q) {
+    // Whether the decoding kernel finishes a q/k/v product left as sums over pieces of K itself (a launch less: the rotation's kernel took 5 to
+    // 6 us of a layer's 63 at 32 rows of the 1.5B shape): steps of one token a sequence that go through that kernel and write their own cache.
+    bool finishes_sums(const StepContext& c, const CacheEntry& entry) const {
+        return c.all_decode && entry.writes && policy().decode_mfma && K::attention_decode_supported.raw(head_dim_) != 0;
+    }
+
+    // product, then bias, position encoding and cache write in their own kernel; leave: where the product may be left as its sums, they are
+    // returned and that is all
+    Product qkv(StepContext& c, const Tensor& x, const CacheEntry& entry, const StepContext::Table& table, Tensor& q, bool leave) {
         const bool own = position_->has_apply();
         const int64_t n = x.shape[0];
         const int total = (n_heads_ + 2 * n_kv_heads_) * head_dim_;
@@ -681,6 +696,7 @@ private:
             sums_ok = x.dtype == BF16 && K::rope_store_takes_sums.raw(BF16, b_qkv_ ? 1 : 0, b_qkv_ ? b_qkv_->t.dtype : 0, tb.rot_dim, tb.style, head_dim_) != 0;
         }
         Product p = linear(c, x, w_qkv_, nullptr, x.dtype, sums_ok);        // may come as its sums over pieces of K
+        if (p.is_sums && leave) return p;
         const void* bias = nullptr;
         int bias_dt = 0;
         if (own) {
@@ -707,6 +723,7 @@ private:
                           write ? table.dev : nullptr, write ? table.width : 0, write ? c.n_seqs : 0, write ? entry.keys.data : nullptr,
                           write ? entry.values.data : nullptr, write ? n_pages : 0, q.data, (int)n, n_heads_, n_kv_heads_, head_dim_, write ? 1 : 0,
                           c.stream);
+        return Product();
     }
 
     // how many partitions a row's pages are dealt out to in the kernels for steps of one token a sequence
@@ -718,7 +735,8 @@ private:
         return n_parts;
     }
 
-    void decode_kernel(StepContext& c, const Tensor& q, const CacheEntry& entry, const int32_t* tok_pos, const int32_t* table, int width,
+    // (sums: the q/k/v product's, [pieces, rows, features], for the kernel to finish in place of q)
+    void decode_kernel(StepContext& c, const Tensor& q, const PartialSums* sums, const CacheEntry& entry, const int32_t* tok_pos, const int32_t* table, int width,
                        Tensor& out) {
         const int n = (int)q.shape[0];
         const int q_blocks = (n_heads_ / n_kv_heads_ + 15) / 16;
@@ -741,6 +759,14 @@ private:
             part_out = c.alloc(F32, {n, n_heads_, n_parts, head_dim_});
             part_ml = c.alloc(F32, {n, n_heads_, n_parts, 2});
         }
+        if (sums) {
+            const Position::Tables tb = position_->tables();
+            K::attention_decode_sums((const float*)sums->sums.data, (int)sums->sums.shape[0], b_qkv_ ? b_qkv_->t.data : nullptr, (const float*)tb.cos.data,
+                                     (const float*)tb.sin.data, (int)tb.cos.shape[0], entry.keys.data, entry.values.data, tok_pos, table, width, n,
+                                     (int)entry.keys.shape[0], window_, scale_, n_parts, part_out.data, part_ml.data, out.data, n_heads_, n_kv_heads_,
+                                     head_dim_, c.stream);
+            return;
+        }
         K::attention_decode(q.data, entry.keys.data, entry.values.data, tok_pos, table, width, n, (int)entry.keys.shape[0], window_, scale_, n_parts,
                             part_out.data, part_ml.data, out.data, n_heads_, n_kv_heads_, head_dim_, c.stream);
     }
@@ -753,7 +779,7 @@ private:
         const int n = (int)q.shape[0], n_pages = (int)entry.keys.shape[0];
         if (extras_) return attend_masked(c, q, entry, table, c.dev.tok_seq, c.dev.tok_pos, head_scale, out, false);
         if (q.dtype == BF16 && c.all_decode && policy().decode_mfma && K::attention_decode_supported.raw(head_dim_))
-            return decode_kernel(c, q, entry, c.dev.tok_pos, table.dev, table.width, out);
+            return decode_kernel(c, q, nullptr, entry, c.dev.tok_pos, table.dev, table.width, out);
         // (not for steps of one token per sequence: tiles of one query are what the plain kernel does anyway,
         // and such a step may be replayed from a graph, which cannot carry the tiles' upload)
         if (q.dtype == BF16 && !c.all_decode && policy().prefill_mfma && scale_ > 0.f && K::attention_prefill_supported.raw(head_dim_)) {
@@ -779,7 +805,7 @@ private:
             Tensor rows_table = c.alloc(I32, {n, table.width});
             Tensor whole((void*)table.dev, I32, {c.n_seqs, table.width});
             k_gather_rows(c, whole, c.dev.last_seq, n, rows_table);
-            return decode_kernel(c, q, entry, c.dev.last_pos, (const int32_t*)rows_table.data, table.width, out);
+            return decode_kernel(c, q, nullptr, entry, c.dev.last_pos, (const int32_t*)rows_table.data, table.width, out);
         }
         if (q.dtype == BF16 && policy().prefill_mfma && scale_ > 0.f && K::attention_prefill_supported.raw(head_dim_)) {
             const int tile = tile_for(c);

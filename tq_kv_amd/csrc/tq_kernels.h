@@ -168,6 +168,12 @@ int tqk_attention_decode(const void* q, const void* keys, const void* values, co
                          const int32_t* page_table, int table_width, int n_seqs, int n_pages, int window,
                          float scale, int n_parts, void* part_out, void* part_ml,
                          void* out, int n_heads, int n_kv_heads, int head_dim, void* stream);
+/* the same with q, k and v given as their product's sums over n_sums pieces of K: bias, rotation in halves over the whole head and the cache
+ * write happen in the kernel (the work of tqk_rope_store_sums for steps of one token a sequence) */
+int tqk_attention_decode_sums(const float* sums, int n_sums, const void* bias, const float* cos_table, const float* sin_table, int max_positions,
+                              void* keys, void* values, const int32_t* tok_pos, const int32_t* page_table, int table_width, int n_seqs,
+                              int n_pages, int window, float scale, int n_parts, void* part_out, void* part_ml,
+                              void* out, int n_heads, int n_kv_heads, int head_dim, void* stream);
 
 /* Prompts: tiles of up to tile_queries (16, 32, 64 or 128) consecutive queries of one sequence
  * (tile i: sequence tile_seq[i], first packed token tile_tok0[i], tile_count[i] queries, none more

@@ -350,12 +350,17 @@ def attention_decode_supported(head_dim):
     return bool(library().tqk_attention_decode_supported(int(head_dim)))
 
 
-def attention_decode(q, keys, values, tok_pos, page_table, window, scale, out, target_blocks=256, n_parts=None):
+def attention_decode(q, keys, values, tok_pos, page_table, window, scale, out, target_blocks=256, n_parts=None, bias=None, cos=None, sin=None):
     """Attention of one new token per sequence (q [B, heads, d] bfloat16, row b belongs to
     sequence b at position tok_pos[b]) over the paged cache; out [B, heads*d].  n_parts: into how many partitions
-    a sequence's pages are dealt (as many as the table is wide: a block of one wave per page)."""
-    n, n_heads, head_dim = q.shape
+    a sequence's pages are dealt (as many as the table is wide: a block of one wave per page).  q may be the PartialSums of the
+    q, k, v product: bias, rotation (cos, sin) and the cache write then happen in the kernel."""
     n_pages, n_kv_heads = keys.shape[0], keys.shape[1]
+    if isinstance(q, PartialSums):
+        head_dim = keys.shape[3]
+        n, n_heads = q.shape[0], q.shape[1] // head_dim - 2 * n_kv_heads
+    else:
+        n, n_heads, head_dim = q.shape
     n_seqs, width = page_table.shape
     if n_seqs != n:
         raise KernelError("attention_decode: %d query rows for %d sequences (one token each is required)" % (n, n_seqs))
@@ -366,8 +371,17 @@ def attention_decode(q, keys, values, tok_pos, page_table, window, scale, out, t
         n_parts = max(1, min((width + 3) // 4, target_blocks // groups))
     part_out = part_ml = None
     if n_parts > 1:
-        part_out = torch.empty((n, n_heads, n_parts, head_dim), dtype=torch.float32, device=q.device)
-        part_ml = torch.empty((n, n_heads, n_parts, 2), dtype=torch.float32, device=q.device)
+        part_out = torch.empty((n, n_heads, n_parts, head_dim), dtype=torch.float32, device=keys.device)
+        part_ml = torch.empty((n, n_heads, n_parts, 2), dtype=torch.float32, device=keys.device)
+    if isinstance(q, PartialSums):
+        _check(library().tqk_attention_decode_sums(
+            _dev(q.sums, "sums", torch.float32), q.sums.shape[0], _opt(bias, "bias", torch.bfloat16), _dev(cos, "cos", torch.float32, (cos.shape[0], head_dim // 2)),
+            _dev(sin, "sin", torch.float32, tuple(cos.shape)), cos.shape[0], _dev(keys, "keys", torch.bfloat16, (n_pages, n_kv_heads, 64, head_dim)),
+            _dev(values, "values", torch.bfloat16, (n_pages, n_kv_heads, head_dim, 64)), _dev(tok_pos, "tok_pos", torch.int32, (n,)),
+            _dev(page_table, "page_table", torch.int32), width, n, n_pages, int(window or 0), ctypes.c_float(scale), n_parts, _opt(part_out, "part_out"),
+            _opt(part_ml, "part_ml"), _dev(out, "out", torch.bfloat16, (n, n_heads * head_dim)), n_heads, n_kv_heads, head_dim, _stream()),
+            "attention_decode")
+        return out
     _check(library().tqk_attention_decode(
         _dev(q, "q", torch.bfloat16), _dev(keys, "keys", torch.bfloat16, (n_pages, n_kv_heads, 64, head_dim)),
         _dev(values, "values", torch.bfloat16, (n_pages, n_kv_heads, head_dim, 64)),
