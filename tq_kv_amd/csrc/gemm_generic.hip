@@ -15,11 +15,14 @@
 // registers whichever kernel it is.
 //
 // For up to 16 rows of x (decoding in the 32-bit path) the weights are the whole cost: a wave takes 16 output features and one
-// group of k and streams their weights from memory into the operands' registers, 16 loads of a KB under way; groups beyond
-// the first meet in a second kernel.  More rows: a block of four waves takes 64 rows by 64 features through LDS; where that gives
+// group of k and streams their weights through LDS, 12 KB of them under way; groups beyond the first meet in a second
+// kernel.  More rows: a block of four waves takes 64 rows by 64 features through LDS; where that gives
 // few blocks they are also dealt out along the groups.  Measured at the 7B layers' sizes: see the kernels.
 #include "common.h"
 #include "tq_kernels.h"
+
+#include <type_traits>
+#include <utility>
 
 #define GT 64      // tile edge
 #define GK 16      // k per stage
@@ -95,6 +98,10 @@ void gemm_generic_kernel(const TX* __restrict__ x, const TW* __restrict__ w, con
 }
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+template <typename F, int... I> __device__ __forceinline__ void each(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, typename F> __device__ __forceinline__ void each(F&& f) { each(f, std::make_integer_sequence<int, N>{}); }
 
 // 16 k more: lane l holds, of both operands, row l % 16 and the four k at 4 (l / 16); of the sums row (of x) l % 16 and the
 // features 4 (l / 16) .. + 3.
@@ -104,57 +111,78 @@ __device__ __forceinline__ void multiply16(floatx4_t& acc, const floatx4_t& w, c
 }
 
 // Up to 16 rows of x: a wave per (16 output features, one group of k).  With one group the result is finished here.
-// Bound by the weights, whose rows it takes 64 bytes at a time out of 16 of them: gate+up of the 7B shape (543 MB), one row, 124 us
-// (4.4 TB/s; 141 with the loads marked read-once, since the other half of a line is the next load's).  With a feature a lane, each
-// reading its own row, it was 131 us for one row, and every further row cost as much again in multiplications.
+// Bound by the weights.  They come in stages of 64 k, 256 contiguous bytes of each of the 16 rows, by loads that end in LDS, three
+// stages on their way while one is multiplied; a piece of 16 bytes lies at its number exclusive-or its row, so that the operands of 16
+// rows meet all banks.  gate+up of the 7B shape (543 MB), one row: 100 us (5.4 TB/s), eight rows 114; 131 and
+// 141 with the operands loaded as the lanes need them, 64 bytes out of 16 rows a load, eight of those under way.
+#define FEW_STAGES 4
 __global__ __launch_bounds__(TQK_WAVE)
 void gemm_few_rows_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ out,
                           int M, int N, int K) {
-    const int lane = threadIdx.x, r16 = lane % 16, k4 = 4 * (lane / 16);
+    constexpr int NS = FEW_STAGES, U = 4;                               // 16 k a step, four steps a stage
+    __shared__ __attribute__((aligned(1024))) float buf0[1024], buf1[1024], buf2[1024], buf3[1024];
+    const int lane = threadIdx.x, r16 = lane % 16, g = lane / 16;
     const int n0 = blockIdx.x * 16;
-    const int k_begin = blockIdx.y * G_GROUP, k_end = min(K, k_begin + G_GROUP);
-    const float* wrow = w + (size_t)min(n0 + r16, N - 1) * K;
-    const float* xrow = x + (size_t)min(r16, M - 1) * K;          // rows past M repeat the last and are dropped
-    floatx4_t group = {0.f, 0.f, 0.f, 0.f};
-    constexpr int U = G_CHUNK / 16;                                     // a chunk's loads together, the next chunk's under way
-    floatx4_t wv[2][U], xv[2][U];
-    auto load = [&](int c0, floatx4_t (&wq)[U], floatx4_t (&xq)[U]) {
+    const int k_begin = blockIdx.y * G_GROUP, k_end = min(K, k_begin + G_GROUP), n_stage = (k_end - k_begin + 63) / 64;
+    const float* xrow = x + (size_t)min(r16, M - 1) * K;                // rows past M repeat the last and are dropped
+    // (rows past N and everything past the last row lie outside of the buffer: nothing is read there)
+    const __amdgpu_buffer_rsrc_t w_mem = __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * K), 0, min(16, N - n0) * K * 4, 0x00020000);
+    uint32_t w_at[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int row = 4 * j + g;
+        w_at[j] = (uint32_t)row * (uint32_t)(K * 4) + ((r16 ^ row) * 16);
+    }
+    auto buf = [&](auto I) -> float* {
+        constexpr int i = decltype(I)::value % NS;
+        if constexpr (i == 0) return buf0; else if constexpr (i == 1) return buf1; else if constexpr (i == 2) return buf2; else return buf3;
+    };
+    floatx4_t xv[NS][U];
+    auto load = [&](auto I, int stage) {
+        const bool there = stage < n_stage;                             // (past the last stage: outside of the buffer, nothing is read)
+        const int k0 = k_begin + (there ? stage * 64 : 0);
+        const uint32_t nowhere = there ? 0u : 0x80000000u;              // (joined to the offsets, so that no branch lies here)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(w_mem, (lds_ptr_t)(buf(I) + j * 256), 16, (int)(w_at[j] | nowhere), k0 * 4, 0, 0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) xv[decltype(I)::value % NS][u] = *reinterpret_cast<const floatx4_t*>(xrow + min(k0 + 16 * u + 4 * g, K - 4));
+    };
+    floatx4_t group = {0.f, 0.f, 0.f, 0.f}, acc = group;
+    // (one straight line from the first product of a chunk to the sum: where a branch lay between, the compiler let the sum read the
+    // last register of a product that was still under way)
+    auto multiply = [&](auto I, int stage) {
+        const float* src = buf(I);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int k = min(c0 + 16 * u + k4, K - 4);                 // (past the end: loaded from inside the row, not used)
-            wq[u] = *reinterpret_cast<const floatx4_t*>(wrow + k);
-            xq[u] = *reinterpret_cast<const floatx4_t*>(xrow + k);
+            const u32x4_t wq = *reinterpret_cast<const u32x4_t*>(src + r16 * 64 + ((4 * u + g) ^ r16) * 4);
+            const uint32_t in = k_begin + stage * 64 + 16 * u + 4 * g < k_end ? 0xffffffffu : 0u;       // past k_end both operands are nothing
+            multiply16(acc, __builtin_bit_cast(floatx4_t, wq & in), __builtin_bit_cast(floatx4_t, __builtin_bit_cast(u32x4_t, xv[decltype(I)::value % NS][u]) & in));
         }
     };
-    // (one straight line from the first product to the sum: where a branch lay between, the compiler let the sum read the last
-    // register of a product that was still under way)
-    auto add = [&](int c0, floatx4_t (&wq)[U], floatx4_t (&xq)[U]) {
-        if (c0 + G_CHUNK > k_end) {                                     // a last chunk that is not full: zeros add nothing
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (c0 + 16 * u + k4 >= k_end) wq[u] = xq[u] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-        }
-        floatx4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int u = 0; u < U; ++u) multiply16(acc, wq[u], xq[u]);
-        group += acc;
-    };
-    load(k_begin, wv[0], xv[0]);
-    for (int c0 = k_begin; c0 < k_end; c0 += 2 * G_CHUNK) {
-        load(c0 + G_CHUNK, wv[1], xv[1]);
-        __builtin_amdgcn_sched_barrier(0);
-        add(c0, wv[0], xv[0]);
-        if (c0 + G_CHUNK >= k_end) break;
-        load(c0 + 2 * G_CHUNK, wv[0], xv[0]);
-        __builtin_amdgcn_sched_barrier(0);
-        add(c0 + G_CHUNK, wv[1], xv[1]);
+    each<NS - 1>([&](auto S) { load(S, S); });
+    for (int s0 = 0; s0 < n_stage; s0 += NS) {
+        each<NS>([&](auto S) {
+            constexpr int h = decltype(S)::value;
+            load(std::integral_constant<int, h + NS - 1>{}, s0 + h + NS - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt(0x0f70 | ((8 * (NS - 1)) & 15) | (((8 * (NS - 1)) >> 4) << 14));      // this stage's loads: eight of each later one may be under way
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(S, s0 + h);
+            if constexpr (h % 2 == 1) {
+                group += acc;
+                acc = floatx4_t{0.f, 0.f, 0.f, 0.f};
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
     }
+    __builtin_amdgcn_s_waitcnt(0x0f70);                                 // nothing is on its way into LDS any more
     if (r16 >= M) return;
     const bool whole = gridDim.y == 1;
     float* dst = out + ((size_t)blockIdx.y * M + r16) * N;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int n = n0 + k4 + i;
+        const int n = n0 + 4 * g + i;
         if (n < N) dst[n] = whole && bias ? group[i] + bias[n] : group[i];
     }
 }
