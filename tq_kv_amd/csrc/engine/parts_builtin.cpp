@@ -754,6 +754,10 @@ private:
         // few sequences: a partition per page of the table, which the kernel gives a block of one wave each (faster up to
         // four sequences of 2100 positions at the 7B sizes, slower from eight on)
         if (width > 1 && (long long)groups * width <= 640) n_parts = width;
+        // pages so small that a compute unit brings in all that the table can name while a merge would be launched: one block a row
+        // and kv head (heads of 32, 8 pages of 8 KB: 3.4 against 5.1 us for 30 positions, 4.7 against 5.2 for 500; heads of 64, twice
+        // as much: 7.6 against 5.9 for 500)
+        if ((long long)width * TQE_PAGE * head_dim_ * 4 <= 64 * 1024) n_parts = 1;
         Tensor part_out, part_ml;
         if (n_parts > 1) {
             part_out = c.alloc(F32, {n, n_heads_, n_parts, head_dim_});
