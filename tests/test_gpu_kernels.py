@@ -633,6 +633,7 @@ def test_product_of_many_rows(m, n, k):
 
 
 @pytest.mark.parametrize("m,inter,k", [(1025, 18944, 512), (800, 4112, 512), (257, 18944, 256), (300, 4112, 512), (513, 8208, 768), (145, 18944, 512),
+                                       (240, 18912, 256), (193, 18960, 768), (239, 18944, 1280),
                                        (129, 16, 256), (257, 48, 1280)])
 def test_gated_product_of_many_rows(m, inter, k):
     x, w = rand(m, k, seed=62, dtype=torch.bfloat16), rand(2 * inter, k, seed=63, scale=0.05, dtype=torch.bfloat16)

@@ -14,6 +14,11 @@
 //    LDS), four stages in turn, one barrier a stage.  A load takes eight whole 128-byte lines of x; the 16-byte pieces of a row
 //    are exchanged within it (piece c of row r lies at c ^ ((r / 2) % 8)) so that the waves' reads of 16 rows of one k step meet
 //    all banks once.  A wave reads its operands PD groups ahead, across the barrier too.
+//  - WN = 5 with 15 groups of rows (240): gated products of one such row of blocks, where what a compute unit brings in binds and not
+//    the products: every block needs all of x, so few, even blocks count (18944 gated features: 237 blocks of 80; K of 3584, us against the
+//    best tile of four waves: 129 rows 77 against 84, 170: 71 against 86, 232: 74 against 93).  Without a second block on the unit its
+//    rate is lower, so that from two rows of blocks on it loses (17920 x 1536, 440 rows: 38 against 34.5), and so do products
+//    without a gate (4608 x 3584, 1800 rows: 67 against 62).
 //  - WM = 2: a second row of four waves on the next MT groups of rows, 256 rows a block, one block a compute unit; the two
 //    waves of a column meet each other's weights in the first-level cache, and a unit brings in a third less than two blocks
 //    of WM = 1 would (1.36 against 1.31 PFLOP/s at 8000 x 37888 x 3584).
@@ -89,19 +94,20 @@ __device__ __forceinline__ void write_rows(const PromptArgs& p, const floatx4_t 
     }
 }
 
-template <int MT, int NT, int WM, int EPI>
-__global__ __launch_bounds__(256 * WM, WM == 1 ? 2 : 1)
+template <int MT, int NT, int WM, int WN, int EPI>
+__global__ __launch_bounds__(TQK_WAVE * WN * WM, WM == 1 && WN == 4 ? 2 : 1)
 void prompt_product_kernel(const PromptArgs p) {
     constexpr int NS = PROMPT_STAGES, WD = 4;
-    constexpr int DMA = (MT + 1) / 2;               // loads of 1 KB by which a wave helps to bring in a stage
-    constexpr int STAGE = WM * DMA * 4096;          // bytes: [rows][8 pieces of 16 bytes]
-    constexpr int PD = (2 * MT) % 4 == 0 ? 4 : MT;  // operands read ahead; a divisor of a stage's groups
+    constexpr int DMA = (2 * MT + WN - 1) / WN;     // loads of 1 KB by which a wave helps to bring in a stage
+    constexpr int STAGE = WM * WN * DMA * 1024;     // bytes: [rows][8 pieces of 16 bytes]
+    constexpr int PD = (2 * MT) % 4 == 0 ? 4 : (2 * MT) % 6 == 0 ? 6 : 5;          // operands read ahead; a divisor of a stage's groups
+    static_assert((2 * MT) % PD == 0, "");
     constexpr int GROUPS = 2 * MT, SYNC = GROUPS - PD;
     constexpr int TW = EPI == PROMPT_GATED ? NT / 2 : NT;       // a wave's tiles of the output
     static_assert(NT <= MT && (EPI != PROMPT_GATED || NT % 2 == 0), "");
     __shared__ __attribute__((aligned(1024))) char buf0[STAGE], buf1[STAGE], buf2[STAGE], buf3[STAGE];
     const int lane = threadIdx.x % TQK_WAVE, wv = __builtin_amdgcn_readfirstlane(threadIdx.x / TQK_WAVE);
-    const int wave = wv % 4, wm = wv / 4;
+    const int wave = wv % WN, wm = wv / WN;
     const int r16 = lane % 16, K = p.K;
 
     // Blocks are dealt to the eight dies in turn: each die takes a run of tiles, rows fastest inside bands of 1024 rows, so
@@ -118,7 +124,7 @@ void prompt_product_kernel(const PromptArgs p) {
     const int k_begin = blockIdx.y * p.k_per_split, n_stage = min(K - k_begin, p.k_per_split) / 64;
 
     const int n_out = EPI == PROMPT_GATED ? p.N / 2 : p.N, part_tiles = n_out / 16;
-    const int tile0 = (tn * 4 + wave) * TW;
+    const int tile0 = (tn * WN + wave) * TW;
     // where the wave's tiles begin, in bytes (tiles past the end repeat the last one; their results are dropped)
     uint32_t w_at[NT];
 #pragma unroll
@@ -130,10 +136,12 @@ void prompt_product_kernel(const PromptArgs p) {
     uint32_t x_at[DMA];
     const char* x0 = (const char*)(p.x + (size_t)tm * (WM * MT * 16) * K + k_begin);
     {
-        const int piece = (lane % 8) ^ ((4 * (wv % 2) + lane / 16) % 8);
         const int last = p.M - 1 - tm * (WM * MT * 16);
 #pragma unroll
-        for (int i = 0; i < DMA; ++i) x_at[i] = (uint32_t)min((i * 4 * WM + wv) * 8 + lane / 8, last) * (uint32_t)(K * 2) + piece * 16;
+        for (int i = 0; i < DMA; ++i) {
+            const int j = i * WN * WM + wv;
+            x_at[i] = (uint32_t)min(j * 8 + lane / 8, last) * (uint32_t)(K * 2) + ((lane % 8) ^ ((4 * (j % 2) + lane / 16) % 8)) * 16;
+        }
     }
     const __amdgpu_buffer_rsrc_t x_mem = __builtin_amdgcn_make_buffer_rsrc((void*)x0, 0, 0x7fffffff, 0x00020000);
     const __amdgpu_buffer_rsrc_t w_mem = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, 0, 0x7fffffff, 0x00020000);
@@ -143,7 +151,7 @@ void prompt_product_kernel(const PromptArgs p) {
     };
     // (past the last stage the last one is brought in again, into an array that is free, and not read: the count of loads stays)
     auto load_x = [&](auto I, int i, int stage) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(x_mem, (lds_ptr_t)(buf(I) + wv * 1024 + i * (4096 * WM)), 16, (int)x_at[i], min(stage, n_stage - 1) * 128, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(x_mem, (lds_ptr_t)(buf(I) + wv * 1024 + i * (1024 * WN * WM)), 16, (int)x_at[i], min(stage, n_stage - 1) * 128, 0, 0);
     };
     bf16x8_t w[WD][NT];
     auto load_w = [&](int step, int t, bf16x8_t& to) {
@@ -208,7 +216,7 @@ void prompt_product_kernel(const PromptArgs p) {
     // A product's D[feature][row]: a lane holds row r16 and the features 4 (lane / 16) .. + 3 of a tile.
     const int col = 4 * (lane / 16), row0 = (tm * WM + wm) * MT * 16;
     char* turn = (wv % 2 ? buf1 : buf0) + wv / 2 * 16 * (TW * 32 + 16);
-    static_assert(16 * (TW * 32 + 16) * 2 * WM <= STAGE, "");
+    static_assert(16 * (TW * 32 + 16) * ((WN * WM + 1) / 2) <= STAGE, "");
     if constexpr (EPI != PROMPT_GATED) {
         if (p.sums) {
             float* y = p.sums + (size_t)blockIdx.y * p.M * p.N;
@@ -259,9 +267,10 @@ __global__ void prompt_finish_kernel(const float* __restrict__ partial, TY* __re
 // at 232, 300, 1024, 2048 and 8000 rows of the four 7B products the rule takes the fastest or one within 4 % of it, but for
 // the gated product of 300 to 600 rows (within 10 %).
 struct PromptPlan { int config, splits, k_per_split; };
-struct PromptConfig { int mt, nt, wm; double rate; };
+struct PromptConfig { int mt, nt, wm, wn; double rate; };
 static const PromptConfig CONFIGS[] = {
-    {8, 4, 2, 1.00}, {8, 4, 1, 0.96}, {8, 3, 2, 0.95}, {8, 3, 1, 0.90}, {6, 4, 1, 0.84}, {8, 2, 1, 0.78}, {5, 4, 1, 0.72}, {4, 4, 1, 0.66}, {5, 2, 1, 0.58},
+    {8, 4, 2, 4, 1.00}, {8, 4, 1, 4, 0.96}, {8, 3, 2, 4, 0.95}, {8, 3, 1, 4, 0.90}, {6, 4, 1, 4, 0.84},
+    {8, 2, 1, 4, 0.78}, {5, 4, 1, 4, 0.72}, {4, 4, 1, 4, 0.66}, {5, 2, 1, 4, 0.58}, {15, 2, 1, 5, 0.79},
 };
 #define PROMPT_CONFIGS ((int)(sizeof(CONFIGS) / sizeof(CONFIGS[0])))
 #define PROMPT_UNITS 256
@@ -274,7 +283,8 @@ static PromptPlan prompt_plan(int M, int N, int K, bool gated) {
     for (int i = 0; i < PROMPT_CONFIGS; ++i) {
         const PromptConfig& c = CONFIGS[i];
         if (gated && c.nt % 2) continue;
-        const long long rows = 16LL * c.mt * c.wm, width = 64LL * (gated ? c.nt / 2 : c.nt), n_out = gated ? N / 2 : N;
+        if (c.wn == 5 && (!gated || M > 16 * c.mt)) continue;
+        const long long rows = 16LL * c.mt * c.wm, width = 16LL * c.wn * (gated ? c.nt / 2 : c.nt), n_out = gated ? N / 2 : N;
         const long long tiles = ((M + rows - 1) / rows) * ((n_out + width - 1) / width);
         if (tiles > 0x7fffffffLL) continue;
         for (int splits = 1; splits <= (gated ? 1 : PROMPT_MAX_SPLITS) && splits <= turns; ++splits) {
@@ -282,7 +292,7 @@ static PromptPlan prompt_plan(int M, int N, int K, bool gated) {
             if (per * (splits - 1) >= turns) continue;                                                // an empty piece
             const double rounds = (double)((tiles * splits + PROMPT_UNITS - 1) / PROMPT_UNITS);
             // (us: 256 units at the best tile's rate are 1.4 PFLOP/s)
-            double us = rounds * (double)(c.mt * c.nt * c.wm) / c.rate * (double)(per * PROMPT_K + (gated && c.wm == 2 ? 600 : 300)) * 3.7e-4;
+            double us = rounds * (c.mt * c.nt * c.wm * c.wn / 4.0) / c.rate * (double)(per * PROMPT_K + (gated && c.wm == 2 ? 600 : 300)) * 3.7e-4;
             if (splits > 1) us += (double)splits * M * N * 8.0 / 4.5e6;
             if (us < best_us) { best_us = us; best = {i, splits, (int)(per * PROMPT_K)}; }
         }
@@ -301,15 +311,15 @@ extern "C" int tqk_prompt_takes(int M, int N, int K, int gated) {
 /* Into how many pieces the product's K is cut (1: none, no scratch is needed). */
 extern "C" int tqk_prompt_splits(int M, int N, int K) { return tqk_prompt_takes(M, N, K, 0) ? prompt_plan(M, N, K, false).splits : 1; }
 
-template <int MT, int NT, int WM, int EPI>
+template <int MT, int NT, int WM, int EPI, int WN = 4>
 static void launch(const PromptArgs& a, int splits, hipStream_t s) {
-    prompt_product_kernel<MT, NT, WM, EPI><<<dim3(a.tiles_m * a.tiles_n, splits), 256 * WM, 0, s>>>(a);
+    prompt_product_kernel<MT, NT, WM, WN, EPI><<<dim3(a.tiles_m * a.tiles_n, splits), TQK_WAVE * WN * WM, 0, s>>>(a);
 }
 
 template <int EPI>
 static int launch_plan(PromptArgs a, const PromptPlan& plan, hipStream_t s) {
     const PromptConfig& c = CONFIGS[plan.config];
-    const int rows = 16 * c.mt * c.wm, width = 64 * (EPI == PROMPT_GATED ? c.nt / 2 : c.nt), n_out = EPI == PROMPT_GATED ? a.N / 2 : a.N;
+    const int rows = 16 * c.mt * c.wm, width = 16 * c.wn * (EPI == PROMPT_GATED ? c.nt / 2 : c.nt), n_out = EPI == PROMPT_GATED ? a.N / 2 : a.N;
     a.tiles_m = (a.M + rows - 1) / rows;
     a.tiles_n = (n_out + width - 1) / width;
     a.k_per_split = plan.k_per_split;
@@ -322,7 +332,8 @@ static int launch_plan(PromptArgs a, const PromptPlan& plan, hipStream_t s) {
         case 5: launch<8, 2, 1, EPI>(a, plan.splits, s); break;
         case 6: launch<5, 4, 1, EPI>(a, plan.splits, s); break;
         case 7: launch<4, 4, 1, EPI>(a, plan.splits, s); break;
-        default: launch<5, 2, 1, EPI>(a, plan.splits, s); break;
+        case 8: launch<5, 2, 1, EPI>(a, plan.splits, s); break;
+        default: if constexpr (EPI == PROMPT_GATED) launch<15, 2, 1, EPI, 5>(a, plan.splits, s); break;
     }
     return tqk_check_launch("tqk_prompt product");
 }
