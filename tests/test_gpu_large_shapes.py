@@ -123,6 +123,30 @@ def test_bfloat16_tracks_float32_in_steps_of_17_and_more_rows_at_large_sizes(sha
     torch.testing.assert_close(outs["bfloat16"], outs["float32"], atol=0.03 * max(1.0, scale), rtol=0.03)
 
 
+@pytest.mark.parametrize("n_seqs,longest", [(18, 40), (40, 40), (40, 2500), (100, 40)])
+def test_decoding_steps_on_both_sides_of_every_line_of_the_folded_sums(n_seqs, longest):
+    """The q/k/v product's sums are finished by the attention kernel at 40 rows of short sequences, and by a kernel of their own where the
+    attention's blocks are of one wave (18 rows), where the table names many pages (one sequence of 2500) and where there are more blocks than
+    compute units (100 rows): two decoding steps each, every row against the float32 path."""
+    raw = two_layer("qwen2.5:7b")
+    tensors = sharpened(tensors_for(raw, 8))
+    first = [helpers.random_tokens(longest if i == 5 else 1 + i % 3, raw["vocab_size"], 300 + i) for i in range(n_seqs)]
+    nxt = [[(17 * i + 3 + 5 * j) % raw["vocab_size"] for i in range(n_seqs)] for j in range(2)]
+    outs = {}
+    for dtype in ("float32", "bfloat16"):
+        eng = Engine(build(raw, dtype, tensors), max_tokens=64 * n_seqs + 2624)
+        slots = [eng.open() for _ in first]
+        eng.step([(s, p, []) for s, p in zip(slots, first)])
+        got = [eng.step([(s, [t], [0]) for s, t in zip(slots, step)]) for step in nxt]
+        outs[dtype] = torch.cat(got).cpu()
+        for s in slots:
+            eng.close(s)
+        del eng
+        torch.cuda.empty_cache()
+    rms, worst = row_errors(outs["bfloat16"], outs["float32"])
+    assert rms.max().item() < 0.07 and worst.max().item() < 0.35, (rms.max().item(), worst.max().item())
+
+
 @pytest.mark.parametrize("shape", ["qwen2.5:7b", "qwen2.5:1.5b", "qwen2.5:32b"])
 def test_float32_path_equals_plain_at_large_sizes(shape):
     raw = two_layer(shape)

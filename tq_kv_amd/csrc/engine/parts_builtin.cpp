@@ -515,7 +515,7 @@ public:
                          table.dev, table.width, entry.keys.data, entry.values.data, n_pages, q.data, (int)n, n_heads_, n_kv_heads_, head_dim_,
                          (int)hidden_, c.stream);
         } else {
-            Product sums = qkv(c, x.x, entry, table, q, !last_rows && finishes_sums(c, entry));
+            Product sums = qkv(c, x.x, entry, table, q, !last_rows && finishes_sums(c, entry, table.width));
             if (sums.is_sums) {
                 // (the product's sums, the biases, the rotation and the cache write are the attention kernel's)
                 Tensor y = c.alloc(dtype, {n, (int64_t)n_heads_ * value_dim_});
@@ -676,10 +676,22 @@ private:
         return it->second;
     }
 
-    // Whether the decoding kernel finishes a q/k/v product left as sums over pieces of K itself (a launch less: the rotation's kernel took 5 to
-    // 6 us of a layer's 63 at 32 rows of the 1.5B shape): steps of one token a sequence that go through that kernel and write their own cache.
-    bool finishes_sums(const StepContext& c, const CacheEntry& entry) const {
-        return c.all_decode && entry.writes && policy().decode_mfma && K::attention_decode_supported.raw(head_dim_) != 0;
+    // Whether the decoding kernel finishes a q/k/v product left as sums over pieces of K itself (a launch less): steps of one token a sequence
+    // that go through that kernel and write their own cache.  A block then waits for its row's sums before it asks for a page, so not
+    // where that costs more than the launch (ms a step, launch -> folded, heads of 128; every rule's both sides):
+    //  - blocks of one wave, two or three rounds of loads on 64 lanes: 7B sizes, 17 and 20 rows of 200 positions 3.368 -> 3.393 and
+    //    3.400 -> 3.435; 24 rows, blocks of four waves, 3.495 -> 3.425;
+    //  - more blocks than units: 7B, 96 rows after 256, up to 1024 and 2048 positions 4.968 -> 4.974, 5.432 -> 5.460 and 6.621 -> 6.795, 128 rows
+    //    5.412 -> 5.456, 5.972 -> 5.989 and 7.344 -> 7.593;
+    //  - more than 24 pages a unit: 7B, 48 rows of 2048 positions 4.490 -> 4.520, 64 rows 4.990 -> 5.032; 1.5B, 96 rows 3.376 -> 3.438; 32B with 8
+    //    layers, 32 rows 2.136 -> 2.156.  Up to that: 7B, 32 rows of 2048 positions 4.026 -> 3.979, 64 rows of up to 1024 4.309 -> 4.287; 1.5B,
+    //    32 and 128 of those 1.963 -> 1.901 and 3.192 -> 3.194; 32B, 32 of those 2.001 -> 1.992.
+    bool finishes_sums(const StepContext& c, const CacheEntry& entry, int width) const {
+        if (!(c.all_decode && entry.writes && policy().decode_mfma && K::attention_decode_supported.raw(head_dim_) != 0)) return false;
+        const int units = 256, n_parts = decode_parts(c.n_tokens, width);
+        const long long groups = (long long)c.n_tokens * n_kv_heads_ * ((n_heads_ / n_kv_heads_ + 15) / 16);
+        const bool one_wave = n_parts > 1 && n_parts >= width;
+        return !one_wave && groups <= units && groups * width <= 24LL * units;
     }
 
     // product, then bias, position encoding and cache write in their own kernel; leave: where the product may be left as its sums, they are
@@ -735,10 +747,8 @@ private:
         return n_parts;
     }
 
-    // (sums: the q/k/v product's, [pieces, rows, features], for the kernel to finish in place of q)
-    void decode_kernel(StepContext& c, const Tensor& q, const PartialSums* sums, const CacheEntry& entry, const int32_t* tok_pos, const int32_t* table, int width,
-                       Tensor& out) {
-        const int n = (int)q.shape[0];
+    // into how many partitions the decoding kernel deals a row's pages
+    int decode_parts(int n, int width) const {
         const int q_blocks = (n_heads_ / n_kv_heads_ + 15) / 16;
         const int groups = std::max(1, n * n_kv_heads_ * q_blocks);
         const int target_blocks = 256;
@@ -758,6 +768,14 @@ private:
         // and kv head (heads of 32, 8 pages of 8 KB: 3.4 against 5.1 us for 30 positions, 4.7 against 5.2 for 500; heads of 64, twice
         // as much: 7.6 against 5.9 for 500)
         if ((long long)width * TQE_PAGE * head_dim_ * 4 <= 64 * 1024) n_parts = 1;
+        return n_parts;
+    }
+
+    // (sums: the q/k/v product's, [pieces, rows, features], for the kernel to finish in place of q)
+    void decode_kernel(StepContext& c, const Tensor& q, const PartialSums* sums, const CacheEntry& entry, const int32_t* tok_pos, const int32_t* table, int width,
+                       Tensor& out) {
+        const int n = (int)q.shape[0];
+        const int n_parts = decode_parts(n, width);
         Tensor part_out, part_ml;
         if (n_parts > 1) {
             part_out = c.alloc(F32, {n, n_heads_, n_parts, head_dim_});
