@@ -7,6 +7,8 @@ import torch
 
 import gpu_common as G
 import plain_qwen2 as plain
+from tq_kv_amd import Model
+from tq_kv_amd.config import catalog
 
 pytestmark = pytest.mark.gpu
 
@@ -495,3 +497,29 @@ def test_decode_steps_of_a_hundred_and_more_sequences(name, sharp, dtype, n_seqs
         eng.close(slots[i])
     eng.cache.check()
     assert eng.cache.slots.n_held == 0
+
+
+# ---- tuning the library -----------------------------------------------------------------------------
+@pytest.mark.parametrize("inter,packed,want", [(512, True, 0), (264, True, 2), (512, False, 4)])
+def test_tuning_takes_every_product_that_goes_to_the_library(inter, packed, want):
+    """Products that the kernel for prompts takes are left out; not so a gate and up whose halves are no whole tiles (inter of 264, whose
+    down product has K of 264, too), nor weights that were loaded without a packed copy, whatever the switch says by then."""
+    from tq_kv_amd import POLICY, tracing
+    raw = dict(catalog.find("qwen2.5:1.5b"), num_hidden_layers=2, vocab_size=512, hidden_size=256, intermediate_size=inter, num_attention_heads=4,
+               num_key_value_heads=2, head_dim=64)
+    old = POLICY["packed"]
+    POLICY["packed"] = packed
+    try:
+        model = Model.random(raw, seed=0, dtype="bfloat16", device="cuda:0")
+    finally:
+        POLICY["packed"] = old
+    events, was_on = [], tracing.enabled()
+    tracing.set_sink(lambda name: events.append(name.decode()), lambda: None)
+    try:
+        assert tracing.enable()
+        model.tune_library(300)
+    finally:
+        tracing.enable(False)
+        tracing.set_sink(None, None)
+        tracing.enable(was_on)
+    assert events == ["tune-library"] * want

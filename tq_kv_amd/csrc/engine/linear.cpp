@@ -101,6 +101,13 @@ bool leaves_sums(int64_t x_rows, const Weight& w) {
     return prompt_rows(x_rows, w) && K::prompt_splits.raw((int)x_rows, (int)w.n, (int)w.k) > 1;
 }
 
+bool prompt_product(int64_t x_rows, const ProductShape& shape) {
+    const Policy& p = policy();
+    if (shape.weight->defined()) return prompt_rows(x_rows, *shape.weight, shape.gated);
+    if (!p.prompt || !p.packed || !p.skinny || x_rows <= mid_max_rows() || x_rows > INT32_MAX || shape.n > INT32_MAX || shape.k > INT32_MAX) return false;
+    return K::prompt_takes.raw((int)x_rows, (int)shape.n, (int)shape.k, shape.gated ? 1 : 0) != 0;
+}
+
 void classify_step(StepContext& c, int64_t hidden) {
     const Policy& p = policy();
     c.fuse_small = p.fused && c.act_dtype == BF16 && c.all_decode && c.n_tokens <= skinny_max_rows() && hidden % 32 == 0;

@@ -56,6 +56,9 @@ bool fusable(int64_t x_rows, const Weight& w, bool adds = false);
 // Whether a product of x_rows rows goes through a kernel that can leave its sums over pieces of K to the next norm: the one for
 // mid-sized steps, or the one for prompts where it cuts K.
 bool leaves_sums(int64_t x_rows, const Weight& w);
+// Whether the kernel for prompts takes a part's product of x_rows rows: the library is then not asked.  Before the weight is loaded: whether it
+// will, as the policy stands.
+bool prompt_product(int64_t x_rows, const ProductShape& shape);
 // What kind of step this is for the parts' folding: small (norms and residual sums folded into
 // the products), mid (sums over pieces of K may be left to the next kernel: any step of more rows), or neither.
 void classify_step(StepContext& c, int64_t hidden);

@@ -1,6 +1,7 @@
 #include "model.h"
 
 #include <algorithm>
+#include <set>
 
 #include "kernels.h"
 #include "trace.h"
@@ -223,13 +224,13 @@ void Model::tune_library(int64_t rows, hipStream_t stream) {
     if (dtype != BF16 || !on_gpu || !policy().library) return;
     const int64_t own_rows = policy().mid && policy().packed ? mid_max_rows() : skinny_max_rows();
     if (rows <= own_rows) return;
-    std::vector<std::pair<int64_t, int64_t>> shapes;
-    for (const auto& b : blocks_) b->product_shapes(shapes);
-    std::sort(shapes.begin(), shapes.end());
-    shapes.erase(std::unique(shapes.begin(), shapes.end()), shapes.end());
+    std::vector<ProductShape> products;
+    for (const auto& b : blocks_) b->product_shapes(products);
+    std::set<std::pair<int64_t, int64_t>> shapes;
+    for (const ProductShape& p : products)
+        if (!prompt_product(rows, p)) shapes.insert({p.n, p.k});
     for (const auto& nk : shapes) {
-        // (the library is not asked for what the own kernel for prompts takes)
-        if (policy().prompt && policy().packed && K::prompt_takes.raw((int)std::min<int64_t>(rows, INT32_MAX), (int)nk.first, (int)nk.second, 0)) continue;
+        Span span("tune-library");
         library_tune(rows, nk.first, nk.second, BF16, stream);
     }
 }

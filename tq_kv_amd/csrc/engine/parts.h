@@ -119,11 +119,20 @@ struct Stream {
 // ---- building --------------------------------------------------------------------------------
 class Part;
 class Position;
+struct Weight;
 
 struct BuildEnv {
     int act_dtype = BF16;
     bool null_device = false;
     std::map<std::string, std::shared_ptr<Part>> shared;       // parts without weights (position tables) shared between layers
+};
+
+// A matrix product of a part: the sizes n, k of its weight, the weight (not defined before it is loaded), and whether it is a gate's
+// and up's product that the gate is applied to.
+struct ProductShape {
+    int64_t n, k;
+    const Weight* weight;
+    bool gated = false;
 };
 
 class Part {
@@ -141,8 +150,8 @@ public:
     // ("qkv.weight"): for inspection
     virtual OwnedPtr held(const std::string& name) const { (void)name; return nullptr; }
     virtual Json describe() const;
-    // the matrix products the part runs through linear(): (n, k) of each weight (what the library can be tuned for)
-    virtual void product_shapes(std::vector<std::pair<int64_t, int64_t>>& out) const { (void)out; }
+    // the matrix products the part runs through linear() and its like (what the library can be tuned for)
+    virtual void product_shapes(std::vector<ProductShape>& out) const { (void)out; }
 };
 
 class Norm : public Part {

@@ -449,11 +449,11 @@ public:
         return nullptr;
     }
     const char* trace_name() const override { return "attn"; }             // the reference's span, src/models/turbo_generic.rs:1920
-    void product_shapes(std::vector<std::pair<int64_t, int64_t>>& out) const override {
+    void product_shapes(std::vector<ProductShape>& out) const override {
         int64_t n = (int64_t)n_heads_ * head_dim_ + (gated_ ? n_heads_ : 0);
         if (own_kv_) n += (int64_t)n_kv_heads_ * head_dim_ + (values_are_keys_ ? 0 : (int64_t)n_kv_heads_ * value_dim_);
-        out.push_back({projected_ ? (n + 15) / 16 * 16 : n, hidden_});
-        out.push_back({hidden_, (int64_t)n_heads_ * value_dim_});
+        out.push_back({projected_ ? (n + 15) / 16 * 16 : n, hidden_, &w_qkv_});
+        out.push_back({hidden_, (int64_t)n_heads_ * value_dim_, &w_o_});
     }
 
     CacheNeed cache_need() const override {
@@ -899,9 +899,9 @@ public:
         return nullptr;
     }
     const char* trace_name() const override { return "attn-mlp"; }         // the reference's span, src/models/turbo_generic.rs:1922
-    void product_shapes(std::vector<std::pair<int64_t, int64_t>>& out) const override {
-        out.push_back({2 * inter_, hidden_});
-        out.push_back({hidden_, inter_});
+    void product_shapes(std::vector<ProductShape>& out) const override {
+        out.push_back({2 * inter_, hidden_, &w_gate_up_, true});
+        out.push_back({hidden_, inter_, &w_down_});
     }
 
     bool folds_norm(const StepContext& c) const override { return fusable(c.n_tokens, w_gate_up_); }
@@ -1003,7 +1003,7 @@ public:
         j.set("parts", parts);
         return j;
     }
-    void product_shapes(std::vector<std::pair<int64_t, int64_t>>& out) const override {
+    void product_shapes(std::vector<ProductShape>& out) const override {
         for (const Role& r : roles_) r.part->product_shapes(out);
     }
     CacheNeed cache_need() const override { return mixer_->cache_need(); }

@@ -154,10 +154,10 @@ public:
         return nullptr;
     }
     const char* trace_name() const override { return "attn"; }
-    void product_shapes(std::vector<std::pair<int64_t, int64_t>>& out) const override {
-        out.push_back({in_cols_ ? in_cols_ : (q_rank_ ? q_rank_ : q_cols()) + kv_rank_ + dr_ + gate_cols(), hidden_});
-        if (q_rank_) out.push_back({q_cols(), q_rank_});
-        out.push_back({hidden_, (int64_t)n_heads_ * dv_});
+    void product_shapes(std::vector<ProductShape>& out) const override {
+        out.push_back({in_cols_ ? in_cols_ : (q_rank_ ? q_rank_ : q_cols()) + kv_rank_ + dr_ + gate_cols(), hidden_, &w_in_});
+        if (q_rank_) out.push_back({q_cols(), q_rank_, &w_uq_});
+        out.push_back({hidden_, (int64_t)n_heads_ * dv_, &w_o_});
     }
 
     CacheNeed cache_need() const override {

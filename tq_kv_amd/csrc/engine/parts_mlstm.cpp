@@ -89,9 +89,9 @@ public:
         return it == stored_.end() ? nullptr : it->second;
     }
     const char* trace_name() const override { return "mlstm"; }
-    void product_shapes(std::vector<std::pair<int64_t, int64_t>>& out) const override {
-        out.push_back({(2LL * heads_ * d_ + 2LL * heads_ * dv_ + 2LL * heads_ + 15) / 16 * 16, hidden_});
-        out.push_back({hidden_, (int64_t)heads_ * dv_});
+    void product_shapes(std::vector<ProductShape>& out) const override {
+        out.push_back({(2LL * heads_ * d_ + 2LL * heads_ * dv_ + 2LL * heads_ + 15) / 16 * 16, hidden_, &w_in_});
+        out.push_back({hidden_, (int64_t)heads_ * dv_, &w_o_});
     }
     CacheNeed cache_need() const override {
         CacheNeed n;

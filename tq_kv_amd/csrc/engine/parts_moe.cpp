@@ -157,7 +157,7 @@ public:
         return nullptr;
     }
     const char* trace_name() const override { return "attn-mlp"; }
-    void product_shapes(std::vector<std::pair<int64_t, int64_t>>& out) const override {
+    void product_shapes(std::vector<ProductShape>& out) const override {
         if (shared_) shared_->product_shapes(out);
     }
 

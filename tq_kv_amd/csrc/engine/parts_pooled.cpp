@@ -119,9 +119,9 @@ public:
         return it == stored_.end() ? nullptr : it->second;
     }
     const char* trace_name() const override { return "attn"; }
-    void product_shapes(std::vector<std::pair<int64_t, int64_t>>& out) const override {
-        out.push_back({(int64_t)(n_heads_ + n_kv_heads_) * head_dim_ + (int64_t)n_kv_heads_ * value_dim_, hidden_});
-        out.push_back({hidden_, (int64_t)n_heads_ * value_dim_});
+    void product_shapes(std::vector<ProductShape>& out) const override {
+        out.push_back({(int64_t)(n_heads_ + n_kv_heads_) * head_dim_ + (int64_t)n_kv_heads_ * value_dim_, hidden_, &w_qkv_});
+        out.push_back({hidden_, (int64_t)n_heads_ * value_dim_, &w_o_});
     }
     CacheNeed cache_need() const override {
         const int rows = TQE_PAGE + K::pooled_rows.raw(pool_);
@@ -245,7 +245,7 @@ public:
         return j;
     }
     const char* trace_name() const override { return "attn"; }
-    void product_shapes(std::vector<std::pair<int64_t, int64_t>>& out) const override {
+    void product_shapes(std::vector<ProductShape>& out) const override {
         for (int i = 0; i < 2; ++i) part_[i]->product_shapes(out);
     }
     // the pages of the one that keeps pages; the two states one behind the other

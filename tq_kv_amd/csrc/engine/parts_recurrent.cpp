@@ -135,9 +135,9 @@ public:
         return it == stored_.end() ? nullptr : it->second;
     }
     const char* trace_name() const override { return "rglru"; }
-    void product_shapes(std::vector<std::pair<int64_t, int64_t>>& out) const override {
-        out.push_back({2 * width_, hidden_});
-        out.push_back({hidden_, width_});
+    void product_shapes(std::vector<ProductShape>& out) const override {
+        out.push_back({2 * width_, hidden_, &w_yx_});
+        out.push_back({hidden_, width_, &w_o_});
     }
     CacheNeed cache_need() const override {
         CacheNeed n;
@@ -259,9 +259,9 @@ public:
         return it == stored_.end() ? nullptr : it->second;
     }
     const char* trace_name() const override { return "mamba2"; }
-    void product_shapes(std::vector<std::pair<int64_t, int64_t>>& out) const override {
-        out.push_back({(total_ + 15) / 16 * 16, hidden_});
-        out.push_back({hidden_, inner_});
+    void product_shapes(std::vector<ProductShape>& out) const override {
+        out.push_back({(total_ + 15) / 16 * 16, hidden_, &w_in_});
+        out.push_back({hidden_, inner_, &w_o_});
     }
     CacheNeed cache_need() const override {
         CacheNeed n;

@@ -102,9 +102,9 @@ public:
         return nullptr;
     }
     const char* trace_name() const override { return "attn-mlp"; }
-    void product_shapes(std::vector<std::pair<int64_t, int64_t>>& out) const override {
-        out.push_back({inter_, hidden_});
-        out.push_back({hidden_, inter_});
+    void product_shapes(std::vector<ProductShape>& out) const override {
+        out.push_back({inter_, hidden_, &w_up_});
+        out.push_back({hidden_, inter_, &w_down_});
     }
     bool adds_to_stream(const StepContext& c) const override { return fusable(c.n_tokens, w_down_, true) || leaves_sums(c.n_tokens, w_down_); }
     Tensor forward(StepContext& c, const Activation& x, Stream* stream) override {
@@ -177,7 +177,7 @@ public:
         j.set("parts", parts);
         return j;
     }
-    void product_shapes(std::vector<std::pair<int64_t, int64_t>>& out) const override {
+    void product_shapes(std::vector<ProductShape>& out) const override {
         for (const Role& r : roles_) r.part->product_shapes(out);
     }
     CacheNeed cache_need() const override { return mixer_->cache_need(); }

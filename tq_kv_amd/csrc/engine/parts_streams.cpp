@@ -209,7 +209,7 @@ public:
         j.set("parts", parts);
         return j;
     }
-    void product_shapes(std::vector<std::pair<int64_t, int64_t>>& out) const override {
+    void product_shapes(std::vector<ProductShape>& out) const override {
         for (const Role& r : roles_) r.part->product_shapes(out);
     }
     // the mixer's need, and behind its state the row of the kept token

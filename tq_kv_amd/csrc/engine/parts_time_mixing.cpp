@@ -129,9 +129,9 @@ public:
         return it == stored_.end() ? nullptr : it->second;
     }
     const char* trace_name() const override { return "linear-attn"; }
-    void product_shapes(std::vector<std::pair<int64_t, int64_t>>& out) const override {
-        out.push_back({(int64_t)heads_ * d_, hidden_});
-        out.push_back({hidden_, (int64_t)heads_ * d_});
+    void product_shapes(std::vector<ProductShape>& out) const override {
+        out.push_back({(int64_t)heads_ * d_, hidden_, &w_in_[0]});
+        out.push_back({hidden_, (int64_t)heads_ * d_, &w_o_});
     }
     CacheNeed cache_need() const override {
         CacheNeed n;
