@@ -2,16 +2,20 @@
 whole requests, the last 32 tokens one by one, batches of unequal lengths whose
 shorter requests end earlier (batch after batch, slots used again), long decoding,
 the first tokens of a sequence, generation through the entry point."""
+import ctypes
+
+import numpy as np
 import pytest
 import torch
 
 import gpu_common as G
 import plain_qwen2 as plain
-from tq_kv_amd import Model
+from tq_kv_amd import Engine, Model, native
 from tq_kv_amd.config import catalog
 
 pytestmark = pytest.mark.gpu
 
+DEV = "cuda"
 DTYPES = ["float32", "bfloat16"]
 CASES = [("A", False), ("A", True), ("B", False), ("B", True), ("C", False), ("C", True)]
 LENS = {"A": [5, 11, 17, 64, 65, 100], "B": [1, 7, 20, 33, 64, 90], "C": [70, 129, 333, 600]}
@@ -523,3 +527,27 @@ def test_tuning_takes_every_product_that_goes_to_the_library(inter, packed, want
         tracing.set_sink(None, None)
         tracing.enable(was_on)
     assert events == ["tune-library"] * want
+
+
+# ---- a caller's own memory --------------------------------------------------------------------------
+def test_many_logits_into_memory_that_begins_at_any_float():
+    """200 wanted rows go to the kernel for prompts where the caller's memory begins at a multiple of 16 bytes, else to the library: the same
+    logits either way, but for the order of float32 sums of 256 products (each of them below 2^-24 of the sum of the terms' sizes)."""
+    raw = dict(catalog.find("qwen2.5:1.5b"), num_hidden_layers=1, vocab_size=512, hidden_size=256, intermediate_size=512, num_attention_heads=4,
+               num_key_value_heads=2, head_dim=64)
+    eng = Engine(Model.random(raw, seed=0, dtype="bfloat16", device="cuda:0"), max_tokens=256)
+    tokens = np.asarray([(7 * i) % 512 for i in range(200)], dtype=np.int32)
+    want = np.arange(200, dtype=np.int32)
+    got = []
+    for offset in (0, 1):
+        buf = torch.full((200 * 512 + 8,), float("nan"), device=DEV)
+        slot = eng.open()
+        one = lambda v: np.asarray([v], dtype=np.int32)
+        slots, n_new, n_want, kept = one(slot), one(200), one(200), ctypes.c_void_p(0)
+        native.check(eng._lib.tqe_step(eng.handle, 1, native._ptr(slots), native._ptr(n_new), native._ptr(tokens), native._ptr(n_want), native._ptr(want),
+                                       None, ctypes.c_void_p(buf.data_ptr() + 4 * offset), 0, ctypes.byref(kept), eng._stream()))
+        eng.close(slot)
+        assert torch.isnan(buf[:offset]).all() and torch.isnan(buf[offset + 200 * 512:]).all()
+        got.append(buf[offset:offset + 200 * 512].reshape(200, 512))
+    # hidden states after the last norm are below 16, the head's weights N(0, 0.02): the terms' sizes sum to less than 256 x 16 x 0.1
+    assert (got[0] - got[1]).abs().max().item() <= 2.0 ** -24 * 256 * 16 * 0.1 * 16

@@ -96,6 +96,10 @@ static bool prompt_rows(int64_t x_rows, const Weight& w, bool gated = false) {
     return K::prompt_takes.raw((int)x_rows, (int)w.n, (int)w.k, gated ? 1 : 0) != 0;
 }
 
+// Whether a tensor begins at a multiple of 16 bytes, as the kernel for prompts wants it.  A step's own tensors do; a caller's memory (logits written
+// in place, a part called by itself) need not, and goes to the library as products that the kernel does not take.
+static bool at_16(const Tensor& t) { return ((uintptr_t)t.data & 15) == 0; }
+
 bool leaves_sums(int64_t x_rows, const Weight& w) {
     if (mid_rows(x_rows, w)) return true;
     return prompt_rows(x_rows, w) && K::prompt_splits.raw((int)x_rows, (int)w.n, (int)w.k) > 1;
@@ -214,7 +218,7 @@ Product linear(StepContext& c, const Tensor& x, const Weight& w, const Tensor* b
             return p;
         }
         if (mid_ok(x, w)) return k_mid_store(c, x, w, out_dtype, leave_sums, out);
-        if (prompt_rows(m, w)) return k_prompt_store(c, x, w, out_dtype, leave_sums, out);
+        if (prompt_rows(m, w) && at_16(x) && (!out || at_16(*out))) return k_prompt_store(c, x, w, out_dtype, leave_sums, out);
         if (!w.rows && m > mid_max_rows() && policy().library && !null_device() && w.n % 8 == 0) {
             // the rows were given up and this is a prompt: the rows come back for the length of this product (the weight
             // read and written once more, against reading it once per 128 rows of x)
@@ -339,7 +343,7 @@ Tensor gated_linear(StepContext& c, const Tensor& x, const Weight& w, const Gate
     Tensor act = c.alloc(x.dtype, {m, inter});
     if (skinny_ok(x, w)) { k_fused_gated(c, x, nullptr, w, act, gate); return act; }
     if (mid_ok(x, w)) { k_mid_gated(c, x, w, act, gate); return act; }
-    if (x.dtype == BF16 && prompt_rows(m, w, true)) {
+    if (x.dtype == BF16 && prompt_rows(m, w, true) && at_16(x)) {
         K::prompt_gated_act(x.data, w.packed->t.data, act.data, (int)m, (int)w.n, (int)w.k, gate.kind, gate.limit, gate.alpha, c.stream);
         return act;
     }
@@ -374,7 +378,7 @@ Tensor activated_linear(StepContext& c, const Tensor& x, const Weight& w, const 
         K::mid_store_act(x.data, w.packed->t.data, act.data, (int)m, (int)w.n, (int)w.k, scratch.data, gate.kind, gate.limit, gate.alpha, c.stream);
         return act;
     }
-    if (x.dtype == BF16 && prompt_rows(m, w)) {
+    if (x.dtype == BF16 && prompt_rows(m, w) && at_16(x)) {
         Tensor act = c.alloc(BF16, {m, w.n});
         const int splits = K::prompt_splits.raw((int)m, (int)w.n, (int)w.k);
         Tensor scratch;
