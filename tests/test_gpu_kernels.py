@@ -422,6 +422,28 @@ def test_attention_generic_two_sequences_share_nothing():
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("d", [64, 30])
+def test_attention_generic_keys_and_values_at_any_element(dtype, d):
+    """Keys and values that do not begin at a multiple of four elements are read one by one: the bits of those that do."""
+    nh, nkv, act = 4, 2, DT[dtype]
+    keys, values = rand(3, nkv, 64, d, seed=20, dtype=act), rand(3, nkv, d, 64, seed=21, dtype=act)
+    q, table, pos = rand(3, nh, d, seed=22, dtype=act), ints([[2, 0, 1]]), ints([0, 70, 155])
+
+    def moved(t, by):
+        buf = torch.zeros(t.numel() + 8, dtype=act, device=DEV)
+        buf[by:by + t.numel()] = t.flatten()
+        return buf[by:by + t.numel()].view(t.shape)
+
+    def run(k, v):
+        out = torch.empty(3, nh * d, dtype=act, device=DEV)
+        return K.attention(q, k, v, ints([0, 0, 0]), pos, table, 0, 0.2, out)
+
+    want = run(keys, values)
+    assert torch.equal(run(moved(keys, 1), values), want) and torch.equal(run(keys, moved(values, 1)), want)
+    assert torch.equal(run(moved(keys, 2), moved(values, 3)), want)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("inter", [250, 18944, 8])
 def test_swiglu(dtype, inter):
     act = DT[dtype]

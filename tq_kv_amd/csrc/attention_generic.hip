@@ -22,7 +22,7 @@
 #define ATT_WAVES 4
 #define ATT_MAX_D 256
 
-// four elements that lie together, at a multiple of their size
+// four elements that lie together, at a multiple of four elements
 __device__ __forceinline__ float4 load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 __device__ __forceinline__ float4 load4(const bf16_t* p) {
     const uint2 v = *reinterpret_cast<const uint2*>(p);
@@ -39,7 +39,7 @@ __global__ __launch_bounds__(ATT_WAVES * TQK_WAVE)
 void attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ keys, const T* __restrict__ values,
                               const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ tok_pos,
                               const int32_t* __restrict__ page_table, int table_width, int window, float scale,
-                              T* __restrict__ out, int n_tokens, int n_heads, int n_kv_heads, int head_dim) {
+                              T* __restrict__ out, int n_tokens, int n_heads, int n_kv_heads, int head_dim, int wide_keys, int wide_values) {
     __shared__ __attribute__((aligned(16))) float q_lds[ATT_WAVES][ATT_MAX_D];
     const int wave = threadIdx.x / TQK_WAVE, lane = threadIdx.x % TQK_WAVE;
     const int t = blockIdx.x * ATT_WAVES + wave;
@@ -75,7 +75,7 @@ void attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ key
             const T* kr = keys + base + (size_t)lane * head_dim;
             float dot = 0.f;
             int i = 0;
-            if (head_dim % 4 == 0) {
+            if (wide_keys) {
 #pragma unroll 8
                 for (; i < head_dim; i += 4) {
                     const float4 k = load4(kr + i), qv4 = *reinterpret_cast<const float4*>(qf + i);
@@ -107,13 +107,15 @@ void attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ key
                 // four positions from a multiple of four lie together
                 int jj = first_key;
                 for (; jj < n_keys && jj % 4 != 0; ++jj) one(jj);
+                if (wide_values) {
 #pragma unroll 4
-                for (; jj + 4 <= n_keys; jj += 4) {
-                    const float4 v = load4(row + value_place(jj));
-                    sum = fmaf(lane_value(p, jj), v.x, sum);
-                    sum = fmaf(lane_value(p, jj + 1), v.y, sum);
-                    sum = fmaf(lane_value(p, jj + 2), v.z, sum);
-                    sum = fmaf(lane_value(p, jj + 3), v.w, sum);
+                    for (; jj + 4 <= n_keys; jj += 4) {
+                        const float4 v = load4(row + value_place(jj));
+                        sum = fmaf(lane_value(p, jj), v.x, sum);
+                        sum = fmaf(lane_value(p, jj + 1), v.y, sum);
+                        sum = fmaf(lane_value(p, jj + 2), v.z, sum);
+                        sum = fmaf(lane_value(p, jj + 3), v.w, sum);
+                    }
                 }
                 for (; jj < n_keys; ++jj) one(jj);
             }
@@ -144,14 +146,17 @@ extern "C" int tqk_attention(const void* q, const void* keys, const void* values
     if (n_tokens == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
     dim3 grid((n_tokens + ATT_WAVES - 1) / ATT_WAVES, n_heads);
+    // four elements a load where keys and values begin at a multiple of four elements (a caller's memory need not) and rows of keys do, too
+    const size_t four = act_dtype == TQK_F32 ? 16 : 8;
+    const int wide_keys = head_dim % 4 == 0 && (uintptr_t)keys % four == 0, wide_values = (uintptr_t)values % four == 0;
     if (act_dtype == TQK_F32)
         attention_generic_kernel<float><<<grid, ATT_WAVES * TQK_WAVE, 0, s>>>(
             (const float*)q, (const float*)keys, (const float*)values, tok_seq, tok_pos, page_table, table_width,
-            window, scale, (float*)out, n_tokens, n_heads, n_kv_heads, head_dim);
+            window, scale, (float*)out, n_tokens, n_heads, n_kv_heads, head_dim, wide_keys, wide_values);
     else if (act_dtype == TQK_BF16)
         attention_generic_kernel<bf16_t><<<grid, ATT_WAVES * TQK_WAVE, 0, s>>>(
             (const bf16_t*)q, (const bf16_t*)keys, (const bf16_t*)values, tok_seq, tok_pos, page_table, table_width,
-            window, scale, (bf16_t*)out, n_tokens, n_heads, n_kv_heads, head_dim);
+            window, scale, (bf16_t*)out, n_tokens, n_heads, n_kv_heads, head_dim, wide_keys, wide_values);
     else
         return tqk_fail("tqk_attention: unknown dtype %d", act_dtype);
     return tqk_check_launch("tqk_attention");
