@@ -4,9 +4,12 @@ kernel library for its limits when it checks a configuration."""
 import ctypes
 import json
 import os
+import re
 import shutil
+import subprocess
 
 from tq_kv_amd import kernels, native
+from tq_kv_amd.csrc import build
 
 CONFIG = {"architectures": ["Qwen2ForCausalLM"], "model_type": "qwen2", "hidden_size": 64, "num_hidden_layers": 1, "num_attention_heads": 2,
           "num_key_value_heads": 1, "intermediate_size": 96, "vocab_size": 50, "max_position_embeddings": 64, "rms_norm_eps": 1e-6,
@@ -54,3 +57,24 @@ def test_the_engine_asks_its_loader_for_the_kernels_when_it_finds_none(tmp_path,
     assert sorted(os.listdir(os.path.join(str(tmp_path), "c"))) == ["config.json", "model.safetensors"]
     assert write("d") == 0 and calls == ["cannot", "can"]
     assert lib.tqe_kernel_library() == path.value
+
+
+def test_the_float32_product_of_few_rows_issues_its_loads_in_the_stages_order(tmp_path):
+    """Its waits let the 24 youngest loads be under way, which are the three later stages' only while every stage's eight loads are issued
+    together, in the stages' order, from the first one on: read off the compiled kernel."""
+    asm = os.path.join(str(tmp_path), "gemm_generic.s")
+    subprocess.run([build._hipcc()] + build.HIPCC_FLAGS + ["-I", build.HERE, "--offload-device-only", "-S", os.path.join(build.HERE, "gemm_generic.hip"), "-o", asm],
+                   check=True, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
+    with open(asm) as f:
+        body = re.search(r"^_Z20gemm_few_rows_kernel\w+:[^\n]*\n(.*?)^\.Lfunc_end", f.read(), re.S | re.M).group(1)
+    kinds = {"buffer_load_dwordx4": "w", "global_load_dwordx4": "x"}
+    events = []
+    for line in body.splitlines():
+        word = line.split()[:2]
+        if word and word[0] in kinds:
+            events.append(kinds[word[0]])
+        elif word and word[0] == "s_waitcnt" and "vmcnt" in line:
+            events.append(word[1])
+    stage = ["w"] * 4 + ["x"] * 4
+    # three stages ahead, then four turns of a stage's loads and the wait for the one three before it, then the wait for all
+    assert events[:3 * 8 + 4 * 9 + 1] == stage * 3 + (stage + ["vmcnt(24)"]) * 4 + ["vmcnt(0)"]

@@ -149,8 +149,7 @@ void gemm_few_rows_kernel(const float* __restrict__ x, const float* __restrict__
         for (int u = 0; u < U; ++u) xv[decltype(I)::value % NS][u] = *reinterpret_cast<const floatx4_t*>(xrow + min(k0 + 16 * u + 4 * g, K - 4));
     };
     floatx4_t group = {0.f, 0.f, 0.f, 0.f}, acc = group;
-    // (one straight line from the first product of a chunk to the sum: where a branch lay between, the compiler let the sum read the
-    // last register of a product that was still under way)
+    // (no branch in a stage: every stage issues its eight loads and multiplies, past the end what is nothing)
     auto multiply = [&](auto I, int stage) {
         const float* src = buf(I);
 #pragma unroll
@@ -160,8 +159,14 @@ void gemm_few_rows_kernel(const float* __restrict__ x, const float* __restrict__
             multiply16(acc, __builtin_bit_cast(floatx4_t, wq & in), __builtin_bit_cast(floatx4_t, __builtin_bit_cast(u32x4_t, xv[decltype(I)::value % NS][u]) & in));
         }
     };
-    each<NS - 1>([&](auto S) { load(S, S); });
-    for (int s0 = 0; s0 < n_stage; s0 += NS) {
+    // The waits below count eight loads a stage in the stages' order.  Barriers keep the scheduler to it, and there is no test in front
+    // of the loop (n_stage is at least 1): behind one the compiler had put all loads of x after all those of the weights.
+    each<NS - 1>([&](auto S) {
+        load(S, S);
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    int s0 = 0;
+    do {
         each<NS>([&](auto S) {
             constexpr int h = decltype(S)::value;
             load(std::integral_constant<int, h + NS - 1>{}, s0 + h + NS - 1);
@@ -175,7 +180,8 @@ void gemm_few_rows_kernel(const float* __restrict__ x, const float* __restrict__
             }
             __builtin_amdgcn_sched_barrier(0);
         });
-    }
+        s0 += NS;
+    } while (s0 < n_stage);
     __builtin_amdgcn_s_waitcnt(0x0f70);                                 // nothing is on its way into LDS any more
     if (r16 >= M) return;
     const bool whole = gridDim.y == 1;
