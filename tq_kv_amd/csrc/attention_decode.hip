@@ -110,11 +110,7 @@ __device__ __forceinline__ void finish_row(const DecodeSums& in, int seq, int po
         if (kind != 2 && pos < in.max_positions) {
             const float c[4] = {c4.x, c4.y, c4.z, c4.w}, sn[4] = {s4.x, s4.y, s4.z, s4.w};
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const float x0 = lo[k], x1 = hi[k];
-                lo[k] = x0 * c[k] - x1 * sn[k];
-                hi[k] = x0 * sn[k] + x1 * c[k];
-            }
+            for (int k = 0; k < 4; ++k) rotate_pair(lo[k], hi[k], c[k], sn[k]);
         }
         uint32_t l[4], h[4];
 #pragma unroll

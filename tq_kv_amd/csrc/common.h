@@ -45,6 +45,15 @@ __device__ __forceinline__ int first_seen(int pos, int window, int chunk) {
     return chunk > 0 ? max(lo, pos - pos % chunk) : lo;
 }
 
+// ---- rotation ----------------------------------------------------------------------
+// A pair x0, x1 turned by an angle, with the roundings in one place: the kernels that write a step's keys from a product that was left as its sums, and
+// from a whole one, then write the same bits (left to itself the compiler joins a multiplication and the addition one way or the other).
+__device__ __forceinline__ void rotate_pair(float& x0, float& x1, float cos, float sin) {
+    const float a = x0, b = x1;
+    x0 = fmaf(a, cos, -(b * sin));
+    x1 = fmaf(a, sin, b * cos);
+}
+
 // ---- reductions ---------------------------------------------------------------
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

@@ -488,11 +488,7 @@ __global__ void rope_store_halves_bf16_kernel(const bf16_t* __restrict__ qkv, co
         const float4 s4 = *reinterpret_cast<const float4*>(sin_table + (size_t)pos * half + i);
         const float c[4] = {c4.x, c4.y, c4.z, c4.w}, sn[4] = {s4.x, s4.y, s4.z, s4.w};
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const float x0 = lo[k], x1 = hi[k];
-            lo[k] = x0 * c[k] - x1 * sn[k];
-            hi[k] = x0 * sn[k] + x1 * c[k];
-        }
+        for (int k = 0; k < 4; ++k) rotate_pair(lo[k], hi[k], c[k], sn[k]);
     }
     uint32_t lo_bits[4], hi_bits[4];
 #pragma unroll
