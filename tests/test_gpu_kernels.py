@@ -351,6 +351,39 @@ def test_decoding_attention_finishes_the_products_sums(d, nh, nkv, n_sums, with_
     assert torch.equal(cache[0], keys) and torch.equal(cache[1], values) and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("n,width,n_parts", [(64, 64, 1), (64, 64, 4), (17, 130, 3), (64, 8, 1), (128, 64, 1), (128, 8, 1), (8, 8, 8), (40, 64, 64)])
+def test_decoding_attention_finishes_sums_before_many_whole_pages(n, width, n_parts):
+    """The same at the 7B heads with pages read once past the caches and through LDS (a table as wide as that, most of it unused), up to 440
+    positions a row of which the last has just been written by the block that reads it, several pages a wave, and where the kernel for given
+    queries takes blocks of two waves (512 blocks and more) or one (a partition a page)."""
+    d, nh, nkv, most = 128, 28, 4, min(width, 9)
+    last = [(128 + 131 * i) % (64 * most - 55) for i in range(n)]
+    g = torch.Generator().manual_seed(75)
+    ids = torch.randperm(n * most, generator=g).tolist()
+    table = ints([[ids[i * most + j] if 64 * j <= p else -1 for j in range(width)] for i, p in enumerate(last)])
+    pos, total = ints(last), (nh + 2 * nkv) * d
+    sums = K.PartialSums(rand(3, n, total, seed=76), torch.bfloat16)
+    bias = rand(total, seed=77, dtype=torch.bfloat16)
+    c, s_ = plain.rope_tables(d, 1e4, 64 * most)
+    cos, sin = c.to(DEV), s_.to(DEV)
+    cache = rand(n * most, nkv, 64, d, seed=78, dtype=torch.bfloat16), rand(n * most, nkv, d, 64, seed=79, dtype=torch.bfloat16)
+    keys, values = cache[0].clone(), cache[1].clone()
+    q = torch.empty(n, nh, d, dtype=torch.bfloat16, device=DEV)
+    K.rope_store(sums, bias, cos, sin, d, K.STYLE_HALVES, ints(range(n)), pos, table, keys, values, q, nh, nkv, d)
+    want = torch.empty(n, nh * d, dtype=torch.bfloat16, device=DEV)
+    K.attention_decode(q, keys, values, pos, table, 0, d ** -0.5, want, n_parts=n_parts)
+    got = torch.full((n, nh * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    K.attention_decode(sums, cache[0], cache[1], pos, table, 0, d ** -0.5, got, n_parts=n_parts, bias=bias, cos=cos, sin=sin)
+    assert torch.equal(cache[0], keys) and torch.equal(cache[1], values)
+    if n_parts == 1 and n * nkv >= 512:
+        # pages meet in two waves there and in four here, each with maxima of its own: a probability is rounded to bfloat16 (2^-9) relative to
+        # another maximum, so an average of values may move by twice that of their mean size, and by a step of its own (at most 2^-7)
+        slack = 2.0 ** -8 * values.float().abs().max() + 2.0 ** -7 * want.float().abs()
+        assert ((got.float() - want.float()).abs() <= slack).all()
+    else:
+        assert torch.equal(got, want)
+
+
 def attention_reference(q, k, v, pos, window, scale, cap=0.0):
     """q [T, nh, d] at absolute positions pos over k, v [nkv, S, d]: plain softmax attention (cap > 0: of cap tanh(score / cap))."""
     nh = q.shape[1]
