@@ -97,9 +97,9 @@ def test_a_wrong_kv_head_is_noticed_at_the_large_sizes(shape):
 @pytest.mark.parametrize("shape,n_seqs", [("qwen2.5:7b", 20), ("qwen2.5:32b", 40), ("qwen2.5:7b", 100), ("qwen2.5:7b", 128),
                                           ("qwen2.5:7b", 129), ("qwen2.5:1.5b", 200)])
 def test_bfloat16_tracks_float32_in_steps_of_17_and_more_rows_at_large_sizes(shape, n_seqs):
-    """The kernels for 17 to 128 rows at the real widths (sums over pieces of K finished by the norm
-    and the rotation kernels, the head product with float32 output), and the steps beyond them (129 and
-    200 rows: eager, the library's products): a short prompt step of 24 tokens, then two decoding steps
+    """The kernels for 17 to 128 rows at the real widths (sums over pieces of K finished by the norm's kernel and by the
+    decoding attention or the rotation's kernel, the head product with float32 output), and the steps beyond them (129 and
+    200 rows: eager, the products of the kernel for prompts): a short prompt step of 24 tokens, then two decoding steps
     of n_seqs rows."""
     raw = two_layer(shape)
     tensors = tensors_for(raw, 5)
@@ -315,12 +315,23 @@ def test_a_step_of_more_than_three_thousand_tokens_takes_the_wide_tiles():
     torch.testing.assert_close(got, want, atol=2e-5 * max(1.0, want.abs().max().item()), rtol=2e-5)
 
 
+@pytest.fixture(params=[True, False])
+def prompt_kernel(request):
+    """The kernel for prompts, switched on and off."""
+    from tq_kv_amd import POLICY
+    old = POLICY["prompt"]
+    POLICY["prompt"] = request.param
+    yield request.param
+    POLICY["prompt"] = old
+
+
 @pytest.mark.parametrize("shape", ["qwen2.5:7b", "qwen2.5:1.5b"])
-def test_a_model_without_weight_rows_gives_the_same_results(shape):
-    """POLICY["keep_rows"] off: the rows of packed weights are given back, and a product of more than
-    128 rows (a prompt) gets them back from the packed copy for its own length and goes to the library
-    as it would have.  So every step is equal bit for bit either way; the prompt of 300 tokens is also
-    compared with the plain implementation as the other bfloat16 runs here are."""
+def test_a_model_without_weight_rows_gives_the_same_results(shape, prompt_kernel):
+    """POLICY["keep_rows"] off: the rows of packed weights are given back.  A product of more than 128 rows (a prompt) is the prompt
+    kernel's, which reads the packed copy either way; with that kernel off (POLICY["prompt"]) the product gets the rows
+    back from the packed copy for its own length and goes to the library as it would have.  So every step is equal bit for bit
+    with and without rows; the prompt of 300 tokens is also compared with the plain implementation as the other
+    bfloat16 runs here are."""
     from tq_kv_amd import POLICY
     raw = two_layer(shape)
     tensors = sharpened(tensors_for(raw, 6))
