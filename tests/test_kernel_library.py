@@ -8,6 +8,7 @@ import re
 import shutil
 import subprocess
 
+import test_gpu_kernels
 from tq_kv_amd import kernels, native
 from tq_kv_amd.csrc import build
 
@@ -78,3 +79,15 @@ def test_the_float32_product_of_few_rows_issues_its_loads_in_the_stages_order(tm
     stage = ["w"] * 4 + ["x"] * 4
     # three stages ahead, then four turns of a stage's loads and the wait for the one three before it, then the wait for all
     assert events[:3 * 8 + 4 * 9 + 1] == stage * 3 + (stage + ["vmcnt(24)"]) * 4 + ["vmcnt(0)"]
+
+
+def test_the_sizes_of_the_prompt_products_tests_take_every_tile():
+    """The choice is made on the host: every tile of the table is taken by some size, the ones without a gate both with K whole and (where real
+    sizes do that) in pieces."""
+    lib = kernels.library()
+    whole = {kernels.prompt_tile(*size) for size in test_gpu_kernels.PROMPT_SIZES if lib.tqk_prompt_splits(*size) == 1}
+    cut = [kernels.prompt_tile(*size) for size in test_gpu_kernels.PROMPT_SIZES if lib.tqk_prompt_splits(*size) > 1]
+    gated = {kernels.prompt_tile(m, 2 * inter, k, True) for m, inter, k in test_gpu_kernels.PROMPT_GATED_SIZES}
+    assert whole == set(range(9)) and len(cut) == 7 and set(cut) >= {1, 3, 4, 5, 6, 8}
+    assert gated == {0, 1, 4, 5, 6, 7, 8, 9}            # three tiles a wave have no gate and up side by side; the last is the gate's alone
+    assert kernels.prompt_tile(129, 16, 250) == -1

@@ -311,6 +311,9 @@ extern "C" int tqk_prompt_takes(int M, int N, int K, int gated) {
 /* Into how many pieces the product's K is cut (1: none, no scratch is needed). */
 extern "C" int tqk_prompt_splits(int M, int N, int K) { return tqk_prompt_takes(M, N, K, 0) ? prompt_plan(M, N, K, false).splits : 1; }
 
+/* Which tile the product takes (an index of the table above; -1: sizes that are not taken): for tests. */
+extern "C" int tqk_prompt_tile(int M, int N, int K, int gated) { return tqk_prompt_takes(M, N, K, gated) ? prompt_plan(M, N, K, gated != 0).config : -1; }
+
 template <int MT, int NT, int WM, int EPI, int WN = 4>
 static void launch(const PromptArgs& a, int splits, hipStream_t s) {
     prompt_product_kernel<MT, NT, WM, WN, EPI><<<dim3(a.tiles_m * a.tiles_n, splits), TQK_WAVE * WN * WM, 0, s>>>(a);

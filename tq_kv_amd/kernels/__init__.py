@@ -572,6 +572,11 @@ def prompt_takes(m, n, k, gated=False):
     return bool(library().tqk_prompt_takes(int(m), int(n), int(k), 1 if gated else 0))
 
 
+def prompt_tile(m, n, k, gated=False):
+    """Which of its tiles the kernel for prompts takes for a product of these sizes (-1: none)."""
+    return int(library().tqk_prompt_tile(int(m), int(n), int(k), 1 if gated else 0))
+
+
 def prompt_store(x, weight, out=None, finish=True, gate=None, limit=0.0, alpha=1.0):
     """out[M,N] = x weight^T (gate: that activation of it) for many rows of bfloat16; weight: a PackedWeight; out: bfloat16 or float32,
     made here (bfloat16) if not given.  finish=False: as mid_store's."""
