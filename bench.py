@@ -203,7 +203,7 @@ def main():
 
     def prefill_point(T, runs):
         if not args.no_tune:
-            # products of more rows than the own kernels take are the library's: let it try its kernels once for the
+            # products that the kernel for prompts does not take are the library's: let it try its kernels once for the
             # shapes of the measured prompt pass
             note("library tuning for %d rows" % T)
             model.tune_library(T)
@@ -234,6 +234,10 @@ def main():
         b_tps, b_sec, _ = decode(engine, random_prompts(z["V"], [long_ctx] * 8), 32, 4)
         points.update(decode_point("decode_b8_8k", z, b_tps, b_sec, 8 * (long_ctx + 4 + 16.0)))
     packed = bool(POLICY["packed"])
+    # whether the prompt pass leaves the library anything to tune
+    own_products = packed and bool(POLICY["prompt"]) and all(
+        K.prompt_takes(args.prompt_len, n, k, gated)
+        for n, k, gated in (((z["nh"] + 2 * z["nkv"]) * z["d"], z["H"], False), (z["H"], z["nh"] * z["d"], False), (2 * z["I"], z["H"], True), (z["H"], z["I"], False)))
     engine = model = None
     release()
 
@@ -296,7 +300,7 @@ def main():
                    "layers": z["L"], "layers_of_shape": full_layers, "hidden": z["H"], "heads": z["nh"], "kv_heads": z["nkv"],
                    "head_dim": z["d"], "intermediate": z["I"], "vocab": z["V"], "prompt_len": args.prompt_len,
                    "new_tokens": total_new, "weights": "random N(0,0.02)", "sampling": "greedy",
-                   "library_tuning": not args.no_tune, "packed_weight_copy": packed, "position_table": raw["max_position_embeddings"]},
+                   "library_tuning": not args.no_tune and not own_products, "packed_weight_copy": packed, "position_table": raw["max_position_embeddings"]},
         "prefill": prefill,
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": PEAK["hbm_gbs"], "unit": "GB/s",
                      "frac": round(achieved / PEAK["hbm_gbs"], 4), "frac_of_probe": of_probe(achieved, "hbm_read_gbs")},

@@ -764,9 +764,12 @@ private:
         // few sequences: a partition per page of the table, which the kernel gives a block of one wave each (faster up to
         // four sequences of 2100 positions at the 7B sizes, slower from eight on)
         if (width > 1 && (long long)groups * width <= 640) n_parts = width;
-        // pages so small that a compute unit brings in all that the table can name while a merge would be launched: one block a row
-        // and kv head (heads of 32, 8 pages of 8 KB: 3.4 against 5.1 us for 30 positions, 4.7 against 5.2 for 500; heads of 64, twice
-        // as much: 7.6 against 5.9 for 500)
+        // pages so small that a compute unit brings in all that the table can name while a merge would be launched: one block a row and kv
+        // head.  us against pages dealt out, 1 to 64 rows, few and all positions of the table used: heads of 32, 8 pages 3.3 to 3.7 against 5.0
+        // to 5.9 and 4.6 to 6.1 against 5.1 to 7.4; heads of 64, 4 pages 4.2 to 4.6 against 6.8 to 8.6 and 5.9 to 6.9 against 7.0 to 9.1; heads
+        // of 128, 2 pages 5.8 to 6.8 against 7.9 to 10.3 and 6.8 to 8.2 against 7.9 to 11.0.  Twice as many pages lose where they are used: heads
+        // of 64 7.6 to 8.8 against 6.2 to 8.1 up to 32 rows, heads of 128 8.7 against 8.4 for one row.  Decoding steps have tables of 8 pages or
+        // more, so there it is heads of 32; the other sizes meet it in the last rows of short prompts.
         if ((long long)width * TQE_PAGE * head_dim_ * 4 <= 64 * 1024) n_parts = 1;
         return n_parts;
     }

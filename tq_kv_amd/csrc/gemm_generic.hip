@@ -6,13 +6,13 @@
 // v_mfma_f32_16x16x4_f32, whose products and sums are float32 ones (no reduced-precision mode of the matrix cores
 // is used anywhere here).  Everything else: LDS-tiled, 64x64 outputs per block, 4x4 per thread, float32 FMA.
 //
-// The order of summation is fixed, and is the same for all numbers of rows, so that a result does
-// not depend on M, on where a row stands in the batch, or on which kernel computed it: k is
+// The order of summation is fixed and the same for all numbers of rows, so that a result does
+// not depend on M or on where a row stands in the batch: k is
 // cut into chunks of 128 and groups of 8 chunks; a chunk is summed from zero, a group is the sum of its chunks in order,
 // the result the sum of the groups in order (and then the bias).  Within a chunk the FMA kernel goes by increasing k; the
 // matrix-core kernels take 16 k at a time, four instructions of which number i adds the k with k % 4 == i to what the ones
 // before it left (a lane then reads its operands of all four as 16 contiguous bytes), with the same operands in the same
-// registers whichever kernel it is.
+// registers in both, so those two give the same bits.  Which of the two orders a product gets is a matter of types, K and addresses alone.
 //
 // For up to 16 rows of x (decoding in the 32-bit path) the weights are the whole cost: a wave takes 16 output features and one
 // group of k and streams their weights through LDS, 12 KB of them under way; groups beyond the first meet in a second

@@ -14,14 +14,19 @@
 //    LDS), four stages in turn, one barrier a stage.  A load takes eight whole 128-byte lines of x; the 16-byte pieces of a row
 //    are exchanged within it (piece c of row r lies at c ^ ((r / 2) % 8)) so that the waves' reads of 16 rows of one k step meet
 //    all banks once.  A wave reads its operands PD groups ahead, across the barrier too.
-//  - WN = 5 with 15 groups of rows (240): gated products of one such row of blocks, where what a compute unit brings in binds and not
-//    the products: every block needs all of x, so few, even blocks count (18944 gated features: 237 blocks of 80; K of 3584, us against the
-//    best tile of four waves: 129 rows 77 against 84, 170: 71 against 86, 232: 74 against 93).  Without a second block on the unit its
-//    rate is lower, so that from two rows of blocks on it loses (17920 x 1536, 440 rows: 38 against 34.5), and so do products
-//    without a gate (4608 x 3584, 1800 rows: 67 against 62).
+//  - WN = 5 with 15 groups of rows (240): gated products of one such row of blocks and no more blocks than units, where what a compute unit
+//    brings in binds and not the products: every block needs all of x, so few, even blocks count.  us at 129, 170, 232 rows against the best
+//    tile of four waves: 18944 gated features (237 blocks of 80) x K of 3584 73, 73, 74 against 80, 84, 90; 17920 x 5120 100, 102, 104 against
+//    115, 120, 127; 20480 x 3584 75, 78, 80 against 80, 84, 90; 16640 x 2048 43, 45, 46 against 42, 47, 51; 17920 x 1536 36, 39, 39 against
+//    36, 38, 41.  With more blocks than units it loses (22016 x 4096 144, 144, 147 against 96, 100, 112), and from two rows of blocks on, too,
+//    since a block alone on its unit has a lower rate (17920 x 1536, 440 rows: 38 against 34.5).  Products without a gate have too few blocks
+//    of that height: with every number of pieces of K tried at 129 to 240 rows, q/k/v and o lose at all three Qwen2.5 shapes (7B, 232 rows:
+//    25.0 against 18.9 and 23.5 against 15.8) and down at the 1.5B one (27 against 19); the other two are within 4 % (50.6 against 50.1, 85.6
+//    against 89.3).
 //  - WM = 2: a second row of four waves on the next MT groups of rows, 256 rows a block, one block a compute unit; the two
 //    waves of a column meet each other's weights in the first-level cache, and a unit brings in a third less than two blocks
-//    of WM = 1 would (1.36 against 1.31 PFLOP/s at 8000 x 37888 x 3584).
+//    of WM = 1 would.  Worth a little where K is long (8000 x 3584 x 18944: 861 us against 869), not where it is short (8000 x 37888 x 3584
+//    without a gate 1585 against 1565; 8000 x 4608 x 3584, where blocks of that size do not go round evenly, 226 against 195).
 //
 // The waits are counted by hand where LDS is concerned (a wave knows how many loads it has issued since the stage it
 // waits for) and by the compiler for the registers; each stage is an array of its own, so that the compiler can tell the
@@ -263,9 +268,10 @@ __global__ void prompt_finish_kernel(const float* __restrict__ partial, TY* __re
 // measured (8000 rows of the 7B products, corrected for the last round), relative to the best; smaller tiles bring more bytes in for
 // a product.  The start and end of a block cost as much as 300 k; 600 for a gated block that has its unit to itself (wm = 2), since then
 // nothing else runs on the unit while the gate is applied (8000 x 1536 x 17920 gated: 393 us against 350 with blocks of four waves;
-// K of 3584: 1620 against 1550).  Cutting K adds the pieces' sums, written and read as float32.  Against all tiles tried one by one
+// 37888 x 3584 1638 against 1539).  Cutting K adds the pieces' sums, written and read as float32.  Against all tiles tried one by one
 // at 232, 300, 1024, 2048 and 8000 rows of the four 7B products the rule takes the fastest or one within 4 % of it, but for
-// the gated product of 300 to 600 rows (within 10 %).
+// the gated product of 300 to 600 rows (within 10 %).  Elsewhere it can be further off: gated 24576 x 3072 and 22016 x 4096 at 170 rows
+// 90 and 115 us, with another tile 78 and 100; o and q/k/v of the 1.5B shape, finished here, up to 2 us of 11 slower in pieces than whole.
 struct PromptPlan { int config, splits, k_per_split; };
 struct PromptConfig { int mt, nt, wm, wn; double rate; };
 static const PromptConfig CONFIGS[] = {
