@@ -236,7 +236,7 @@ def main():
     packed = bool(POLICY["packed"])
     # whether the prompt pass leaves the library anything to tune
     own_products = packed and bool(POLICY["prompt"]) and all(
-        K.prompt_takes(args.prompt_len, n, k, gated)
+        K.prompt_pays(args.prompt_len, n, k, gated)
         for n, k, gated in (((z["nh"] + 2 * z["nkv"]) * z["d"], z["H"], False), (z["H"], z["nh"] * z["d"], False), (2 * z["I"], z["H"], True), (z["H"], z["I"], False)))
     engine = model = None
     release()

@@ -504,10 +504,11 @@ def test_decode_steps_of_a_hundred_and_more_sequences(name, sharp, dtype, n_seqs
 
 
 # ---- tuning the library -----------------------------------------------------------------------------
-@pytest.mark.parametrize("inter,packed,want", [(512, True, 0), (264, True, 2), (512, False, 4)])
+@pytest.mark.parametrize("inter,packed,want", [(256, True, 0), (512, True, 1), (264, True, 2), (512, False, 4)])
 def test_tuning_takes_every_product_that_goes_to_the_library(inter, packed, want):
-    """Products that the kernel for prompts takes are left out; not so a gate and up whose halves are no whole tiles (inter of 264, whose
-    down product has K of 264, too), nor weights that were loaded without a packed copy, whatever the switch says by then."""
+    """Products that the kernel for prompts takes whatever follows them are left out; not so one that is small and cut into pieces (down, K of 512), a
+    gate and up whose halves are no whole tiles (inter of 264, whose down product has K of 264, too), nor weights that were loaded without a
+    packed copy, whatever the switch says by then."""
     from tq_kv_amd import POLICY, tracing
     raw = dict(catalog.find("qwen2.5:1.5b"), num_hidden_layers=2, vocab_size=512, hidden_size=256, intermediate_size=inter, num_attention_heads=4,
                num_key_value_heads=2, head_dim=64)

@@ -46,6 +46,23 @@ def test_rms_norm_part(dtype):
     torch.testing.assert_close(got.float().cpu(), plain.rms_norm((want_h + d.float()).cpu()[[4, 1]], w["weight"], 1e-4), **TOL[dtype])
 
 
+@pytest.mark.parametrize("hidden,inter,own", [(2048, 1024, True), (8192, 64, False), (4096, 256, False)])
+def test_gated_feed_forward_of_prompts_either_side_of_the_products_rule(hidden, inter, own):
+    """200 rows in bfloat16: gate and up through the kernel for prompts, or (few features, long K) through the library and the gate's kernel; the down
+    product, which nothing takes as its sums here, whole, in pieces, or the library's."""
+    from tq_kv_amd import kernels
+    assert kernels.prompt_pays(200, 2 * inter, hidden, True) == own
+    env = BuildEnv(DEV, torch.bfloat16)
+    ff = env.build("feed_forward", PartSpec("gated_silu", {"hidden": hidden, "inter": inter}))
+    w = load_random(ff, "bfloat16", 3, std=0.02)
+    x = torch.randn(200, hidden, generator=torch.Generator().manual_seed(4)).bfloat16().to(DEV)
+    gate, up, down = (next(v for k, v in w.items() if name in k).to(DEV).double() for name in ("gate", "up", "down"))
+    want = (torch.nn.functional.silu(x.double() @ gate.t()) * (x.double() @ up.t())) @ down.t()
+    got = ff.forward(x).double()
+    # gate, up, their product and the result are each rounded to bfloat16 (2^-9 of a value at most): four such errors, which do not add up in full
+    assert ((got - want).norm() / want.norm()).item() < 4 * 2.0 ** -9
+
+
 def test_rotary_part_tables():
     env = BuildEnv(DEV, torch.float32)
     rot = env.build("position", PartSpec("rotary", {"theta": 1e6, "rot_dim": 48, "max_positions": 300, "style": "halves"}))

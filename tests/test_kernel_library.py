@@ -8,6 +8,8 @@ import re
 import shutil
 import subprocess
 
+import pytest
+
 import test_gpu_kernels
 from tq_kv_amd import kernels, native
 from tq_kv_amd.csrc import build
@@ -91,3 +93,14 @@ def test_the_sizes_of_the_prompt_products_tests_take_every_tile():
     assert whole == set(range(9)) and len(cut) == 7 and set(cut) >= {1, 3, 4, 5, 6, 8}
     assert gated == {0, 1, 4, 5, 6, 7, 8, 9}            # three tiles a wave have no gate and up side by side; the last is the gate's alone
     assert kernels.prompt_tile(129, 16, 250) == -1
+
+
+@pytest.mark.parametrize("m,n,k,gated,pays", [
+    (200, 512, 4096, False, False), (129, 128, 2048, False, False), (8000, 32, 1024, False, False), (1024, 16, 512, False, False),  # small and cut
+    (2048, 512, 256, False, True), (300, 512, 256, False, True),                                                                  # not cut
+    (129, 3584, 18944, False, True), (300, 3584, 18944, False, True), (232, 1536, 8960, False, True),                             # cut and large
+    (200, 128, 8192, True, False), (129, 2048, 8192, True, False), (512, 1024, 4096, True, False),                                # long K, few blocks
+    (129, 37888, 3584, True, True), (255, 37888, 3584, True, True), (1023, 17920, 1536, True, True), (768, 55296, 5120, True, True),
+    (129, 37888, 3584 + 32, True, False), (129, 24, 256, False, False)])                                                           # not taken at all
+def test_which_products_pay_in_the_kernel_for_prompts(m, n, k, gated, pays):
+    assert kernels.prompt_pays(m, n, k, gated) == pays

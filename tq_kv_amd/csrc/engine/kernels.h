@@ -36,6 +36,7 @@ TQ_KERNEL(mid_store, cptr, cptr, void*, int, int, int, int, void*, int, void*);
 TQ_KERNEL(mid_gated, cptr, cptr, void*, int, int, int, void*, void*);
 TQ_QUERY(int, prompt_takes, int, int, int, int);
 TQ_QUERY(int, prompt_splits, int, int, int);
+TQ_QUERY(int, prompt_pays, int, int, int, int);
 TQ_KERNEL(prompt_store, cptr, cptr, void*, int, int, int, int, void*, int, void*);
 TQ_KERNEL(prompt_store_act, cptr, cptr, void*, int, int, int, void*, int, float, float, void*);
 TQ_KERNEL(prompt_gated_act, cptr, cptr, void*, int, int, int, int, float, float, void*);

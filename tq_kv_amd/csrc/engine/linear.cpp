@@ -100,6 +100,11 @@ static bool prompt_rows(int64_t x_rows, const Weight& w, bool gated = false) {
 // in place, a part called by itself) need not, and goes to the library as products that the kernel does not take.
 static bool at_16(const Tensor& t) { return ((uintptr_t)t.data & 15) == 0; }
 
+// Whether such a product is worth it where its sums are finished at once (with the library switched off everything is).
+static bool prompt_pays(int64_t x_rows, const Weight& w, bool gated = false) {
+    return !policy().library || K::prompt_pays.raw((int)x_rows, (int)w.n, (int)w.k, gated ? 1 : 0) != 0;
+}
+
 bool leaves_sums(int64_t x_rows, const Weight& w) {
     if (mid_rows(x_rows, w)) return true;
     return prompt_rows(x_rows, w) && K::prompt_splits.raw((int)x_rows, (int)w.n, (int)w.k) > 1;
@@ -107,9 +112,9 @@ bool leaves_sums(int64_t x_rows, const Weight& w) {
 
 bool prompt_product(int64_t x_rows, const ProductShape& shape) {
     const Policy& p = policy();
-    if (shape.weight->defined()) return prompt_rows(x_rows, *shape.weight, shape.gated);
+    if (shape.weight->defined()) return prompt_rows(x_rows, *shape.weight, shape.gated) && prompt_pays(x_rows, *shape.weight, shape.gated);
     if (!p.prompt || !p.packed || !p.skinny || x_rows <= mid_max_rows() || x_rows > INT32_MAX || shape.n > INT32_MAX || shape.k > INT32_MAX) return false;
-    return K::prompt_takes.raw((int)x_rows, (int)shape.n, (int)shape.k, shape.gated ? 1 : 0) != 0;
+    return K::prompt_pays.raw((int)x_rows, (int)shape.n, (int)shape.k, shape.gated ? 1 : 0) != 0;
 }
 
 void classify_step(StepContext& c, int64_t hidden) {
@@ -218,7 +223,7 @@ Product linear(StepContext& c, const Tensor& x, const Weight& w, const Tensor* b
             return p;
         }
         if (mid_ok(x, w)) return k_mid_store(c, x, w, out_dtype, leave_sums, out);
-        if (prompt_rows(m, w) && at_16(x) && (!out || at_16(*out))) return k_prompt_store(c, x, w, out_dtype, leave_sums, out);
+        if (prompt_rows(m, w) && at_16(x) && (!out || at_16(*out)) && (leave_sums || prompt_pays(m, w))) return k_prompt_store(c, x, w, out_dtype, leave_sums, out);
         if (!w.rows && m > mid_max_rows() && policy().library && !null_device() && w.n % 8 == 0) {
             // the rows were given up and this is a prompt: the rows come back for the length of this product (the weight
             // read and written once more, against reading it once per 128 rows of x)
@@ -343,7 +348,7 @@ Tensor gated_linear(StepContext& c, const Tensor& x, const Weight& w, const Gate
     Tensor act = c.alloc(x.dtype, {m, inter});
     if (skinny_ok(x, w)) { k_fused_gated(c, x, nullptr, w, act, gate); return act; }
     if (mid_ok(x, w)) { k_mid_gated(c, x, w, act, gate); return act; }
-    if (x.dtype == BF16 && prompt_rows(m, w, true) && at_16(x)) {
+    if (x.dtype == BF16 && prompt_rows(m, w, true) && at_16(x) && prompt_pays(m, w, true)) {
         K::prompt_gated_act(x.data, w.packed->t.data, act.data, (int)m, (int)w.n, (int)w.k, gate.kind, gate.limit, gate.alpha, c.stream);
         return act;
     }
@@ -378,6 +383,7 @@ Tensor activated_linear(StepContext& c, const Tensor& x, const Weight& w, const 
         K::mid_store_act(x.data, w.packed->t.data, act.data, (int)m, (int)w.n, (int)w.k, scratch.data, gate.kind, gate.limit, gate.alpha, c.stream);
         return act;
     }
+    // (in pieces or not: the kernel that adds them up applies the activation, which a library's product would need a kernel for, too)
     if (x.dtype == BF16 && prompt_rows(m, w) && at_16(x)) {
         Tensor act = c.alloc(BF16, {m, w.n});
         const int splits = K::prompt_splits.raw((int)m, (int)w.n, (int)w.k);
@@ -411,7 +417,7 @@ static bool pieces_pay(const Weight& w) {
 void add_product(StepContext& c, Stream& stream, const Tensor& x, const Weight& w) {
     if (x.shape[0] > skinny_max_rows() || pieces_pay(w)) {
         const bool leave = stream.next_norm && stream.next_norm->takes_partial_sums();
-        Product p = x.shape[0] > mid_max_rows() ? k_prompt_store(c, x, w, BF16, leave, nullptr) : k_mid_store(c, x, w, BF16, leave, nullptr);
+        Product p = x.shape[0] > mid_max_rows() ? linear(c, x, w, nullptr, BF16, leave) : k_mid_store(c, x, w, BF16, leave, nullptr);
         stream.pending = p.is_sums ? Pending::of(p.sums) : Pending::of(p.t);
         stream.invalidate();
         return;

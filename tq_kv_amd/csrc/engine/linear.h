@@ -11,7 +11,8 @@
 //            copy of the weight, packed at loading time in the order its lanes take it.
 //   bfloat16, more rows up to what the kernel for mid-sized steps takes, where the weight has a packed copy
 //         -> the hand-written kernel that stages x in LDS and streams the packed weights
-//   bfloat16, more rows (prompts, large decoding batches), where the weight has a packed copy and K is a multiple of 256
+//   bfloat16, more rows (prompts, large decoding batches), where the weight has a packed copy, K is a multiple of 256, and the kernel pays:
+//   K whole, its sums left to the next kernel, or the product large (tqk_prompt_pays)
 //         -> the hand-written kernel that shares x in LDS and streams the packed weights (prompt_product.hip)
 //   bfloat16, more rows of other shapes, or without a packed copy
 //         -> the library GEMM (hipBLASLt), float32 accumulation; float32 output where logits are wanted
@@ -56,7 +57,7 @@ bool fusable(int64_t x_rows, const Weight& w, bool adds = false);
 // Whether a product of x_rows rows goes through a kernel that can leave its sums over pieces of K to the next norm: the one for
 // mid-sized steps, or the one for prompts where it cuts K.
 bool leaves_sums(int64_t x_rows, const Weight& w);
-// Whether the kernel for prompts takes a part's product of x_rows rows: the library is then not asked.  Before the weight is loaded: whether it
+// Whether the kernel for prompts takes a part's product of x_rows rows, whatever follows it: the library is then not asked.  Before the weight is loaded: whether it
 // will, as the policy stands.
 bool prompt_product(int64_t x_rows, const ProductShape& shape);
 // What kind of step this is for the parts' folding: small (norms and residual sums folded into

@@ -272,7 +272,7 @@ __global__ void prompt_finish_kernel(const float* __restrict__ partial, TY* __re
 // at 232, 300, 1024, 2048 and 8000 rows of the four 7B products the rule takes the fastest or one within 4 % of it, but for
 // the gated product of 300 to 600 rows (within 10 %).  Elsewhere it can be further off: gated 24576 x 3072 and 22016 x 4096 at 170 rows
 // 90 and 115 us, with another tile 78 and 100; o and q/k/v of the 1.5B shape, finished here, up to 2 us of 11 slower in pieces than whole.
-struct PromptPlan { int config, splits, k_per_split; };
+struct PromptPlan { int config, splits, k_per_split; double us; };
 struct PromptConfig { int mt, nt, wm, wn; double rate; };
 static const PromptConfig CONFIGS[] = {
     {8, 4, 2, 4, 1.00}, {8, 4, 1, 4, 0.96}, {8, 3, 2, 4, 0.95}, {8, 3, 1, 4, 0.90}, {6, 4, 1, 4, 0.84},
@@ -283,8 +283,7 @@ static const PromptConfig CONFIGS[] = {
 #define PROMPT_MAX_SPLITS 16
 
 static PromptPlan prompt_plan(int M, int N, int K, bool gated) {
-    PromptPlan best = {0, 1, K};
-    double best_us = 1e30;
+    PromptPlan best = {0, 1, K, 1e30};
     const long long turns = K / PROMPT_K;
     for (int i = 0; i < PROMPT_CONFIGS; ++i) {
         const PromptConfig& c = CONFIGS[i];
@@ -300,7 +299,7 @@ static PromptPlan prompt_plan(int M, int N, int K, bool gated) {
             // (us: 256 units at the best tile's rate are 1.4 PFLOP/s)
             double us = rounds * (c.mt * c.nt * c.wm * c.wn / 4.0) / c.rate * (double)(per * PROMPT_K + (gated && c.wm == 2 ? 600 : 300)) * 3.7e-4;
             if (splits > 1) us += (double)splits * M * N * 8.0 / 4.5e6;
-            if (us < best_us) { best_us = us; best = {i, splits, (int)(per * PROMPT_K)}; }
+            if (us < best.us) best = {i, splits, (int)(per * PROMPT_K), us};
         }
     }
     return best;
@@ -316,6 +315,23 @@ extern "C" int tqk_prompt_takes(int M, int N, int K, int gated) {
 
 /* Into how many pieces the product's K is cut (1: none, no scratch is needed). */
 extern "C" int tqk_prompt_splits(int M, int N, int K) { return tqk_prompt_takes(M, N, K, 0) ? prompt_plan(M, N, K, false).splits : 1; }
+
+/* Whether a product that is taken is worth it where its pieces' sums are not left to another kernel; else the library is the faster one (its first
+ * choice for a shape, us in replayed graphs, weights from memory).
+ * Cut into pieces, the second kernel that adds them up takes 3.6 us and more: of 921 sizes (16 to 16384 features, K of 256 to 18944, 129 to 8000
+ * rows) the 362 cut ones that the plan puts below 18 us with it are 1.17 times as slow as the library (200 x 512 x 4096 13.4 us against 8.3,
+ * 129 x 128 x 2048 8.8 against 5.9), the 156 above 1.49 times as fast, the 403 whole ones 1.17 times; left to the next kernel cut ones are 1.49
+ * times as fast, two of 520 slower.
+ * A gate cannot be applied to pieces, so K is whole however few blocks there are: measured against what the same product without
+ * the gate would take in pieces, and 5 us for a gate of its own.  Of 687 gated sizes those refused are 1.37 times as slow as the library with its gate's
+ * kernel (200 x 64 x 8192 36 us against 13, 129 x 1024 x 8192 57 against 30), the others 1.33 times as fast; the factor 1.3 lies above
+ * what the large products reach (1.16), which are to stay. */
+extern "C" int tqk_prompt_pays(int M, int N, int K, int gated) {
+    if (!tqk_prompt_takes(M, N, K, gated)) return 0;
+    const PromptPlan plan = prompt_plan(M, N, K, gated != 0);
+    if (!gated) return plan.splits == 1 || plan.us + 3.6 >= 18.0;
+    return plan.us <= 1.3 * prompt_plan(M, N, K, false).us + 5.0;
+}
 
 /* Which tile the product takes (an index of the table above; -1: sizes that are not taken): for tests. */
 extern "C" int tqk_prompt_tile(int M, int N, int K, int gated) { return tqk_prompt_takes(M, N, K, gated) ? prompt_plan(M, N, K, gated != 0).config : -1; }

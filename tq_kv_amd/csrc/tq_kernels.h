@@ -123,6 +123,7 @@ int tqk_mid_gated(const void* x, const void* w_packed, void* y, int M, int N, in
  * tqk_prompt_store_act: bfloat16, an activation of the product (TQK_GATE_*). */
 int tqk_prompt_takes(int M, int N, int K, int gated);
 int tqk_prompt_splits(int M, int N, int K);
+int tqk_prompt_pays(int M, int N, int K, int gated);       /* whether it is faster than a library's where its pieces' sums are not left */
 int tqk_prompt_tile(int M, int N, int K, int gated);       /* which of its tiles it takes, for tests */
 int tqk_prompt_store(const void* x, const void* w_packed, void* y, int y_dtype, int M, int N, int K, void* scratch, int finish, void* stream);
 int tqk_prompt_store_act(const void* x, const void* w_packed, void* y, int M, int N, int K, void* scratch, int gate, float limit, float alpha, void* stream);

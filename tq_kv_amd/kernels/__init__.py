@@ -572,6 +572,12 @@ def prompt_takes(m, n, k, gated=False):
     return bool(library().tqk_prompt_takes(int(m), int(n), int(k), 1 if gated else 0))
 
 
+def prompt_pays(m, n, k, gated=False):
+    """Whether the kernel for prompts is faster than a library's for a product of these sizes that is finished at once (its pieces' sums not left to
+    another kernel): the engine sends the others to the library."""
+    return bool(library().tqk_prompt_pays(int(m), int(n), int(k), 1 if gated else 0))
+
+
 def prompt_tile(m, n, k, gated=False):
     """Which of its tiles the kernel for prompts takes for a product of these sizes (-1: none)."""
     return int(library().tqk_prompt_tile(int(m), int(n), int(k), 1 if gated else 0))
