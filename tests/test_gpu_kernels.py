@@ -731,6 +731,31 @@ def test_product_of_17_to_128_rows(m, n, k):
         K.mid_store(x, w, out)
 
 
+# Wide products, whose waves take 1, 2 or more tiles each by the number of rows, and gated ones of 3 to 8 waves a block; K that ends in the middle of
+# a stage of 64, before the ring of stages is full (96, 160) and after it has gone round (416, 928).
+@pytest.mark.parametrize("m", [17, 33, 65, 128])
+@pytest.mark.parametrize("n,k", [(16400, 160), (20000, 416), (40010, 352), (77000, 928), (152064, 96)])
+def test_wide_products_of_17_to_128_rows(m, n, k):
+    x, w = rand(m, k, seed=44, dtype=torch.bfloat16), rand(n, k, seed=45, scale=0.05, dtype=torch.bfloat16)
+    out = torch.full((m + 1, n), float("nan"), device=DEV)
+    K.mid_store(x, K.pack_weight(w), out[:m])
+    # up to 928 sums in float32, each rounded to 2^-24 of a sum of size about 3
+    torch.testing.assert_close(out[:m].double(), x.double() @ w.double().t(), atol=928 * 3 * 2.0 ** -24, rtol=1e-5)
+    assert torch.isnan(out[m]).all()
+
+
+@pytest.mark.parametrize("m", [17, 33, 65, 128])
+@pytest.mark.parametrize("inter,k", [(8960, 160), (9000, 96), (12000, 416), (17000, 224), (24560, 352), (30000, 64)])
+def test_gated_products_of_17_to_128_rows_by_waves(m, inter, k):
+    x = rand(m, k, seed=46, scale=1.5, dtype=torch.bfloat16)
+    w = rand(2 * inter, k, seed=47, scale=0.4 / math.sqrt(k), dtype=torch.bfloat16)
+    out = torch.full((m + 1, inter), float("nan"), dtype=torch.bfloat16, device=DEV)
+    K.mid_gated(x, K.pack_weight(w, parts=2), out[:m])
+    gu = (x.double() @ w.double().t()).float().to(torch.bfloat16).float()
+    torch.testing.assert_close(out[:m].float(), F.silu(gu[:, :inter]) * gu[:, inter:], atol=3e-2, rtol=3e-2)      # as the other gated products
+    assert torch.isnan(out[m]).all()
+
+
 @pytest.mark.parametrize("m", [17, 40, 64, 65, 90, 128])
 @pytest.mark.parametrize("inter,k", [(112, 64), (18944, 3584), (100, 96), (200, 1312), (18, 1312), (50, 2048), (7, 96)])
 def test_gated_product_of_17_to_128_rows(m, inter, k):

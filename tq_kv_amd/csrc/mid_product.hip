@@ -5,11 +5,19 @@
 // packed in the lanes' order ([tile of 16 rows][K/32][lane][8 values], see skinny_fused.hip).
 //
 // With this many rows x is no longer small beside a tile of weights: every wave needs all of it.
-// So a block is 4 to 8 waves that walk K together in chunks of 128; each chunk of x is staged once
-// per block in LDS, in the order the lanes read it ([16 rows][k step][lane] x 16 bytes, so both
-// the block's write and the waves' reads are linear), double buffered with one barrier per
-// chunk, while each wave multiplies its own tiles of 16 output features with it.  The loads of
-// the next two chunks are under way while the current one is multiplied.
+// So a block is 3 to 8 waves that walk K together, each with its own tiles of 16 output features,
+// and one or two more waves that do nothing but bring x in, 64 k a stage, into a ring in LDS with
+// loads that end there (a load takes eight whole lines of 128 bytes, of eight rows; the 16-byte pieces
+// of a row are exchanged within it so that the reads of 16 rows of one k step meet all banks once).
+// What binds such a block is what a compute unit brings in, weights and x together: with x in whole
+// lines 38 GB/s at 64 rows and 53 at 256, in pieces of 64 bytes of 16 rows, which is what the matrix
+// cores' order asks for, 33 and 36 (a bare loop of such loads).  The waves that multiply count no load
+// but their weights', 8 steps of 32 k ahead, and meet once a stage.  Against a kernel whose waves
+// brought x in between their weights, through registers, us at 32, 64 and 128 rows: gate+up of the 7B
+// shape 47, 54, 69 -> 44, 46, 55; down 24.9, 28.7, 40.0 -> 24.2, 26.3, 34.4; q/k/v 9.7, 11.3, 17.2 ->
+// 8.8, 10.1, 14.5; o 8.4, 10.2, 13.9 -> 7.6, 8.6, 11.6; gate+up of the 1.5B shape 17.9, 22.8, 29.3 ->
+// 12.8, 15.6, 21.6.  Measured and left: 2, 4, 6 and 12 steps of weights ahead (within 1 %), 4 and 8 stages
+// of x (the same), counts in LDS in place of the barrier, so that the waves may run apart (2 to 15 % slower).
 //
 // v_mfma_f32_16x16x32_bf16: A = a tile of w (16 features x 32 k), B = 32 k x 16 rows of x, so
 // D[n][m] is a tile of y^T: lane l holds row m = l%16 of its 16-row group and the four features
@@ -20,24 +28,19 @@
 // (store, or the gate: silu(gate) * up of src/models/turbo_generic.rs:105-111).  The number of
 // splits depends on the product's shape alone, never on M, so a row's result does not depend on
 // the batch it is in.
-//
-// Beyond 64 rows (8 row groups) every compute unit pulls all of x through its first-level cache
-// beside its own share of the weights (0.9 MB beside 1.15 MB at 128 rows of the 7B gate+up
-// product), and that path, not HBM, sets the time: 4.1 TB/s of weights at 128 rows against 4.9 at
-// 64.  Measured there and left: reads of x two steps ahead, one or two extra waves that only bring
-// x in, a deeper ring of LDS operands (the waves wait for x behind the weights in the same
-// queue, whoever asks for it).
 #include "common.h"
 #include "tq_kernels.h"
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 enum { MID_STORE = 0, MID_GATED = 1 };
-#define MID_CHUNK 128           // k per stage
-#define MID_MIN_WAVES 4          // waves per block: from the product's shape (mid_plan)
+#define MID_CHUNK 128           // K is cut into multiples of it
+#define MID_MIN_WAVES 4          // waves per block that multiply: from the product's shape (mid_plan, mid_waves)
 #define MID_MAX_WAVES 8
+#define MID_LEAST_WAVES 3        // where K is whole
 #define MID_MAX_ROWS 128
 
 struct MidArgs {
@@ -67,187 +70,9 @@ __device__ __forceinline__ float finished(const Gate& gate, float sum) {
     return gate.activated ? act_value(gate.kind, gate.limit, gate.alpha, to_float(from_float<bf16_t>(sum))) : sum;
 }
 
-// MT: groups of 16 rows of x (2: up to 32 rows, 4: up to 64, 8: up to 128).  TN: tiles of 16
-// features per wave (gated: the gate tile and its up tile).
-// PAR: 256-thread groups of the block that bring x in (2 in a block of 8 waves, else 1).
-template <int MT, int TN, int EPI, typename TY, int PAR>
-__global__ __launch_bounds__(MID_MAX_WAVES * TQK_WAVE)
-void mid_product_kernel(const MidArgs p) {
-    constexpr int SLOTS = MT * 256;                 // 16-byte pieces of a chunk of x: [row group][k step][lane]
-    constexpr bool WIDE = MT > 4;                   // 8 row groups: registers are short, see below
-    constexpr int XS = WIDE ? MT / PAR : SLOTS / (MID_MIN_WAVES * TQK_WAVE);       // pieces of x per thread at most
-    static_assert(EPI != MID_GATED || TN == 2, "a gated block holds pairs of tiles");
-    extern __shared__ u32x4_t xs[];                 // [2][SLOTS]
-    const int lane = threadIdx.x % TQK_WAVE, wave = threadIdx.x / TQK_WAVE;
-    const int n_waves = blockDim.x / TQK_WAVE;
-    const int row = lane % 16, kgrp = lane / 16;
-    const int K = p.K;
-    const bf16_t* px = p.x;
-    if (EPI == MID_STORE && p.group_rows) px += (size_t)((int)blockIdx.x * n_waves * TN * 16 / p.group_rows) * p.x_group_stride;
-    const int k_begin = blockIdx.y * p.k_per_split, k_end = min(K, k_begin + p.k_per_split);
-
-    const int n_out = EPI == MID_GATED ? p.N / 2 : p.N;             // features one part of the weight has
-    const int part_tiles = (n_out + 15) / 16;
-    const int tile0 = (blockIdx.x * n_waves + wave) * (EPI == MID_GATED ? 1 : TN);
-    const int n_lo0 = tile0 * 16;
-    const size_t tile_size = (size_t)(K / 32) * 512;
-    const bf16_t* wtile[TN];
-#pragma unroll
-    for (int t = 0; t < TN; ++t) {
-        // tiles past the end repeat the last one; their results are dropped
-        const int tile = EPI == MID_GATED ? t * part_tiles + min(tile0, part_tiles - 1) : min(tile0 + t, part_tiles - 1);
-        wtile[t] = p.w + (size_t)tile * tile_size + lane * 8;
-    }
-    // Up to 4 row groups: a thread's pieces of a chunk of x are those at its number plus multiples of
-    // the block's size; rows past M repeat the last row.  Pieces past the chunk's end (whole waves
-    // of them, with more than 4 waves) are loaded again and not stored.
-    const bf16_t* xsrc[WIDE ? 1 : XS];
-    int xk[WIDE ? 1 : XS];
-    if constexpr (!WIDE) {
-#pragma unroll
-        for (int i = 0; i < XS; ++i) {
-            const int s = min((int)threadIdx.x + i * (int)blockDim.x, SLOTS - 1);
-            const int mt = s / 256, ks = (s / 64) % 4, ln = s % 64;
-            xk[i] = ks * 32 + (ln / 16) * 8;
-            xsrc[i] = px + (size_t)min(mt * 16 + ln % 16, p.M - 1) * K;
-        }
-    }
-    // 8 row groups: the block's first 256 threads bring x in, thread t piece t ([k step][lane]) of
-    // every row group, so that its pieces lie 16 rows apart and need one address; in a block of 8
-    // waves the second 256 threads take every other row group (PAR = 2).
-    const int st_half = threadIdx.x / 256;
-    const bool stages = st_half < PAR;
-    const int st_row = threadIdx.x % 16, st_k = ((threadIdx.x / 64) % 4) * 32 + ((threadIdx.x % 64) / 16) * 8;
-    floatx4_t acc[TN][MT];
-#pragma unroll
-    for (int t = 0; t < TN; ++t)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[t][mt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-
-    // Loads past the end of K stay inside the row (and are valid memory); x is zeroed there as it
-    // goes into LDS, so they add nothing.  Nothing is under a condition: the waits can be counted.
-    // (Measured: with the loads of a wave whose pieces all lie past the chunk left out under a
-    // condition, the compiler waits for all loads at every use, and a step of 64 rows at the 7B
-    // sizes takes 16.6 ms instead of 4.1.)
-    auto load_x = [&](int c, u32x4_t (&xr)[XS]) {
-        if constexpr (WIDE) {
-            if (!stages) return;
-            const uint32_t kk = (uint32_t)min(c + st_k, K - 8);
-#pragma unroll
-            for (int i = 0; i < XS; ++i) {
-                const uint32_t r = (uint32_t)min((i * PAR + st_half) * 16 + st_row, p.M - 1);
-                xr[i] = *reinterpret_cast<const u32x4_t*>(px + (r * (uint32_t)K + kk));
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < XS; ++i) xr[i] = *reinterpret_cast<const u32x4_t*>(xsrc[i] + min(c + xk[i], K - 8));
-        }
-    };
-    auto store_x = [&](int c, int buf, const u32x4_t (&xr)[XS]) {
-        if constexpr (WIDE) {
-            if (!stages) return;
-            const bool past = c + st_k >= k_end;
-#pragma unroll
-            for (int i = 0; i < XS; ++i) xs[buf * SLOTS + (i * PAR + st_half) * 256 + threadIdx.x % 256] = past ? u32x4_t{0, 0, 0, 0} : xr[i];
-        } else {
-#pragma unroll
-            for (int i = 0; i < XS; ++i) {
-                u32x4_t v = xr[i];
-                if (c + xk[i] >= k_end) v = u32x4_t{0, 0, 0, 0};
-                const int s = threadIdx.x + i * blockDim.x;
-                if (s < SLOTS) xs[buf * SLOTS + s] = v;
-            }
-        }
-    };
-    auto load_w = [&](int c, bf16x8_t (&a)[TN][4]) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const size_t at = (size_t)min(c / 32 + u, K / 32 - 1) * 512;
-#pragma unroll
-            for (int t = 0; t < TN; ++t) a[t][u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wtile[t] + at));      // read once
-        }
-    };
-    // x comes from LDS four row groups at a time (two where registers are short), the next ones on
-    // their way while these are multiplied.
-    // RING (8 row groups, where registers are short): a k step's weight registers are asked for
-    // again, for the chunk after those under way, as soon as its products are issued, so that two
-    // register sets keep nearly two chunks on their way.
-    constexpr bool RING = WIDE;
-    auto multiply = [&](int buf, bf16x8_t (&a)[TN][4], int refill_c) {
-        constexpr int G = RING && TN > 1 ? 2 : (MT < 4 ? MT : 4), NG = MT / G, STEPS = 4 * NG;
-        u32x4_t bx[2][G];
-#pragma unroll
-        for (int g = 0; g < G; ++g) bx[0][g] = xs[buf * SLOTS + (g * 4) * 64 + lane];
-#pragma unroll
-        for (int st = 0; st < STEPS; ++st) {
-            const int u = st / NG, grp = st % NG;
-            if (st + 1 < STEPS) {
-                const int u1 = (st + 1) / NG, grp1 = (st + 1) % NG;
-#pragma unroll
-                for (int g = 0; g < G; ++g) bx[(st + 1) & 1][g] = xs[buf * SLOTS + ((grp1 * G + g) * 4 + u1) * 64 + lane];
-            }
-#pragma unroll
-            for (int g = 0; g < G; ++g)
-#pragma unroll
-                for (int t = 0; t < TN; ++t)
-                    acc[t][grp * G + g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][u], __builtin_bit_cast(bf16x8_t, bx[st & 1][g]),
-                                                                                  acc[t][grp * G + g], 0, 0, 0);
-            if constexpr (RING) {
-                if (grp == NG - 1) {
-                    const size_t at = (size_t)min(refill_c / 32 + u, K / 32 - 1) * 512;
-#pragma unroll
-                    for (int t = 0; t < TN; ++t) a[t][u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wtile[t] + at));      // read once
-                }
-                __builtin_amdgcn_sched_barrier(0);       // or the reads of many steps are issued at once and held
-            }
-        }
-    };
-
-    // Chunk j is multiplied while the weights of chunks j+1 and j+2 and x of chunk j+2 are on their
-    // way: what a step waits for was asked for two steps (weights) or one step (x, which comes
-    // from the cache) earlier.  Three register sets of weights, two of x and two LDS buffers take
-    // turns, so six steps are written out for the names to come round.
-    // With 8 row groups the registers hold one set of x only: the next chunk's x is asked for at the
-    // start of a step and stored at its end (XA = 1), and the weights go round as said above, in
-    // two sets with two tiles per wave, in three with one.
-    constexpr int XA = RING ? 1 : 2;
-    constexpr int WA = RING && TN > 1 ? 2 : 3;
-    bf16x8_t a[WA][TN][4];
-    u32x4_t xr[XA][XS];
-    load_w(k_begin, a[0]);
-    load_w(k_begin + MID_CHUNK, a[1]);
-    if constexpr (RING && WA == 3) load_w(k_begin + 2 * MID_CHUNK, a[WA - 1]);
-    load_x(k_begin, xr[0]);
-    if constexpr (XA == 2) load_x(k_begin + MID_CHUNK, xr[XA - 1]);
-    store_x(k_begin, 0, xr[0]);
-    __syncthreads();
-#define MID_STEP(J) { \
-        const int c = base + (J) * MID_CHUNK; \
-        load_x(c + XA * MID_CHUNK, xr[XA == 2 ? (J) % 2 : 0]); \
-        if constexpr (!RING) load_w(c + 2 * MID_CHUNK, a[((J) + 2) % WA]); \
-        __builtin_amdgcn_sched_barrier(0); \
-        multiply((J) % 2, a[(J) % WA], c + WA * MID_CHUNK); \
-        store_x(c + MID_CHUNK, ((J) + 1) % 2, xr[XA == 2 ? ((J) + 1) % 2 : 0]); \
-        __syncthreads(); }
-    int base = k_begin, left = (k_end - k_begin + MID_CHUNK - 1) / MID_CHUNK;
-    for (; left >= 6; left -= 6, base += 6 * MID_CHUNK) {
-        MID_STEP(0) MID_STEP(1) MID_STEP(2) MID_STEP(3) MID_STEP(4) MID_STEP(5)
-    }
-    if (left > 0) {
-        MID_STEP(0)
-        if (left > 1) {
-            MID_STEP(1)
-            if (left > 2) {
-                MID_STEP(2)
-                if (left > 3) {
-                    MID_STEP(3)
-                    if (left > 4) MID_STEP(4)
-                }
-            }
-        }
-    }
-#undef MID_STEP
-
+// What a wave does with its sums: acc[t][mt] holds row mt * 16 + lane % 16 and the four features 4 * (lane / 16) .. + 3 of tile t.
+template <int MT, int TN, int EPI, typename TY>
+__device__ __forceinline__ void mid_write(const MidArgs& p, floatx4_t (&acc)[TN][MT], int n_lo0, int n_out, int row, int kgrp) {
     const int nb = 4 * kgrp;
     if (gridDim.y > 1) {
         const bool vec = p.N % 4 == 0 && n_out % 4 == 0;           // the up rows' sums start at n_out
@@ -300,8 +125,14 @@ void mid_product_kernel(const MidArgs p) {
             const int n = n_lo0 + nb;
             if (m >= p.M) continue;
             float o[4];
+            // (which gate is asked once, not for every value)
+            if (p.gate == TQK_GATE_SILU) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) o[r] = gate_times_up(Gate{p.gate, p.gate_limit, p.gate_alpha, 0}, acc[0][mt][r], acc[TN - 1][mt][r]);
+                for (int r = 0; r < 4; ++r) o[r] = gate_times_up(Gate{TQK_GATE_SILU, 0.f, 1.f, 0}, acc[0][mt][r], acc[TN - 1][mt][r]);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[r] = gate_times_up(Gate{p.gate, p.gate_limit, p.gate_alpha, 0}, acc[0][mt][r], acc[TN - 1][mt][r]);
+            }
             bf16_t* dst = y + (size_t)m * n_out + n;
             if (vec && n + 3 < n_out) { *reinterpret_cast<uint2*>(dst) = pack4_bf16(o[0], o[1], o[2], o[3]); continue; }
 #pragma unroll
@@ -309,6 +140,132 @@ void mid_product_kernel(const MidArgs p) {
                 if (n + r < n_out) dst[r] = from_float<bf16_t>(o[r]);
         }
     }
+}
+
+// Stages of 64 k of x in LDS: as many as a wave's count of loads under way reaches, six at most.
+constexpr int mid_stages(int mt, int xw) { return 2 * mt / xw > 15 ? 5 : 6; }
+
+// MT: groups of 16 rows of x (2: up to 32 rows, 4: up to 64, 8: up to 128).  TN: tiles of 16 features per wave (gated: the gate tile and its up
+// tile).  XW waves of the block bring x in and do nothing else; WAVES others at most multiply.
+template <int MT, int TN, int EPI, typename TY, int XW, int WAVES>
+__global__ __launch_bounds__((WAVES + XW) * TQK_WAVE)
+void mid_product_kernel(const MidArgs p) {
+    constexpr int NS = mid_stages(MT, XW), STAGE = MT * 2048, DMA = 2 * MT / XW;
+    __shared__ __attribute__((aligned(1024))) char ring[NS * STAGE];        // [NS][rows][8 pieces of 16 bytes]
+    const int lane = threadIdx.x % TQK_WAVE, wv = __builtin_amdgcn_readfirstlane(threadIdx.x / TQK_WAVE);
+    const int n_waves = blockDim.x / TQK_WAVE - XW;
+    const int K = p.K;
+    const int k_begin = blockIdx.y * p.k_per_split, n_step = min(K - k_begin, p.k_per_split) / 32, n_stage = (n_step + 1) / 2;
+    if (wv >= n_waves) {
+        const bf16_t* px = p.x + k_begin;
+        if (EPI == MID_STORE && p.group_rows) px += (size_t)((int)blockIdx.x * n_waves * TN * 16 / p.group_rows) * p.x_group_stride;
+        const __amdgpu_buffer_rsrc_t x_mem = __builtin_amdgcn_make_buffer_rsrc((void*)px, 0, 0x7fffffff, 0x00020000);
+        const int xw = wv - n_waves;
+        uint32_t x_at[DMA];
+#pragma unroll
+        for (int i = 0; i < DMA; ++i) {
+            const int j = i * XW + xw;
+            x_at[i] = (uint32_t)min(j * 8 + lane / 8, p.M - 1) * (uint32_t)(K * 2) + ((lane % 8) ^ ((4 * (j % 2) + lane / 16) % 8)) * 16;
+        }
+        auto load = [&](int stage) {
+            char* to = ring + (stage % NS) * STAGE + xw * 1024;
+            if (2 * stage + 1 == n_step) {          // half a stage is left: the other half's pieces are the same again, and not read
+#pragma unroll
+                for (int i = 0; i < DMA; ++i) x_at[i] -= (((lane % 8) ^ ((4 * ((i * XW + xw) % 2) + lane / 16) % 8)) & 4) * 16;
+            }
+#pragma unroll
+            for (int i = 0; i < DMA; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(x_mem, (lds_ptr_t)(to + i * XW * 1024), 16, (int)x_at[i], stage * 128, 0, 0);
+        };
+        for (int s = 0; s < NS - 1 && s < n_stage; ++s) load(s);
+        for (int s = 0; s < n_stage; ++s) {
+            constexpr int left = (NS - 2) * DMA;
+            static_assert(left < 64, "");
+            if (s + NS - 1 <= n_stage) __builtin_amdgcn_s_waitcnt(0x0f70 | (left & 15) | ((left >> 4) << 14));
+            else __builtin_amdgcn_s_waitcnt(0x0f70);
+            __builtin_amdgcn_s_barrier();
+            if (s + NS - 1 < n_stage) load(s + NS - 1);         // into the place of stage s - 1, which everybody has read
+        }
+        return;
+    }
+
+    const int row = lane % 16, kgrp = lane / 16;
+    const int n_out = EPI == MID_GATED ? p.N / 2 : p.N;
+    const int part_tiles = (n_out + 15) / 16;
+    const int tile0 = (blockIdx.x * n_waves + wv) * (EPI == MID_GATED ? 1 : TN);
+    const int n_lo0 = tile0 * 16;
+    const size_t tile_size = (size_t)(K / 32) * 512;
+    const bf16_t* wtile[TN];
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+        const int tile = EPI == MID_GATED ? t * part_tiles + min(tile0, part_tiles - 1) : min(tile0 + t, part_tiles - 1);
+        wtile[t] = p.w + (size_t)tile * tile_size + (size_t)(k_begin / 32) * 512 + lane * 8;
+    }
+    floatx4_t acc[TN][MT];
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[t][mt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    constexpr int WD = TN > 2 ? 4 : 8;              // steps of 32 k of weights under way
+    bf16x8_t w[WD][TN];
+    auto load_w = [&](int step, int t) {
+        return __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wtile[t] + (size_t)min(step, n_step - 1) * 512));      // read once
+    };
+#pragma unroll
+    for (int s = 0; s < WD; ++s)
+#pragma unroll
+        for (int t = 0; t < TN; ++t) w[s][t] = load_w(s, t);
+
+    const int at0 = row * 128 + (kgrp ^ (row / 2)) * 16, at1 = at0 ^ 64;
+    const char* from = ring;
+    auto stage = [&](int s, int h, bool last) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");              // what LDS holds has changed
+        __builtin_amdgcn_sched_barrier(0);
+        // (both steps' operands are asked for together where the registers hold them)
+        constexpr bool BOTH = MT * TN < 16;
+        bf16x8_t x[2][MT];
+        auto read = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) x[u][mt] = *reinterpret_cast<const bf16x8_t*>(from + (u ? at1 : at0) + mt * 2048);
+        };
+        if (BOTH) {
+            read(0);
+            read(1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            if (!BOTH) read(u);
+            if (last && u == 1 && 2 * s + 1 == n_step) {         // K ends in the middle of the stage
+                const bf16x8_t none = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) x[u][mt] = none;
+#pragma unroll
+                for (int t = 0; t < TN; ++t) w[2 * h + u][t] = none;
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int t = 0; t < TN; ++t) acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[2 * h + u][t], x[u][mt], acc[t][mt], 0, 0, 0);
+            if (!last) {
+#pragma unroll
+                for (int t = 0; t < TN; ++t) w[2 * h + u][t] = load_w(2 * s + u + WD, t);
+            }
+        }
+        from = from == ring + (NS - 1) * STAGE ? ring : from + STAGE;
+    };
+    constexpr int H = WD / 2;
+    int s = 0;
+    for (; s + H <= n_step / 2; s += H) {
+#pragma unroll
+        for (int h = 0; h < H; ++h) stage(s + h, h, false);
+    }
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+        if (s + h < n_stage) stage(s + h, h, true);
+    mid_write<MT, TN, EPI, TY>(p, acc, n_lo0, n_out, row, kgrp);
 }
 
 // Adds the splits' sums in split order and finishes as the product kernel does without splits.
@@ -411,12 +368,8 @@ static size_t mid_scratch_bytes(int M, int N, int K, bool gated) {
     return splits > 1 && M > 0 ? (size_t)splits * M * N * sizeof(float) : 0;
 }
 
-template <int MT, int TN, int EPI, typename TY>
-static int launch_mid(const MidArgs& a, const MidPlan& plan, bool finish, hipStream_t s) {
-    dim3 grid(plan.blocks, plan.splits);
-    constexpr int PAR8 = (MT > 4) ? 2 : 1;
-    if (PAR8 == 2 && plan.waves == MID_MAX_WAVES) mid_product_kernel<MT, TN, EPI, TY, PAR8><<<grid, plan.waves * TQK_WAVE, 2 * MT * 256 * 16, s>>>(a);
-    else mid_product_kernel<MT, TN, EPI, TY, 1><<<grid, plan.waves * TQK_WAVE, 2 * MT * 256 * 16, s>>>(a);
+template <int EPI, typename TY>
+static int finish_mid(const MidArgs& a, const MidPlan& plan, bool finish, hipStream_t s) {
     if (tqk_check_launch("tqk_mid product")) return -1;
     if (plan.splits > 1 && finish) {
         const size_t total = (size_t)a.M * (EPI == MID_GATED ? a.N / 2 : a.N);
@@ -426,16 +379,52 @@ static int launch_mid(const MidArgs& a, const MidPlan& plan, bool finish, hipStr
     return 0;
 }
 
+template <int MT, int TN, int EPI, typename TY, int WAVES>
+static int launch_mid(const MidArgs& a, const MidPlan& plan, bool finish, hipStream_t s) {
+    constexpr int XW = MT > 4 && WAVES == MID_MAX_WAVES ? 2 : 1;
+    mid_product_kernel<MT, TN, EPI, TY, XW, WAVES><<<dim3(plan.blocks, plan.splits), (plan.waves + XW) * TQK_WAVE, 0, s>>>(a);
+    return finish_mid<EPI, TY>(a, plan, finish, s);
+}
+
+// The most tiles a wave takes of a wide product, and with how many waves beside it at most: as many as the registers hold with x's rows.
+template <int MT> struct MidWide { enum { tn = MT == 2 ? 5 : MT == 4 ? 6 : 3, waves = MT == 2 ? 8 : 7 }; };
+
+// Tiles per wave and waves per block of a product whose K is whole (a sum's order does not depend on them).  A block brings in all of x beside
+// its own weights, so what the busiest unit brings in is rounds of blocks times (tiles of a block + groups of rows of x), each 32 K bytes.
+// us at 32, 64 and 128 rows, against two tiles a wave and as many waves as leave the fewest units idle: the 7B head 194, 231, 236 -> 172, 178,
+// 219; the 1.5B one 89, 105, 115 -> 83, 91, 112; gate+up of the 1.5B shape (187 blocks of three waves for 140 of four) 15.7, 19.5, 25.9 ->
+// 12.8, 15.6, 21.6.
+static void mid_waves(MidPlan& plan, int N, bool gated, int mt, int wide_tn, int wide_waves) {
+    const int tiles = ((gated ? N / 2 : N) + 15) / 16;
+    int best = 1 << 30;
+    const int tns[3] = {1, 2, wide_tn};
+    for (int i = 0; i < (gated ? 1 : 3); ++i)
+        for (int waves = MID_LEAST_WAVES; waves <= (i == 2 ? wide_waves : MID_MAX_WAVES); ++waves) {
+            const int tn = gated ? 2 : tns[i];
+            const int items = gated ? tiles : (tiles + tn - 1) / tn, blocks = (items + waves - 1) / waves, rounds = (blocks + MID_UNITS - 1) / MID_UNITS;
+            const int cost = rounds * (waves * tn + mt);
+            if (cost < best) { best = cost; plan.tn = tn; plan.waves = waves; plan.blocks = blocks; }
+        }
+}
+
+template <int MT, int EPI, typename TY>
+static int launch_rows(const MidArgs& a, MidPlan plan, bool finish, hipStream_t s) {
+    constexpr int W = MID_MAX_WAVES;
+    constexpr bool GATED = EPI == MID_GATED;
+    using Wide = MidWide<MT>;
+    if (plan.splits == 1 && !a.group_rows) mid_waves(plan, a.N, GATED, MT, Wide::tn, Wide::waves);
+    if (GATED || plan.tn == 2) return launch_mid<MT, 2, EPI, TY, W>(a, plan, finish, s);
+    if constexpr (!GATED) {
+        if (plan.tn == Wide::tn) return launch_mid<MT, Wide::tn, EPI, TY, Wide::waves>(a, plan, finish, s);
+        return launch_mid<MT, 1, EPI, TY, W>(a, plan, finish, s);
+    }
+    return -1;
+}
+
 template <int EPI, typename TY>
 static int launch_rows(const MidArgs& a, const MidPlan& plan, bool finish, hipStream_t s) {
-    if constexpr (EPI == MID_GATED) {
-        if (a.M > 64) return launch_mid<8, 2, EPI, TY>(a, plan, finish, s);
-        return a.M > 32 ? launch_mid<4, 2, EPI, TY>(a, plan, finish, s) : launch_mid<2, 2, EPI, TY>(a, plan, finish, s);
-    } else {
-        if (a.M > 64) return plan.tn == 2 ? launch_mid<8, 2, EPI, TY>(a, plan, finish, s) : launch_mid<8, 1, EPI, TY>(a, plan, finish, s);
-        if (a.M > 32) return plan.tn == 2 ? launch_mid<4, 2, EPI, TY>(a, plan, finish, s) : launch_mid<4, 1, EPI, TY>(a, plan, finish, s);
-        return plan.tn == 2 ? launch_mid<2, 2, EPI, TY>(a, plan, finish, s) : launch_mid<2, 1, EPI, TY>(a, plan, finish, s);
-    }
+    if (a.M > 64) return launch_rows<8, EPI, TY>(a, plan, finish, s);
+    return a.M > 32 ? launch_rows<4, EPI, TY>(a, plan, finish, s) : launch_rows<2, EPI, TY>(a, plan, finish, s);
 }
 
 static int check_mid(const MidArgs& a, const void* scratch, bool gated, bool finish, const char* what) {
