@@ -325,7 +325,7 @@ def paged(k, v, page_ids, n_pages, dtype):
 
 
 @pytest.mark.parametrize("d,nh,nkv", [(128, 28, 4), (128, 12, 2), (64, 40, 2), (32, 3, 1), (96, 4, 4), (256, 2, 1)])
-@pytest.mark.parametrize("n_sums,with_bias,window,n_parts", [(1, True, 0, 1), (7, True, 0, 2), (4, False, 70, 3), (5, True, 0, 8)])
+@pytest.mark.parametrize("n_sums,with_bias,window,n_parts", [(1, True, 0, 1), (7, True, 0, 2), (4, False, 70, 3), (5, True, 0, 8), (9, False, 0, 3)])
 def test_decoding_attention_finishes_the_products_sums(d, nh, nkv, n_sums, with_bias, window, n_parts):
     """Against the rotation's kernel followed by the attention alone: the outputs and what lies in the cache.  Positions at the edges of pages,
     a row without earlier positions, heads in one group of 16 and in more, more partitions than pages."""

@@ -30,6 +30,7 @@
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
+typedef floatx4_t floatx4_any_t __attribute__((aligned(4)));         // at any float's address
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ int wave_of_block() { return threadIdx.x / TQK_WAVE; }
@@ -54,84 +55,120 @@ struct DecodeSums {
     bf16_t *keys, *values;          // the cache, to write
 };
 
-// Twice four values of the row, D / 2 apart, at their rounding to bfloat16 and the bias added: the pieces in their order, all of up to
-// eight under way together with the bias and the angles.
+// A block's part of that work: the queries of its heads (n_live of them from head0 on) into LDS, rows of D + 8, and the row's new key and value
+// behind them; where the block reads the row's own position (owner), also into the cache.  A job is twice four values, D / 2 apart, that
+// rotate with each other.  The first job's loads are issued by `ask`, so that a page's loads can be on their way behind them while the sums
+// are added up by `finish`: the block does not read what it writes to the cache, it takes the new key and value out of LDS.
 template <int D>
-__device__ __forceinline__ void finished8(const DecodeSums& in, size_t at, size_t feature, float (&lo)[4], float (&hi)[4]) {
-    constexpr int BATCH = 8;
-    uint2 b_lo = make_uint2(0, 0), b_hi = b_lo;
-    if (in.bias) {
-        b_lo = *reinterpret_cast<const uint2*>(in.bias + feature);
-        b_hi = *reinterpret_cast<const uint2*>(in.bias + feature + D / 2);
-    }
-    floatx4_t a = {0.f, 0.f, 0.f, 0.f}, b = a;
-    for (int s = 0; s < in.n; s += BATCH) {
-        floatx4_t pa[BATCH], pb[BATCH];
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u) {
-            const float* src = in.sums + (size_t)min(s + u, in.n - 1) * in.stride + at;
-            pa[u] = *reinterpret_cast<const floatx4_t*>(src);
-            pb[u] = *reinterpret_cast<const floatx4_t*>(src + D / 2);
-        }
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u) {
-            const bool there = s + u < in.n;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) { a[k] = there ? a[k] + pa[u][k] : a[k]; b[k] = there ? b[k] + pb[u][k] : b[k]; }
-        }
-    }
-    const float bias_lo[4] = {__uint_as_float(b_lo.x << 16), __uint_as_float(b_lo.x & 0xffff0000u), __uint_as_float(b_lo.y << 16), __uint_as_float(b_lo.y & 0xffff0000u)};
-    const float bias_hi[4] = {__uint_as_float(b_hi.x << 16), __uint_as_float(b_hi.x & 0xffff0000u), __uint_as_float(b_hi.y << 16), __uint_as_float(b_hi.y & 0xffff0000u)};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        lo[k] = to_float(from_float<bf16_t>(a[k]));
-        hi[k] = to_float(from_float<bf16_t>(b[k]));
-        if (in.bias) { lo[k] += bias_lo[k]; hi[k] += bias_hi[k]; }
-    }
-}
+struct RowFinish {
+    static constexpr int PER = D / 8, BATCH = 8;
+    const DecodeSums& in;
+    const int seq, head0, n_live, kvh, n_heads, n_kv_heads;
+    uint2 b_lo, b_hi;
+    floatx4_t pa[BATCH], pb[BATCH];
 
-// A block's part of that work: the queries of its heads (n_live of them from head0 on) into LDS, rows of D + 8; and where the block reads the
-// row's own position (owner), the position's key and value into the cache.  (Blocks that share a kv head and a page write the
-// same values; each reads its own writes, behind a barrier.)
-template <int D>
-__device__ __forceinline__ void finish_row(const DecodeSums& in, int seq, int pos, int page, bool owner, int head0, int n_live, int kvh, int n_heads,
-                                           int n_kv_heads, bf16_t* q_lds) {
-    constexpr int PER = D / 8;          // pieces of four and four values, half a head apart, that rotate with each other
-    const size_t row = (size_t)seq * (n_heads + 2 * n_kv_heads) * D;
-    const int jobs = (n_live + (owner ? 2 : 0)) * PER;
-    for (int job = threadIdx.x; job < jobs; job += blockDim.x) {
-        const int which = job / PER, i = (job % PER) * 4;
-        const int kind = which < n_live ? 0 : which - n_live + 1;
-        const size_t feature = (size_t)(kind == 0 ? head0 + which : n_heads + (kind - 1) * n_kv_heads + kvh) * D + i;
-        float lo[4], hi[4];
-        const size_t angle = (size_t)min(pos, in.max_positions - 1) * (D / 2) + i;
-        const float4 c4 = *reinterpret_cast<const float4*>(in.cos_table + angle), s4 = *reinterpret_cast<const float4*>(in.sin_table + angle);
-        finished8<D>(in, row + feature, feature, lo, hi);
-        if (kind != 2 && pos < in.max_positions) {
-            const float c[4] = {c4.x, c4.y, c4.z, c4.w}, sn[4] = {s4.x, s4.y, s4.z, s4.w};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) rotate_pair(lo[k], hi[k], c[k], sn[k]);
-        }
-        uint32_t l[4], h[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) { l[k] = float_to_bf16_bits(lo[k]); h[k] = float_to_bf16_bits(hi[k]); }
-        if (kind == 2) {
-            bf16_t* dst = in.values + ((size_t)page * n_kv_heads + kvh) * TQK_PAGE * D + value_place(pos % TQK_PAGE);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                dst[(size_t)(i + k) * TQK_PAGE].bits = (uint16_t)l[k];
-                dst[(size_t)(i + D / 2 + k) * TQK_PAGE].bits = (uint16_t)h[k];
+    __device__ __forceinline__ size_t feature_of(int job) const {
+        const int which = min(job / PER, n_live + 1), i = (job % PER) * 4;
+        return (size_t)(which < n_live ? head0 + which : n_heads + (which - n_live) * n_kv_heads + kvh) * D + i;
+    }
+    // the bias and up to eight pieces, all under way together
+    __device__ __forceinline__ void ask(int job, int s0) {
+        const size_t feature = feature_of(job), at = (size_t)seq * (n_heads + 2 * n_kv_heads) * D + feature;
+        if (s0 == 0) {
+            b_lo = b_hi = make_uint2(0, 0);
+            if (in.bias) {
+                b_lo = *reinterpret_cast<const uint2*>(in.bias + feature);
+                b_hi = *reinterpret_cast<const uint2*>(in.bias + feature + D / 2);
             }
-            continue;
         }
-        bf16_t* dst = kind == 0 ? q_lds + which * (D + 8) : in.keys + (((size_t)page * n_kv_heads + kvh) * TQK_PAGE + pos % TQK_PAGE) * D;
-        *reinterpret_cast<uint2*>(dst + i) = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
-        *reinterpret_cast<uint2*>(dst + i + D / 2) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+        auto half = [&](int u0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = u0; u < u0 + BATCH / 2; ++u) {
+                const float* src = in.sums + (size_t)min(s0 + u, in.n - 1) * in.stride + at;
+                pa[u] = *reinterpret_cast<const floatx4_t*>(src);
+                pb[u] = *reinterpret_cast<const floatx4_t*>(src + D / 2);
+            }
+        };
+        half(0);
+        if (s0 + BATCH / 2 < in.n) half(BATCH / 2);
     }
-    __builtin_amdgcn_s_waitcnt(0x0f70);         // the writes have left for the memory that the block's loads come from
-    __syncthreads();
-}
+    // the values at their rounding to bfloat16 and the bias added: the pieces in their order
+    __device__ __forceinline__ void sum(int job, float (&lo)[4], float (&hi)[4]) {
+        floatx4_t a = {0.f, 0.f, 0.f, 0.f}, b = a;
+        auto add = [&](int s) {
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u) {
+                const bool there = s + u < in.n;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) { a[k] = there ? a[k] + pa[u][k] : a[k]; b[k] = there ? b[k] + pb[u][k] : b[k]; }
+            }
+        };
+        add(0);
+        for (int s = BATCH; s < in.n; s += BATCH) {
+            ask(job, s);
+            add(s);
+        }
+        const float bias_lo[4] = {__uint_as_float(b_lo.x << 16), __uint_as_float(b_lo.x & 0xffff0000u), __uint_as_float(b_lo.y << 16), __uint_as_float(b_lo.y & 0xffff0000u)};
+        const float bias_hi[4] = {__uint_as_float(b_hi.x << 16), __uint_as_float(b_hi.x & 0xffff0000u), __uint_as_float(b_hi.y << 16), __uint_as_float(b_hi.y & 0xffff0000u)};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            lo[k] = to_float(from_float<bf16_t>(a[k]));
+            hi[k] = to_float(from_float<bf16_t>(b[k]));
+            if (in.bias) { lo[k] += bias_lo[k]; hi[k] += bias_hi[k]; }
+        }
+    }
+    // (c4, s4: the angles of the first job, asked for before)
+    __device__ __forceinline__ void finish(int pos, int page, bool owner, float4 c4, float4 s4, bf16_t* q_lds, bf16_t* new_lds) {
+        const int jobs = (n_live + (owner ? 2 : 0)) * PER;
+        auto one = [&](int job) __attribute__((always_inline)) {
+            const int which = job / PER, i = (job % PER) * 4;
+            const int kind = which < n_live ? 0 : which - n_live + 1;
+            float lo[4], hi[4];
+            sum(job, lo, hi);
+            if (kind != 2 && pos < in.max_positions) {
+                const float c[4] = {c4.x, c4.y, c4.z, c4.w}, sn[4] = {s4.x, s4.y, s4.z, s4.w};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) rotate_pair(lo[k], hi[k], c[k], sn[k]);
+            }
+            uint32_t l[4], h[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { l[k] = float_to_bf16_bits(lo[k]); h[k] = float_to_bf16_bits(hi[k]); }
+            const uint2 l4 = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16)), h4 = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+            bf16_t* dst = kind == 0 ? q_lds + which * (D + 8) : new_lds + (kind - 1) * D;
+            *reinterpret_cast<uint2*>(dst + i) = l4;
+            *reinterpret_cast<uint2*>(dst + i + D / 2) = h4;
+            // (blocks that share a kv head and a page write the same values)
+            if (kind == 1) {
+                bf16_t* key = in.keys + (((size_t)page * n_kv_heads + kvh) * TQK_PAGE + pos % TQK_PAGE) * D;
+                *reinterpret_cast<uint2*>(key + i) = l4;
+                *reinterpret_cast<uint2*>(key + i + D / 2) = h4;
+            } else if (kind == 2) {
+                bf16_t* value = in.values + ((size_t)page * n_kv_heads + kvh) * TQK_PAGE * D + value_place(pos % TQK_PAGE);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    value[(size_t)(i + k) * TQK_PAGE].bits = (uint16_t)l[k];
+                    value[(size_t)(i + D / 2 + k) * TQK_PAGE].bits = (uint16_t)h[k];
+                }
+            }
+        };
+        if ((int)threadIdx.x < jobs) one(threadIdx.x);          // (apart, so that its waits are counted and leave a page's loads under way)
+        for (int job = threadIdx.x + blockDim.x; job < jobs; job += blockDim.x) {
+            ask(job, 0);
+            const size_t angle = (size_t)min(pos, in.max_positions - 1) * (D / 2) + (job % PER) * 4;
+            c4 = *reinterpret_cast<const float4*>(in.cos_table + angle);
+            s4 = *reinterpret_cast<const float4*>(in.sin_table + angle);
+            one(job);
+        }
+        __syncthreads();
+    }
+};
 
+// With a page or two a wave the kernel is bound by what a block does one thing after the other, not by bytes.  Stamps of one launch (32 rows of up to
+// 1024 positions, 12 heads on 2, sums of 3 pieces, us from its start, the last block): position known 1.9, loads asked for 5.6, sums finished
+// 6.5, page there 7.1, page done 8.7, written 9.8.  A page that is not whole took 4 us longer while each of its values was compared with the
+// positions (bits to keep are found once for all elements now), the sums 1.3 in front of the page's loads instead of over them, and the
+// waves' results 1.3 when one wave added up all of them.  ms a step, together: 7B, 1, 8 and 64 sequences 2.882 -> 2.832, 3.130 -> 3.058 and
+// 3.921 -> 3.793; 1.5B, 32 sequences 1.766 -> 1.657; 32B with 8 layers, 16 sequences 1.843 -> 1.816.
 // SUMS: q, k and v come as `in` and are finished here (keys and values are then written, too, so nothing promises that they are not).
 template <int D, bool NT, int W, bool SUMS>
 __global__ __launch_bounds__(AD_WAVES * TQK_WAVE)
@@ -143,23 +180,34 @@ void attention_decode_kernel(const DecodeSums in, const bf16_t* __restrict__ q, 
                              bf16_t* __restrict__ out) {
     constexpr int KB = D / 32;          // k-blocks of the score product
     constexpr int DB = D / 16;          // 16-element blocks of the output
-    constexpr int ROW = DB * 4 + 2;     // floats a lane hands over: its out^T values, m, l
     // Head size 128: a page comes in with loads of 1 KB of contiguous memory each and goes through LDS into the matrix
     // cores' order, a region of 16 KB per wave (see below); the waves' results change hands through the same memory.
     // (Worth it where the step reads so much that the memory's rate counts, which is where the loads are marked as
     // read-once, NT: 64 sequences of 2100 positions 56.2 -> 49.7 us, 128 sequences 106 -> 89 us; 8 sequences 13.2 -> 14.2.)
     constexpr bool VIA_LDS = D == 128 && NT;
-    constexpr int XCH = (W > 1 ? W - 1 : 1) * TQK_WAVE * ROW;
-    constexpr int TURN = VIA_LDS ? W * 4096 : 0;                 // floats: 1024 pieces of 16 bytes a wave
-    __shared__ __attribute__((aligned(16))) float lds_all[XCH > TURN ? XCH : TURN];
-    float* const xch = lds_all;
-    u32x4_t* const turn = reinterpret_cast<u32x4_t*>(lds_all) + wave_of_block() * 1024;
-    const int wave = threadIdx.x / TQK_WAVE, lane = threadIdx.x % TQK_WAVE;
+    constexpr bool EARLY = SUMS && D <= 128;           // the first page is asked for while the sums are added up: where the registers hold both
+    constexpr int XCH_WAVE = DB * TQK_WAVE + TQK_WAVE / 2;      // pieces of 16 bytes a wave hands over: its out^T values, m, l
+    constexpr int XCH = W > 1 ? W * XCH_WAVE : 1, TURN = VIA_LDS ? W * 1024 : 0;
+    __shared__ u32x4_t lds_all[XCH > TURN ? XCH : TURN];
+    floatx4_t* const xch = reinterpret_cast<floatx4_t*>(lds_all);
+    u32x4_t* const turn = lds_all + wave_of_block() * 1024;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TQK_WAVE), lane = threadIdx.x % TQK_WAVE;
     const int col = lane % 16, g = lane / 16;
     const int part = blockIdx.x;
     const int kvh = blockIdx.y / q_blocks, qb = blockIdx.y % q_blocks;
     const int seq = blockIdx.z;
     const int n_rep = n_heads / n_kv_heads;
+    // What a block waits for before its pages is a chain of loads that miss all caches, about a microsecond each, so nothing waits that need not:
+    // without a window the wave's first page is asked for together with the position, and the sums before both.
+    const int32_t* pages = page_table + (size_t)seq * table_width;
+    int page = 0;
+    if (window == 0) page = __builtin_amdgcn_readfirstlane(pages[min(part + wave * n_parts, table_width - 1)]);
+    __shared__ __attribute__((aligned(16))) bf16_t q_lds[SUMS ? 16 * (D + 8) : 8], new_lds[SUMS ? 2 * D : 8];
+    RowFinish<SUMS ? D : 32> finish = {in, seq, kvh * n_rep + qb * 16, min(16, n_rep - qb * 16), kvh, n_heads, n_kv_heads};
+    if constexpr (EARLY) {
+        finish.ask(threadIdx.x, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    }
     const int pos = __builtin_amdgcn_readfirstlane(tok_pos[seq]);
     const int lo = window > 0 ? max(0, pos - window + 1) : 0;
     // exponentials to base 2 (one instruction each): the scores carry log2(e), and so do the running
@@ -171,22 +219,59 @@ void attention_decode_kernel(const DecodeSums in, const bf16_t* __restrict__ q, 
     const bool head_live = rep < n_rep;
     const int head = kvh * n_rep + (head_live ? rep : 0);
 
-    const int last_page = pos / TQK_PAGE;
-    const int start_page = lo / TQK_PAGE + part + wave * n_parts;       // this wave's first page
+    const int first_page = lo / TQK_PAGE, last_page = pos / TQK_PAGE;
+    const int start_page = first_page + part + wave * n_parts;          // this wave's first page
+    if (window > 0) page = __builtin_amdgcn_readfirstlane(pages[min(start_page, table_width - 1)]);
 
     float m = -INFINITY, l = 0.f;
     floatx4_t o[DB];
 #pragma unroll
     for (int i = 0; i < DB; ++i) o[i] = floatx4_t{0.f, 0.f, 0.f, 0.f};
 
-    __shared__ __attribute__((aligned(16))) bf16_t q_lds[SUMS ? 16 * (D + 8) : 8];
-    if constexpr (SUMS) {
-        const int first_page = lo / TQK_PAGE;
-        if (first_page + part <= last_page) {           // (the same for the block: one without pages has nothing to finish)
-            const int page = __builtin_amdgcn_readfirstlane(page_table[(size_t)seq * table_width + last_page]);
-            const bool owner = (last_page - first_page) % n_parts == part && page >= 0;
-            finish_row<D>(in, seq, pos, page, owner, kvh * n_rep + qb * 16, min(16, n_rep - qb * 16), kvh, n_heads, n_kv_heads, q_lds);
+    // all of a page's loads together, so that they are in flight together
+    bf16x8_t ka[4][KB], va[DB][2];
+    u32x4_t kr[VIA_LDS ? 16 : 1], vr[VIA_LDS ? 16 : 1];
+    auto load_page = [&](int page, int lane) __attribute__((always_inline)) {
+        const int col = lane % 16, g = lane / 16;
+        const size_t at = ((size_t)page * n_kv_heads + kvh) * TQK_PAGE * D;
+        const bf16_t *kp = keys + at, *vp = values + at;
+        if constexpr (VIA_LDS) {
+            // A load of a wave takes 1 KB of contiguous memory (four key rows, eight value rows): the memory serves
+            // such loads at 6.9 TB/s and loads of 64 bytes out of each of 16 rows, which is what the matrix cores'
+            // order asks of a page as it lies in the cache, at 5.9.  The pieces of 16 bytes then go through the wave's
+            // region of LDS to the lanes that need them, XOR-swizzled so that neither the writes nor the reads meet
+            // a bank twice: the keys first, and the values through the same region once the scores are done.
+            const u32x4_t* kg = reinterpret_cast<const u32x4_t*>(kp) + lane;
+            const u32x4_t* vg = reinterpret_cast<const u32x4_t*>(vp) + lane;
+#pragma unroll
+            for (int j = 0; j < 16; ++j) kr[j] = __builtin_nontemporal_load(kg + j * 64);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) vr[j] = __builtin_nontemporal_load(vg + j * 64);
+        } else {
+            auto load = [](const bf16_t* p) { return NT ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(p)) : *reinterpret_cast<const bf16x8_t*>(p); };
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int kb = 0; kb < KB; ++kb) ka[t][kb] = load(kp + (size_t)(t * 16 + col) * D + kb * 32 + g * 8);
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+#pragma unroll
+                for (int pr = 0; pr < 2; ++pr) va[db][pr] = load(vp + (size_t)(db * 16 + col) * TQK_PAGE + pr * 32 + g * 8);
         }
+    };
+
+    if constexpr (SUMS) {
+        const int row_page = __builtin_amdgcn_readfirstlane(pages[last_page]);
+        const size_t angle = (size_t)min(pos, in.max_positions - 1) * (D / 2) + (threadIdx.x % (D / 8)) * 4;
+        const float4 c4 = *reinterpret_cast<const float4*>(in.cos_table + angle), s4 = *reinterpret_cast<const float4*>(in.sin_table + angle);
+        __builtin_amdgcn_sched_barrier(0);
+        if (!EARLY) finish.ask(threadIdx.x, 0);
+        // (a wave without a page asks for a few lines of some page, so that the count of loads under way is the same)
+        const bool live = start_page <= last_page && page >= 0;
+        if (EARLY) load_page(live ? page : 0, live ? lane : 0);
+        __builtin_amdgcn_sched_barrier(0);
+        const bool owner = (last_page - first_page) % n_parts == part && row_page >= 0;
+        finish.finish(pos, row_page, owner, c4, s4, q_lds, new_lds);
     }
 
     if (start_page <= last_page) {
@@ -199,32 +284,18 @@ void attention_decode_kernel(const DecodeSums in, const bf16_t* __restrict__ q, 
         for (int kb = 0; kb < KB; ++kb)
             bq[kb] = head_live ? *reinterpret_cast<const bf16x8_t*>(SUMS ? q_lds + col * (D + 8) + g * 8 + kb * 32 : qrow + kb * 32) : zero.v;
 
-        const int32_t* pages = page_table + (size_t)seq * table_width;
-        const size_t page_stride = (size_t)n_kv_heads * TQK_PAGE * D;
         for (int pg = start_page; pg <= last_page; pg += W * n_parts) {
-            const int page = __builtin_amdgcn_readfirstlane(pages[pg]);        // the same in all lanes: the page's address is then a scalar
-            if (page < 0) continue;                     // the host never lets this happen
-            const bf16_t* kp = keys + (size_t)page * page_stride + (size_t)kvh * TQK_PAGE * D;
-            const bf16_t* vp = values + (size_t)page * page_stride + (size_t)kvh * TQK_PAGE * D;
+            const int next_pg = pg + W * n_parts;
+            const int next = __builtin_amdgcn_readfirstlane(pages[min(next_pg, last_page)]);        // the same in all lanes: the page's address is then a scalar
+            const int here = page;
+            page = next;
+            if (here < 0) continue;                     // the host never lets this happen
+            if (!EARLY || pg != start_page) load_page(here, lane);
             const int key0 = pg * TQK_PAGE;
-            const bool edge = key0 < lo || key0 + TQK_PAGE - 1 > pos;
+            const bool newest = SUMS && pg == last_page;            // its last key and value are those that the block has finished itself
+            const bool edge = newest || key0 < lo || key0 + TQK_PAGE - 1 > pos;
 
-            // all of the page's loads first, so that they are in flight together
-            bf16x8_t ka[4][KB], va[DB][2];
-            u32x4_t vr[VIA_LDS ? 16 : 1];
             if constexpr (VIA_LDS) {
-                // A load of a wave takes 1 KB of contiguous memory (four key rows, eight value rows): the memory serves
-                // such loads at 6.9 TB/s and loads of 64 bytes out of each of 16 rows, which is what the matrix cores'
-                // order asks of a page as it lies in the cache, at 5.9.  The pieces of 16 bytes then go through the wave's
-                // region of LDS to the lanes that need them, XOR-swizzled so that neither the writes nor the reads meet
-                // a bank twice: the keys first, and the values through the same region once the scores are done.
-                const u32x4_t* kg = reinterpret_cast<const u32x4_t*>(kp) + lane;
-                const u32x4_t* vg = reinterpret_cast<const u32x4_t*>(vp) + lane;
-                u32x4_t kr[16];
-#pragma unroll
-                for (int j = 0; j < 16; ++j) kr[j] = NT ? __builtin_nontemporal_load(kg + j * 64) : kg[j * 64];
-#pragma unroll
-                for (int j = 0; j < 16; ++j) vr[j] = NT ? __builtin_nontemporal_load(vg + j * 64) : vg[j * 64];
 #pragma unroll
                 for (int j = 0; j < 16; ++j) {
                     const int key = 4 * j + lane / 16, oct = lane % 16;
@@ -240,17 +311,16 @@ void attention_decode_kernel(const DecodeSums in, const bf16_t* __restrict__ q, 
                         ka[t][kb] = __builtin_bit_cast(bf16x8_t, piece);
                     }
                 __builtin_amdgcn_wave_barrier();
-            } else {
+            }
+            if (newest) {
+                const int at = pos % TQK_PAGE;
 #pragma unroll
-                for (int t = 0; t < 4; ++t)
+                for (int kb = 0; kb < KB; ++kb) {
+                    const bf16x8_t k = *reinterpret_cast<const bf16x8_t*>(new_lds + kb * 32 + g * 8);
 #pragma unroll
-                    for (int kb = 0; kb < KB; ++kb)
-                        ka[t][kb] = NT ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(kp + (size_t)(t * 16 + col) * D + kb * 32 + g * 8)) : *reinterpret_cast<const bf16x8_t*>(kp + (size_t)(t * 16 + col) * D + kb * 32 + g * 8);
-#pragma unroll
-                for (int db = 0; db < DB; ++db)
-#pragma unroll
-                    for (int pr = 0; pr < 2; ++pr)
-                        va[db][pr] = NT ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(vp + (size_t)(db * 16 + col) * TQK_PAGE + pr * 32 + g * 8)) : *reinterpret_cast<const bf16x8_t*>(vp + (size_t)(db * 16 + col) * TQK_PAGE + pr * 32 + g * 8);
+                    for (int t = 0; t < 4; ++t)
+                        if (at == t * 16 + col) ka[t][kb] = k;
+                }
             }
 
             // scores^T for the page's four groups of 16 keys
@@ -319,73 +389,101 @@ void attention_decode_kernel(const DecodeSums in, const bf16_t* __restrict__ q, 
                     }
                 __builtin_amdgcn_wave_barrier();
             }
+            if (edge) {
+                // Which of a lane's values count, and which one is the new one, is the same for all elements of the head, so it is found once, as
+                // bits to keep and to put in pairs of values.
+                uint32_t keep[2][4], put[2][4];
+#pragma unroll
+                for (int pr = 0; pr < 2; ++pr)
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        const int j = key0 + (2 * pr + w / 2) * 16 + g * 4 + 2 * (w % 2);
+                        const int in0 = j >= lo && j <= pos, in1 = j + 1 >= lo && j + 1 <= pos;
+                        put[pr][w] = !newest ? 0u : j == pos ? 0xffffu : j + 1 == pos ? 0xffff0000u : 0u;
+                        keep[pr][w] = ((in0 ? 0xffffu : 0u) | (in1 ? 0xffff0000u : 0u)) & ~put[pr][w];
+                    }
+#pragma unroll
+                for (int db = 0; db < DB; ++db) {
+                    const uint32_t v = SUMS ? new_lds[D + db * 16 + col].bits * 0x10001u : 0u;
+#pragma unroll
+                    for (int pr = 0; pr < 2; ++pr) {
+                        u32x4_t u = __builtin_bit_cast(u32x4_t, va[db][pr]);
+#pragma unroll
+                        for (int w = 0; w < 4; ++w) u[w] = (u[w] & keep[pr][w]) | (SUMS ? v & put[pr][w] : 0u);
+                        va[db][pr] = __builtin_bit_cast(bf16x8_t, u);
+                    }
+                }
+            }
 #pragma unroll
             for (int db = 0; db < DB; ++db) {
                 o[db][0] *= alpha; o[db][1] *= alpha; o[db][2] *= alpha; o[db][3] *= alpha;
 #pragma unroll
-                for (int pr = 0; pr < 2; ++pr) {
-                    pack8 av;
-                    av.v = va[db][pr];
-                    if (edge) {
-#pragma unroll
-                        for (int i = 0; i < 8; ++i) {
-                            const int j = key0 + (2 * pr + i / 4) * 16 + g * 4 + (i % 4);
-                            if (j < lo || j > pos) av.u[i] = 0;
-                        }
-                    }
-                    o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av.v, pb[pr].v, o[db], 0, 0, 0);
-                }
+                for (int pr = 0; pr < 2; ++pr) o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[db][pr], pb[pr].v, o[db], 0, 0, 0);
             }
         }
         l += __shfl_xor(l, 16, TQK_WAVE);
         l += __shfl_xor(l, 32, TQK_WAVE);
     }
 
-    // the waves' results into wave 0, in wave order
-    if (VIA_LDS && W > 1) __syncthreads();          // (the memory they change hands through is the regions of the pages)
-    if (wave > 0) {
-        float* mine = xch + ((size_t)(wave - 1) * TQK_WAVE + lane) * ROW;
+    // The waves' results meet in wave order, each wave taking its share of the elements.
+    if constexpr (W > 1) {
+        if (VIA_LDS) __syncthreads();               // (the memory they change hands through is the regions of the pages)
+        floatx4_t* mine = xch + (size_t)wave * XCH_WAVE + lane;
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) mine[db * 4 + r] = o[db][r];
-        mine[DB * 4] = m;
-        mine[DB * 4 + 1] = l;
+        for (int db = 0; db < DB; ++db) mine[db * TQK_WAVE] = o[db];
+        float* ml = reinterpret_cast<float*>(xch + (size_t)wave * XCH_WAVE + DB * TQK_WAVE);
+        ml[lane] = m;
+        ml[TQK_WAVE + lane] = l;
+        __syncthreads();
     }
-    __syncthreads();
     const size_t row = ((size_t)seq * n_heads + head) * n_parts + part;
-    if (wave == 0) {
+    bool some[W];                                   // whether a wave had a page
+    float of_others[W], of_sum[W];                  // what the sum so far and the wave's are multiplied by
+    if constexpr (W > 1) {
+        const float* ml = reinterpret_cast<const float*>(xch + DB * TQK_WAVE) + lane;
+        m = ml[0];
+        l = ml[TQK_WAVE];
+#pragma unroll
         for (int w = 1; w < W; ++w) {
-            const float* theirs = xch + ((size_t)(w - 1) * TQK_WAVE + lane) * ROW;
-            const float m2 = theirs[DB * 4], l2 = theirs[DB * 4 + 1];
-            if (m2 == -INFINITY) continue;
+            const float m2 = ml[(size_t)w * XCH_WAVE * 4], l2 = ml[(size_t)w * XCH_WAVE * 4 + TQK_WAVE];
             const float mn = fmaxf(m, m2);
-            const float a1 = __builtin_amdgcn_exp2f(m - mn), a2 = __builtin_amdgcn_exp2f(m2 - mn);
-#pragma unroll
-            for (int db = 0; db < DB; ++db)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) o[db][r] = o[db][r] * a1 + theirs[db * 4 + r] * a2;
-            l = l * a1 + l2 * a2;
+            some[w] = m2 != -INFINITY;
+            of_sum[w] = __builtin_amdgcn_exp2f(m - mn);
+            of_others[w] = __builtin_amdgcn_exp2f(m2 - mn);
+            if (!some[w]) continue;
+            l = l * of_sum[w] + l2 * of_others[w];
             m = mn;
         }
-        if (!head_live) return;
+    }
+    if (!head_live) return;
+#pragma unroll
+    for (int d0 = 0; d0 < DB; d0 += W) {
+        const int db = d0 + (W > 1 ? wave : 0);
+        if (DB % W != 0 && db >= DB) break;
+        floatx4_t v = o[d0];
+        if constexpr (W > 1) {
+            const floatx4_t* from = xch + (size_t)db * TQK_WAVE + lane;
+            v = from[0];
+#pragma unroll
+            for (int w = 1; w < W; ++w) {
+                const floatx4_t theirs = from[(size_t)w * XCH_WAVE];
+                if (some[w]) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] = v[r] * of_sum[w] + theirs[r] * of_others[w];
+                }
+            }
+        }
         if (n_parts == 1) {
             // the only partition: this is the result, out[head, element db*16 + 4g + r]
-            bf16_t* po = out + ((size_t)seq * n_heads + head) * D;
+            bf16_t* po = out + ((size_t)seq * n_heads + head) * D + db * 16 + g * 4;
             const float inv = 1.f / l;
 #pragma unroll
-            for (int db = 0; db < DB; ++db)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) po[db * 16 + g * 4 + r] = from_float<bf16_t>(o[db][r] * inv);
+            for (int r = 0; r < 4; ++r) po[r] = from_float<bf16_t>(v[r] * inv);
         } else {
-            float* po = part_out + row * D;
-#pragma unroll
-            for (int db = 0; db < DB; ++db)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) po[db * 16 + g * 4 + r] = o[db][r];
-            if (g == 0) { part_ml[row * 2] = m; part_ml[row * 2 + 1] = l; }
+            *reinterpret_cast<floatx4_any_t*>(part_out + row * D + db * 16 + g * 4) = v;
         }
     }
+    if (n_parts > 1 && wave == 0 && g == 0) { part_ml[row * 2] = m; part_ml[row * 2 + 1] = l; }
 }
 
 // out[seq, head, :] = sum_p exp(m_p - M) o_p / sum_p exp(m_p - M) l_p, partitions in order.
