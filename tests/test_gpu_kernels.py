@@ -800,6 +800,24 @@ def test_unfinished_sums_of_a_product_are_finished_by_the_next_norm(m, n, k):
     torch.testing.assert_close(n1.float(), n2.float(), atol=1e-3, rtol=2 ** -7)
 
 
+@pytest.mark.parametrize("rows", [3, 64, 65])
+@pytest.mark.parametrize("hidden,n_sums", [(4, 1), (68, 5), (1536, 14), (3584, 16), (3584, 17), (4096, 4), (4100, 9), (5120, 8), (8192, 33)])
+def test_the_norm_adds_up_any_number_of_pieces(rows, hidden, n_sums):
+    """Against the pieces added in order in float32, rounded and given as a plain update: more and fewer pieces than are under way together, rows
+    that end within a wave and rows of more values than a block has threads for, both sides of the rule by rows."""
+    sums, h = rand(n_sums, rows, hidden, seed=90), rand(rows, hidden, seed=91, scale=2.0)
+    nw = (1 + rand(hidden, seed=92, scale=0.1)).to(torch.bfloat16)
+    total = torch.zeros_like(sums[0])
+    for piece in sums:
+        total += piece
+    h1, h2 = h.clone(), h.clone()
+    out1 = K.add_rmsnorm(h1, total.to(torch.bfloat16), nw, 1e-6, torch.empty(rows, hidden, dtype=torch.bfloat16, device=DEV), write_back=True)
+    out2 = K.add_rmsnorm(h2, K.PartialSums(sums, torch.bfloat16), nw, 1e-6, torch.empty(rows, hidden, dtype=torch.bfloat16, device=DEV), write_back=True)
+    assert torch.equal(h1, h2)
+    # the squares are added in another order, so a value may round to its neighbour: a step of bfloat16 is at most 2^-7 of it
+    assert ((out1.float() - out2.float()).abs() <= out1.float().abs() * 2 ** -7).all()
+
+
 @pytest.mark.parametrize("nh,nkv,d,k", [(28, 4, 128, 3584), (3, 1, 32, 2048), (6, 2, 64, 1056)])
 def test_unfinished_sums_of_q_k_v_are_finished_by_the_rotation_kernel(nh, nkv, d, k):
     m, n_pages = 20, 24

@@ -133,6 +133,41 @@ extern "C" int tqk_finish_logits(float* logits, int n_rows, int vocab, const flo
 // added as any other update: the product's own finishing pass and its round trip disappear.
 struct PartSums { const float* sums; int n; size_t stride; };       // stride: rows * hidden
 
+// Four values of each piece, up to MAX pieces under way together: the small kernels that add pieces up are bound by how many loads they
+// wait for one after the other (each misses every cache, about a microsecond), so they ask for all pieces at once, together with whatever
+// else they need, and look at them afterwards.
+template <int MAX>
+struct Pieces {
+    float4 p[MAX];
+    __device__ __forceinline__ void ask(const PartSums& ps, size_t at, int s0) {
+        const float* from = ps.sums + (size_t)s0 * ps.stride + at;
+#pragma unroll
+        for (int u = 0; u < MAX; ++u) {
+            if (s0 + u >= ps.n) break;              // (none is read that is not there: many rows are bound by bytes)
+            p[u] = *reinterpret_cast<const float4*>(from + (size_t)u * ps.stride);
+        }
+    }
+    // added in their order
+    __device__ __forceinline__ void add(const PartSums& ps, int s0, float4& a) const {
+#pragma unroll
+        for (int u = 0; u < MAX; ++u) {
+            const bool there = s0 + u < ps.n;
+            a.x = there ? a.x + p[u].x : a.x; a.y = there ? a.y + p[u].y : a.y;
+            a.z = there ? a.z + p[u].z : a.z; a.w = there ? a.w + p[u].w : a.w;
+        }
+    }
+    // the sum of all pieces, the first of which have been asked for
+    __device__ __forceinline__ float4 sum(const PartSums& ps, size_t at) {
+        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+        add(ps, 0, a);
+        for (int s = MAX; s < ps.n; s += MAX) {
+            ask(ps, at, s);
+            add(ps, s, a);
+        }
+        return a;
+    }
+};
+
 template <typename TA>
 __device__ __forceinline__ float summed(const PartSums& ps, size_t at) {
     float a = 0.f;
@@ -191,7 +226,8 @@ template <> __device__ __forceinline__ void store4<bf16_t>(bf16_t* p, float a, f
     *reinterpret_cast<uint2*>(p) = o;
 }
 
-template <typename TA, typename TW, int VPT>
+// SUMS: the update is a product's pieces, so many of them under way together (0: it is not; VPT is 1 or 2 otherwise).
+template <typename TA, typename TW, int VPT, int SUMS>
 __global__ void add_rmsnorm_vec_kernel(float* __restrict__ h, const TA* __restrict__ delta, const PartSums ps,
                                        const TW* __restrict__ weight, float eps,
                                        const int32_t* __restrict__ rows, int hidden,
@@ -202,40 +238,43 @@ __global__ void add_rmsnorm_vec_kernel(float* __restrict__ h, const TA* __restri
     float* hr = h ? h + row * hidden : nullptr;
     const TA* dr = delta ? delta + row * hidden : nullptr;
     TA* o = out + (size_t)r * hidden;
+    // Everything is asked for before anything is looked at, the norm's weight too.  (Lanes past the row repeat its last values and drop them.)
+    constexpr bool EARLY_W = VPT <= 4;
     float v[VPT][4];
+    float4 hv[VPT];
+    Vec4<TA> d[VPT];
+    Vec4<TW> w[VPT];
+    auto place = [&](int j) { return min((int)(j * blockDim.x + threadIdx.x) * 4, hidden - 4); };
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        const int i = place(j);
+        hv[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (hr) hv[j] = *reinterpret_cast<const float4*>(hr + i);
+        if (!SUMS && dr) d[j].v = *reinterpret_cast<const decltype(d[j].v)*>(dr + i);
+        if (EARLY_W) w[j].v = *reinterpret_cast<const decltype(w[j].v)*>(weight + i);
+    }
+    if constexpr (SUMS > 0) {
+        Pieces<SUMS> p[VPT];
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) p[j].ask(ps, row * hidden + place(j), 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+            const float4 a = p[j].sum(ps, row * hidden + place(j));
+            hv[j].x += to_float(from_float<TA>(a.x)); hv[j].y += to_float(from_float<TA>(a.y));
+            hv[j].z += to_float(from_float<TA>(a.z)); hv[j].w += to_float(from_float<TA>(a.w));
+        }
+    }
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
         const int i = (j * blockDim.x + threadIdx.x) * 4;
+        if (!SUMS && dr) { hv[j].x += d[j].get(0); hv[j].y += d[j].get(1); hv[j].z += d[j].get(2); hv[j].w += d[j].get(3); }
         if (i < hidden) {
-            float4 hv = hr ? *reinterpret_cast<const float4*>(hr + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-            if (dr) {
-                Vec4<TA> d;
-                d.v = *reinterpret_cast<const decltype(d.v)*>(dr + i);
-                hv.x += d.get(0); hv.y += d.get(1); hv.z += d.get(2); hv.w += d.get(3);
-            }
-            if (ps.sums) {
-                float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-                const float* at = ps.sums + row * hidden + i;
-                int s = 0;
-                for (; s + 4 <= ps.n; s += 4) {             // four loads under way together, added in order
-                    float4 part[4];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) part[u] = *reinterpret_cast<const float4*>(at + (size_t)(s + u) * ps.stride);
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) { a.x += part[u].x; a.y += part[u].y; a.z += part[u].z; a.w += part[u].w; }
-                }
-                for (; s < ps.n; ++s) {
-                    const float4 part = *reinterpret_cast<const float4*>(at + (size_t)s * ps.stride);
-                    a.x += part.x; a.y += part.y; a.z += part.z; a.w += part.w;
-                }
-                hv.x += to_float(from_float<TA>(a.x)); hv.y += to_float(from_float<TA>(a.y));
-                hv.z += to_float(from_float<TA>(a.z)); hv.w += to_float(from_float<TA>(a.w));
-            }
-            if (write_back) *reinterpret_cast<float4*>(hr + i) = hv;
-            v[j][0] = hv.x; v[j][1] = hv.y; v[j][2] = hv.z; v[j][3] = hv.w;
-            ss += hv.x * hv.x + hv.y * hv.y + hv.z * hv.z + hv.w * hv.w;
+            if (write_back) *reinterpret_cast<float4*>(hr + i) = hv[j];
+            ss += hv[j].x * hv[j].x + hv[j].y * hv[j].y + hv[j].z * hv[j].z + hv[j].w * hv[j].w;
         }
+        v[j][0] = hv[j].x; v[j][1] = hv[j].y; v[j][2] = hv[j].z; v[j][3] = hv[j].w;
     }
     const float total = block_sum(ss, scratch);
     const float rms = sqrtf(total / (float)hidden + eps);
@@ -243,13 +282,13 @@ __global__ void add_rmsnorm_vec_kernel(float* __restrict__ h, const TA* __restri
     for (int j = 0; j < VPT; ++j) {
         const int i = (j * blockDim.x + threadIdx.x) * 4;
         if (i < hidden) {
-            Vec4<TW> w;
-            w.v = *reinterpret_cast<const decltype(w.v)*>(weight + i);
-            store4<TA>(o + i, (v[j][0] / rms) * w.get(0), (v[j][1] / rms) * w.get(1),
-                       (v[j][2] / rms) * w.get(2), (v[j][3] / rms) * w.get(3));
+            if (!EARLY_W) w[j].v = *reinterpret_cast<const decltype(w[j].v)*>(weight + i);
+            store4<TA>(o + i, (v[j][0] / rms) * w[j].get(0), (v[j][1] / rms) * w[j].get(1),
+                       (v[j][2] / rms) * w[j].get(2), (v[j][3] / rms) * w[j].get(3));
         }
     }
 }
+
 
 static int add_rmsnorm(float* h, const void* delta, const PartSums ps, int act_dtype, const void* weight,
                        int weight_dtype, float eps, const int32_t* rows, int n_rows,
@@ -265,13 +304,18 @@ static int add_rmsnorm(float* h, const void* delta, const PartSums ps, int act_d
     const bool aligned = ((((uintptr_t)h) | ((uintptr_t)delta) | ((uintptr_t)weight) | ((uintptr_t)out) | ((uintptr_t)ps.sums)) & 15) == 0;
     const int code = act_dtype * 2 + weight_dtype;
     if (hidden % 4 == 0 && hidden <= 8192 && aligned) {
-        // sums of a product: several times the bytes per row, and few rows: more threads per row
-        const int threads = ps.sums ? 1024 : 256;
-#define LAUNCHV(TA, TW, VPT) add_rmsnorm_vec_kernel<TA, TW, VPT><<<n_rows, threads, 0, s>>>( \
+        // Sums of a product are several times the bytes per row, of few rows: a thread for every four values (no more, waves without any cost time
+        // too) and all pieces asked for together, with the norm's weight.  32 rows of 1536, 14 and 3 pieces: 4.64 -> 4.04 us (a step of
+        // the 1.5B shape 0.7 % less); 64 rows of 3584, 9 and 7 pieces: 5.16 either way, what a compute unit brings in of its row.  More rows than that
+        // are bound by bytes: 232 rows of 3584, 6 and 3 pieces 7.24 us with all of them under way, 7.0 with four.
+        const int threads = !ps.sums ? 256 : hidden < 4096 ? (hidden / 4 + TQK_WAVE - 1) / TQK_WAVE * TQK_WAVE : 1024;
+#define LAUNCHV(TA, TW, VPT, SUMS) add_rmsnorm_vec_kernel<TA, TW, VPT, SUMS><<<n_rows, threads, 0, s>>>( \
         h, (const TA*)delta, ps, (const TW*)weight, eps, rows, hidden, (TA*)out, write_back)
 #define PICK(TA, TW) do { const int per = (hidden + threads * 4 - 1) / (threads * 4); \
-        if (per <= 1) LAUNCHV(TA, TW, 1); else if (per <= 2) LAUNCHV(TA, TW, 2); \
-        else if (per <= 4) LAUNCHV(TA, TW, 4); else LAUNCHV(TA, TW, 8); } while (0)
+        if (ps.sums && n_rows > 64) { if (per <= 1) LAUNCHV(TA, TW, 1, 4); else LAUNCHV(TA, TW, 2, 4); } \
+        else if (ps.sums) { if (per <= 1) LAUNCHV(TA, TW, 1, 16); else LAUNCHV(TA, TW, 2, 8); } \
+        else if (per <= 1) LAUNCHV(TA, TW, 1, 0); else if (per <= 2) LAUNCHV(TA, TW, 2, 0); \
+        else if (per <= 4) LAUNCHV(TA, TW, 4, 0); else LAUNCHV(TA, TW, 8, 0); } while (0)
         switch (code) {
             case 0: PICK(float, float); break;
             case 1: PICK(float, bf16_t); break;
