@@ -431,6 +431,30 @@ def test_attention_generic(dtype, nh, nkv, d, window):
     assert (other[59] - want[59]).abs().max() > 0.1
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("d,window", [(48, 0), (128, 0), (128, 130), (256, 600)])
+def test_attention_generic_gives_few_queries_the_bits_of_many(dtype, d, window):
+    """A wave for each stripe of pages or one wave for all of them: one page, a page for some stripes, for all, and several for some; the
+    first page in any stripe (windows); values against the reference as well."""
+    nh, nkv, act, n = 4, 2, DT[dtype], 1100
+    k, v = rand(nkv, n, d, seed=23).to(act).float().cpu(), rand(nkv, n, d, seed=24).to(act).float().cpu()
+    page_ids = list(reversed(range(18)))
+    keys, values = paged(k, v, page_ids, 18, act)
+    pos = torch.tensor([0, 5, 63, 64, 200, 511, 512, 575, 800, 1099] * 13)
+    q = rand(len(pos), nh, d, seed=25).to(act)
+    table, scale = ints([page_ids]), d ** -0.5
+
+    def run(rows):
+        out = torch.empty(len(rows), nh * d, dtype=act, device=DEV)
+        return K.attention(q[rows].contiguous(), keys, values, ints([0] * len(rows)), pos[rows].to(torch.int32).to(DEV), table, window, scale, out)
+
+    many = run(list(range(len(pos))))                        # 520 waves' worth: one wave each
+    few = torch.cat([run(list(range(i, i + 5))) for i in range(0, 10, 5)])
+    assert torch.equal(few, many[:10])
+    want = attention_reference(q[:10].float().cpu(), k, v, pos[:10], window, scale)
+    torch.testing.assert_close(few.float().cpu(), want, **TOL[dtype])
+
+
 def test_attention_generic_two_sequences_share_nothing():
     nh, nkv, d = 4, 2, 32
     ka, va = rand(nkv, 100, d, seed=15).cpu(), rand(nkv, 100, d, seed=16).cpu()

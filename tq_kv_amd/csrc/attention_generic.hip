@@ -12,14 +12,17 @@
 //
 // Work of one wave: keys are taken in blocks of 64 (one page); lane j computes the
 // score of key j of the block, the softmax runs online over blocks, then lane c
-// accumulates output element c (+64, +128, ...) over the block's keys.  The order of
-// operations for a query depends only on its position, never on the batch.
+// accumulates output element c (+64, +128, ...) over the block's keys.  Pages are dealt to
+// eight stripes by their number, each walked on its own, and the stripes meet in their order: either
+// one wave walks all of them (many queries), or a wave each (few queries).  The order of
+// operations for a query depends only on its position, never on the batch or on which of the two it is.
 // Cache pages: keys [kv head][position][head_dim], values [kv head][head_dim][place of
 // the position] (value_place in common.h).
 #include "common.h"
 #include "tq_kernels.h"
 
 #define ATT_WAVES 4
+#define ATT_STRIPES 8
 #define ATT_MAX_D 256
 
 // four elements that lie together, at a multiple of four elements
@@ -32,41 +35,26 @@ __device__ __forceinline__ float4 load4(const bf16_t* p) {
 // lane j's value, j the same for the whole wave
 __device__ __forceinline__ float lane_value(float v, int j) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), j)); }
 
-// Bound by latency (one wave walks a query's pages): loads of four elements, several of them under way, took the float32
-// step of one token after 300 (28 heads of 128) from 116 to 39 us and the prompt of 300 from 437 to 191 us against loads of one.
-template <typename T>
-__global__ __launch_bounds__(ATT_WAVES * TQK_WAVE)
-void attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ keys, const T* __restrict__ values,
-                              const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ tok_pos,
-                              const int32_t* __restrict__ page_table, int table_width, int window, float scale,
-                              T* __restrict__ out, int n_tokens, int n_heads, int n_kv_heads, int head_dim, int wide_keys, int wide_values) {
-    __shared__ __attribute__((aligned(16))) float q_lds[ATT_WAVES][ATT_MAX_D];
-    const int wave = threadIdx.x / TQK_WAVE, lane = threadIdx.x % TQK_WAVE;
-    const int t = blockIdx.x * ATT_WAVES + wave;
-    const int head = blockIdx.y;
-    const bool live = t < n_tokens;
-    if (live) {
-        const T* qv = q + ((size_t)t * n_heads + head) * head_dim;
-        for (int i = lane; i < head_dim; i += TQK_WAVE) q_lds[wave][i] = to_float(qv[i]);
-    }
-    __syncthreads();
-    if (!live) return;
+// What a stripe leaves: maximum, sum, and this lane's output elements.
+struct Stripe {
+    float m, l, acc[ATT_MAX_D / TQK_WAVE];
+};
 
-    const int pos = tok_pos[t];
-    const int32_t* pages = page_table + (size_t)tok_seq[t] * table_width;
-    const int kvh = head / (n_heads / n_kv_heads);
-    const int lo = window > 0 ? max(0, pos - window + 1) : 0;
-    const size_t page_stride = (size_t)n_kv_heads * TQK_PAGE * head_dim;
-    const float* qf = q_lds[wave];
-
+// The pages of one stripe for one query: its values in LDS (qf), keys lo .. pos.
+// UNROLL: loads of four elements of a key under way together.
+template <typename T, int UNROLL>
+__device__ __forceinline__ Stripe walk(int stripe, const float* qf, const T* keys, const T* values, const int32_t* pages, int pos, int lo, int kvh,
+                                       int n_kv_heads, int head_dim, float scale, int wide_keys, int wide_values, int lane) {
     constexpr int NACC = ATT_MAX_D / TQK_WAVE;
-    float acc[NACC];
+    const size_t page_stride = (size_t)n_kv_heads * TQK_PAGE * head_dim;
+    Stripe r;
 #pragma unroll
-    for (int i = 0; i < NACC; ++i) acc[i] = 0.f;
-    float m = -INFINITY, l = 0.f;
-
-    for (int kb = (lo / TQK_PAGE) * TQK_PAGE; kb <= pos; kb += TQK_PAGE) {
-        const int page = pages[kb / TQK_PAGE];
+    for (int i = 0; i < NACC; ++i) r.acc[i] = 0.f;
+    r.m = -INFINITY;
+    r.l = 0.f;
+    const int first = lo / TQK_PAGE;
+    for (int pg = first + (stripe - first % ATT_STRIPES + ATT_STRIPES) % ATT_STRIPES; pg * TQK_PAGE <= pos; pg += ATT_STRIPES) {
+        const int kb = pg * TQK_PAGE, page = pages[pg];
         const int j = kb + lane;
         const bool valid = j >= lo && j <= pos && page >= 0;
         const size_t base = (size_t)(page < 0 ? 0 : page) * page_stride + (size_t)kvh * TQK_PAGE * head_dim;
@@ -76,7 +64,7 @@ void attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ key
             float dot = 0.f;
             int i = 0;
             if (wide_keys) {
-#pragma unroll 8
+#pragma unroll UNROLL
                 for (; i < head_dim; i += 4) {
                     const float4 k = load4(kr + i), qv4 = *reinterpret_cast<const float4*>(qf + i);
                     dot = fmaf(qv4.x, k.x, dot);
@@ -88,18 +76,18 @@ void attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ key
             for (; i < head_dim; ++i) dot = fmaf(qf[i], to_float(kr[i]), dot);
             s = dot * scale;
         }
-        const float m_new = fmaxf(m, wave_max(s));     // finite: the block holds at least key lo or kb
+        const float m_new = fmaxf(r.m, wave_max(s));    // finite: the page holds at least one key of lo .. pos
         const float p = valid ? expf(s - m_new) : 0.f;
-        const float alpha = expf(m - m_new);            // exp(-inf) = 0 on the first block
-        l = l * alpha + wave_sum(p);
-        m = m_new;
+        const float alpha = expf(r.m - m_new);          // exp(-inf) = 0 on the stripe's first page
+        r.l = fmaf(r.l, alpha, wave_sum(p));
+        r.m = m_new;
         const int n_keys = min(TQK_PAGE, pos - kb + 1);
         const int first_key = max(0, lo - kb);           // keys before the window are never read
         const T* vb = values + base;
 #pragma unroll
         for (int a = 0; a < NACC; ++a) {
             const int c = lane + a * TQK_WAVE;
-            float sum = acc[a] * alpha;
+            float sum = r.acc[a] * alpha;
             if (a * TQK_WAVE < head_dim) {
                 // (lanes past the head read its last row and drop the result)
                 const T* row = vb + (size_t)min(c, head_dim - 1) * TQK_PAGE;
@@ -108,7 +96,7 @@ void attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ key
                 int jj = first_key;
                 for (; jj < n_keys && jj % 4 != 0; ++jj) one(jj);
                 if (wide_values) {
-#pragma unroll 4
+#pragma unroll UNROLL / 2
                     for (; jj + 4 <= n_keys; jj += 4) {
                         const float4 v = load4(row + value_place(jj));
                         sum = fmaf(lane_value(p, jj), v.x, sum);
@@ -119,14 +107,93 @@ void attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ key
                 }
                 for (; jj < n_keys; ++jj) one(jj);
             }
-            acc[a] = sum;
+            r.acc[a] = sum;
         }
     }
+    return r;
+}
+
+// The next stripe joins the ones before it: what the sums so far and the stripe's are multiplied by.
+__device__ __forceinline__ void join(float& m, float& l, float stripe_m, float stripe_l, float& of_sum, float& of_stripe) {
+    const float mn = fmaxf(m, stripe_m);
+    of_sum = expf(m - mn);                              // exp(-inf) = 0 for the first one
+    of_stripe = expf(stripe_m - mn);
+    l = fmaf(l, of_sum, stripe_l * of_stripe);
+    m = mn;
+}
+
+// Bound by latency, a page costs a wave 8 us: the float32 step of one token after 300 (28 heads of 128) takes 17.6 us with a wave per stripe and
+// 16 loads under way, 45.9 with one wave for all and 8; the prompt of 300 190 us.
+// SPLIT: a block of a wave per stripe for one query.
+template <typename T, bool SPLIT>
+__global__ __launch_bounds__((SPLIT ? ATT_STRIPES : ATT_WAVES) * TQK_WAVE)
+void attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ keys, const T* __restrict__ values,
+                              const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ tok_pos,
+                              const int32_t* __restrict__ page_table, int table_width, int window, float scale,
+                              T* __restrict__ out, int n_tokens, int n_heads, int n_kv_heads, int head_dim, int wide_keys, int wide_values) {
+    constexpr int NACC = ATT_MAX_D / TQK_WAVE;
+    __shared__ __attribute__((aligned(16))) float q_lds[SPLIT ? 1 : ATT_WAVES][ATT_MAX_D];
+    const int wave = threadIdx.x / TQK_WAVE, lane = threadIdx.x % TQK_WAVE;
+    const int t = SPLIT ? blockIdx.x : blockIdx.x * ATT_WAVES + wave;
+    const int head = blockIdx.y;
+    const bool live = t < n_tokens;
+    float* qf = q_lds[SPLIT ? 0 : wave];
+    if (live) {
+        const T* qv = q + ((size_t)t * n_heads + head) * head_dim;
+        for (int i = SPLIT ? threadIdx.x : lane; i < head_dim; i += SPLIT ? blockDim.x : TQK_WAVE) qf[i] = to_float(qv[i]);
+    }
+    __syncthreads();
+    if (!live) return;
+
+    const int pos = tok_pos[t];
+    const int32_t* pages = page_table + (size_t)tok_seq[t] * table_width;
+    const int kvh = head / (n_heads / n_kv_heads);
+    const int lo = window > 0 ? max(0, pos - window + 1) : 0;
     T* o = out + ((size_t)t * n_heads + head) * head_dim;
+    float m = -INFINITY, l = 0.f, of_sum, of_stripe;
+
+    if constexpr (SPLIT) {
+        __shared__ float met[ATT_STRIPES][ATT_MAX_D], ml[ATT_STRIPES][2];
+        const bool alone = lo / TQK_PAGE == pos / TQK_PAGE;             // one page: its stripe is the result
+        if (alone && wave > 0) return;
+        const Stripe r = walk<T, 16>(alone ? lo / TQK_PAGE % ATT_STRIPES : wave, qf, keys, values, pages, pos, lo, kvh, n_kv_heads, head_dim, scale, wide_keys, wide_values, lane);
+        if (alone) {
 #pragma unroll
-    for (int a = 0; a < NACC; ++a) {
-        const int c = lane + a * TQK_WAVE;
-        if (c < head_dim) o[c] = from_float<T>(acc[a] / l);
+            for (int a = 0; a < NACC; ++a) {
+                const int c = lane + a * TQK_WAVE;
+                if (c < head_dim) o[c] = from_float<T>(r.acc[a] / r.l);
+            }
+            return;
+        }
+#pragma unroll
+        for (int a = 0; a < NACC; ++a) met[wave][lane + a * TQK_WAVE] = r.acc[a];
+        if (lane == 0) { ml[wave][0] = r.m; ml[wave][1] = r.l; }
+        __syncthreads();
+        float acc = 0.f;
+        const int c = threadIdx.x;
+        if (c >= head_dim) return;
+        for (int s = 0; s < ATT_STRIPES; ++s) {
+            if (ml[s][0] == -INFINITY) continue;        // no page
+            join(m, l, ml[s][0], ml[s][1], of_sum, of_stripe);
+            acc = fmaf(acc, of_sum, met[s][c] * of_stripe);
+        }
+        o[c] = from_float<T>(acc / l);
+    } else {
+        float acc[NACC];
+#pragma unroll
+        for (int a = 0; a < NACC; ++a) acc[a] = 0.f;
+        for (int s = 0; s < ATT_STRIPES; ++s) {
+            const Stripe r = walk<T, 8>(s, qf, keys, values, pages, pos, lo, kvh, n_kv_heads, head_dim, scale, wide_keys, wide_values, lane);
+            if (r.m == -INFINITY) continue;
+            join(m, l, r.m, r.l, of_sum, of_stripe);
+#pragma unroll
+            for (int a = 0; a < NACC; ++a) acc[a] = fmaf(acc[a], of_sum, r.acc[a] * of_stripe);
+        }
+#pragma unroll
+        for (int a = 0; a < NACC; ++a) {
+            const int c = lane + a * TQK_WAVE;
+            if (c < head_dim) o[c] = from_float<T>(acc[a] / l);
+        }
     }
 }
 
@@ -145,19 +212,22 @@ extern "C" int tqk_attention(const void* q, const void* keys, const void* values
     TQK_REQUIRE(window >= 0, "tqk_attention: negative window");
     if (n_tokens == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
-    dim3 grid((n_tokens + ATT_WAVES - 1) / ATT_WAVES, n_heads);
+    // A wave per stripe (45.9 -> 17.6 us, one token after 300, 28 heads) while no unit gets more than two blocks of them; the results are the same.
+    // One page is one wave's work either way.
+    const bool split = (long long)n_tokens * n_heads <= 512;
+    const dim3 grid(split ? n_tokens : (n_tokens + ATT_WAVES - 1) / ATT_WAVES, n_heads);
     // four elements a load where keys and values begin at a multiple of four elements (a caller's memory need not) and rows of keys do, too
     const size_t four = act_dtype == TQK_F32 ? 16 : 8;
     const int wide_keys = head_dim % 4 == 0 && (uintptr_t)keys % four == 0, wide_values = (uintptr_t)values % four == 0;
-    if (act_dtype == TQK_F32)
-        attention_generic_kernel<float><<<grid, ATT_WAVES * TQK_WAVE, 0, s>>>(
-            (const float*)q, (const float*)keys, (const float*)values, tok_seq, tok_pos, page_table, table_width,
-            window, scale, (float*)out, n_tokens, n_heads, n_kv_heads, head_dim, wide_keys, wide_values);
-    else if (act_dtype == TQK_BF16)
-        attention_generic_kernel<bf16_t><<<grid, ATT_WAVES * TQK_WAVE, 0, s>>>(
-            (const bf16_t*)q, (const bf16_t*)keys, (const bf16_t*)values, tok_seq, tok_pos, page_table, table_width,
-            window, scale, (bf16_t*)out, n_tokens, n_heads, n_kv_heads, head_dim, wide_keys, wide_values);
-    else
+#define LAUNCH(T, SPLIT) attention_generic_kernel<T, SPLIT><<<grid, (SPLIT ? ATT_STRIPES : ATT_WAVES) * TQK_WAVE, 0, s>>>( \
+            (const T*)q, (const T*)keys, (const T*)values, tok_seq, tok_pos, page_table, table_width, \
+            window, scale, (T*)out, n_tokens, n_heads, n_kv_heads, head_dim, wide_keys, wide_values)
+    if (act_dtype == TQK_F32) {
+        if (split) LAUNCH(float, true); else LAUNCH(float, false);
+    } else if (act_dtype == TQK_BF16) {
+        if (split) LAUNCH(bf16_t, true); else LAUNCH(bf16_t, false);
+    } else
+#undef LAUNCH
         return tqk_fail("tqk_attention: unknown dtype %d", act_dtype);
     return tqk_check_launch("tqk_attention");
 }
