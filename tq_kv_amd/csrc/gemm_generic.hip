@@ -194,9 +194,10 @@ void gemm_few_rows_kernel(const float* __restrict__ x, const float* __restrict__
 }
 
 // More rows: 64 rows by 64 features a block, each of four waves 32 by 32.  Stages of 32 k go through registers into LDS, two in turn;
-// a row's 128 bytes lie 144 apart, so that the 16 rows of an operand meet all banks.  blockIdx.z: the block's share of the
+// a row's 128 bytes lie 144 apart, so that the 16 rows of an operand meet all banks.  blockIdx.y: the block's share of the
 // groups; with more than one share every group's sums go to scratch on their own.  Bound by the matrix cores (157 TFLOP/s in
-// float32): gate+up of the 7B shape at 300 rows 836 us = 97 TFLOP/s, and 2108 us through the FMA kernel above; down 287 and 1663.
+// float32): gate+up of the 7B shape at 300 rows 805 us = 101 TFLOP/s (855 with the
+// rows' tiles of some features far apart), and 2108 us through the FMA kernel above; down 287 and 1663.
 #define GM_LINE 36              // floats from row to row in LDS
 __global__ __launch_bounds__(256)
 void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ out,
@@ -204,9 +205,19 @@ void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, c
     __shared__ __attribute__((aligned(16))) float lds[2][2][GT * GM_LINE];     // [stage][x, w]
     const int tid = threadIdx.x, lane = tid % TQK_WAVE, wave = tid / TQK_WAVE;
     const int r16 = lane % 16, k4 = 4 * (lane / 16);
-    const int m0 = blockIdx.y * GT, n0 = blockIdx.x * GT, wm = wave / 2 * 32, wn = wave % 2 * 32;
-    const int k_begin = blockIdx.z * groups_per_share * G_GROUP, k_end = min(K, k_begin + groups_per_share * G_GROUP);
-    const bool shared_out = gridDim.z > 1;
+    // Blocks are dealt to the eight dies in turn: all rows' tiles of some features go to one die one after the other, so that the weights come out
+    // of its second-level cache for all but the first.
+    const int tiles_m = (M + GT - 1) / GT, tiles_n = (N + GT - 1) / GT;
+    int tm, tn;
+    {
+        const int n = tiles_m * tiles_n, die = blockIdx.x % 8, at = blockIdx.x / 8, each_die = n / 8, more = n % 8;
+        const int id = die * each_die + min(die, more) + at;
+        tm = id % tiles_m;
+        tn = id / tiles_m;
+    }
+    const int m0 = tm * GT, n0 = tn * GT, wm = wave / 2 * 32, wn = wave % 2 * 32;
+    const int k_begin = blockIdx.y * groups_per_share * G_GROUP, k_end = min(K, k_begin + groups_per_share * G_GROUP);
+    const bool shared_out = gridDim.y > 1;
     // what a thread brings in: of rows tid / 8 and 32 + tid / 8 of both tiles the four k at 4 (tid % 8) (rows past the end repeat the last)
     const int sr = tid / 8, sk = 4 * (tid % 8);
     const float* src[2][2];
@@ -354,7 +365,7 @@ extern "C" int tqk_gemm(const void* x, int x_dtype, const void* w, int w_dtype, 
         const float *xf = (const float*)x, *wf = (const float*)w, *bf = (const float*)bias;
         float* out = shares > 1 ? (float*)scratch : (float*)y;
         if (M <= 16 && shares == groups) gemm_few_rows_kernel<<<dim3((N + 15) / 16, groups), TQK_WAVE, 0, s>>>(xf, wf, bf, out, M, N, K);
-        else gemm_f32_kernel<<<dim3((N + GT - 1) / GT, (M + GT - 1) / GT, shares), 256, 0, s>>>(xf, wf, bf, out, M, N, K, (groups + shares - 1) / shares);
+        else gemm_f32_kernel<<<dim3(((N + GT - 1) / GT) * ((M + GT - 1) / GT), shares), 256, 0, s>>>(xf, wf, bf, out, M, N, K, (groups + shares - 1) / shares);
         if (tqk_check_launch("tqk_gemm float32")) return -1;
         if (shares == 1) return 0;
         const size_t total = (size_t)M * N;
