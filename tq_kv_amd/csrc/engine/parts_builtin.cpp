@@ -677,21 +677,20 @@ private:
     }
 
     // Whether the decoding kernel finishes a q/k/v product left as sums over pieces of K itself (a launch less): steps of one token a sequence
-    // that go through that kernel and write their own cache.  A block then waits for its row's sums before it asks for a page, so not
-    // where that costs more than the launch (ms a step, launch -> folded, heads of 128; every rule's both sides):
-    //  - blocks of one wave, two or three rounds of loads on 64 lanes: 7B sizes, 17 and 20 rows of 200 positions 3.368 -> 3.393 and
-    //    3.400 -> 3.435; 24 rows, blocks of four waves, 3.495 -> 3.425;
-    //  - more blocks than units: 7B, 96 rows after 256, up to 1024 and 2048 positions 4.968 -> 4.974, 5.432 -> 5.460 and 6.621 -> 6.795, 128 rows
-    //    5.412 -> 5.456, 5.972 -> 5.989 and 7.344 -> 7.593;
-    //  - more than 24 pages a unit: 7B, 48 rows of 2048 positions 4.490 -> 4.520, 64 rows 4.990 -> 5.032; 1.5B, 96 rows 3.376 -> 3.438; 32B with 8
-    //    layers, 32 rows 2.136 -> 2.156.  Up to that: 7B, 32 rows of 2048 positions 4.026 -> 3.979, 64 rows of up to 1024 4.309 -> 4.287; 1.5B,
-    //    32 and 128 of those 1.963 -> 1.901 and 3.192 -> 3.194; 32B, 32 of those 2.001 -> 1.992.
+    // that go through that kernel and write their own cache.  A block asks for its first page while its row's sums are on their way, so the launch
+    // is saved but for the work that blocks of one row then do each for themselves.  Not where that costs more than the launch (ms a step, launch ->
+    // folded, heads of 128; every rule's both sides):
+    //  - blocks of one wave, two or three rounds of loads on 64 lanes (before a page was asked for ahead): 7B sizes, 17 and 20 rows of 200
+    //    positions 3.368 -> 3.393 and 3.400 -> 3.435; 24 rows, blocks of four waves, 3.495 -> 3.425;
+    //  - more blocks than units: 7B, 72 rows of 64 positions 3.803 -> 3.851, 120 of 1024 5.282 -> 5.342, 80 of up to 1024 4.345 -> 4.332; 32B with 8
+    //    layers, 60 of 1024 2.158 -> 2.176.  Up to that, of any length: 7B, 48 and 64 rows of 2048 positions 4.238 -> 4.179 and 4.588 -> 4.569;
+    //    1.5B, 96 of 2048 2.836 -> 2.778 and 64 of 4096 2.882 -> 2.816; 32B, 20 and 32 of 2048 1.991 -> 1.940 and 2.118 -> 2.095.
     bool finishes_sums(const StepContext& c, const CacheEntry& entry, int width) const {
         if (!(c.all_decode && entry.writes && policy().decode_mfma && K::attention_decode_supported.raw(head_dim_) != 0)) return false;
         const int units = 256, n_parts = decode_parts(c.n_tokens, width);
         const long long groups = (long long)c.n_tokens * n_kv_heads_ * ((n_heads_ / n_kv_heads_ + 15) / 16);
         const bool one_wave = n_parts > 1 && n_parts >= width;
-        return !one_wave && groups <= units && groups * width <= 24LL * units;
+        return !one_wave && groups <= units;
     }
 
     // product, then bias, position encoding and cache write in their own kernel; leave: where the product may be left as its sums, they are
