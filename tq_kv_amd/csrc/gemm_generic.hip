@@ -196,8 +196,9 @@ void gemm_few_rows_kernel(const float* __restrict__ x, const float* __restrict__
 // More rows: 64 rows by 64 features a block, each of four waves 32 by 32.  Stages of 32 k go through registers into LDS, two in turn;
 // a row's 128 bytes lie 144 apart, so that the 16 rows of an operand meet all banks.  blockIdx.y: the block's share of the
 // groups; with more than one share every group's sums go to scratch on their own.  Bound by the matrix cores (157 TFLOP/s in
-// float32): gate+up of the 7B shape at 300 rows 805 us = 101 TFLOP/s (855 with the
-// rows' tiles of some features far apart), and 2108 us through the FMA kernel above; down 287 and 1663.
+// float32): gate+up of the 7B shape at 300 rows 750 us = 109 TFLOP/s (827 with the
+// rows' tiles of some features far apart and loads one stage ahead: a stage is hardly longer than a load takes), and 2108 us through the FMA kernel above; down
+// 465 with the groups' sums (495), 40 rows 206 and 108 (229 and 111).  Blocks of 160 rows by 64 features took 967 us: fewer waves lose more than the bytes saved.
 #define GM_LINE 36              // floats from row to row in LDS
 __global__ __launch_bounds__(256)
 void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ out,
@@ -226,23 +227,23 @@ void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, c
         src[0][i] = x + (size_t)min(m0 + sr + 32 * i, M - 1) * K;
         src[1][i] = w + (size_t)min(n0 + sr + 32 * i, N - 1) * K;
     }
-    floatx4_t ahead[2][2];
-    auto load = [&](int k0) {
+    floatx4_t ahead[2][2][2];          // [stage % 2]: a stage's loads are issued two stages before it
+    auto load = [&](int k0, int to) {
         const int k = min(k0 + sk, K - 4);          // past K: read from inside the row, zeros in its place
         const bool in = k0 + sk < K;
 #pragma unroll
         for (int o = 0; o < 2; ++o)
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                ahead[o][i] = *reinterpret_cast<const floatx4_t*>(src[o][i] + k);
-                if (!in) ahead[o][i] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+                ahead[to][o][i] = *reinterpret_cast<const floatx4_t*>(src[o][i] + k);
+                if (!in) ahead[to][o][i] = floatx4_t{0.f, 0.f, 0.f, 0.f};
             }
     };
     auto put = [&](int stage) {
 #pragma unroll
         for (int o = 0; o < 2; ++o)
 #pragma unroll
-            for (int i = 0; i < 2; ++i) *reinterpret_cast<floatx4_t*>(&lds[stage][o][(sr + 32 * i) * GM_LINE + sk]) = ahead[o][i];
+            for (int i = 0; i < 2; ++i) *reinterpret_cast<floatx4_t*>(&lds[stage][o][(sr + 32 * i) * GM_LINE + sk]) = ahead[stage][o][i];
     };
     floatx4_t acc[2][2], group[2][2], total[2][2];
 #pragma unroll
@@ -263,7 +264,8 @@ void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, c
                 }
         }
     };
-    load(k_begin);
+    load(k_begin, 0);
+    load(k_begin + 32, 1);
     put(0);
     __syncthreads();
     for (int c0 = k_begin; c0 < k_end; c0 += G_CHUNK) {
@@ -271,7 +273,7 @@ void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, c
 #pragma unroll
         for (int q = 0; q < G_CHUNK / 32; ++q) {
             const int stage = q % 2;
-            load(c0 + 32 * (q + 1));
+            load(c0 + 32 * (q + 2), stage);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 floatx4_t xv[2], wv[2];
