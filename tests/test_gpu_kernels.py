@@ -3,6 +3,7 @@ sizes other than the tiny models': widths and vocabularies that are no power of 
 head sizes in steps of 16, odd numbers of heads and groups.  Inputs are made so that a
 fault shows: one far key that dominates, keys just inside and just outside a window,
 pages in scrambled order, NaN in everything that must not be read."""
+import ctypes
 import math
 
 import pytest
@@ -382,6 +383,36 @@ def test_decoding_attention_finishes_sums_before_many_whole_pages(n, width, n_pa
         assert ((got.float() - want.float()).abs() <= slack).all()
     else:
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("n_parts", [2, 3, 4, 5, 8, 11, 17, 20])
+def test_partitions_are_merged_with_every_product_rounded(n_parts):
+    """The merge's bits from the partitions' results as the kernel left them: maxima, then in the partitions' order the weighted outputs, each
+    product and each sum rounded, and the weights' sum with fused ones.  Values that change sign from page to page, so that what a sum
+    loses shows in its bfloat16 result; 1 to 20 pages a row, so that partitions without pages are among them."""
+    d, nh, nkv, width, n = 128, 28, 4, 20, 32
+    last = [(97 * i) % (64 * width) for i in range(n)]
+    table = ints([[i * width + j for j in range(width)] for i in range(n)])
+    keys = rand(n * width, nkv, 64, d, seed=94, scale=0.3, dtype=torch.bfloat16)
+    sign = 1.0 - 2.0 * (torch.arange(n * width, device=DEV) % 2).float()
+    values = ((rand(n * width, nkv, d, 64, seed=95, scale=0.05) + 1) * sign[:, None, None, None]).to(torch.bfloat16)
+    q = rand(n, nh, d, seed=96, dtype=torch.bfloat16)
+    part_out = torch.empty(n, nh, n_parts, d, device=DEV)
+    part_ml = torch.empty(n, nh, n_parts, 2, device=DEV)
+    out = torch.empty(n, nh * d, dtype=torch.bfloat16, device=DEV)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    pos = ints(last)
+    assert K.library().tqk_attention_decode(p(q), p(keys), p(values), p(pos), p(table), width, n, n * width, 0, ctypes.c_float(d ** -0.5), n_parts,
+                                            p(part_out), p(part_ml), p(out), nh, nkv, d, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    most = part_ml[..., 0].amax(-1)
+    total, weights = torch.zeros(n, nh, d, device=DEV), torch.zeros(n, nh, device=DEV)
+    for i in range(n_parts):
+        live = torch.isfinite(part_ml[..., i, 0])
+        w = torch.where(live, torch.exp2(part_ml[..., i, 0] - most), torch.zeros_like(most))
+        weights = torch.where(live, (w.double() * part_ml[..., i, 1].double() + weights.double()).float(), weights)
+        product = w[..., None] * part_out[:, :, i]
+        total = torch.where(live[..., None], total + product, total)
+    assert torch.equal(out.reshape(n, nh, d), (total / weights[..., None]).to(torch.bfloat16))
 
 
 def attention_reference(q, k, v, pos, window, scale, cap=0.0):

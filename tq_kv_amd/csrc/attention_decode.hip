@@ -486,10 +486,17 @@ void attention_decode_kernel(const DecodeSums in, const bf16_t* __restrict__ q, 
     if (n_parts > 1 && wave == 0 && g == 0) { part_ml[row * 2] = m; part_ml[row * 2 + 1] = l; }
 }
 
+// sum + weight * value, each rounded on its own whatever the code around it is (the weights' sum is fused): a decoding step's bits go by it.
+__device__ __forceinline__ float added(float sum, float weight, float value) {
+#pragma clang fp contract(off)
+    return sum + weight * value;
+}
+
 // out[seq, head, :] = sum_p exp(m_p - M) o_p / sum_p exp(m_p - M) l_p, partitions in order.
 // Bound by the loads it waits for one after the other (each misses every cache), so those of up to 16 partitions are asked for
 // together, and up to eight partitions take one round for maxima, sums and outputs alike: with four partitions of 32 rows and 12 heads a step of the 1.5B
-// shape takes 1.65 -> 1.605 ms against a loop that took eight at a time and a remainder one after the other.  A partition without keys (m = -inf) has weight 0 and its (unwritten) output is not looked at.
+// shape takes 1.65 -> 1.605 ms against a loop that took eight at a time and a remainder one after the other.  A partition without keys (m = -inf)
+// has weight 0 and its (unwritten) output is not looked at.
 template <int BATCH, bool ONE_ROUND>
 __global__ void attention_merge_kernel(const float* __restrict__ part_out, const float* __restrict__ part_ml,
                                        int n_parts, int head_dim, bf16_t* __restrict__ out) {
@@ -522,8 +529,8 @@ __global__ void attention_merge_kernel(const float* __restrict__ part_out, const
             for (int u = 0; u < BATCH; ++u) {
                 const bool live = s[u].x != -INFINITY && p0 + u < n_parts;
                 const float wgt = live ? __builtin_amdgcn_exp2f(s[u].x - M) : 0.f;
-                denom = live ? denom + wgt * s[u].y : denom;
-                acc = live ? acc + wgt * v[u] : acc;
+                denom = live ? fmaf(wgt, s[u].y, denom) : denom;
+                acc = live ? added(acc, wgt, v[u]) : acc;
             }
         }
         out[row * head_dim + c] = from_float<bf16_t>(acc / denom);
