@@ -6,6 +6,7 @@ pages in scrambled order, NaN in everything that must not be read."""
 import ctypes
 import math
 
+import numpy as np
 import pytest
 import torch
 import torch.nn.functional as F
@@ -871,6 +872,48 @@ def test_the_norm_adds_up_any_number_of_pieces(rows, hidden, n_sums):
     assert torch.equal(h1, h2)
     # the squares are added in another order, so a value may round to its neighbour: a step of bfloat16 is at most 2^-7 of it
     assert ((out1.float() - out2.float()).abs() <= out1.float().abs() * 2 ** -7).all()
+
+
+@pytest.mark.parametrize("rows", [5, 70])
+@pytest.mark.parametrize("hidden,n_sums", [(64, 0), (1024, 0), (3584, 0), (8192, 0), (68, 5), (1536, 3), (3584, 16), (4096, 4), (5120, 9), (8192, 14)])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_the_norm_adds_squares_in_one_order(dtype, hidden, n_sums, rows):
+    """The bits of the vectorised norm from its operations one by one: a thread's squares of four fused in the order y, x, z, w, its fours added, then the
+    lanes' sums by halves and the waves' one after the other; mean, root, two divisions' roundings."""
+    act, eps = DT[dtype], 1e-6
+    h, nw = rand(rows, hidden, seed=97, scale=1.5), 1 + rand(hidden, seed=98, scale=0.1)
+    if n_sums:
+        sums = rand(n_sums, rows, hidden, seed=99)
+        total = torch.zeros_like(h)
+        for piece in sums:
+            total += piece
+        update, threads = K.PartialSums(sums, act), 1024
+    else:
+        total = rand(rows, hidden, seed=99)
+        update, threads = total.to(act), 256
+    stream = (h + total.to(act).float()).cpu().numpy()
+    h2, out = h.clone(), torch.empty(rows, hidden, dtype=act, device=DEV)
+    K.add_rmsnorm(h2, update, nw, eps, out, write_back=True)
+    f32, f64 = np.float32, np.float64
+    padded = np.zeros((rows, -(-hidden // (4 * threads)) * threads, 4), f32)
+    padded[:, :hidden // 4] = stream.reshape(rows, -1, 4)
+    x, y, z, w = (padded[..., i].astype(f64) for i in range(4))
+    four = (y * y).astype(f32)
+    for v in (x, z, w):
+        four = (v * v + four).astype(f32)                      # fused: the product is exact in 64 bits
+    lanes = np.zeros((rows, threads), f32)
+    for j in range(four.shape[1] // threads):
+        lanes += four[:, j * threads:(j + 1) * threads]
+    lanes = lanes.reshape(rows, -1, 64)
+    for step in (32, 16, 8, 4, 2, 1):
+        lanes = lanes + lanes[..., np.arange(64) ^ step]
+    ss = np.zeros(rows, f32)
+    for wave in range(lanes.shape[1]):
+        ss += lanes[:, wave, 0]
+    rms = np.sqrt(ss / f32(hidden) + f32(eps))
+    want = (stream / rms[:, None]) * nw.cpu().numpy()
+    assert torch.equal(h2.cpu(), torch.from_numpy(stream))
+    assert torch.equal(out.cpu(), torch.from_numpy(want).to(act))
 
 
 @pytest.mark.parametrize("nh,nkv,d,k", [(28, 4, 128, 3584), (3, 1, 32, 2048), (6, 2, 64, 1056)])

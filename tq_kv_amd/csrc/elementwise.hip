@@ -226,6 +226,10 @@ template <> __device__ __forceinline__ void store4<bf16_t>(bf16_t* p, float a, f
     *reinterpret_cast<uint2*>(p) = o;
 }
 
+// Sum of four squares, fused in this order by name: what the compiler fuses of a plain expression changes with the code around it, and the bits of
+// all that follows the norm with it.
+__device__ __forceinline__ float squares(float4 v) { return fmaf(v.w, v.w, fmaf(v.z, v.z, fmaf(v.x, v.x, v.y * v.y))); }
+
 // SUMS: the update is a product's pieces, so many of them under way together (0: it is not; VPT is 1 or 2 otherwise).
 template <typename TA, typename TW, int VPT, int SUMS>
 __global__ void add_rmsnorm_vec_kernel(float* __restrict__ h, const TA* __restrict__ delta, const PartSums ps,
@@ -272,7 +276,7 @@ __global__ void add_rmsnorm_vec_kernel(float* __restrict__ h, const TA* __restri
         if (!SUMS && dr) { hv[j].x += d[j].get(0); hv[j].y += d[j].get(1); hv[j].z += d[j].get(2); hv[j].w += d[j].get(3); }
         if (i < hidden) {
             if (write_back) *reinterpret_cast<float4*>(hr + i) = hv[j];
-            ss += hv[j].x * hv[j].x + hv[j].y * hv[j].y + hv[j].z * hv[j].z + hv[j].w * hv[j].w;
+            ss += squares(hv[j]);
         }
         v[j][0] = hv[j].x; v[j][1] = hv[j].y; v[j][2] = hv[j].z; v[j][3] = hv[j].w;
     }
@@ -288,7 +292,6 @@ __global__ void add_rmsnorm_vec_kernel(float* __restrict__ h, const TA* __restri
         }
     }
 }
-
 
 static int add_rmsnorm(float* h, const void* delta, const PartSums ps, int act_dtype, const void* weight,
                        int weight_dtype, float eps, const int32_t* rows, int n_rows,
