@@ -874,7 +874,7 @@ def test_the_norm_adds_up_any_number_of_pieces(rows, hidden, n_sums):
     assert ((out1.float() - out2.float()).abs() <= out1.float().abs() * 2 ** -7).all()
 
 
-@pytest.mark.parametrize("rows", [5, 70])
+@pytest.mark.parametrize("rows", [5, 70, 257])
 @pytest.mark.parametrize("hidden,n_sums", [(64, 0), (1024, 0), (3584, 0), (8192, 0), (68, 5), (1536, 3), (3584, 16), (4096, 4), (5120, 9), (8192, 14)])
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_the_norm_adds_squares_in_one_order(dtype, hidden, n_sums, rows):

@@ -135,36 +135,28 @@ struct PartSums { const float* sums; int n; size_t stride; };       // stride: r
 
 // Four values of each piece, up to MAX pieces under way together: the small kernels that add pieces up are bound by how many loads they
 // wait for one after the other (each misses every cache, about a microsecond), so they ask for all pieces at once, together with whatever
-// else they need, and look at them afterwards.
+// else they need, and look at them afterwards.  row: where the row begins in the first of `left` pieces, the same for the wave; i: the lane's
+// value in the row.  A piece that is not there costs a branch and no more: many rows are bound by bytes, few by instructions.  (Written out by the
+// template: a loop that is left early keeps the pieces in memory.)
 template <int MAX>
 struct Pieces {
     float4 p[MAX];
-    __device__ __forceinline__ void ask(const PartSums& ps, size_t at, int s0) {
-        const float* from = ps.sums + (size_t)s0 * ps.stride + at;
-#pragma unroll
-        for (int u = 0; u < MAX; ++u) {
-            if (s0 + u >= ps.n) break;              // (none is read that is not there: many rows are bound by bytes)
-            p[u] = *reinterpret_cast<const float4*>(from + (size_t)u * ps.stride);
+    template <int U = 0>
+    __device__ __forceinline__ void ask(const PartSums& ps, size_t row, int left, uint32_t i) {
+        if (left <= U) return;
+        p[U] = *reinterpret_cast<const float4*>(ps.sums + row + i);
+        if constexpr (U + 1 < MAX) {
+            size_t next = row + ps.stride;
+            asm("" : "+s"(next));               // (or all pieces' places are worked out in front of the first load, a hundred instructions)
+            ask<U + 1>(ps, next, left, i);
         }
     }
     // added in their order
-    __device__ __forceinline__ void add(const PartSums& ps, int s0, float4& a) const {
-#pragma unroll
-        for (int u = 0; u < MAX; ++u) {
-            const bool there = s0 + u < ps.n;
-            a.x = there ? a.x + p[u].x : a.x; a.y = there ? a.y + p[u].y : a.y;
-            a.z = there ? a.z + p[u].z : a.z; a.w = there ? a.w + p[u].w : a.w;
-        }
-    }
-    // the sum of all pieces, the first of which have been asked for
-    __device__ __forceinline__ float4 sum(const PartSums& ps, size_t at) {
-        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-        add(ps, 0, a);
-        for (int s = MAX; s < ps.n; s += MAX) {
-            ask(ps, at, s);
-            add(ps, s, a);
-        }
-        return a;
+    template <int U = 0>
+    __device__ __forceinline__ void add(int left, float4& a) const {
+        if (left <= U) return;
+        a.x += p[U].x; a.y += p[U].y; a.z += p[U].z; a.w += p[U].w;
+        if constexpr (U + 1 < MAX) add<U + 1>(left, a);
     }
 };
 
@@ -242,31 +234,45 @@ __global__ void add_rmsnorm_vec_kernel(float* __restrict__ h, const TA* __restri
     float* hr = h ? h + row * hidden : nullptr;
     const TA* dr = delta ? delta + row * hidden : nullptr;
     TA* o = out + (size_t)r * hidden;
-    // Everything is asked for before anything is looked at, the norm's weight too.  (Lanes past the row repeat its last values and drop them.)
+    // Everything is asked for before anything is looked at, the norm's weight too.  (Lanes past the row repeat its last values and drop them, and so do
+    // waves past it, but for those of rows narrower than a block and the second half of long rows of sums: elsewhere the branch costs more.)
     constexpr bool EARLY_W = VPT <= 4;
     float v[VPT][4];
     float4 hv[VPT];
     Vec4<TA> d[VPT];
     Vec4<TW> w[VPT];
     auto place = [&](int j) { return min((int)(j * blockDim.x + threadIdx.x) * 4, hidden - 4); };
+    const int wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x);
+    auto live = [&](int j) { return (SUMS == 0 ? VPT > 1 : j == 0 || SUMS < 8) || (j * (int)blockDim.x + wave0) * 4 < hidden; };
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
         const int i = place(j);
         hv[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (!live(j)) continue;
         if (hr) hv[j] = *reinterpret_cast<const float4*>(hr + i);
         if (!SUMS && dr) d[j].v = *reinterpret_cast<const decltype(d[j].v)*>(dr + i);
         if (EARLY_W) w[j].v = *reinterpret_cast<const decltype(w[j].v)*>(weight + i);
     }
     if constexpr (SUMS > 0) {
         Pieces<SUMS> p[VPT];
+        float4 a[VPT];
 #pragma unroll
-        for (int j = 0; j < VPT; ++j) p[j].ask(ps, row * hidden + place(j), 0);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int j = 0; j < VPT; ++j) a[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+        size_t at = row * hidden;
+        for (int left = ps.n; left > 0; left -= SUMS, at += SUMS * ps.stride) {
+#pragma unroll
+            for (int j = 0; j < VPT; ++j)
+                if (live(j)) p[j].ask(ps, at, left, place(j));
+            asm("" : "+s"(left));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < VPT; ++j)
+                if (live(j)) p[j].add(left, a[j]);
+        }
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
-            const float4 a = p[j].sum(ps, row * hidden + place(j));
-            hv[j].x += to_float(from_float<TA>(a.x)); hv[j].y += to_float(from_float<TA>(a.y));
-            hv[j].z += to_float(from_float<TA>(a.z)); hv[j].w += to_float(from_float<TA>(a.w));
+            hv[j].x += to_float(from_float<TA>(a[j].x)); hv[j].y += to_float(from_float<TA>(a[j].y));
+            hv[j].z += to_float(from_float<TA>(a[j].z)); hv[j].w += to_float(from_float<TA>(a[j].w));
         }
     }
     float ss = 0.f;
@@ -309,13 +315,15 @@ static int add_rmsnorm(float* h, const void* delta, const PartSums ps, int act_d
     if (hidden % 4 == 0 && hidden <= 8192 && aligned) {
         // Sums of a product are several times the bytes per row, of few rows: a thread for every four values (no more, waves without any cost time
         // too) and all pieces asked for together, with the norm's weight.  32 rows of 1536, 14 and 3 pieces: 4.64 -> 4.04 us (a step of
-        // the 1.5B shape 0.7 % less); 64 rows of 3584, 9 and 7 pieces: 5.16 either way, what a compute unit brings in of its row.  More rows than that
-        // are bound by bytes: 232 rows of 3584, 6 and 3 pieces 7.24 us with all of them under way, 7.0 with four.
+        // the 1.5B shape 0.7 % less); 64 rows of 3584, 9 and 7 pieces: 5.16 either way, what a compute unit brings in of its row.  With more rows
+        // than units other blocks' waves hide a round and their number counts: 2048 rows of 3584, 5120 and 8192 values, 3 pieces, 29.5, 41.3
+        // and 65.8 us with all of them under way, 25.8, 34.9 and 57.4 with four; up to 232 rows it is 4.6 either way, 5.3 against 5.7, 7.3 against 7.1,
+        // and with 9 pieces 6.3 either way, 10.9 against 11.0 and 16.1 against 16.0 (65 rows 4.6 against 4.8, 5.4 against 6.3, 7.0 either way).
         const int threads = !ps.sums ? 256 : hidden < 4096 ? (hidden / 4 + TQK_WAVE - 1) / TQK_WAVE * TQK_WAVE : 1024;
 #define LAUNCHV(TA, TW, VPT, SUMS) add_rmsnorm_vec_kernel<TA, TW, VPT, SUMS><<<n_rows, threads, 0, s>>>( \
         h, (const TA*)delta, ps, (const TW*)weight, eps, rows, hidden, (TA*)out, write_back)
 #define PICK(TA, TW) do { const int per = (hidden + threads * 4 - 1) / (threads * 4); \
-        if (ps.sums && n_rows > 64) { if (per <= 1) LAUNCHV(TA, TW, 1, 4); else LAUNCHV(TA, TW, 2, 4); } \
+        if (ps.sums && n_rows > 256) { if (per <= 1) LAUNCHV(TA, TW, 1, 4); else LAUNCHV(TA, TW, 2, 4); } \
         else if (ps.sums) { if (per <= 1) LAUNCHV(TA, TW, 1, 16); else LAUNCHV(TA, TW, 2, 8); } \
         else if (per <= 1) LAUNCHV(TA, TW, 1, 0); else if (per <= 2) LAUNCHV(TA, TW, 2, 0); \
         else if (per <= 4) LAUNCHV(TA, TW, 4, 0); else LAUNCHV(TA, TW, 8, 0); } while (0)
