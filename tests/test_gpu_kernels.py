@@ -487,6 +487,29 @@ def test_attention_generic_gives_few_queries_the_bits_of_many(dtype, d, window):
     torch.testing.assert_close(few.float().cpu(), want, **TOL[dtype])
 
 
+@pytest.mark.parametrize("n", [2, 200])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("what,pages", [("-inf", (0, 1, 2, 9, 21)), ("-inf", (6, 14)), ("nan", (0, 1, 2, 9, 21)), ("nan", (6, 14))])
+def test_attention_generic_takes_pages_of_infinite_scores(dtype, what, pages, n):
+    """Keys of whole pages at -inf, so that their scores are: they have weight 0 wherever they lie (first page of the context or of a stripe of
+    pages, the last one, pages next to each other, all of a stripe).  Not-a-numbers show.  A wave a query (200 x 3 heads) and one for each stripe."""
+    nh, nkv, d, act, s = 3, 1, 64, DT[dtype], 1400
+    k, v = rand(nkv, s, d, seed=100).to(act).float().cpu(), rand(nkv, s, d, seed=101).to(act).float().cpu()
+    q = rand(n, nh, d, seed=102).to(act).float().cpu()
+    q[..., 0] = q[..., 0].abs() + 0.1                       # so that a key's -inf in element 0 is a score of -inf
+    for page in pages:
+        k[:, 64 * page:64 * page + 64, 0] = float(what)
+    page_ids = list(range(22))
+    keys, values = paged(k, v, page_ids, 22, act)
+    pos = torch.tensor([1399, 1330] * (n // 2))
+    out = torch.empty(n, nh * d, dtype=act, device=DEV)
+    K.attention(q.to(act).to(DEV), keys, values, ints([0] * n), pos.to(torch.int32).to(DEV), ints([page_ids]), 0, d ** -0.5, out)
+    if what == "nan":
+        assert torch.isnan(out).all()
+    else:
+        torch.testing.assert_close(out.float().cpu(), attention_reference(q, k, v, pos, 0, d ** -0.5), **TOL[dtype])
+
+
 def test_attention_generic_two_sequences_share_nothing():
     nh, nkv, d = 4, 2, 32
     ka, va = rand(nkv, 100, d, seed=15).cpu(), rand(nkv, 100, d, seed=16).cpu()

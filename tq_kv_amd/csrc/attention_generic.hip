@@ -35,6 +35,13 @@ __device__ __forceinline__ float4 load4(const bf16_t* p) {
 // lane j's value, j the same for the whole wave
 __device__ __forceinline__ float lane_value(float v, int j) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), j)); }
 
+// What scores are taken from before their exponential: the maximum so far, or 0 while every score is -inf (a stripe may begin with such pages), so that
+// those have weight 0 and what follows counts as if they were not there.
+__device__ __forceinline__ float from_max(float m) { return m == -INFINITY ? 0.f : m; }
+
+// A stripe's first page from `first` on.
+__device__ __forceinline__ int page_of(int stripe, int first) { return first + (stripe - first % ATT_STRIPES + ATT_STRIPES) % ATT_STRIPES; }
+
 // What a stripe leaves: maximum, sum, and this lane's output elements.
 struct Stripe {
     float m, l, acc[ATT_MAX_D / TQK_WAVE];
@@ -52,8 +59,7 @@ __device__ __forceinline__ Stripe walk(int stripe, const float* qf, const T* key
     for (int i = 0; i < NACC; ++i) r.acc[i] = 0.f;
     r.m = -INFINITY;
     r.l = 0.f;
-    const int first = lo / TQK_PAGE;
-    for (int pg = first + (stripe - first % ATT_STRIPES + ATT_STRIPES) % ATT_STRIPES; pg * TQK_PAGE <= pos; pg += ATT_STRIPES) {
+    for (int pg = page_of(stripe, lo / TQK_PAGE); pg * TQK_PAGE <= pos; pg += ATT_STRIPES) {
         const int kb = pg * TQK_PAGE, page = pages[pg];
         const int j = kb + lane;
         const bool valid = j >= lo && j <= pos && page >= 0;
@@ -76,9 +82,9 @@ __device__ __forceinline__ Stripe walk(int stripe, const float* qf, const T* key
             for (; i < head_dim; ++i) dot = fmaf(qf[i], to_float(kr[i]), dot);
             s = dot * scale;
         }
-        const float m_new = fmaxf(r.m, wave_max(s));    // finite: the page holds at least one key of lo .. pos
-        const float p = valid ? expf(s - m_new) : 0.f;
-        const float alpha = expf(r.m - m_new);          // exp(-inf) = 0 on the stripe's first page
+        const float m_new = fmaxf(r.m, wave_max(s)), m_at = from_max(m_new);
+        const float p = valid ? expf(s - m_at) : 0.f;
+        const float alpha = expf(r.m - m_at);           // exp(-inf) = 0 on the stripe's first page
         r.l = fmaf(r.l, alpha, wave_sum(p));
         r.m = m_new;
         const int n_keys = min(TQK_PAGE, pos - kb + 1);
@@ -115,9 +121,9 @@ __device__ __forceinline__ Stripe walk(int stripe, const float* qf, const T* key
 
 // The next stripe joins the ones before it: what the sums so far and the stripe's are multiplied by.
 __device__ __forceinline__ void join(float& m, float& l, float stripe_m, float stripe_l, float& of_sum, float& of_stripe) {
-    const float mn = fmaxf(m, stripe_m);
-    of_sum = expf(m - mn);                              // exp(-inf) = 0 for the first one
-    of_stripe = expf(stripe_m - mn);
+    const float mn = fmaxf(m, stripe_m), at = from_max(mn);
+    of_sum = expf(m - at);                              // exp(-inf) = 0 for the first one
+    of_stripe = expf(stripe_m - at);
     l = fmaf(l, of_sum, stripe_l * of_stripe);
     m = mn;
 }
@@ -145,7 +151,7 @@ void attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ key
     __syncthreads();
     if (!live) return;
 
-    const int pos = tok_pos[t];
+    const int pos = __builtin_amdgcn_readfirstlane(tok_pos[t]);
     const int32_t* pages = page_table + (size_t)tok_seq[t] * table_width;
     const int kvh = head / (n_heads / n_kv_heads);
     const int lo = window > 0 ? max(0, pos - window + 1) : 0;
@@ -173,7 +179,7 @@ void attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ key
         const int c = threadIdx.x;
         if (c >= head_dim) return;
         for (int s = 0; s < ATT_STRIPES; ++s) {
-            if (ml[s][0] == -INFINITY) continue;        // no page
+            if (page_of(s, lo / TQK_PAGE) * TQK_PAGE > pos) continue;
             join(m, l, ml[s][0], ml[s][1], of_sum, of_stripe);
             acc = fmaf(acc, of_sum, met[s][c] * of_stripe);
         }
@@ -183,8 +189,8 @@ void attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ key
 #pragma unroll
         for (int a = 0; a < NACC; ++a) acc[a] = 0.f;
         for (int s = 0; s < ATT_STRIPES; ++s) {
+            if (page_of(s, lo / TQK_PAGE) * TQK_PAGE > pos) continue;
             const Stripe r = walk<T, 8>(s, qf, keys, values, pages, pos, lo, kvh, n_kv_heads, head_dim, scale, wide_keys, wide_values, lane);
-            if (r.m == -INFINITY) continue;
             join(m, l, r.m, r.l, of_sum, of_stripe);
 #pragma unroll
             for (int a = 0; a < NACC; ++a) acc[a] = fmaf(acc[a], of_sum, r.acc[a] * of_stripe);
