@@ -487,6 +487,24 @@ def test_attention_generic_gives_few_queries_the_bits_of_many(dtype, d, window):
     torch.testing.assert_close(few.float().cpu(), want, **TOL[dtype])
 
 
+@pytest.mark.parametrize("few", [True, False])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("d", [4, 12, 36, 64, 100, 116, 148, 196, 250, 256])
+def test_attention_generic_at_any_head_size_and_context(d, dtype, few):
+    """Head sizes and contexts that end in every kind of remainder of the loads taken together (16, 8, 4 and single ones), with and without a
+    window that begins inside a page."""
+    nh, nkv, act, s = 2, 1, DT[dtype], 200
+    k, v = rand(nkv, s, d, seed=103).to(act).float().cpu(), rand(nkv, s, d, seed=104).to(act).float().cpu()
+    page_ids = [2, 0, 3, 1]
+    keys, values = paged(k, v, page_ids, 4, act)
+    pos = torch.tensor([0, 2, 3, 6, 14, 15, 16, 31, 34, 47, 50, 62, 63, 64, 100, 127, 191, 199] * (1 if few else 15))
+    q = rand(len(pos), nh, d, seed=105).to(act).float().cpu()
+    for window in (0, 37):
+        out = torch.empty(len(pos), nh * d, dtype=act, device=DEV)
+        K.attention(q.to(act).to(DEV), keys, values, ints([0] * len(pos)), pos.to(torch.int32).to(DEV), ints([page_ids]), window, d ** -0.5, out)
+        torch.testing.assert_close(out.float().cpu(), attention_reference(q, k, v, pos, window, d ** -0.5), **TOL[dtype])
+
+
 @pytest.mark.parametrize("n", [2, 200])
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("what,pages", [("-inf", (0, 1, 2, 9, 21)), ("-inf", (6, 14)), ("nan", (0, 1, 2, 9, 21)), ("nan", (6, 14))])

@@ -35,6 +35,39 @@ __device__ __forceinline__ float4 load4(const bf16_t* p) {
 // lane j's value, j the same for the whole wave
 __device__ __forceinline__ float lane_value(float v, int j) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), j)); }
 
+// dot + the product of 4 N elements, in their order, N loads under way together
+template <int N, typename T>
+__device__ __forceinline__ float key_dot(const float* q, const T* k, float dot) {
+    float4 kv[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) kv[u] = load4(k + 4 * u);
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        const float4 qv = *reinterpret_cast<const float4*>(q + 4 * u);
+        dot = fmaf(qv.x, kv[u].x, dot);
+        dot = fmaf(qv.y, kv[u].y, dot);
+        dot = fmaf(qv.z, kv[u].z, dot);
+        dot = fmaf(qv.w, kv[u].w, dot);
+    }
+    return dot;
+}
+
+// sum + the weighted values of 4 N positions from j on (a multiple of four), in their order, N loads under way together
+template <int N, typename T>
+__device__ __forceinline__ float value_sum(const T* row, float p, int j, float sum) {
+    float4 v[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) v[u] = load4(row + value_place(j + 4 * u));
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        sum = fmaf(lane_value(p, j + 4 * u), v[u].x, sum);
+        sum = fmaf(lane_value(p, j + 4 * u + 1), v[u].y, sum);
+        sum = fmaf(lane_value(p, j + 4 * u + 2), v[u].z, sum);
+        sum = fmaf(lane_value(p, j + 4 * u + 3), v[u].w, sum);
+    }
+    return sum;
+}
+
 // What scores are taken from before their exponential: the maximum so far, or 0 while every score is -inf (a stripe may begin with such pages), so that
 // those have weight 0 and what follows counts as if they were not there.
 __device__ __forceinline__ float from_max(float m) { return m == -INFINITY ? 0.f : m; }
@@ -70,14 +103,11 @@ __device__ __forceinline__ Stripe walk(int stripe, const float* qf, const T* key
             float dot = 0.f;
             int i = 0;
             if (wide_keys) {
-#pragma unroll UNROLL
-                for (; i < head_dim; i += 4) {
-                    const float4 k = load4(kr + i), qv4 = *reinterpret_cast<const float4*>(qf + i);
-                    dot = fmaf(qv4.x, k.x, dot);
-                    dot = fmaf(qv4.y, k.y, dot);
-                    dot = fmaf(qv4.z, k.z, dot);
-                    dot = fmaf(qv4.w, k.w, dot);
-                }
+                // (fewer loads at a time for what is left of the head, or of a small one, and not one)
+                if (UNROLL > 8) for (; i + 64 <= head_dim; i += 64) dot = key_dot<16>(qf + i, kr + i, dot);
+                for (; i + 32 <= head_dim; i += 32) dot = key_dot<8>(qf + i, kr + i, dot);
+                for (; i + 16 <= head_dim; i += 16) dot = key_dot<4>(qf + i, kr + i, dot);
+                for (; i < head_dim; i += 4) dot = key_dot<1>(qf + i, kr + i, dot);
             }
             for (; i < head_dim; ++i) dot = fmaf(qf[i], to_float(kr[i]), dot);
             s = dot * scale;
@@ -102,14 +132,9 @@ __device__ __forceinline__ Stripe walk(int stripe, const float* qf, const T* key
                 int jj = first_key;
                 for (; jj < n_keys && jj % 4 != 0; ++jj) one(jj);
                 if (wide_values) {
-#pragma unroll UNROLL / 2
-                    for (; jj + 4 <= n_keys; jj += 4) {
-                        const float4 v = load4(row + value_place(jj));
-                        sum = fmaf(lane_value(p, jj), v.x, sum);
-                        sum = fmaf(lane_value(p, jj + 1), v.y, sum);
-                        sum = fmaf(lane_value(p, jj + 2), v.z, sum);
-                        sum = fmaf(lane_value(p, jj + 3), v.w, sum);
-                    }
+                    if (UNROLL > 8) for (; jj + 32 <= n_keys; jj += 32) sum = value_sum<8>(row, p, jj, sum);
+                    for (; jj + 16 <= n_keys; jj += 16) sum = value_sum<4>(row, p, jj, sum);
+                    for (; jj + 4 <= n_keys; jj += 4) sum = value_sum<1>(row, p, jj, sum);
                 }
                 for (; jj < n_keys; ++jj) one(jj);
             }
@@ -128,8 +153,9 @@ __device__ __forceinline__ void join(float& m, float& l, float stripe_m, float s
     m = mn;
 }
 
-// Bound by latency, a page costs a wave 8 us: the float32 step of one token after 300 (28 heads of 128) takes 17.6 us with a wave per stripe and
-// 16 loads under way, 45.9 with one wave for all and 8; the prompt of 300 190 us.
+// Bound by latency, a page costs a wave 6 us: the float32 step of four tokens after 300 (28 heads of 128) takes 13.6 us with a wave per stripe and
+// up to 16 loads under way, 37.0 with one wave for all and up to 8.  What is left of a head or a page after the last 16 loads goes by
+// 8 and 4 before single ones: one after the other it was most of the time of small heads and short contexts (heads of 32, 20 positions 5.4 -> 4.5 us).
 // SPLIT: a block of a wave per stripe for one query.
 template <typename T, bool SPLIT>
 __global__ __launch_bounds__((SPLIT ? ATT_STRIPES : ATT_WAVES) * TQK_WAVE)
@@ -138,20 +164,19 @@ void attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ key
                               const int32_t* __restrict__ page_table, int table_width, int window, float scale,
                               T* __restrict__ out, int n_tokens, int n_heads, int n_kv_heads, int head_dim, int wide_keys, int wide_values) {
     constexpr int NACC = ATT_MAX_D / TQK_WAVE;
-    __shared__ __attribute__((aligned(16))) float q_lds[SPLIT ? 1 : ATT_WAVES][ATT_MAX_D];
-    const int wave = threadIdx.x / TQK_WAVE, lane = threadIdx.x % TQK_WAVE;
+    __shared__ __attribute__((aligned(16))) float q_lds[SPLIT ? ATT_STRIPES : ATT_WAVES][ATT_MAX_D];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TQK_WAVE), lane = threadIdx.x % TQK_WAVE;
     const int t = SPLIT ? blockIdx.x : blockIdx.x * ATT_WAVES + wave;
     const int head = blockIdx.y;
-    const bool live = t < n_tokens;
-    float* qf = q_lds[SPLIT ? 0 : wave];
-    if (live) {
-        const T* qv = q + ((size_t)t * n_heads + head) * head_dim;
-        for (int i = SPLIT ? threadIdx.x : lane; i < head_dim; i += SPLIT ? blockDim.x : TQK_WAVE) qf[i] = to_float(qv[i]);
-    }
-    __syncthreads();
-    if (!live) return;
+    if (t >= n_tokens) return;
+    // (every wave keeps a copy of its query: nobody waits for anybody, and waves without a page are gone at once)
+    float* qf = q_lds[wave];
+    const T* qv = q + ((size_t)t * n_heads + head) * head_dim;
+    for (int i = lane; i < head_dim; i += TQK_WAVE) qf[i] = to_float(qv[i]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 
-    const int pos = __builtin_amdgcn_readfirstlane(tok_pos[t]);
+    const int pos = tok_pos[t];
     const int32_t* pages = page_table + (size_t)tok_seq[t] * table_width;
     const int kvh = head / (n_heads / n_kv_heads);
     const int lo = window > 0 ? max(0, pos - window + 1) : 0;
@@ -218,8 +243,10 @@ extern "C" int tqk_attention(const void* q, const void* keys, const void* values
     TQK_REQUIRE(window >= 0, "tqk_attention: negative window");
     if (n_tokens == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
-    // A wave per stripe (45.9 -> 17.6 us, one token after 300, 28 heads) while no unit gets more than two blocks of them; the results are the same.
-    // One page is one wave's work either way.
+    // A wave per stripe while no unit gets more than two blocks of them; the results are the same.  us with a wave per stripe and with one for all,
+    // float32, 28 heads of 128: 504 waves of queries after 20, 128, 300 and 1500 positions 6.3, 12.1, 23.0, 97 and 7.3, 18.7, 37.5, 173; 616 of them 6.8, 19.5,
+    // 39.4, 137 and 7.3, 18.8, 37.7, 173; 1008 of them 7.5, 21.2, 41.5, 187 and 7.3, 19.1, 37.6, 173.  Heads of 32: 512 4.5, 6.5, 9.2, 29 and 4.9, 8.9, 15.9, 61;
+    // 616 4.9, 10.1, 14.9, 40 and 4.9, 9.0, 16.1, 60; 2048 7.4, 18.5, 28.1, 97 and 5.6, 11.9, 23.3, 96.  bfloat16 alike.
     const bool split = (long long)n_tokens * n_heads <= 512;
     const dim3 grid(split ? n_tokens : (n_tokens + ATT_WAVES - 1) / ATT_WAVES, n_heads);
     // four elements a load where keys and values begin at a multiple of four elements (a caller's memory need not) and rows of keys do, too
