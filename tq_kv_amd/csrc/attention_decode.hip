@@ -169,8 +169,10 @@ struct RowFinish {
 // positions (bits to keep are found once for all elements now), the sums 1.3 in front of the page's loads instead of over them, and the
 // waves' results 1.3 when one wave added up all of them.  ms a step, together: 7B, 1, 8 and 64 sequences 2.882 -> 2.832, 3.130 -> 3.058 and
 // 3.921 -> 3.793; 1.5B, 32 sequences 1.766 -> 1.657; 32B with 8 layers, 16 sequences 1.843 -> 1.816.
-// SUMS: q, k and v come as `in` and are finished here (keys and values are then written, too, so nothing promises that they are not).
-template <int D, bool NT, int W, bool SUMS>
+// SUMS: q, k and v come as `in` and are finished here (keys and values are then written, too, so nothing promises that they are not); SUMS_EARLY: the
+// first page is asked for while the sums are added up.
+enum { NO_SUMS = 0, SUMS_FIRST = 1, SUMS_EARLY = 2 };
+template <int D, bool NT, int W, int SUMS>
 __global__ __launch_bounds__(AD_WAVES * TQK_WAVE)
 void attention_decode_kernel(const DecodeSums in, const bf16_t* __restrict__ q, const bf16_t* keys,
                              const bf16_t* values, const int32_t* __restrict__ tok_pos,
@@ -185,7 +187,7 @@ void attention_decode_kernel(const DecodeSums in, const bf16_t* __restrict__ q, 
     // (Worth it where the step reads so much that the memory's rate counts, which is where the loads are marked as
     // read-once, NT: 64 sequences of 2100 positions 56.2 -> 49.7 us, 128 sequences 106 -> 89 us; 8 sequences 13.2 -> 14.2.)
     constexpr bool VIA_LDS = D == 128 && NT;
-    constexpr bool EARLY = SUMS && D <= 128;           // the first page is asked for while the sums are added up: where the registers hold both
+    constexpr bool EARLY = SUMS == SUMS_EARLY;
     constexpr int XCH_WAVE = DB * TQK_WAVE + TQK_WAVE / 2;      // pieces of 16 bytes a wave hands over: its out^T values, m, l
     constexpr int XCH = W > 1 ? W * XCH_WAVE : 1, TURN = VIA_LDS ? W * 1024 : 0;
     __shared__ u32x4_t lds_all[XCH > TURN ? XCH : TURN];
@@ -198,7 +200,7 @@ void attention_decode_kernel(const DecodeSums in, const bf16_t* __restrict__ q, 
     const int seq = blockIdx.z;
     const int n_rep = n_heads / n_kv_heads;
     // What a block waits for before its pages is a chain of loads that miss all caches, about a microsecond each, so nothing waits that need not:
-    // without a window the wave's first page is asked for together with the position, and the sums before both.
+    // without a window the name of the wave's first page is asked for first, then the sums, then the position, and none is looked at before.
     const int32_t* pages = page_table + (size_t)seq * table_width;
     int page = 0;
     if (window == 0) page = __builtin_amdgcn_readfirstlane(pages[min(part + wave * n_parts, table_width - 1)]);
@@ -573,8 +575,13 @@ static int attention_decode(const DecodeSums& in, const void* q, const void* key
     const bool one = n_parts > 1 && n_parts >= table_width;
     // Sums are finished by blocks of four waves alone: fewer lanes take the heads' values in two or three rounds (20 rows of 200 positions at the
     // 7B sizes, blocks of one wave: 3.435 ms a step against 3.400 with the rotation's own kernel).
+    // The first page beside the sums, where the registers hold both (heads up to 128) and a unit gets one block: with both there is room for one only.  us
+    // beside and after the sums, 8 kv heads of 128: 64 rows of up to 24, 200 and 1000 positions 13.6, 18.9, 45.1 and 8.5, 14.5, 46.5, 100 rows
+    // 25.7, 33.7, 73.3 and 14.3, 31.3, 73.9; 4 kv heads, 100 rows 13.2, 17.5, 40.7 and 8.1, 13.5, 40.9.  One block a unit: see the kernel.
+    const bool early = in.sums && (long long)n_seqs * n_kv_heads * q_blocks * n_parts <= 256;
 #define LAUNCH_W(DD, W, SUMS) { if (nt) LAUNCH_S(DD, true, W, SUMS); else LAUNCH_S(DD, false, W, SUMS); }
-#define LAUNCH(DD) { if (in.sums) LAUNCH_W(DD, 4, true) else if (one) LAUNCH_W(DD, 1, false) else if (two) LAUNCH_W(DD, 2, false) else LAUNCH_W(DD, 4, false) }
+#define LAUNCH(DD) { if (early && DD <= 128) LAUNCH_W(DD, 4, (DD <= 128 ? SUMS_EARLY : SUMS_FIRST)) else if (in.sums) LAUNCH_W(DD, 4, SUMS_FIRST) \
+        else if (one) LAUNCH_W(DD, 1, NO_SUMS) else if (two) LAUNCH_W(DD, 2, NO_SUMS) else LAUNCH_W(DD, 4, NO_SUMS) }
     switch (head_dim) {
         case 32: LAUNCH(32); break;
         case 64: LAUNCH(64); break;
