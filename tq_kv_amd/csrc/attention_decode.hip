@@ -488,17 +488,19 @@ void attention_decode_kernel(const DecodeSums in, const bf16_t* __restrict__ q, 
     if (n_parts > 1 && wave == 0 && g == 0) { part_ml[row * 2] = m; part_ml[row * 2 + 1] = l; }
 }
 
-// sum + weight * value, each rounded on its own whatever the code around it is (the weights' sum is fused): a decoding step's bits go by it.
-__device__ __forceinline__ float added(float sum, float weight, float value) {
+// weight * value, rounded whatever is done with it (the compiler would fuse it with the sum it goes into): a decoding step's bits go by it.
+__device__ __forceinline__ float rounded_product(float weight, float value) {
 #pragma clang fp contract(off)
-    return sum + weight * value;
+    return weight * value;
 }
 
 // out[seq, head, :] = sum_p exp(m_p - M) o_p / sum_p exp(m_p - M) l_p, partitions in order.
 // Bound by the loads it waits for one after the other (each misses every cache), so those of up to 16 partitions are asked for
-// together, and up to eight partitions take one round for maxima, sums and outputs alike: with four partitions of 32 rows and 12 heads a step of the 1.5B
-// shape takes 1.65 -> 1.605 ms against a loop that took eight at a time and a remainder one after the other.  A partition without keys (m = -inf)
-// has weight 0 and its (unwritten) output is not looked at.
+// together, and up to 16 partitions take one round for maxima, sums and outputs alike: with four partitions of 32 rows and 12 heads a step of the 1.5B
+// shape takes 1.65 -> 1.605 ms against a loop that took eight at a time and a remainder one after the other.  More go by 16 and what is left by 8: in a
+// second round of 16, 17 partitions took longer than in that loop (attention and merge of 3 rows, 8 heads of 32 6.7 us, 7.1, now 6.7; 4 heads of 96, which
+// two waves share now, 8.7, 9.3, 7.2).  A partition without keys (m = -inf) has weight 0 and its (unwritten) output is not looked at.
+template <int N> struct Count { static constexpr int n = N; };
 template <int BATCH, bool ONE_ROUND>
 __global__ void attention_merge_kernel(const float* __restrict__ part_out, const float* __restrict__ part_ml,
                                        int n_parts, int head_dim, bf16_t* __restrict__ out) {
@@ -513,11 +515,13 @@ __global__ void attention_merge_kernel(const float* __restrict__ part_out, const
     for (int c = threadIdx.x; c < head_dim; c += blockDim.x) {
         float acc = 0.f, denom = 0.f;
         const float* po = part_out + row * n_parts * head_dim + c;
-        for (int p0 = 0; p0 < n_parts; p0 += BATCH) {
-            float2 s[BATCH];
-            float v[BATCH];
+        // (written out for B partitions from p0 on: what is left after rounds of 16 goes by 8)
+        auto round = [&](int p0, auto batch) __attribute__((always_inline)) {
+            constexpr int B = decltype(batch)::n;
+            float2 s[B];
+            float v[B];
 #pragma unroll
-            for (int u = 0; u < BATCH; ++u) {
+            for (int u = 0; u < B; ++u) {
                 const int p = min(p0 + u, n_parts - 1);
                 s[u] = ml[p];
                 v[u] = po[(size_t)p * head_dim];
@@ -525,16 +529,20 @@ __global__ void attention_merge_kernel(const float* __restrict__ part_out, const
             __builtin_amdgcn_sched_barrier(0);
             if (ONE_ROUND) {
 #pragma unroll
-                for (int u = 0; u < BATCH; ++u) M = fmaxf(M, s[u].x);
+                for (int u = 0; u < B; ++u) M = fmaxf(M, s[u].x);
             }
 #pragma unroll
-            for (int u = 0; u < BATCH; ++u) {
+            for (int u = 0; u < B; ++u) {
                 const bool live = s[u].x != -INFINITY && p0 + u < n_parts;
                 const float wgt = live ? __builtin_amdgcn_exp2f(s[u].x - M) : 0.f;
-                denom = live ? fmaf(wgt, s[u].y, denom) : denom;
-                acc = live ? added(acc, wgt, v[u]) : acc;
+                denom = fmaf(wgt, s[u].y, denom);
+                acc += live ? rounded_product(wgt, v[u]) : 0.f;
             }
-        }
+        };
+        // (a loop where there is one round, too: without it maxima are looked at before outputs are asked for)
+        int p0 = 0;
+        for (; ONE_ROUND ? p0 < n_parts : p0 + BATCH <= n_parts; p0 += BATCH) round(p0, Count<BATCH>{});
+        if (!ONE_ROUND) for (; p0 < n_parts; p0 += 8) round(p0, Count<8>{});
         out[row * head_dim + c] = from_float<bf16_t>(acc / denom);
     }
 }
@@ -594,10 +602,11 @@ static int attention_decode(const DecodeSums& in, const void* q, const void* key
 #undef LAUNCH
     if (tqk_check_launch("tqk_attention_decode")) return -1;
     if (n_parts == 1) return 0;
-    const int threads = head_dim >= 128 ? 128 : 64;
+    const int threads = head_dim > 64 ? 128 : 64;
 #define MERGE(BATCH, ONE) attention_merge_kernel<BATCH, ONE><<<n_seqs * n_heads, threads, 0, s>>>((const float*)part_out, (const float*)part_ml, n_parts, head_dim, (bf16_t*)out)
     if (n_parts <= 4) MERGE(4, true);
     else if (n_parts <= 8) MERGE(8, true);
+    else if (n_parts <= 16) MERGE(16, true);
     else MERGE(16, false);
 #undef MERGE
     return tqk_check_launch("tqk_attention_decode merge");
