@@ -393,16 +393,25 @@ template <int MT> struct MidWide { enum { tn = MT == 2 ? 5 : MT == 4 ? 6 : 3, wa
 // its own weights, so what the busiest unit brings in is rounds of blocks times (tiles of a block + groups of rows of x), each 32 K bytes.
 // us at 32, 64 and 128 rows, against two tiles a wave and as many waves as leave the fewest units idle: the 7B head 194, 231, 236 -> 172, 178,
 // 219; the 1.5B one 89, 105, 115 -> 83, 91, 112; gate+up of the 1.5B shape (187 blocks of three waves for 140 of four) 15.7, 19.5, 25.9 ->
-// 12.8, 15.6, 21.6.
-static void mid_waves(MidPlan& plan, int N, bool gated, int mt, int wide_tn, int wide_waves) {
+// 12.8, 15.6, 21.6.  Beyond that (us, weights that no cache holds):
+//  - A round more than one costs its start and end, two tiles' worth: 128256 features, K of 4096, 20, 32 and 64 rows 183, 191 and 199 us in two rounds
+//    of two tiles by eight waves, 157, 159 and 164 in one of five or six by six or seven.
+//  - Blocks that lie a power of two from 256 KB on apart ask the same channels of memory at the same time, and up to 64 rows nothing hides it: K of 2048, 32000
+//    features 28.5 and 30.3 us at 20 and 64 rows by eight waves (512 KB), 23.0 and 25.2 by five of two tiles; K of 1024, 64000 features 32.2 in 250
+//    such blocks, 25.3 in 400 others.  At 128 rows 32.2 and 30.0, 38.9 and 36.0, K of 4096 and 32000 features 48.6 and 53.3: not counted there.
+//  - More than two tiles a wave pay for themselves in long runs of K: 152064 features, 64 and 128 rows, K of 512 41.7 and 53.2 us with them, 37.8 and
+//    48.4 without, K of 1024 64.5 and 77.8, 61.3 and 71.5; K of 2048 106.6 and 126.5, 110.5 and 121.8; K of 3584 174 and 212, 203 and 220.
+static void mid_waves(MidPlan& plan, int N, int K, bool gated, int mt, int wide_tn, int wide_waves) {
     const int tiles = ((gated ? N / 2 : N) + 15) / 16;
-    int best = 1 << 30;
+    long long best = 1LL << 62;
     const int tns[3] = {1, 2, wide_tn};
-    for (int i = 0; i < (gated ? 1 : 3); ++i)
+    for (int i = 0; i < (gated ? 1 : K >= 1536 ? 3 : 2); ++i)
         for (int waves = MID_LEAST_WAVES; waves <= (i == 2 ? wide_waves : MID_MAX_WAVES); ++waves) {
             const int tn = gated ? 2 : tns[i];
             const int items = gated ? tiles : (tiles + tn - 1) / tn, blocks = (items + waves - 1) / waves, rounds = (blocks + MID_UNITS - 1) / MID_UNITS;
-            const int cost = rounds * (waves * tn + mt);
+            const long long apart = (long long)waves * tn * K * 32;
+            const bool same_channels = !gated && mt <= 4 && apart >= 256 * 1024 && (apart & (apart - 1)) == 0;
+            const long long cost = (long long)rounds * (waves * tn * (same_channels ? 17 : 10) + mt * 10) + (gated ? 0 : (rounds - 1) * 20);
             if (cost < best) { best = cost; plan.tn = tn; plan.waves = waves; plan.blocks = blocks; }
         }
 }
@@ -412,7 +421,7 @@ static int launch_rows(const MidArgs& a, MidPlan plan, bool finish, hipStream_t 
     constexpr int W = MID_MAX_WAVES;
     constexpr bool GATED = EPI == MID_GATED;
     using Wide = MidWide<MT>;
-    if (plan.splits == 1 && !a.group_rows) mid_waves(plan, a.N, GATED, MT, Wide::tn, Wide::waves);
+    if (plan.splits == 1 && !a.group_rows) mid_waves(plan, a.N, a.K, GATED, MT, Wide::tn, Wide::waves);
     if (GATED || plan.tn == 2) return launch_mid<MT, 2, EPI, TY, W>(a, plan, finish, s);
     if constexpr (!GATED) {
         if (plan.tn == Wide::tn) return launch_mid<MT, Wide::tn, EPI, TY, Wide::waves>(a, plan, finish, s);
