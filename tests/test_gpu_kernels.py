@@ -828,8 +828,8 @@ def test_product_of_17_to_128_rows(m, n, k):
         K.mid_store(x, w, out)
 
 
-# Wide products, whose waves take 1, 2 or more tiles each by the number of rows, and gated ones of 3 to 8 waves a block; K that ends in the middle of
-# a stage of 64, before the ring of stages is full (96, 160) and after it has gone round (416, 928).
+# Wide products, whose waves take 1 or 2 tiles each, and gated ones of 3 to 8 waves a block; K that ends in the middle of a stage of 64, before the ring
+# of stages is full (96, 160) and after it has gone round (416, 928).
 @pytest.mark.parametrize("m", [17, 33, 65, 128])
 @pytest.mark.parametrize("n,k", [(16400, 160), (20000, 416), (40010, 352), (77000, 928), (152064, 96)])
 def test_wide_products_of_17_to_128_rows(m, n, k):
@@ -839,6 +839,31 @@ def test_wide_products_of_17_to_128_rows(m, n, k):
     # up to 928 sums in float32, each rounded to 2^-24 of a sum of size about 3
     torch.testing.assert_close(out[:m].double(), x.double() @ w.double().t(), atol=928 * 3 * 2.0 ** -24, rtol=1e-5)
     assert torch.isnan(out[m]).all()
+
+
+# Long K, so that the weights' registers are asked for again many times and the ring of x goes round: every number of tiles a wave takes at each
+# number of rows' groups (tests/test_kernel_library.py holds the list to that), K in whole stages of 64 and ending in half of one.
+MID_LONG_SIZES = [(m, n, k) for n, k in ((65610, 1568), (152064, 1536), (32000, 2080), (40010, 1568)) for m in (17, 32, 33, 64, 65, 128)]
+
+
+@pytest.mark.parametrize("m,n,k", MID_LONG_SIZES)
+def test_wide_products_of_17_to_128_rows_and_long_k(m, n, k):
+    g = torch.Generator(device=DEV).manual_seed(48)
+    x = torch.randn(m, k, generator=g, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).to(torch.bfloat16)
+    packed = K.pack_weight(w)
+    out = torch.full((m + 1, n), float("nan"), device=DEV)
+    K.mid_store(x, packed, out[:m])
+    out16 = torch.full((m + 1, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    K.mid_store(x, packed, out16[:m])
+    for first in range(0, n, 32768):
+        part = slice(first, min(n, first + 32768))
+        want = x.double() @ w[part].double().t()
+        # float32 sums: each of K additions rounds to 2^-24 of a sum that is at most that of the terms' sizes, and such errors mostly cancel
+        slack = 2.0 ** -22 * (x.double().abs() @ w[part].double().abs().t())
+        assert ((out[:m, part].double() - want).abs() <= slack).all()
+    assert torch.isnan(out[m]).all() and torch.isnan(out16[m].float()).all()
+    assert torch.equal(out16[:m], out[:m].to(torch.bfloat16))
 
 
 @pytest.mark.parametrize("m", [17, 33, 65, 128])

@@ -95,6 +95,16 @@ def test_the_sizes_of_the_prompt_products_tests_take_every_tile():
     assert kernels.prompt_tile(129, 16, 250) == -1
 
 
+def test_the_sizes_of_the_mid_products_tests_take_every_tile():
+    """Tiles a wave takes, by the rows' groups (up to 32, 64 and 128 rows); gated products always take pairs."""
+    taken = {}
+    for m, n, k in test_gpu_kernels.MID_LONG_SIZES:
+        assert kernels.library().tqk_mid_splits(n, k, 0) == 1
+        taken.setdefault(32 if m <= 32 else 64 if m <= 64 else 128, set()).add(kernels.mid_tile(m, n, k)[0])
+    assert taken == {32: {1, 2, 5}, 64: {1, 2, 6}, 128: {1, 2, 3}}
+    assert kernels.mid_tile(64, 2 * 8960, 1536, True) == (2, 3)
+
+
 @pytest.mark.parametrize("m,n,k,gated,pays", [
     (200, 512, 4096, False, False), (129, 128, 2048, False, False), (8000, 32, 1024, False, False), (1024, 16, 512, False, False),  # small and cut
     (2048, 512, 256, False, True), (300, 512, 256, False, True),                                                                  # not cut

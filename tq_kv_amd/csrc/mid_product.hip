@@ -416,12 +416,27 @@ static void mid_waves(MidPlan& plan, int N, int K, bool gated, int mt, int wide_
         }
 }
 
+// The same for the rows that M falls among.
+static void mid_waves(MidPlan& plan, int M, int N, int K, bool gated) {
+    if (M > 64) mid_waves(plan, N, K, gated, 8, MidWide<8>::tn, MidWide<8>::waves);
+    else if (M > 32) mid_waves(plan, N, K, gated, 4, MidWide<4>::tn, MidWide<4>::waves);
+    else mid_waves(plan, N, K, gated, 2, MidWide<2>::tn, MidWide<2>::waves);
+}
+
+/* Which tile a product is given, for tests: 16 times the tiles a wave takes, plus the waves that multiply. */
+extern "C" int tqk_mid_tile(int M, int N, int K, int gated) {
+    if (M <= 0 || M > MID_MAX_ROWS || N <= 0 || K <= 0) return -1;
+    MidPlan plan = mid_plan(N, K, gated != 0);
+    if (plan.splits == 1) mid_waves(plan, M, N, K, gated != 0);
+    return plan.tn * 16 + plan.waves;
+}
+
 template <int MT, int EPI, typename TY>
 static int launch_rows(const MidArgs& a, MidPlan plan, bool finish, hipStream_t s) {
     constexpr int W = MID_MAX_WAVES;
     constexpr bool GATED = EPI == MID_GATED;
     using Wide = MidWide<MT>;
-    if (plan.splits == 1 && !a.group_rows) mid_waves(plan, a.N, a.K, GATED, MT, Wide::tn, Wide::waves);
+    if (plan.splits == 1 && !a.group_rows) mid_waves(plan, a.M, a.N, a.K, GATED);
     if (GATED || plan.tn == 2) return launch_mid<MT, 2, EPI, TY, W>(a, plan, finish, s);
     if constexpr (!GATED) {
         if (plan.tn == Wide::tn) return launch_mid<MT, Wide::tn, EPI, TY, Wide::waves>(a, plan, finish, s);

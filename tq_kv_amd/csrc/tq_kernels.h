@@ -112,6 +112,7 @@ int tqk_fused_qkv(const void* x, const float* ss_parts, int n_ss_parts, float ep
  * float32 [pieces][M][N], 16-byte aligned.  finish == 0: with more than one piece the pieces'
  * sums stay in scratch (tqk_add_rmsnorm_sums adds them up) and y is not written. */
 int tqk_mid_splits(int N, int K, int gated);
+int tqk_mid_tile(int M, int N, int K, int gated);          /* which tile it takes, for tests: 16 * tiles a wave takes + waves that multiply */
 int tqk_mid_store(const void* x, const void* w_packed, void* y, int y_dtype, int M, int N, int K, void* scratch,
                   int finish, void* stream);
 /* y[M, N/2] = silu(gate) * up, w = gate rows then up rows, packed in two parts */

@@ -535,6 +535,12 @@ def _mid_scratch(m, n, k, gated, device):
     return torch.empty((splits, m, n), dtype=torch.float32, device=device) if splits > 1 else None
 
 
+def mid_tile(m, n, k, gated=False):
+    """(tiles of 16 features a wave takes, waves that multiply) of mid_store's product of these sizes (mid_gated's: n counts both parts)."""
+    tile = int(library().tqk_mid_tile(int(m), int(n), int(k), 1 if gated else 0))
+    return tile // 16, tile % 16
+
+
 def mid_store(x, weight, out=None, finish=True):
     """out[M,N] = x weight^T for up to 128 rows of bfloat16; weight: a PackedWeight; out: bfloat16
     or float32, made here (bfloat16) if not given.  finish=False: where the kernel cuts K into
