@@ -33,14 +33,13 @@
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 enum { MID_STORE = 0, MID_GATED = 1 };
 #define MID_CHUNK 128           // K is cut into multiples of it
-#define MID_MIN_WAVES 4          // waves per block that multiply: from the product's shape (mid_plan, mid_waves)
+#define MID_MIN_WAVES 4          // waves per block that multiply: in pieces or groups (mid_plan)
 #define MID_MAX_WAVES 8
-#define MID_LEAST_WAVES 3        // where K is whole
+#define MID_LEAST_WAVES 3        // where K is whole (mid_waves)
 #define MID_MAX_ROWS 128
 
 struct MidArgs {
@@ -285,9 +284,8 @@ __global__ void mid_finish_kernel(const float* __restrict__ partial, void* __res
     else ((TY*)yv)[i] = from_float<TY>(finished(gate, a));
 }
 
-// How a product of this shape is cut: tiles per wave, waves per block, splits of K.  From N and K
-// alone.  Measured: the time is that of the compute unit with the most blocks, so the blocks
-// should fall evenly on the 256 units, and about one block per unit streams fastest.
+// How a product is cut: pieces of K, from N and K alone (the order of a row's sums goes by them, and must not depend on the batch); and of products
+// in pieces or in groups the tiles per wave and waves per block, too (mid_waves has those of the others).
 struct MidPlan { int tn, waves, blocks, splits, k_per_split; };
 #define MID_UNITS 256
 
@@ -302,7 +300,7 @@ static MidPlan mid_plan(int N, int K, bool gated) {
     plan.waves = MID_MAX_WAVES;
     plan.splits = 1;
     if (items >= MID_UNITS * MID_MIN_WAVES) {
-        // enough for every unit: the waves per block and rounds of blocks that leave the fewest idle
+        // enough for every unit.  Groups: the waves per block and rounds of blocks that leave the fewest units idle
         double best = 0.0;
         for (int rounds = 1; rounds <= 8; ++rounds) {
             int waves = (items + MID_UNITS * rounds - 1) / (MID_UNITS * rounds);
@@ -330,24 +328,21 @@ static MidPlan mid_plan(int N, int K, bool gated) {
     }
     if (gated && plan.splits > 1) {
         // A gated product in pieces needs a kernel of its own to add them up and apply the gate (4 to 5 us); where the
-        // blocks of the whole K already cover half the units, that costs more than the pieces gain.  Estimated with a
-        // unit pulling 34 GB/s and the memory giving 6.5 TB/s (a width of 1536 and 8960 gate rows, 55 MB: 15.4 us whole
-        // against 13.9 + 4.6 in three pieces).
+        // blocks of the whole K already cover half the units, that costs more than the pieces gain.  The line is the one of a kernel whose
+        // units pulled 34 GB/s, in blocks of four waves and more, of 6.5 TB/s that the memory gives, and stays where it was, since results' low bits go by
+        // it.  Units pull about 55 GB/s today, x counted, and blocks may have three waves, so whole products are better over more sizes than it
+        // says.  us whole and in pieces, 20, 64 and 128 rows, N of both parts: it takes 17920 x 1536 whole, 11.7, 14.3, 20.1 and 16.7, 23.6, 29.0; 22016 x
+        // 4096 whole, 29.6, 32.8, 42.2 and 34.0, 39.2, 44.4; 4096 x 4096 in pieces, 19.2, 24.8, 34.6 and 15.6, 17.6, 21.4; 9728 x 8192 in pieces, 40.2, 50.0,
+        // 67.4 and 32.3, 36.7, 42.3; but also 12288 x 2048 in pieces, 12.6, 15.8, 22.1 and 15.5, 20.9, 27.3, and 16384 x 4096, 24.3, 29.3, 39.0 and 37.5,
+        // 43.2, 49.5.
         const double bytes = 2.0 * (double)N * (double)K;
         auto time_us = [&](int blocks) { return 4.0 + bytes / (1e6 * (blocks * 0.034 < 6.5 ? blocks * 0.034 : 6.5)); };
-        double best_whole = 1e30;
-        int whole_waves = 0;
+        double whole = 1e30;
         for (int waves = MID_MAX_WAVES; waves >= MID_MIN_WAVES; --waves) {
             const int blocks = (items + waves - 1) / waves;
-            if (blocks > MID_UNITS) continue;
-            const double t = time_us(blocks);
-            if (t < best_whole - 0.1) { best_whole = t; whole_waves = waves; }
+            if (blocks <= MID_UNITS && time_us(blocks) < whole - 0.1) whole = time_us(blocks);
         }
-        if (whole_waves && best_whole < time_us(plan.blocks * plan.splits) + 4.6) {
-            plan.waves = whole_waves;
-            plan.blocks = (items + whole_waves - 1) / whole_waves;
-            plan.splits = 1;
-        }
+        if (whole < time_us(plan.blocks * plan.splits) + 4.6) plan.splits = 1;
     }
     const int per = (chunks + plan.splits - 1) / plan.splits;
     plan.splits = (chunks + per - 1) / per;             // no empty piece
