@@ -680,11 +680,12 @@ private:
     // that go through that kernel and write their own cache.  A block asks for its first page while its row's sums are on their way, so the launch
     // is saved but for the work that blocks of one row then do each for themselves.  Not where that costs more than the launch (ms a step, launch ->
     // folded, heads of 128; every rule's both sides):
-    //  - blocks of one wave, two or three rounds of loads on 64 lanes (before a page was asked for ahead): 7B sizes, 17 and 20 rows of 200
-    //    positions 3.368 -> 3.393 and 3.400 -> 3.435; 24 rows, blocks of four waves, 3.495 -> 3.425;
-    //  - more blocks than units: 7B, 72 rows of 64 positions 3.803 -> 3.851, 120 of 1024 5.282 -> 5.342, 80 of up to 1024 4.345 -> 4.332; 32B with 8
-    //    layers, 60 of 1024 2.158 -> 2.176.  Up to that, of any length: 7B, 48 and 64 rows of 2048 positions 4.238 -> 4.179 and 4.588 -> 4.569;
-    //    1.5B, 96 of 2048 2.836 -> 2.778 and 64 of 4096 2.882 -> 2.816; 32B, 20 and 32 of 2048 1.991 -> 1.940 and 2.118 -> 2.095.
+    //  - blocks of one wave, which the kernel does not have for sums: 7B sizes, 17 and 20 rows of 200 positions 3.26 -> 3.29 and 3.28 -> 3.35, 1.5B, 40 rows
+    //    1.63 -> 1.68 (20 rows 1.45 -> 1.43);
+    //  - more blocks than units and long rows: 7B, 120 rows of 1024 positions 5.28 -> 5.36; 32B with 8 layers, 60 of 1024 2.19 -> 2.20.  (Short ones would
+    //    gain, 72 rows of 64 3.88 -> 3.76, 80 of up to 1024 4.39 -> 4.33: the line is by blocks alone.)  Up to that, of any length: 7B, 48 and 64 rows
+    //    of 2048 positions 4.238 -> 4.179 and 4.588 -> 4.569; 1.5B, 96 of 2048 2.836 -> 2.778 and 64 of 4096 2.882 -> 2.816; 32B, 20 and 32 of 2048
+    //    1.991 -> 1.940 and 2.118 -> 2.095.
     bool finishes_sums(const StepContext& c, const CacheEntry& entry, int width) const {
         if (!(c.all_decode && entry.writes && policy().decode_mfma && K::attention_decode_supported.raw(head_dim_) != 0)) return false;
         const int units = 256, n_parts = decode_parts(c.n_tokens, width);

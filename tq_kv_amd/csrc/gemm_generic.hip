@@ -196,9 +196,10 @@ void gemm_few_rows_kernel(const float* __restrict__ x, const float* __restrict__
 // More rows: 64 rows by 64 features a block, each of four waves 32 by 32.  Stages of 32 k go through registers into LDS, two in turn;
 // a row's 128 bytes lie 144 apart, so that the 16 rows of an operand meet all banks.  blockIdx.y: the block's share of the
 // groups; with more than one share every group's sums go to scratch on their own.  Bound by the matrix cores (157 TFLOP/s in
-// float32): gate+up of the 7B shape at 300 rows 750 us = 109 TFLOP/s (827 with the
-// rows' tiles of some features far apart and loads one stage ahead: a stage is hardly longer than a load takes), and 2108 us through the FMA kernel above; down
-// 465 with the groups' sums (495), 40 rows 206 and 108 (229 and 111).  Blocks of 160 rows by 64 features took 967 us: fewer waves lose more than the bytes saved.
+// float32): gate+up of the 7B shape at 300 rows 750 us = 109 TFLOP/s (826 with the rows' tiles of some features far apart, 805 with loads one stage
+// ahead, as a stage is hardly longer than a load takes, 855 with neither), and 2108 us through the FMA kernel above; down 465 us with the
+// groups' sums written and added (495 with neither), 40 rows 206 and 108 (229 and 111).  Blocks of 160 rows by 64 features took 967 us
+// for gate+up: fewer waves lose more than the bytes saved.
 #define GM_LINE 36              // floats from row to row in LDS
 __global__ __launch_bounds__(256)
 void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ out,
@@ -207,7 +208,10 @@ void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, c
     const int tid = threadIdx.x, lane = tid % TQK_WAVE, wave = tid / TQK_WAVE;
     const int r16 = lane % 16, k4 = 4 * (lane / 16);
     // Blocks are dealt to the eight dies in turn: all rows' tiles of some features go to one die one after the other, so that the weights come out
-    // of its second-level cache for all but the first.
+    // of its second-level cache for all but the first.  37888 features, K of 3584, 300, 1024 and 4096 rows: 826, 2534 and 10307 us with neighbouring
+    // blocks on one row of tiles, 752, 2276 and 9030 so.  Where the weights are small it hardly matters: 512 to 17920 features, 100 to 8192 rows within
+    // 2 %, but for single sizes (3584 features and 2048 rows, 4096 and 4096: 4 and 5 % slower).  (Shares of K read other weights, so it is no loss that
+    // a share's dealing begins at another die where the tiles are no multiple of eight.)
     const int tiles_m = (M + GT - 1) / GT, tiles_n = (N + GT - 1) / GT;
     int tm, tn;
     {
