@@ -18,140 +18,10 @@
 // operations for a query depends only on its position, never on the batch or on which of the two it is.
 // Cache pages: keys [kv head][position][head_dim], values [kv head][head_dim][place of
 // the position] (value_place in common.h).
-#include "common.h"
+#include "attention_walk.h"
 #include "tq_kernels.h"
 
 #define ATT_WAVES 4
-#define ATT_STRIPES 8
-#define ATT_MAX_D 256
-
-// four elements that lie together, at a multiple of four elements
-__device__ __forceinline__ float4 load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
-__device__ __forceinline__ float4 load4(const bf16_t* p) {
-    const uint2 v = *reinterpret_cast<const uint2*>(p);
-    return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u));
-}
-
-// lane j's value, j the same for the whole wave
-__device__ __forceinline__ float lane_value(float v, int j) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), j)); }
-
-// dot + the product of 4 N elements, in their order, N loads under way together
-template <int N, typename T>
-__device__ __forceinline__ float key_dot(const float* q, const T* k, float dot) {
-    float4 kv[N];
-#pragma unroll
-    for (int u = 0; u < N; ++u) kv[u] = load4(k + 4 * u);
-#pragma unroll
-    for (int u = 0; u < N; ++u) {
-        const float4 qv = *reinterpret_cast<const float4*>(q + 4 * u);
-        dot = fmaf(qv.x, kv[u].x, dot);
-        dot = fmaf(qv.y, kv[u].y, dot);
-        dot = fmaf(qv.z, kv[u].z, dot);
-        dot = fmaf(qv.w, kv[u].w, dot);
-    }
-    return dot;
-}
-
-// sum + the weighted values of 4 N positions from j on (a multiple of four), in their order, N loads under way together
-template <int N, typename T>
-__device__ __forceinline__ float value_sum(const T* row, float p, int j, float sum) {
-    float4 v[N];
-#pragma unroll
-    for (int u = 0; u < N; ++u) v[u] = load4(row + value_place(j + 4 * u));
-#pragma unroll
-    for (int u = 0; u < N; ++u) {
-        sum = fmaf(lane_value(p, j + 4 * u), v[u].x, sum);
-        sum = fmaf(lane_value(p, j + 4 * u + 1), v[u].y, sum);
-        sum = fmaf(lane_value(p, j + 4 * u + 2), v[u].z, sum);
-        sum = fmaf(lane_value(p, j + 4 * u + 3), v[u].w, sum);
-    }
-    return sum;
-}
-
-// What scores are taken from before their exponential: the maximum so far, or 0 while every score is -inf (a stripe may begin with such pages), so that
-// those have weight 0 and what follows counts as if they were not there.
-__device__ __forceinline__ float from_max(float m) { return m == -INFINITY ? 0.f : m; }
-
-// A stripe's first page from `first` on.
-__device__ __forceinline__ int page_of(int stripe, int first) { return first + (stripe - first % ATT_STRIPES + ATT_STRIPES) % ATT_STRIPES; }
-
-// What a stripe leaves: maximum, sum, and this lane's output elements.
-struct Stripe {
-    float m, l, acc[ATT_MAX_D / TQK_WAVE];
-};
-
-// The pages of one stripe for one query: its values in LDS (qf), keys lo .. pos.
-// UNROLL: loads of four elements of a key under way together.
-template <typename T, int UNROLL>
-__device__ __forceinline__ Stripe walk(int stripe, const float* qf, const T* keys, const T* values, const int32_t* pages, int pos, int lo, int kvh,
-                                       int n_kv_heads, int head_dim, float scale, int wide_keys, int wide_values, int lane) {
-    constexpr int NACC = ATT_MAX_D / TQK_WAVE;
-    const size_t page_stride = (size_t)n_kv_heads * TQK_PAGE * head_dim;
-    Stripe r;
-#pragma unroll
-    for (int i = 0; i < NACC; ++i) r.acc[i] = 0.f;
-    r.m = -INFINITY;
-    r.l = 0.f;
-    for (int pg = page_of(stripe, lo / TQK_PAGE); pg * TQK_PAGE <= pos; pg += ATT_STRIPES) {
-        const int kb = pg * TQK_PAGE, page = pages[pg];
-        const int j = kb + lane;
-        const bool valid = j >= lo && j <= pos && page >= 0;
-        const size_t base = (size_t)(page < 0 ? 0 : page) * page_stride + (size_t)kvh * TQK_PAGE * head_dim;
-        float s = -INFINITY;
-        if (valid) {
-            const T* kr = keys + base + (size_t)lane * head_dim;
-            float dot = 0.f;
-            int i = 0;
-            if (wide_keys) {
-                // (fewer loads at a time for what is left of the head, or of a small one, and not one)
-                if (UNROLL > 8) for (; i + 64 <= head_dim; i += 64) dot = key_dot<16>(qf + i, kr + i, dot);
-                for (; i + 32 <= head_dim; i += 32) dot = key_dot<8>(qf + i, kr + i, dot);
-                for (; i + 16 <= head_dim; i += 16) dot = key_dot<4>(qf + i, kr + i, dot);
-                for (; i < head_dim; i += 4) dot = key_dot<1>(qf + i, kr + i, dot);
-            }
-            for (; i < head_dim; ++i) dot = fmaf(qf[i], to_float(kr[i]), dot);
-            s = dot * scale;
-        }
-        const float m_new = fmaxf(r.m, wave_max(s)), m_at = from_max(m_new);
-        const float p = valid ? expf(s - m_at) : 0.f;
-        const float alpha = expf(r.m - m_at);           // exp(-inf) = 0 on the stripe's first page
-        r.l = fmaf(r.l, alpha, wave_sum(p));
-        r.m = m_new;
-        const int n_keys = min(TQK_PAGE, pos - kb + 1);
-        const int first_key = max(0, lo - kb);           // keys before the window are never read
-        const T* vb = values + base;
-#pragma unroll
-        for (int a = 0; a < NACC; ++a) {
-            const int c = lane + a * TQK_WAVE;
-            float sum = r.acc[a] * alpha;
-            if (a * TQK_WAVE < head_dim) {
-                // (lanes past the head read its last row and drop the result)
-                const T* row = vb + (size_t)min(c, head_dim - 1) * TQK_PAGE;
-                auto one = [&](int jj) { sum = fmaf(lane_value(p, jj), to_float(row[value_place(jj)]), sum); };
-                // four positions from a multiple of four lie together
-                int jj = first_key;
-                for (; jj < n_keys && jj % 4 != 0; ++jj) one(jj);
-                if (wide_values) {
-                    if (UNROLL > 8) for (; jj + 32 <= n_keys; jj += 32) sum = value_sum<8>(row, p, jj, sum);
-                    for (; jj + 16 <= n_keys; jj += 16) sum = value_sum<4>(row, p, jj, sum);
-                    for (; jj + 4 <= n_keys; jj += 4) sum = value_sum<1>(row, p, jj, sum);
-                }
-                for (; jj < n_keys; ++jj) one(jj);
-            }
-            r.acc[a] = sum;
-        }
-    }
-    return r;
-}
-
-// The next stripe joins the ones before it: what the sums so far and the stripe's are multiplied by.
-__device__ __forceinline__ void join(float& m, float& l, float stripe_m, float stripe_l, float& of_sum, float& of_stripe) {
-    const float mn = fmaxf(m, stripe_m), at = from_max(mn);
-    of_sum = expf(m - at);                              // exp(-inf) = 0 for the first one
-    of_stripe = expf(stripe_m - at);
-    l = fmaf(l, of_sum, stripe_l * of_stripe);
-    m = mn;
-}
 
 // Bound by latency, a page costs a wave 6 us: the float32 step of four tokens after 300 (28 heads of 128) takes 13.6 us with a wave per stripe and
 // up to 16 loads under way, 37.0 with one wave for all and up to 8.  What is left of a head or a page after the last 16 loads goes by
@@ -187,7 +57,7 @@ void attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ key
         __shared__ float met[ATT_STRIPES][ATT_MAX_D], ml[ATT_STRIPES][2];
         const bool alone = lo / TQK_PAGE == pos / TQK_PAGE;             // one page: its stripe is the result
         if (alone && wave > 0) return;
-        const Stripe r = walk<T, 16>(alone ? lo / TQK_PAGE % ATT_STRIPES : wave, qf, keys, values, pages, pos, lo, kvh, n_kv_heads, head_dim, scale, wide_keys, wide_values, lane);
+        const Stripe<NACC> r = walk<T, 16, NACC>(alone ? lo / TQK_PAGE % ATT_STRIPES : wave, qf, keys, values, pages, pos, lo, kvh, n_kv_heads, head_dim, scale, wide_keys, wide_values, lane);
         if (alone) {
 #pragma unroll
             for (int a = 0; a < NACC; ++a) {
@@ -215,7 +85,7 @@ void attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ key
         for (int a = 0; a < NACC; ++a) acc[a] = 0.f;
         for (int s = 0; s < ATT_STRIPES; ++s) {
             if (page_of(s, lo / TQK_PAGE) * TQK_PAGE > pos) continue;
-            const Stripe r = walk<T, 8>(s, qf, keys, values, pages, pos, lo, kvh, n_kv_heads, head_dim, scale, wide_keys, wide_values, lane);
+            const Stripe<NACC> r = walk<T, 8, NACC>(s, qf, keys, values, pages, pos, lo, kvh, n_kv_heads, head_dim, scale, wide_keys, wide_values, lane);
             join(m, l, r.m, r.l, of_sum, of_stripe);
 #pragma unroll
             for (int a = 0; a < NACC; ++a) acc[a] = fmaf(acc[a], of_sum, r.acc[a] * of_stripe);

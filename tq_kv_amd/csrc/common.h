@@ -91,6 +91,11 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
     return total;
 }
 
+// ---- norms ---------------------------------------------------------------------------
+// Sum of four squares, fused in this order by name: what the compiler fuses of a plain expression changes with the code around it, and the bits of
+// all that follows the norm with it.
+__device__ __forceinline__ float squares(float4 v) { return fmaf(v.w, v.w, fmaf(v.z, v.z, fmaf(v.x, v.x, v.y * v.y))); }
+
 // ---- gates of feed-forwards -------------------------------------------------------
 // What a gated feed-forward makes of its gate and up products g and u:
 //   TQK_GATE_SILU     g sigmoid(g) u

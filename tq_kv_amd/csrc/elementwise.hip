@@ -218,10 +218,6 @@ template <> __device__ __forceinline__ void store4<bf16_t>(bf16_t* p, float a, f
     *reinterpret_cast<uint2*>(p) = o;
 }
 
-// Sum of four squares, fused in this order by name: what the compiler fuses of a plain expression changes with the code around it, and the bits of
-// all that follows the norm with it.
-__device__ __forceinline__ float squares(float4 v) { return fmaf(v.w, v.w, fmaf(v.z, v.z, fmaf(v.x, v.x, v.y * v.y))); }
-
 // SUMS: the update is a product's pieces, so many of them under way together (0: it is not; VPT is 1 or 2 otherwise).
 template <typename TA, typename TW, int VPT, int SUMS>
 __global__ void add_rmsnorm_vec_kernel(float* __restrict__ h, const TA* __restrict__ delta, const PartSums ps,
@@ -425,7 +421,7 @@ __global__ void rope_store_kernel(const TA* __restrict__ qkv, const TB* __restri
             const float y = to_float(src[partner]) + (b ? to_float(b[partner]) : 0.f);
             const float c = cos_table[(size_t)pos * half_rot + p];
             const float s = sin_table[(size_t)pos * half_rot + p];
-            x = first ? x * c - y * s : y * s + x * c;
+            x = fmaf(x, c, first ? -(y * s) : y * s);
         }
         dst[(size_t)i * dst_stride] = from_float<TA>(x);
     }

@@ -85,7 +85,17 @@ const float* Engine::step(int n_seqs, const int32_t* slots, const int32_t* n_new
     ctx.stream = stream;
     ctx.staging = &staging_;
     ctx.act_dtype = model->dtype;
-    if (use_graphs && all_one && n_seqs <= mid_max_rows()) {
+    long long n_tokens = 0;
+    for (int i = 0; i < n_seqs; ++i) n_tokens += n_new[i];
+    TqkSmallStep small;
+    if (n_tokens <= Model::SMALL_ROWS && model->has_small_steps() && !trace_enabled() &&
+        (ctx.plan(cache->book, n_seqs, slots, starts.data(), n_new, tokens, want_counts, want_idx, 1), model->small_step(ctx, *cache, small))) {
+        ws_.reset(stream);
+        ctx.ws = &ws_;
+        logits = (const float*)model->forward_small(ctx, small, device_tokens, logits_out).data;
+        last_n_want_ = ctx.n_want;
+        if (use_graphs && all_one && single_.size() < (size_t)MAX_GRAPHS) single_.insert(ctx.shape());
+    } else if (use_graphs && all_one && n_seqs <= mid_max_rows()) {
         logits = graphed_step(ctx, n_seqs, slots, starts.data(), n_new, tokens, want_counts, want_idx, device_tokens, logits_out, stream);
     } else {
         ws_.reset(stream);

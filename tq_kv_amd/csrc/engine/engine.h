@@ -7,6 +7,7 @@
 // against what the cache holds, and returns the logits at the wanted places.
 #pragma once
 #include <list>
+#include <set>
 
 #include "model.h"
 
@@ -39,7 +40,8 @@ public:
     // the next step writes again.  Returns where they are.
     const float* step(int n_seqs, const int32_t* slots, const int32_t* n_new, const int32_t* tokens, const int32_t* want_counts,
                       const int32_t* want_idx, const int32_t* device_tokens, float* logits_out, hipStream_t stream);
-    int n_graphs() const { return (int)graphs_.size(); }
+    // shapes of one-token steps that are ready to be replayed: captured as graphs, or one launch as they are
+    int n_graphs() const { return (int)(graphs_.size() + single_.size()); }
     int last_n_want() const { return last_n_want_; }
 
     static const int GRAPH_WIDTH_STEP = 8;      // page-table widths of graphed steps grow in steps of 8 pages
@@ -61,6 +63,7 @@ private:
     Workspace ws_;
     Staging staging_;
     std::list<Graph> graphs_;            // least recently used first
+    std::set<StepShape> single_;         // shapes of one-token steps that were one launch (MAX_GRAPHS of them at most)
     hipStream_t capture_stream_ = nullptr;
     int last_n_want_ = 0;
 };

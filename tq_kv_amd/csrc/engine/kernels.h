@@ -3,6 +3,7 @@
 // (sizes of scratch memory, what a kernel takes) are plain host functions.
 #pragma once
 #include "core.h"
+#include "../tq_kernels.h"
 
 namespace tq {
 namespace K {
@@ -34,6 +35,9 @@ TQ_KERNEL(fused_qkv, cptr, cf32, int, float, cptr, int, cptr, cf32, cf32, int, c
 TQ_QUERY(int, mid_splits, int, int, int);
 TQ_KERNEL(mid_store, cptr, cptr, void*, int, int, int, int, void*, int, void*);
 TQ_KERNEL(mid_gated, cptr, cptr, void*, int, int, int, void*, void*);
+TQ_QUERY(int, small_step_takes, const TqkSmallStep*);
+TQ_QUERY(int, small_step_pays, const TqkSmallStep*, int, int);
+TQ_KERNEL(small_step, const TqkSmallStep*, void*);
 TQ_QUERY(int, prompt_takes, int, int, int, int);
 TQ_QUERY(int, prompt_splits, int, int, int);
 TQ_QUERY(int, prompt_pays, int, int, int, int);

@@ -28,6 +28,7 @@ int* policy_field(const std::string& name) {
     if (name == "prompt") return &p.prompt;
     if (name == "decode_mfma") return &p.decode_mfma;
     if (name == "prefill_mfma") return &p.prefill_mfma;
+    if (name == "small") return &p.small;
     return nullptr;
 }
 

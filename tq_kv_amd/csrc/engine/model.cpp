@@ -99,7 +99,74 @@ void Model::load(Loaded& tensors, hipStream_t stream) {
     // a tied head's rows are the embedding: they stay whatever the policy says
     head_ = make_weight(spec.head_name.empty() ? embedding_ : need(tensors, spec.head_name), 1, spec.head_name.empty(), stream);
     stream_synchronize(stream);
+    find_small();
     loaded = true;
+}
+
+void Model::find_small() {
+    small_.reset();
+    const ModelSpec& s = spec;
+    if (!on_gpu || stream_position_ || s.has_embedding_scale || s.has_logit_scale || s.has_logit_cap || head_bias_) return;
+    if (embedding_->t.dtype != dtype || !head_.rows || head_.dtype != dtype || s.order.size() > TQK_SMALL_LAYERS || s.hidden_size > INT32_MAX || s.vocab_size > INT32_MAX) return;
+    const Tensor* norm = final_norm_->plain_rms_weight();
+    if (!norm || norm->dtype != dtype) return;
+    std::unique_ptr<TqkSmallStep> m(new TqkSmallStep());
+    m->act_dtype = dtype;
+    m->hidden = (int)s.hidden_size;
+    m->vocab = (int)s.vocab_size;
+    m->embedding = embedding_->t.data;
+    m->head = head_.rows->t.data;
+    m->final_norm = norm->data;
+    m->final_eps = final_norm_->fold_eps();
+    m->n_layers = (int)s.order.size();
+    for (int i = 0; i < m->n_layers; ++i) {
+        const Run& run = s.order[(size_t)i];
+        if (run.add_embedding || run.cache_of >= 0 || !blocks_[(size_t)run.layer]->small_layer(*m, m->layers[i])) return;
+    }
+    m->n_rows = m->n_want = 1;
+    if (K::small_step_takes.raw(m.get()) && (K::small_step_pays.raw(m.get(), 0, 1) || K::small_step_pays.raw(m.get(), 1, 1))) small_ = std::move(m);
+}
+
+bool Model::small_step(const StepContext& c, const CacheStore& cache, TqkSmallStep& step) const {
+    if (!small_ || !policy().small_steps() || c.n_tokens > SMALL_ROWS || c.n_want > c.n_tokens) return false;
+    step = *small_;
+    step.n_rows = c.n_tokens;
+    step.n_want = c.n_want;
+    int n = 0;
+    auto put = [&](const int32_t* from, int count) {
+        const int at = n;
+        if (count > TQK_SMALL_INTS - n) { n = TQK_SMALL_INTS + 1; return 0; }
+        memcpy(step.ints + at, from, (size_t)count * sizeof(int32_t));
+        n += count;
+        return at;
+    };
+    step.tokens = put(c.host.tokens, c.n_tokens);
+    step.tok_seq = n <= TQK_SMALL_INTS ? put(c.host.tok_seq, c.n_tokens) : 0;
+    step.tok_pos = n <= TQK_SMALL_INTS ? put(c.host.tok_pos, c.n_tokens) : 0;
+    step.want = n <= TQK_SMALL_INTS ? put(c.host.want_rows, c.n_want) : 0;
+    std::vector<int> tables;
+    for (const StepContext::Table& t : c.tables) tables.push_back(n <= TQK_SMALL_INTS ? put(t.host, c.n_seqs * t.width) : 0);
+    if (n > TQK_SMALL_INTS) return false;
+    step.n_ints = n;
+    for (int i = 0; i < step.n_layers; ++i) {
+        const CacheEntry& e = cache.entry(i);
+        if (e.kind != CacheNeed::Pages || !e.writes || e.keys.dtype != dtype) return false;
+        step.layers[i].keys = e.keys.data;
+        step.layers[i].values = e.values.data;
+        step.layers[i].table = tables.at((size_t)e.group);
+        step.layers[i].width = c.tables[(size_t)e.group].width;
+    }
+    return K::small_step_takes.raw(&step) != 0 && K::small_step_pays.raw(&step, c.all_decode ? 1 : 0, c.max_end) != 0;
+}
+
+Tensor Model::forward_small(StepContext& c, TqkSmallStep& step, const int32_t* device_tokens, float* out) {
+    Span span("model");
+    Tensor logits(out, F32, {c.n_want, spec.vocab_size});
+    if (!out && c.n_want) logits = c.alloc(F32, {c.n_want, spec.vocab_size});
+    step.device_tokens = device_tokens;
+    step.logits = (float*)logits.data;
+    K::small_step(&step, c.stream);
+    return logits;
 }
 
 OwnedPtr Model::held(const std::string& name) const {

@@ -33,6 +33,12 @@ public:
     // Runs the step's tokens through every run of the order; logits [wanted rows, vocab] float32 for
     // the step's wanted rows, written to `out` (device memory) or to workspace memory.
     Tensor forward(StepContext& c, const CacheStore& cache, float* out = nullptr);
+    // The step in one launch, for small models (small_step.hip): whether that is the way for the planned step, and the step itself.  Nothing
+    // of the plan is uploaded: the step's arrays travel with the launch.  device_tokens: as Engine::step.
+    bool small_step(const StepContext& c, const CacheStore& cache, TqkSmallStep& step) const;
+    Tensor forward_small(StepContext& c, TqkSmallStep& step, const int32_t* device_tokens, float* out);
+    bool has_small_steps() const { return small_ != nullptr; }
+    static const int SMALL_ROWS = 64;           // (more rows are not asked about)
     Json describe() const;
     // Lets the library try its kernels once for every product of the model at `rows` rows (more than the own kernels
     // take: fewer never reach the library) and keep the fastest for later calls.
@@ -46,6 +52,8 @@ private:
     int stream_state_entry_ = -1;               // the cache entry of the stream position's state, if it keeps one
     OwnedPtr embedding_, head_bias_;
     Weight head_;
+    std::unique_ptr<TqkSmallStep> small_;       // the model as that kernel takes it, if it does
+    void find_small();
     Tensor head_logits(StepContext& c, Stream& stream, float* out);
 };
 

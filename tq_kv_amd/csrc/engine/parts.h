@@ -31,6 +31,7 @@
 #include <string>
 #include <vector>
 
+#include "../tq_kernels.h"
 #include "core.h"
 #include "spec.h"
 
@@ -166,6 +167,8 @@ public:
     virtual bool takes_normed_update(const Norm* norm) const { (void)norm; return false; }
     // whether the kernels that add to the stream can prepare this norm, and with what
     virtual bool foldable() const { return false; }
+    // the weight and the eps, where the norm is x / sqrt(mean(x^2) + eps) * weight as stored (for a small model's step in one launch)
+    virtual const Tensor* plain_rms_weight() const { return nullptr; }
     virtual const Tensor* fold_weight() const { return nullptr; }
     virtual float fold_eps() const { return 0.f; }
     bool lazy(const Stream& stream, LazyNorm& out) const;
@@ -220,6 +223,9 @@ public:
     // result is undefined()).  last_rows: keys and values of all tokens go to the cache as always,
     // but the output is computed for the step's last_rows alone.
     virtual Tensor forward(StepContext& c, const Activation& x, const CacheEntry& entry, Stream* stream, bool last_rows) = 0;
+    // Optional: the part as the kernel that runs a small model's whole step takes it.  model: sizes, types and angle tables, filled in by the first
+    // part and the same for all; layer: what is this one's own.  False: not such a part.
+    virtual bool small_layer(TqkSmallStep& model, TqkSmallLayer& layer) const { (void)model; (void)layer; return false; }
 };
 
 class FeedForward : public Part {
@@ -227,6 +233,7 @@ public:
     virtual bool folds_norm(const StepContext& c) const { (void)c; return false; }
     virtual bool adds_to_stream(const StepContext& c) const { (void)c; return false; }
     virtual Tensor forward(StepContext& c, const Activation& x, Stream* stream) = 0;
+    virtual bool small_layer(TqkSmallStep& model, TqkSmallLayer& layer) const { (void)model; (void)layer; return false; }      // (as a mixer's)
     // Optional: scale (forward(x) + beside) out of the part's own last kernel (beside: [tokens, hidden], what another part made of the step).
     // stream and next_norm given: the part may add the sum to the stream and leave next_norm of it there (normed); it then returns nothing.
     virtual bool takes_beside() const { return false; }
@@ -241,6 +248,7 @@ public:
     virtual CacheNeed cache_need() const = 0;
     virtual Norm* first_norm() = 0;
     virtual Mixer* mixer() { return nullptr; }
+    virtual bool small_layer(TqkSmallStep& model, TqkSmallLayer& layer) const { (void)model; (void)layer; return false; }      // (as a mixer's)
     // next_norm: the norm that reads the stream after this block.  last: nothing but the head
     // reads the stream after it.  Returns the stream to go on with.
     virtual Stream* forward(StepContext& c, Stream* stream, const CacheEntry& entry, Norm* next_norm, bool last) = 0;

@@ -95,6 +95,9 @@ static OwnedPtr as_floats(const OwnedPtr& p, hipStream_t stream) {
     return out;
 }
 
+// whether a product's weight is rows of the run's own type
+static bool small_weight(const Weight& w, int dtype) { return w.rows && w.dtype == dtype; }
+
 // ---- RMSNorm -----------------------------------------------------------------------------------
 // As the reference computes it (src/models/turbo_generic.rs:41-51): x / sqrt(mean(x^2) + eps) *
 // weight in float32, cast last; the weight is used as it is stored (no 1 + w).
@@ -157,6 +160,7 @@ public:
     // (the weight as stored, bfloat16, or the sum 1 + w, float32: the kernels that prepare a norm take either)
     bool foldable() const override { return weight_ && (weight_->t.dtype == BF16 || (unit_offset_ && weight_->t.dtype == F32)); }
     const Tensor* fold_weight() const override { return &weight_->t; }
+    const Tensor* plain_rms_weight() const override { return weight_ && !unit_offset_ ? &weight_->t : nullptr; }
     float fold_eps() const override { return eps_; }
 
 private:
@@ -548,6 +552,29 @@ public:
         return linear(c, y, w_o_, b_o_ ? &b_o_->t : nullptr, dtype).t;
     }
 
+    bool small_layer(TqkSmallStep& m, TqkSmallLayer& l) const override {
+        if (extras_ || b_o_ || reads_other_cache || position_->has_apply() || !small_weight(w_qkv_, m.act_dtype) || !small_weight(w_o_, m.act_dtype)) return false;
+        if (b_qkv_ && b_qkv_->t.dtype != m.act_dtype) return false;
+        const Position::Tables tb = position_->tables();
+        if (tb.style != STYLE_HALVES || tb.rot_dim != head_dim_) return false;
+        if (m.n_heads == 0) {
+            m.n_heads = n_heads_;
+            m.n_kv_heads = n_kv_heads_;
+            m.head_dim = head_dim_;
+            m.cos_table = (const float*)tb.cos.data;
+            m.sin_table = (const float*)tb.sin.data;
+            m.max_positions = (int)tb.cos.shape[0];
+        }
+        if (hidden_ != m.hidden || m.n_heads != n_heads_ || m.n_kv_heads != n_kv_heads_ || m.head_dim != head_dim_ || m.cos_table != tb.cos.data || m.sin_table != tb.sin.data)
+            return false;
+        l.qkv = w_qkv_.rows->t.data;
+        l.qkv_bias = b_qkv_ ? b_qkv_->t.data : nullptr;
+        l.o = w_o_.rows->t.data;
+        l.scale = scale_;
+        l.window = window_;
+        return true;
+    }
+
 private:
     // product, then biases, the heads' norm, rotation, value mixing and cache write in one kernel
     void normed_qkv(StepContext& c, const Tensor& x, const CacheEntry& entry, const StepContext::Table& table, Tensor& q) {
@@ -912,6 +939,14 @@ public:
         return (fusable(c.n_tokens, w_down_, true) && fusable(c.n_tokens, w_gate_up_)) || leaves_sums(c.n_tokens, w_down_);
     }
 
+    bool small_layer(TqkSmallStep& m, TqkSmallLayer& l) const override {
+        if (gate_.kind != Gate::SiLU || hidden_ != m.hidden || !small_weight(w_gate_up_, m.act_dtype) || !small_weight(w_down_, m.act_dtype)) return false;
+        if (m.inter == 0) m.inter = (int)inter_;
+        l.gate_up = w_gate_up_.rows->t.data;
+        l.down = w_down_.rows->t.data;
+        return m.inter == inter_;
+    }
+
     Tensor forward(StepContext& c, const Activation& x, Stream* stream) override {
         if (stream && !x.lazy && x.x.shape[0] > skinny_max_rows()) {
             add_product(c, *stream, gated_linear(c, x.x, w_gate_up_, gate_), w_down_);
@@ -1012,6 +1047,16 @@ public:
     CacheNeed cache_need() const override { return mixer_->cache_need(); }
     Norm* first_norm() override { return mixer_norm_.get(); }
     Mixer* mixer() override { return mixer_.get(); }
+    bool small_layer(TqkSmallStep& m, TqkSmallLayer& l) const override {
+        if (!feed_forward_ || post_mixer_norm_ || post_ff_norm_) return false;
+        const Tensor *first = mixer_norm_->plain_rms_weight(), *second = ff_norm_->plain_rms_weight();
+        if (!first || !second || first->dtype != m.act_dtype || second->dtype != m.act_dtype) return false;
+        l.norm1 = first->data;
+        l.norm2 = second->data;
+        l.eps1 = mixer_norm_->fold_eps();
+        l.eps2 = ff_norm_->fold_eps();
+        return mixer_->small_layer(m, l) && feed_forward_->small_layer(m, l);
+    }
 
     Stream* forward(StepContext& c, Stream* stream, const CacheEntry& entry, Norm* next_norm, bool last) override {
         if (last && c.prune_last && policy().prune_last && mixer_->takes_rows) return forward_last_rows(c, stream, entry, next_norm);

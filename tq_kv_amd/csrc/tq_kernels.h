@@ -623,6 +623,32 @@ int tqk_pooled_attention_tiles(const void* q, const void* keys, const void* valu
 int tqk_normed_pair_sum(const void* x, const void* y, int dtype, const float* wx, const float* wy, float eps, float c, void* out, int out_dtype,
                         int n_tokens, int width, void* stream);
 
+/* A whole step of a small pre-norm decoder (grouped-query attention with rotary positions in halves, gated SiLU) in one launch (small_step.hip).
+ * Weights are rows as the checkpoint has them, all of the activation type; gate's rows in front of up's; q's, k's and v's one after the other.  The step's
+ * arrays (tokens, the rows' sequences and positions, the wanted rows, the page tables [sequences][width]) travel with the launch, in `ints` at the
+ * places named; device_tokens: the rows' tokens, on the device instead.  logits [n_want, vocab] float32. */
+enum { TQK_SMALL_LAYERS = 16, TQK_SMALL_INTS = 416 };
+typedef struct {
+    const void *norm1, *qkv, *qkv_bias, *o, *norm2, *gate_up, *down;
+    void *keys, *values;
+    float eps1, eps2, scale;
+    int window, table, width;
+} TqkSmallLayer;
+typedef struct {
+    const void *embedding, *final_norm, *head;
+    const float *cos_table, *sin_table;
+    const int32_t* device_tokens;
+    float* logits;
+    float final_eps;
+    int act_dtype, max_positions, n_layers, hidden, n_heads, n_kv_heads, head_dim, inter, vocab, n_rows, n_want, n_ints;
+    int tokens, tok_seq, tok_pos, want;
+    TqkSmallLayer layers[TQK_SMALL_LAYERS];
+    int32_t ints[TQK_SMALL_INTS];
+} TqkSmallStep;
+int tqk_small_step_takes(const TqkSmallStep* step);
+int tqk_small_step_pays(const TqkSmallStep* step, int decode, int positions);
+int tqk_small_step(const TqkSmallStep* step, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

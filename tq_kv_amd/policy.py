@@ -10,10 +10,11 @@ another; nothing else reads these.  They live in the engine library (tqe_policy_
                          half the weight memory again; a product of more than 128 rows (a prompt) that the kernel for
                          prompts does not take gets the rows back from the packed copy for its own length
   decode_mfma, prefill_mfma   the two matrix-core attention kernels (off: the plain kernel)
+  small                  steps of small models in one launch (they are not while any of the routines above is off)
 """
 from . import native
 
-NAMES = ("skinny", "library", "fused", "prune_last", "packed", "mid", "keep_rows", "decode_mfma", "prefill_mfma", "prompt")
+NAMES = ("skinny", "library", "fused", "prune_last", "packed", "mid", "keep_rows", "decode_mfma", "prefill_mfma", "prompt", "small")
 
 
 class _Policy:
