@@ -3,8 +3,8 @@
 // candle matmuls (src/models/turbo_generic.rs:68-91, 779-781).
 //
 // float32 throughout, K a multiple of 4 and operands at 16 bytes (every product of the float32 path of a usual model):
-// v_mfma_f32_16x16x4_f32, whose products and sums are float32 ones (no reduced-precision mode of the matrix cores
-// is used anywhere here).  Everything else: LDS-tiled, 64x64 outputs per block, 4x4 per thread, float32 FMA.
+// v_mfma_f32_16x16x4_f32, whose products and sums are float32 ones, and for large weights v_mfma_f32_16x16x32_bf16 on numbers taken apart
+// without loss.  Everything else: LDS-tiled, 64x64 outputs per block, 4x4 per thread, float32 FMA.
 //
 // The order of summation is fixed and the same for all numbers of rows, so that a result does
 // not depend on M or on where a row stands in the batch: k is
@@ -12,11 +12,12 @@
 // the result the sum of the groups in order (and then the bias).  Within a chunk the FMA kernel goes by increasing k; the
 // matrix-core kernels take 16 k at a time, four instructions of which number i adds the k with k % 4 == i to what the ones
 // before it left (a lane then reads its operands of all four as 16 contiguous bytes), with the same operands in the same
-// registers in both, so those two give the same bits.  Which of the two orders a product gets is a matter of types, K and addresses alone.
+// registers in both, so those two give the same bits.  Products with large weights (tqk_gemm_takes_apart) go by three bfloat16 numbers for a float32 one, 32 k at a time, again
+// in one order in all their kernels.  Which of the three orders a product gets is a matter of types, N, K and addresses alone.
 //
 // For up to 16 rows of x (decoding in the 32-bit path) the weights are the whole cost: a wave takes 16 output features and one
 // group of k and streams their weights through LDS, 12 KB of them under way; groups beyond the first meet in a second
-// kernel.  More rows: a block of four waves takes 64 rows by 64 features through LDS; where that gives
+// kernel.  More rows: a block of four waves takes 64 rows by 64 features (up to 128, for large weights) through LDS; where that gives
 // few blocks they are also dealt out along the groups.  Measured at the 7B layers' sizes: see the kernels.
 #include "common.h"
 #include "tq_kernels.h"
@@ -110,6 +111,67 @@ __device__ __forceinline__ void multiply16(floatx4_t& acc, const floatx4_t& w, c
     for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], x[i], acc, 0, 0, 0);
 }
 
+// ---- large weights: a float32 number as three bfloat16 ones -----------------------------------------
+// 24 bits are 8 + 8 + 8: p the number cut off after 8 bits (so that nothing overflows), q what is left rounded to 8, t what is left then, exactly.
+// Of the nine products of two numbers' parts the three smallest (below 2^-22 of the whole, on average far less) are left out; the others are exact in
+// float32.  Six bfloat16 instructions stand for eight float32 ones of twice the time each, 2.7 times the rate, and their sums of 32 k at once round less often: error against 64 bits, 2-norm,
+// K of 3584 and 18944, operands N(0, 1) 1.73e-7 and 2.07e-7 (the float32 instructions 2.17e-7 and 2.28e-7), all of one sign 0.52e-7 and 0.64e-7 (0.55e-7 and 0.64e-7), spread over
+// twelve powers of ten 1.30e-7 and 1.65e-7 (1.79e-7 and 2.06e-7), N(0, 1e-33) as N(0, 1).  (With the five small products in a sum of their own 0.98e-7, and 32 registers more.)
+// Infinities have no parts (inf - inf): where a wave's sums are not finite it takes them again with the float32 instructions.
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
+struct Parts { bf16x8_t p, q, t; };
+__device__ __forceinline__ uint32_t high_halves(float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); }
+__device__ __forceinline__ void split2(float a, float b, uint32_t& p, uint32_t& q, uint32_t& t) {
+    p = high_halves(a, b);
+    a -= __uint_as_float(__float_as_uint(a) & 0xffff0000u);
+    b -= __uint_as_float(__float_as_uint(b) & 0xffff0000u);
+    q = (uint32_t)float_to_bf16_bits(a) | (uint32_t)float_to_bf16_bits(b) << 16;
+    a -= __uint_as_float(q << 16);
+    b -= __uint_as_float(q & 0xffff0000u);
+    t = high_halves(a, b);
+}
+__device__ __forceinline__ Parts split8(floatx4_t a, floatx4_t b) {
+    u32x4_t p, q, t;
+    uint32_t pp, qq, tt;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const floatx4_t v = i < 2 ? a : b;
+        split2(v[2 * (i % 2)], v[2 * (i % 2) + 1], pp, qq, tt);
+        p[i] = pp; q[i] = qq; t[i] = tt;
+    }
+    return {__builtin_bit_cast(bf16x8_t, p), __builtin_bit_cast(bf16x8_t, q), __builtin_bit_cast(bf16x8_t, t)};
+}
+// 32 k more: a lane holds, of both operands, row lane % 16 and the eight k at 8 (lane / 16); the smallest products first.
+__device__ __forceinline__ void multiply32(floatx4_t& acc, const Parts& w, const Parts& x) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.t, x.p, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p, x.t, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.q, x.q, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.q, x.p, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p, x.q, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p, x.p, acc, 0, 0, 0);
+}
+__device__ __forceinline__ bool finite(floatx4_t v) {
+    return __builtin_isfinite(v[0]) && __builtin_isfinite(v[1]) && __builtin_isfinite(v[2]) && __builtin_isfinite(v[3]);
+}
+// The sums of k_begin .. k_end (whole groups, or up to K) of 16 rows and 16 features by the float32 instructions, for a wave; xrow, wrow: the lane's rows.
+__device__ __forceinline__ floatx4_t plain_sums(const float* xrow, const float* wrow, int k_begin, int k_end, int k4) {
+    floatx4_t total = {0.f, 0.f, 0.f, 0.f};
+    for (int g0 = k_begin; g0 < k_end; g0 += G_GROUP) {
+        floatx4_t group = {0.f, 0.f, 0.f, 0.f};
+        for (int c0 = g0; c0 < min(g0 + G_GROUP, k_end); c0 += G_CHUNK) {
+            floatx4_t acc = {0.f, 0.f, 0.f, 0.f};
+            for (int k0 = c0; k0 < min(c0 + G_CHUNK, k_end); k0 += 16) {
+                const floatx4_t none = {0.f, 0.f, 0.f, 0.f};
+                const bool in = k0 + k4 < k_end;
+                multiply16(acc, in ? *reinterpret_cast<const floatx4_t*>(wrow + k0 + k4) : none, in ? *reinterpret_cast<const floatx4_t*>(xrow + k0 + k4) : none);
+            }
+            group += acc;
+        }
+        total += group;
+    }
+    return total;
+}
+
 // Up to 16 rows of x: a wave per (16 output features, one group of k).  With one group the result is finished here.
 // Bound by the weights.  They come in stages of 64 k, 256 contiguous bytes of each of the 16 rows, by loads that end in LDS, three
 // stages on their way while one is multiplied; a piece of 16 bytes lies at its number exclusive-or its row, so that the operands of 16
@@ -183,6 +245,134 @@ void gemm_few_rows_kernel(const float* __restrict__ x, const float* __restrict__
         s0 += NS;
     } while (s0 < n_stage);
     __builtin_amdgcn_s_waitcnt(0x0f70);                                 // nothing is on its way into LDS any more
+    if (r16 >= M) return;
+    const bool whole = gridDim.y == 1;
+    float* dst = out + ((size_t)blockIdx.y * M + r16) * N;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int n = n0 + 4 * g + i;
+        if (n < N) dst[n] = whole && bias ? group[i] + bias[n] : group[i];
+    }
+}
+
+// The same by parts in bfloat16, for large weights.  What it spends beside its loads is taking numbers apart, 88 instructions for a stage's weights and as many for its x.
+// ROWS: up to 4, 8 or 16 rows of x.  Of the 16 lanes that hold x's rows four (two) stand for one row where there are few, each takes a quarter (half) of the row's values apart,
+// and the first gets the others' parts by turning the 16 lanes: 40 (56) instructions, and a quarter (half) of the loads.  One row, 4608, 3584 and 37888 features, K of 3584, 18944 and 3584:
+// 16.6, 61 and 102 us (17.2, 62 and 102 with the float32 instructions; 18.9, 66 and 104 without the turning).
+// TAIL: K is no multiple of 64.
+template <bool TAIL, int ROWS>
+__global__ __launch_bounds__(TQK_WAVE)
+void gemm_few_rows_apart_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ out,
+                          int M, int N, int K) {
+    constexpr int NS = FEW_STAGES, U = 4;                               // 16 k a step, four steps a stage
+    __shared__ __attribute__((aligned(1024))) float buf0[1024], buf1[1024], buf2[1024], buf3[1024];
+    const int lane = threadIdx.x, r16 = lane % 16, g = lane / 16;
+    const int n0 = blockIdx.x * 16;
+    const int k_begin = blockIdx.y * G_GROUP, k_end = min(K, k_begin + G_GROUP), n_stage = (k_end - k_begin + 63) / 64;
+    const float* xrow = x + (size_t)min(r16 % ROWS, M - 1) * K;        // rows past M repeat the last and are dropped
+    // (rows past N and everything past the last row lie outside of the buffer: nothing is read there)
+    const __amdgpu_buffer_rsrc_t w_mem = __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * K), 0, min(16, N - n0) * K * 4, 0x00020000);
+    uint32_t w_at[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int row = 4 * j + g;
+        w_at[j] = (uint32_t)row * (uint32_t)(K * 4) + ((r16 ^ row) * 16);
+    }
+    auto buf = [&](auto I) -> float* {
+        constexpr int i = decltype(I)::value % NS;
+        if constexpr (i == 0) return buf0; else if constexpr (i == 1) return buf1; else if constexpr (i == 2) return buf2; else return buf3;
+    };
+    constexpr int XU = ROWS / 4, LOADS = 4 + XU;
+    floatx4_t xv[NS][XU];
+    // where in a stage the lane's four k of part u of its operands lie
+    auto place = [&](int u) { return 32 * (u / 2) + 8 * g + 4 * (u % 2); };
+    auto x_place = [&](int u) { return place(r16 / ROWS * XU + u); };       // (of the x that the lane takes apart)
+    auto load = [&](auto I, int stage) {
+        const bool there = stage < n_stage;                             // (past the last stage: outside of the buffer, nothing is read)
+        const int k0 = k_begin + (there ? stage * 64 : 0);
+        const uint32_t nowhere = there ? 0u : 0x80000000u;              // (joined to the offsets, so that no branch lies here)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(w_mem, (lds_ptr_t)(buf(I) + j * 256), 16, (int)(w_at[j] | nowhere), k0 * 4, 0, 0);
+#pragma unroll
+        for (int u = 0; u < XU; ++u) xv[decltype(I)::value % NS][u] = *reinterpret_cast<const floatx4_t*>(xrow + min(k0 + x_place(u), K - 4));
+    };
+    floatx4_t group = {0.f, 0.f, 0.f, 0.f}, acc = group;
+    // (no branch in a stage: every stage issues its loads and multiplies, past the end what is nothing)
+    auto multiply = [&](auto I, int stage) {
+        const float* src = buf(I);
+        auto inside = [&](int at) { return (TAIL ? k_begin + stage * 64 + at < k_end : stage < n_stage) ? 0xffffffffu : 0u; };      // past k_end both operands are nothing
+        auto masked = [&](floatx4_t v, uint32_t in) { return __builtin_bit_cast(floatx4_t, __builtin_bit_cast(u32x4_t, v) & in); };
+        // (of a whole stage past it one of them alone: sums that are not finite are taken again anyway)
+        floatx4_t wv[U], xs[XU];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            wv[u] = *reinterpret_cast<const floatx4_t*>(src + r16 * 64 + ((place(u) / 4) ^ r16) * 4);
+            if (TAIL) wv[u] = masked(wv[u], inside(place(u)));
+        }
+#pragma unroll
+        for (int u = 0; u < XU; ++u) xs[u] = masked(xv[decltype(I)::value % NS][u], inside(x_place(u)));
+        Parts xp[2];
+        auto turned = [&](auto ctrl, const Parts& from) {
+            u32x4_t p = __builtin_bit_cast(u32x4_t, from.p), q = __builtin_bit_cast(u32x4_t, from.q), t = __builtin_bit_cast(u32x4_t, from.t);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                p[i] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)p[i], decltype(ctrl)::value, 0xf, 0xf, true);
+                q[i] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)q[i], decltype(ctrl)::value, 0xf, 0xf, true);
+                t[i] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)t[i], decltype(ctrl)::value, 0xf, 0xf, true);
+            }
+            return Parts{__builtin_bit_cast(bf16x8_t, p), __builtin_bit_cast(bf16x8_t, q), __builtin_bit_cast(bf16x8_t, t)};
+        };
+        if constexpr (ROWS == 16) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) xp[h] = split8(xs[2 * h], xs[2 * h + 1]);
+        } else if constexpr (ROWS == 8) {
+            xp[0] = split8(xs[0], xs[1]);
+            xp[1] = turned(std::integral_constant<int, 0x128>{}, xp[0]);                        // row_ror:8
+        } else {
+            // (own values first, then those of the lane four on (row_ror:12); the lanes eight on (row_ror:8) hold the other half so)
+            uint32_t own[3][2];
+            split2(xs[0][0], xs[0][1], own[0][0], own[1][0], own[2][0]);
+            split2(xs[0][2], xs[0][3], own[0][1], own[1][1], own[2][1]);
+            u32x4_t parts[3];
+#pragma unroll
+            for (int part = 0; part < 3; ++part)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    parts[part][i] = own[part][i];
+                    parts[part][2 + i] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)own[part][i], 0x12c, 0xf, 0xf, true);
+                }
+            xp[0] = {__builtin_bit_cast(bf16x8_t, parts[0]), __builtin_bit_cast(bf16x8_t, parts[1]), __builtin_bit_cast(bf16x8_t, parts[2])};
+            xp[1] = turned(std::integral_constant<int, 0x128>{}, xp[0]);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) multiply32(acc, split8(wv[2 * h], wv[2 * h + 1]), xp[h]);
+    };
+    // The waits below count LOADS loads a stage in the stages' order.  Barriers keep the scheduler to it, and there is no test in front
+    // of the loop (n_stage is at least 1): behind one the compiler had put all loads of x after all those of the weights.
+    each<NS - 1>([&](auto S) {
+        load(S, S);
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    int s0 = 0;
+    do {
+        each<NS>([&](auto S) {
+            constexpr int h = decltype(S)::value;
+            load(std::integral_constant<int, h + NS - 1>{}, s0 + h + NS - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt(0x0f70 | ((LOADS * (NS - 1)) & 15) | (((LOADS * (NS - 1)) >> 4) << 14));      // this stage's loads: those of each later one may be under way
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(S, s0 + h);
+            if constexpr (h % 2 == 1) {
+                group += acc;
+                acc = floatx4_t{0.f, 0.f, 0.f, 0.f};
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        s0 += NS;
+    } while (s0 < n_stage);
+    __builtin_amdgcn_s_waitcnt(0x0f70);                                 // nothing is on its way into LDS any more
+    if (__any(r16 < M && !finite(group))) group = plain_sums(x + (size_t)min(r16, M - 1) * K, w + (size_t)min(n0 + r16, N - 1) * K, k_begin, k_end, 4 * g);
     if (r16 >= M) return;
     const bool whole = gridDim.y == 1;
     float* dst = out + ((size_t)blockIdx.y * M + r16) * N;
@@ -314,6 +504,166 @@ void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, c
     if (!shared_out) write(out, total, bias != nullptr);
 }
 
+// More rows against large weights, by parts in bfloat16: a block of four waves takes 16 RT rows by 64 FT features, each wave all rows of 16 FT.  A wave's weights come straight from
+// memory to its own registers, which take them apart; x goes through LDS, taken apart once for the block (stages of 64 k, three parts a row of 128 bytes each, pieces of 16
+// bytes at their number exclusive-or half their row, so that the 16 rows of an operand meet all banks; two stages in turn, one barrier each).  Loads are issued
+// half a stage or a stage ahead of being taken apart, which happens beside the products of the half before.  Whole groups' sums wait in LDS too, a float4 of each thread's in turn, where
+// the registers would cost a wave per SIMD.  Bound by the matrix cores' power and by what LDS delivers of x (12 pieces a wave for 48 products: about half the time of those).  us, gate+up of the 7B
+// shape, down, q/k/v and o at 300 rows: 581, 381, 100 and 77 (820, 470, 115 and 97 with the float32 instructions); 2000 rows of o 350 (470).  Weights in whole lines in place of the
+// matrix cores' order: 4 % less, not without LDS between; waves of 48 or 64 features, one to a SIMD: 671 and 717; numbers taken apart in front of the products: 587.
+#define GS_WAVES 4
+template <int RT, int FT, bool TAIL>
+__global__ __launch_bounds__(GS_WAVES * TQK_WAVE, 2)
+void gemm_split_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ out,
+                       int M, int N, int K, int groups_per_share) {
+    constexpr int ROWS = 16 * RT, FEATURES = 16 * FT * GS_WAVES, THREADS = GS_WAVES * TQK_WAVE, XL = ROWS * 16 / THREADS;     // XL: what a thread brings in of x, in four k each
+    __shared__ __attribute__((aligned(16))) char lds[2][3][ROWS * 128];
+    __shared__ floatx4_t totals[FT * RT][THREADS];
+    const int tid = threadIdx.x, lane = tid % TQK_WAVE, wave = tid / TQK_WAVE, r16 = lane % 16, g = lane / 16;
+    const int tiles_m = (M + ROWS - 1) / ROWS, tiles_n = (N + FEATURES - 1) / FEATURES;
+    int tm, tn;                                 // (blocks over the dies as in gemm_f32_kernel)
+    {
+        const int n = tiles_m * tiles_n, die = blockIdx.x % 8, at = blockIdx.x / 8, each_die = n / 8, more = n % 8;
+        const int id = die * each_die + min(die, more) + at;
+        tm = id % tiles_m;
+        tn = id / tiles_m;
+    }
+    const int m0 = tm * ROWS, n0 = tn * FEATURES + wave * 16 * FT;
+    const int k_begin = blockIdx.y * groups_per_share * G_GROUP, k_end = min(K, k_begin + groups_per_share * G_GROUP);
+    const bool shared_out = gridDim.y > 1;
+    const float* wrow[FT];
+#pragma unroll
+    for (int f = 0; f < FT; ++f) wrow[f] = w + (size_t)min(n0 + 16 * f + r16, N - 1) * K;
+    const float* xsrc[XL];
+    int xdst[XL];
+    const int xk = 4 * (tid % 16);
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+        const int row = tid / 16 + i * (THREADS / 16);
+        xsrc[i] = x + (size_t)min(m0 + row, M - 1) * K + xk;
+        xdst[i] = row * 128 + (((xk / 8) ^ ((row >> 1) & 7)) * 16) + (xk & 4) * 2;
+    }
+    const floatx4_t none = {0.f, 0.f, 0.f, 0.f};
+    floatx4_t wv[FT][4], xv[XL];
+    // (past the last stage, and with TAIL past K, the row's last values are read; what lies past k_end counts as nothing when it is taken apart)
+    auto load_w = [&](int k0, int h) {
+#pragma unroll
+        for (int f = 0; f < FT; ++f)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) wv[f][2 * h + u] = *reinterpret_cast<const floatx4_t*>(wrow[f] + min(k0 + 32 * h + 8 * g + 4 * u, K - 4));
+    };
+    auto load_x = [&](int k0, int h) {
+#pragma unroll
+        for (int i = h * XL / 2; i < (h + 1) * XL / 2; ++i) xv[i] = *reinterpret_cast<const floatx4_t*>(xsrc[i] + min(k0, K - 4 - xk));
+    };
+    auto put_x = [&](int k0, int to, int h) {
+        const bool in = !TAIL || k0 + xk < k_end;
+#pragma unroll
+        for (int i = h * XL / 2; i < (h + 1) * XL / 2; ++i) {
+            const floatx4_t v = in ? xv[i] : none;
+            uint2 p, q, t;
+            split2(v[0], v[1], p.x, q.x, t.x);
+            split2(v[2], v[3], p.y, q.y, t.y);
+            *reinterpret_cast<uint2*>(&lds[to][0][xdst[i]]) = p;
+            *reinterpret_cast<uint2*>(&lds[to][1][xdst[i]]) = q;
+            *reinterpret_cast<uint2*>(&lds[to][2][xdst[i]]) = t;
+        }
+    };
+    floatx4_t acc[FT][RT], group[FT][RT];
+#pragma unroll
+    for (int f = 0; f < FT; ++f)
+#pragma unroll
+        for (int a = 0; a < RT; ++a) {
+            acc[f][a] = group[f][a] = none;
+            totals[f * RT + a][tid] = none;
+        }
+    auto write = [&](float* y, int f, int a, floatx4_t v, bool with_bias, int k0, int k1) {
+        const int m = m0 + 16 * a + r16;
+        if (__any(!finite(v))) v = plain_sums(x + (size_t)min(m, M - 1) * K, wrow[f], k0, k1, 4 * g);
+        if (m >= M) return;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int n = n0 + 16 * f + 4 * g + i;
+            if (n < N) y[(size_t)m * N + n] = with_bias ? v[i] + bias[n] : v[i];
+        }
+    };
+    Parts wp[FT], ahead[FT];                  // the weights' parts of the half stage at hand, and of the next one
+    auto take_apart = [&](Parts (&to)[FT], int k0, int h) {
+#pragma unroll
+        for (int f = 0; f < FT; ++f) {
+            const bool in0 = !TAIL || k0 + 32 * h + 8 * g < k_end, in1 = !TAIL || k0 + 32 * h + 8 * g + 4 < k_end;
+            to[f] = split8(in0 ? wv[f][2 * h] : none, in1 ? wv[f][2 * h + 1] : none);
+        }
+    };
+    load_x(k_begin, 0);
+    load_x(k_begin, 1);
+    load_w(k_begin, 0);
+    load_w(k_begin, 1);
+    put_x(k_begin, 0, 0);
+    put_x(k_begin, 0, 1);
+    load_x(k_begin + 64, 0);
+    load_x(k_begin + 64, 1);
+    take_apart(wp, k_begin, 0);
+    load_w(k_begin + 64, 0);
+    __syncthreads();
+    for (int c0 = k_begin; c0 < k_end; c0 += G_CHUNK) {
+#pragma unroll
+        for (int stage = 0; stage < 2; ++stage) {
+            const int k0 = c0 + 64 * stage;
+            if (!TAIL && stage == 1 && k0 >= k_end) break;          // (K ends with half a chunk)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                // the next half's weights and half of the next stage's x are taken apart beside this half's products
+                take_apart(ahead, k0 + 64 * h, 1 - h);
+                load_w(k0 + 64 + 64 * h, 1 - h);
+                put_x(k0 + 64, stage ^ 1, h);                       // (what that part of LDS held has been multiplied: a barrier lies between)
+                load_x(k0 + 128, h);
+                Parts xp[RT];
+#pragma unroll
+                for (int a = 0; a < RT; ++a) {
+                    const int row = 16 * a + r16, at = row * 128 + (((4 * h + g) ^ ((row >> 1) & 7)) * 16);
+                    xp[a] = {*reinterpret_cast<const bf16x8_t*>(&lds[stage][0][at]), *reinterpret_cast<const bf16x8_t*>(&lds[stage][1][at]),
+                             *reinterpret_cast<const bf16x8_t*>(&lds[stage][2][at])};
+#pragma unroll
+                    for (int f = 0; f < FT; ++f) multiply32(acc[f][a], wp[f], xp[a]);
+                }
+                // a product's instruction takes the matrix cores 16 cycles and the wave 4: three others beside each
+                __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+#pragma unroll
+                for (int a = 0; a < RT; ++a) {
+#pragma unroll
+                    for (int i = 0; i < 6 * FT; ++i) {
+                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
+                    }
+                    __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+                }
+#pragma unroll
+                for (int f = 0; f < FT; ++f) wp[f] = ahead[f];
+            }
+            __syncthreads();
+        }
+        const int done = c0 + G_CHUNK;
+        const bool end = done % G_GROUP == 0 || done >= k_end;
+#pragma unroll
+        for (int f = 0; f < FT; ++f)
+#pragma unroll
+            for (int a = 0; a < RT; ++a) {
+                group[f][a] += acc[f][a];
+                acc[f][a] = none;
+                if (!end) continue;
+                if (shared_out) write(out + (size_t)(c0 / G_GROUP) * M * N, f, a, group[f][a], false, c0 / G_GROUP * G_GROUP, min(done, k_end));
+                else totals[f * RT + a][tid] += group[f][a];
+                group[f][a] = none;
+            }
+    }
+    if (shared_out) return;
+#pragma unroll
+    for (int f = 0; f < FT; ++f)
+#pragma unroll
+        for (int a = 0; a < RT; ++a) write(out, f, a, totals[f * RT + a][tid], bias != nullptr, k_begin, k_end);
+}
+
 __global__ void gemm_few_rows_sum_kernel(const float* __restrict__ group_sums, const float* __restrict__ bias,
                                          float* __restrict__ y, int n_groups, int M, int N) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -329,13 +679,35 @@ static bool f32_case(int x_dtype, int w_dtype, const void* bias, int bias_dtype,
            ((((uintptr_t)x) | ((uintptr_t)w)) & 15) == 0;
 }
 
+// Whether a product's numbers are taken apart: where its weights are large (4 MB).  Below it launches are what a product costs, and the kernel for a small model's
+// whole step (small_step.hip) has the order of the float32 instructions.
+extern "C" int tqk_gemm_takes_apart(int N, int K) { return (long long)N * K >= 1 << 20; }
+
+// Tiles of 16 rows and of 16 features a wave of gemm_split_kernel takes, in blocks of four waves side by side: the largest that leaves every unit a block.  us with 64 rows by 128
+// features everywhere, and so: 300 rows of 1536 x 1536 39.0 and 25.1, 64 and 24 rows of 3584 x 3584 39.0 and 27.8, 33.5 and 25.2 (31.8, 32.1 and 31.3 with the float32 instructions).
+// 9 to 16 rows go there with one tile of each where that gives every unit two blocks (of whole groups): 16 rows of 37888 x 3584, 3584 x 18944, 152064 x 3584, 4608 x 3584 and 3584 x 3584
+// 124, 66, 512, 21.1 and 17.8, through the kernel for few rows 140, 77, 558, 19.7 and 16.8 (139, 76, 548, 18.8 and 16.3 with the float32 instructions).
+struct SplitTile { int rows, features; };
+static SplitTile split_tile(int M, int N, int K) {
+    const int groups = (K + G_GROUP - 1) / G_GROUP;
+    auto blocks = [&](SplitTile t) { return (long long)((M + 16 * t.rows - 1) / (16 * t.rows)) * ((N + 64 * t.features - 1) / (64 * t.features)) * groups; };
+    if (M <= 16) return M > 8 && blocks({1, 1}) >= 512 ? SplitTile{1, 1} : SplitTile{0, 0};
+    const SplitTile all[] = {{4, 2}, {2, 2}, {4, 1}, {2, 1}};
+    for (const SplitTile& t : all)
+        if ((t.rows == 2 || M > 32) && blocks(t) >= 256) return t;
+    return {2, 1};
+}
+
 // Into how many shares the groups are dealt for M rows: few rows, one a group; more, so that there are about four blocks a compute
-// unit (one: 280 blocks of 300 x 3584 leave most units idle while a few do a second block), no more than there are groups.
+// unit (one: 280 blocks of 300 x 3584 leave most units idle while a few do a second block) and two of the larger ones that take numbers apart, no more than there are groups.
 static int f32_shares(int M, int N, int K) {
     const int groups = (K + G_GROUP - 1) / G_GROUP;
     if (M <= 16) return groups;
-    const long long tiles = (long long)((M + GT - 1) / GT) * ((N + GT - 1) / GT);
-    const int want = (int)(tiles >= 1024 ? 1 : (1024 + tiles - 1) / tiles), per = (groups + want - 1) / want;
+    const bool apart = tqk_gemm_takes_apart(N, K);
+    const SplitTile t = split_tile(M, N, K);
+    const int rows = apart ? 16 * t.rows : GT, features = apart ? 64 * t.features : GT, blocks = apart ? 512 : 1024;
+    const long long tiles = (long long)((M + rows - 1) / rows) * ((N + features - 1) / features);
+    const int want = (int)(tiles >= blocks ? 1 : (blocks + tiles - 1) / tiles), per = (groups + want - 1) / want;
     return (groups + per - 1) / per;
 }
 
@@ -370,8 +742,31 @@ extern "C" int tqk_gemm(const void* x, int x_dtype, const void* w, int w_dtype, 
         TQK_REQUIRE(groups <= 65535, "tqk_gemm: K=%d is more than the grid takes", K);
         const float *xf = (const float*)x, *wf = (const float*)w, *bf = (const float*)bias;
         float* out = shares > 1 ? (float*)scratch : (float*)y;
-        if (M <= 16 && shares == groups) gemm_few_rows_kernel<<<dim3((N + 15) / 16, groups), TQK_WAVE, 0, s>>>(xf, wf, bf, out, M, N, K);
-        else gemm_f32_kernel<<<dim3(((N + GT - 1) / GT) * ((M + GT - 1) / GT), shares), 256, 0, s>>>(xf, wf, bf, out, M, N, K, (groups + shares - 1) / shares);
+        const bool apart = tqk_gemm_takes_apart(N, K);
+        const int per = (groups + shares - 1) / shares;
+        SplitTile t = apart ? split_tile(M, N, K) : SplitTile{0, 0};
+        if (apart && t.rows == 0 && shares < groups) t = {1, 1};             // (few rows without scratch: one block walks all of K)
+        if (t.rows == 0 && M <= 16 && shares == groups) {
+            const dim3 grid((N + 15) / 16, groups);
+            if (!apart) gemm_few_rows_kernel<<<grid, TQK_WAVE, 0, s>>>(xf, wf, bf, out, M, N, K);
+            else {
+#define LAUNCH(ROWS) do { if (K % 64) gemm_few_rows_apart_kernel<true, ROWS><<<grid, TQK_WAVE, 0, s>>>(xf, wf, bf, out, M, N, K); \
+        else gemm_few_rows_apart_kernel<false, ROWS><<<grid, TQK_WAVE, 0, s>>>(xf, wf, bf, out, M, N, K); } while (0)
+                if (M <= 4) LAUNCH(4);
+                else if (M <= 8) LAUNCH(8);
+                else LAUNCH(16);
+#undef LAUNCH
+            }
+        } else if (apart) {
+            const dim3 grid(((N + 64 * t.features - 1) / (64 * t.features)) * ((M + 16 * t.rows - 1) / (16 * t.rows)), shares);
+#define LAUNCH(RT, FT) do { if (K % 64) gemm_split_kernel<RT, FT, true><<<grid, GS_WAVES * TQK_WAVE, 0, s>>>(xf, wf, bf, out, M, N, K, per); \
+        else gemm_split_kernel<RT, FT, false><<<grid, GS_WAVES * TQK_WAVE, 0, s>>>(xf, wf, bf, out, M, N, K, per); } while (0)
+            if (t.rows == 1) LAUNCH(1, 1);
+            else if (t.rows == 4) { if (t.features == 2) LAUNCH(4, 2); else LAUNCH(4, 1); }
+            else if (t.features == 2) LAUNCH(2, 2);
+            else LAUNCH(2, 1);
+#undef LAUNCH
+        } else gemm_f32_kernel<<<dim3(((N + GT - 1) / GT) * ((M + GT - 1) / GT), shares), 256, 0, s>>>(xf, wf, bf, out, M, N, K, (groups + shares - 1) / shares);
         if (tqk_check_launch("tqk_gemm float32")) return -1;
         if (shares == 1) return 0;
         const size_t total = (size_t)M * N;

@@ -464,6 +464,8 @@ extern "C" int tqk_small_step_takes(const TqkSmallStep* step) {
     const int q = p.n_heads * p.head_dim, whole = 64 / size;
     if (p.hidden % whole || p.inter % whole || q % whole || (p.n_kv_heads * p.head_dim * 2) % 16) return 0;
     if (small_layout(p).bytes > 160 * 1024) return 0;
+    // (larger products have another order of summation there)
+    if (p.act_dtype == TQK_F32 && (tqk_gemm_takes_apart(p.vocab, p.hidden) || tqk_gemm_takes_apart(2 * p.inter, p.hidden) || tqk_gemm_takes_apart(q + 2 * p.n_kv_heads * p.head_dim, p.hidden))) return 0;
     return 1;
 }
 
