@@ -255,7 +255,6 @@ void small_step_kernel(const TqkSmallStep p) {
         one.ask();
         return one;
     };
-    SmallProduct<T, 1> w_qkv = product(p.layers[0].qkv, qkv, hidden, row_tiles);
     for (int i = tid; i < p.n_ints; i += SS_THREADS) ints[i] = p.ints[i];
     for (int i = tid; i < p.n_layers * (int)(sizeof(TqkSmallLayer) / 4); i += SS_THREADS)
         reinterpret_cast<int32_t*>(lds + at.layers)[i] = reinterpret_cast<const int32_t*>(p.layers)[i];
@@ -318,6 +317,7 @@ void small_step_kernel(const TqkSmallStep p) {
         for (int i = 0; i < (int)(sizeof(l) / 4); ++i)
             reinterpret_cast<int32_t*>(&l)[i] = __builtin_amdgcn_readfirstlane(reinterpret_cast<const int32_t*>(layers + layer)[i]);
         const int32_t* table = ints + l.table;
+        SmallProduct<T, 1> w_qkv = product(l.qkv, qkv, hidden, row_tiles);
         for (int r = wave; r < rows; r += SS_WAVES) norm_row(r, r, norms + 2 * layer * hidden, l.eps1);
         lds_barrier();
         float* bf = reinterpret_cast<float*>(b);
@@ -431,11 +431,6 @@ void small_step_kernel(const TqkSmallStep p) {
         SmallProduct<T, 1> w_down = product(l.down, hidden, inter, row_tiles);
         lds_barrier();
         w_down.run(act, ld_act, rows, add_to_stream);
-        if (layer + 1 < p.n_layers) {
-            const uint64_t next = (uint64_t)layers[layer + 1].qkv;
-            w_qkv = product((const void*)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(next >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)next)),
-                            qkv, hidden, row_tiles);
-        }
         lds_barrier();
     }
 
