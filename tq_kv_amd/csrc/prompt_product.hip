@@ -14,7 +14,7 @@
 //    LDS), four stages in turn, one barrier a stage.  A load takes eight whole 128-byte lines of x; the 16-byte pieces of a row
 //    are exchanged within it (piece c of row r lies at c ^ ((r / 2) % 8)) so that the waves' reads of 16 rows of one k step meet
 //    all banks once.  A wave reads its operands PD groups ahead, across the barrier too.
-//  - WN = 5 with 15 groups of rows (240): gated products of one such row of blocks and no more blocks than units, where what a compute unit
+//  - WN = 5 with 15 groups of rows (240; in ten waves for up to 160, 192 and 256 rows, see five_wide): gated products of one such row of blocks and no more blocks than units, where what a compute unit
 //    brings in binds and not the products: every block needs all of x, so few, even blocks count.  us at 129, 170, 232 rows against the best
 //    tile of four waves: 18944 gated features (237 blocks of 80) x K of 3584 73, 73, 74 against 80, 84, 90; 17920 x 5120 100, 102, 104 against
 //    115, 120, 127; 20480 x 3584 75, 78, 80 against 80, 84, 90; 16640 x 2048 43, 45, 46 against 42, 47, 51; 17920 x 1536 36, 39, 39 against
@@ -22,7 +22,8 @@
 //    since a block alone on its unit has a lower rate (17920 x 1536, 440 rows: 38 against 34.5).  Products without a gate have too few blocks
 //    of that height: with every number of pieces of K tried at 129 to 240 rows, q/k/v and o lose at all three Qwen2.5 shapes (7B, 232 rows:
 //    25.0 against 18.9 and 23.5 against 15.8) and down at the 1.5B one (27 against 19); the other two are within 4 % (50.6 against 50.1, 85.6
-//    against 89.3).
+//    against 89.3).  Ten waves: 18944 x 3584 at 129, 170 and 256 rows 74, 75 and 83 against 87 and 86 with 240 rows in five waves and 96 with the best tile of
+//    four, 16640 x 2048 42, 46 and 49 against 50, 49 and 62, 17920 x 1536 35, 38 and 41 against 40, 39 and 44; at 232 rows the same as five.
 //  - WM = 2: a second row of four waves on the next MT groups of rows, 256 rows a block, one block a compute unit; the two
 //    waves of a column meet each other's weights in the first-level cache, and a unit brings in a third less than two blocks
 //    of WM = 1 would.  Worth a little where K is long (8000 x 3584 x 18944: 861 us against 869), not where it is short (8000 x 37888 x 3584
@@ -276,19 +277,28 @@ struct PromptPlan { int config, splits, k_per_split; double us; };
 struct PromptConfig { int mt, nt, wm, wn; double rate; };
 static const PromptConfig CONFIGS[] = {
     {8, 4, 2, 4, 1.00}, {8, 4, 1, 4, 0.96}, {8, 3, 2, 4, 0.95}, {8, 3, 1, 4, 0.90}, {6, 4, 1, 4, 0.84},
-    {8, 2, 1, 4, 0.78}, {5, 4, 1, 4, 0.72}, {4, 4, 1, 4, 0.66}, {5, 2, 1, 4, 0.58}, {15, 2, 1, 5, 0.79},
+    {8, 2, 1, 4, 0.78}, {5, 4, 1, 4, 0.72}, {4, 4, 1, 4, 0.66}, {5, 2, 1, 4, 0.58}, {15, 2, 1, 5, 0.79},     // (the last: five_wide)
 };
 #define PROMPT_CONFIGS ((int)(sizeof(CONFIGS) / sizeof(CONFIGS[0])))
 #define PROMPT_UNITS 256
 #define PROMPT_MAX_SPLITS 16
 
+// The gated tile of five waves side by side has all rows in one block, as high as they are many: two rows of five waves for up to 160, 192 and 256, whose ten
+// waves lie more evenly on the four SIMDs than five do (three and two against two and one), and one of five for up to 240, which brings weights in once.
+static PromptConfig five_wide(int M) {
+    if (M <= 160) return {5, 2, 2, 5, 0.62};
+    if (M <= 192) return {6, 2, 2, 5, 0.72};
+    if (M <= 240) return {15, 2, 1, 5, 0.79};
+    return {8, 2, 2, 5, 0.84};
+}
+
 static PromptPlan prompt_plan(int M, int N, int K, bool gated) {
     PromptPlan best = {0, 1, K, 1e30};
     const long long turns = K / PROMPT_K;
     for (int i = 0; i < PROMPT_CONFIGS; ++i) {
-        const PromptConfig& c = CONFIGS[i];
+        const PromptConfig c = CONFIGS[i].wn == 5 ? five_wide(M) : CONFIGS[i];
         if (gated && c.nt % 2) continue;
-        if (c.wn == 5 && (!gated || M > 16 * c.mt)) continue;
+        if (c.wn == 5 && (!gated || M > 256)) continue;
         const long long rows = 16LL * c.mt * c.wm, width = 16LL * c.wn * (gated ? c.nt / 2 : c.nt), n_out = gated ? N / 2 : N;
         const long long tiles = ((M + rows - 1) / rows) * ((n_out + width - 1) / width);
         if (tiles > 0x7fffffffLL) continue;
@@ -297,7 +307,7 @@ static PromptPlan prompt_plan(int M, int N, int K, bool gated) {
             if (per * (splits - 1) >= turns) continue;                                                // an empty piece
             const double rounds = (double)((tiles * splits + PROMPT_UNITS - 1) / PROMPT_UNITS);
             // (us: 256 units at the best tile's rate are 1.4 PFLOP/s)
-            double us = rounds * (c.mt * c.nt * c.wm * c.wn / 4.0) / c.rate * (double)(per * PROMPT_K + (gated && c.wm == 2 ? 600 : 300)) * 3.7e-4;
+            double us = rounds * (c.mt * c.nt * c.wm * c.wn / 4.0) / c.rate * (double)(per * PROMPT_K + (gated && c.wm == 2 && c.wn == 4 ? 600 : 300)) * 3.7e-4;
             if (splits > 1) us += (double)splits * M * N * 8.0 / 4.5e6;
             if (us < best.us) best = {i, splits, (int)(per * PROMPT_K), us};
         }
@@ -343,7 +353,7 @@ static void launch(const PromptArgs& a, int splits, hipStream_t s) {
 
 template <int EPI>
 static int launch_plan(PromptArgs a, const PromptPlan& plan, hipStream_t s) {
-    const PromptConfig& c = CONFIGS[plan.config];
+    const PromptConfig c = CONFIGS[plan.config].wn == 5 ? five_wide(a.M) : CONFIGS[plan.config];
     const int rows = 16 * c.mt * c.wm, width = 16 * c.wn * (EPI == PROMPT_GATED ? c.nt / 2 : c.nt), n_out = EPI == PROMPT_GATED ? a.N / 2 : a.N;
     a.tiles_m = (a.M + rows - 1) / rows;
     a.tiles_n = (n_out + width - 1) / width;
@@ -358,7 +368,14 @@ static int launch_plan(PromptArgs a, const PromptPlan& plan, hipStream_t s) {
         case 6: launch<5, 4, 1, EPI>(a, plan.splits, s); break;
         case 7: launch<4, 4, 1, EPI>(a, plan.splits, s); break;
         case 8: launch<5, 2, 1, EPI>(a, plan.splits, s); break;
-        default: if constexpr (EPI == PROMPT_GATED) launch<15, 2, 1, EPI, 5>(a, plan.splits, s); break;
+        default:
+            if constexpr (EPI == PROMPT_GATED) {
+                if (c.mt == 5) launch<5, 2, 2, EPI, 5>(a, plan.splits, s);
+                else if (c.mt == 6) launch<6, 2, 2, EPI, 5>(a, plan.splits, s);
+                else if (c.mt == 8) launch<8, 2, 2, EPI, 5>(a, plan.splits, s);
+                else launch<15, 2, 1, EPI, 5>(a, plan.splits, s);
+            }
+            break;
     }
     return tqk_check_launch("tqk_prompt product");
 }
