@@ -356,8 +356,10 @@ void attention_decode_kernel(const DecodeSums in, const bf16_t* __restrict__ q, 
                         mx = fmaxf(mx, s[t][r]);
                     }
             }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, TQK_WAVE));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, TQK_WAVE));
+            float2 both = with_lane_16(mx);
+            mx = fmaxf(both.x, both.y);
+            both = with_lane_32(mx);
+            mx = fmaxf(both.x, both.y);
             // mx is finite: the page holds at least one key of [lo, pos]
             const float alpha = __builtin_amdgcn_exp2f(m - mx);     // 2^(-inf) = 0 on the wave's first page
             m = mx;
@@ -423,8 +425,10 @@ void attention_decode_kernel(const DecodeSums in, const bf16_t* __restrict__ q, 
                 for (int pr = 0; pr < 2; ++pr) o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[db][pr], pb[pr].v, o[db], 0, 0, 0);
             }
         }
-        l += __shfl_xor(l, 16, TQK_WAVE);
-        l += __shfl_xor(l, 32, TQK_WAVE);
+        float2 both = with_lane_16(l);
+        l = both.x + both.y;
+        both = with_lane_32(l);
+        l = both.x + both.y;
     }
 
     // The waves' results meet in wave order, each wave taking its share of the elements.

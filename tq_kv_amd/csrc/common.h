@@ -4,8 +4,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <type_traits>
-
 #define TQK_WAVE 64
 #define TQK_PAGE 64
 
@@ -57,21 +55,31 @@ __device__ __forceinline__ void rotate_pair(float& x0, float& x1, float cos, flo
 }
 
 // ---- reductions ---------------------------------------------------------------
-// Over a wave, every lane gets the result: lanes 32 apart first, then 16, 8, 4, 2 and 1.  The partner's value comes by the vector unit's own lane
-// moves: a swap of halves or of rows of 16, a turn of a row by 8, and by 4 (lanes 8 apart are equal by then, so that
-// is the partner's value too), and a permutation of four.  A shuffle through LDS takes 36 ns of a wave's time, six of them 0.2 us.
+// Lane moves of the vector unit: a shuffle through LDS takes 36 ns of a wave's time, one after the other where sums depend on each other.
+// A lane's value and that of the lane 32 (16) away, the lower one first, the same for both.
+__device__ __forceinline__ float2 with_lane_32(float v) {
+    const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return make_float2(__uint_as_float(both[0]), __uint_as_float(both[1]));
+}
+__device__ __forceinline__ float2 with_lane_16(float v) {
+    const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return make_float2(__uint_as_float(both[0]), __uint_as_float(both[1]));
+}
+template <int CTRL> __device__ __forceinline__ float moved(float v) { return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CTRL, 0xf, 0xf, true)); }
+__device__ __forceinline__ float lane_xor_8(float v) { return moved<0x128>(v); }                      // row_ror:8
+__device__ __forceinline__ float lane_xor_4(float v) { return moved<0x1b>(moved<0x141>(v)); }         // row_half_mirror (xor 7), quad_perm:[3,2,1,0] (xor 3)
+
+// Over a wave, every lane gets the result: lanes 32 apart first, then 16, 8, 4, 2 and 1 (lanes 8 apart are equal by the time 4 is come to, so that a turn of 16 lanes by 4
+// brings the partner's value too).
 template <typename F> __device__ __forceinline__ float wave_reduce(float v, F&& op) {
-    const uint32_t u = __float_as_uint(v);
-    const auto halves = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-    v = op(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
-    const uint32_t w = __float_as_uint(v);
-    const auto rows = __builtin_amdgcn_permlane16_swap(w, w, false, false);
-    v = op(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
-    auto moved = [&](auto ctrl) { return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), decltype(ctrl)::value, 0xf, 0xf, true)); };
-    v = op(v, moved(std::integral_constant<int, 0x128>{}));         // row_ror:8
-    v = op(v, moved(std::integral_constant<int, 0x124>{}));         // row_ror:4
-    v = op(v, moved(std::integral_constant<int, 0x4e>{}));          // quad_perm:[2,3,0,1]
-    v = op(v, moved(std::integral_constant<int, 0xb1>{}));          // quad_perm:[1,0,3,2]
+    float2 both = with_lane_32(v);
+    v = op(both.x, both.y);
+    both = with_lane_16(v);
+    v = op(both.x, both.y);
+    v = op(v, lane_xor_8(v));
+    v = op(v, moved<0x124>(v));         // row_ror:4
+    v = op(v, moved<0x4e>(v));          // quad_perm:[2,3,0,1]
+    v = op(v, moved<0xb1>(v));          // quad_perm:[1,0,3,2]
     return v;
 }
 __device__ __forceinline__ float wave_sum(float v) { return wave_reduce(v, [](float a, float b) { return a + b; }); }

@@ -269,13 +269,15 @@ void skinny_fused_kernel(const FusedArgs p) {
             ssq.x += v.x; ssq.y += v.y; ssq.z += v.z; ssq.w += v.w;
         }
         // lanes with equal lane%4 hold the same rows: add them up, fixed order
-#pragma unroll
-        for (int d = 4; d < TQK_WAVE; d *= 2) {
-            ssq.x += __shfl_xor(ssq.x, d, TQK_WAVE);
-            ssq.y += __shfl_xor(ssq.y, d, TQK_WAVE);
-            ssq.z += __shfl_xor(ssq.z, d, TQK_WAVE);
-            ssq.w += __shfl_xor(ssq.w, d, TQK_WAVE);
-        }
+        auto over_lanes = [](float& v) {
+            v += lane_xor_4(v);
+            v += lane_xor_8(v);
+            float2 both = with_lane_16(v);
+            v = both.x + both.y;
+            both = with_lane_32(v);
+            v = both.x + both.y;
+        };
+        over_lanes(ssq.x); over_lanes(ssq.y); over_lanes(ssq.z); over_lanes(ssq.w);
     }
 
     // add the waves' partial tiles up in wave order
@@ -356,9 +358,8 @@ void skinny_fused_kernel(const FusedArgs p) {
         }
         if (p.ss_out) {
             // this block's columns of row m: the four lanes of the row, in lane order
-            const float s1 = __shfl_xor(sq, 16, TQK_WAVE);
-            const float s2 = __shfl_xor(sq, 32, TQK_WAVE);
-            const float s3 = __shfl_xor(s1, 32, TQK_WAVE);
+            // (read in the first 16 lanes: the values of the lanes 16, 32 and 48 on)
+            const float s1 = with_lane_16(sq).y, s2 = with_lane_32(sq).y, s3 = with_lane_32(s1).y;
             if (kgrp == 0 && m < p.M) p.ss_out[(size_t)blockIdx.x * 16 + m] = ((sq + s1) + s2) + s3;
         }
     } else {    // EPI_QKV
