@@ -664,12 +664,30 @@ void gemm_split_kernel(const float* __restrict__ x, const float* __restrict__ w,
         for (int a = 0; a < RT; ++a) write(out, f, a, totals[f * RT + a][tid], bias != nullptr, k_begin, k_end);
 }
 
+// The groups' sums in their order.  Eight loads under way together: one after the other they were most of the time (19 groups of one row of 3584 5.6 -> 4.7 us).
 __global__ void gemm_few_rows_sum_kernel(const float* __restrict__ group_sums, const float* __restrict__ bias,
                                          float* __restrict__ y, int n_groups, int M, int N) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (size_t)M * N) return;
+    const size_t group = (size_t)M * N;
+    const float* from = group_sums + i;
     float total = 0.f;
-    for (int g = 0; g < n_groups; ++g) total += group_sums[(size_t)g * M * N + i];
+    int g = 0;
+    for (; g + 8 <= n_groups; g += 8, from += 8 * group) {
+        float sums[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) sums[u] = from[u * group];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) total += sums[u];
+    }
+    // (what is left likewise: the last group again where there are fewer, not added)
+    if (g < n_groups) {
+        float sums[7];
+#pragma unroll
+        for (int u = 0; u < 7; ++u) sums[u] = from[min(u, n_groups - 1 - g) * group];
+#pragma unroll
+        for (int u = 0; u < 7; ++u) total = g + u < n_groups ? total + sums[u] : total;
+    }
     if (bias) total += bias[i % N];
     y[i] = total;
 }
