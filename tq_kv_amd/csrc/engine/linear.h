@@ -4,7 +4,7 @@
 // (src/models/turbo_generic.rs:68-91).  Here:
 //
 //   float32 anywhere (the 32-bit path, or a weight stored in 32-bit)
-//         -> the hand-written FMA kernel (no matrix cores, fixed summation order)
+//         -> the hand-written kernels of gemm_generic.hip (float32 sums in a fixed order; large weights: every number as three bfloat16 ones)
 //   bfloat16, few rows (decoding, chosen logit rows; as many as the skinny kernel takes)
 //         -> the hand-written weight-streaming MFMA kernel (alone here, with the neighbouring
 //            norm, residual sum, gate or rotation folded in where parts ask).  It reads a second

@@ -4,7 +4,7 @@
 // microsecond and costs two to four in a replayed graph, and about as much again on the host.  One block on one compute unit runs
 // the step with barriers in place of launches.  It pulls weights and does a row's work at a fraction of the chip's rate, so this is the better way only
 // while that takes no longer than the launches it stands for: tqk_small_step_pays says where that is.  Two layers of 64 values, 3 sequences after
-// 20 tokens: 22.2 us in bfloat16 and 32.7 in float32 for what a replayed graph of 21 kernels does in 65 and 81; three of 96: 34.3 and 62.5 for 76 and 110.
+// 20 tokens: 22.2 us in bfloat16 and 30.2 in float32 for what a replayed graph of 21 kernels does in 65 and 81; three of 96: 34.3 and 62.5 for 76 and 110.
 // What a phase between two barriers takes (three of 96, bfloat16, us): norm 0.6 to 0.8, q/k/v 0.6, rotation 0.7, attention 2.6, o 1.2,
 // gate and up 1.5, down 1.3, none of it bytes or products but a wave's instructions one after the other, 4 and more cycles each.
 //
