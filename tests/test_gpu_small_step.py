@@ -1,6 +1,6 @@
-"""Steps of small models in one launch (csrc/small_step.hip) against the same steps through the kernels of larger ones: in float32 the same
-bits, in bfloat16 as far apart as its roundings make two orders of summation.  Shapes with 16 to 64 values a head, widths that are and
-are not whole steps of the matrix cores, more tiles than waves; steps of 1 to 64 rows on both sides of every change of the kernel."""
+"""Steps of small models in one launch (csrc/small_step.hip) against the same steps through the kernels of larger ones: the same bits.  Shapes with 16 to
+64 values a head, widths that are and are not whole steps of the matrix cores, more tiles than waves, K that other kernels deal out to
+waves or cut into pieces; steps of 1 to 64 rows on both sides of every change of the kernels that the step stands for.  Which way a step went is counted."""
 import pytest
 import torch
 
@@ -9,6 +9,7 @@ from tq_kv_amd import POLICY, Engine, Model
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
+PAGE = 64
 
 
 def shape(hidden, inter, heads, kv_heads, head_dim, layers, vocab=97, window=None, tied=False):
@@ -19,77 +20,146 @@ def shape(hidden, inter, heads, kv_heads, head_dim, layers, vocab=97, window=Non
     return cfg
 
 
+# (and the most rows whose stream and products fit the unit's LDS, float32 and bfloat16)
 SHAPES = {
-    "a": helpers.TINY_A, "b": helpers.TINY_B,
-    "one head": shape(32, 32, 1, 1, 32, 1, vocab=16),
-    "more tiles than waves": shape(96, 288, 4, 2, 64, 2, vocab=700, window=70),
-    "wide": shape(160, 192, 5, 5, 32, 3, tied=True),
-    "no whole step of k": shape(48, 80, 4, 2, 20, 2),              # float32 alone: bfloat16 takes 32 k at a time
-    "many layers": shape(32, 64, 2, 1, 16, 16),
+    "a": (helpers.TINY_A, 64, 64), "b": (helpers.TINY_B, 64, 64),
+    "one head": (shape(32, 32, 1, 1, 32, 1, vocab=16), 64, 64),
+    "more tiles than waves": (shape(96, 224, 3, 1, 64, 2, vocab=700, window=70), 48, 48),
+    "wide": (shape(160, 192, 5, 5, 32, 3, tied=True), 32, 32),
+    "k dealt out to waves": (shape(256, 512, 4, 2, 64, 2, window=9), 19, 0),                # (bfloat16 keeps the order of the kernels that deal it out)
+    "k in pieces": (shape(64, 1024, 2, 1, 32, 2), 16, 0),
+    "many heads": (shape(32, 32, 28, 4, 8, 2, window=40), 48, 64),
+    "more heads than a tile": (shape(32, 32, 20, 1, 32, 2, window=40), 16, 0),
+    "no whole step of k": (shape(48, 80, 4, 2, 20, 2), 64, 0),              # float32 alone: bfloat16 takes 32 k at a time
+    "many layers": (shape(32, 64, 2, 1, 16, 16), 64, 64),
 }
 
 
-def close(a, b, dtype, what):
-    if dtype == "float32":
-        assert torch.equal(a, b), what
-    else:                # (one rounding in a few hundred differs by a step of 2^-8; two such runs stay within a tenth of the logits' spread)
-        assert (a - b).abs().max() <= 0.1 * b.std(), what
+class policy:
+    def __init__(self, **values):
+        self.values = values
+
+    def __enter__(self):
+        self.old = {n: POLICY[n] for n in self.values}
+        POLICY.update(self.values)
+
+    def __exit__(self, *_):
+        POLICY.update(self.old)
+
+
+class Steps:
+    """An engine's steps, and how many of them the one launch should take."""
+
+    def __init__(self, model, cfg, dtype, most, always):
+        self.eng, self.most, self.expected = Engine(model, max_tokens=1024), most, 0
+        self.always = always
+        self.furthest = PAGE if dtype == "bfloat16" and cfg["head_dim"] in (32, 64) else 1 << 30       # those heads' attention is of one page there
+
+    def __call__(self, items, **kw):
+        self.expected += self.always and sum(len(t) for _, t, _ in items) <= self.most and max(self.eng.length(s) + len(t) for s, t, _ in items) <= self.furthest
+        return self.eng.step(items, **kw)
+
+    def done(self, slots):
+        for s in slots:
+            self.eng.close(s)
+        self.eng.cache.check()
+        assert self.eng.n_small_steps == self.expected
 
 
 def steps(eng, vocab, count):
     """Prompts of several lengths, a chunk after them, single tokens from the host and from the device, wanted places out of order and none."""
-    out, slots = [], [eng.open() for _ in range(3)]
+    out, slots = [], [eng.eng.open() for _ in range(3)]
     tok = lambda n, s: helpers.random_tokens(n, vocab, s)
-    out.append(eng.step([(slots[0], tok(count, 1), [count - 1, 0] if count > 1 else [0])]))
-    out.append(eng.step([(slots[1], tok(1, 2), [0]), (slots[0], tok(min(7, 65 - count), 3), [])]))
-    out.append(eng.step([(slots[2], tok(9, 4), [8, 3]), (slots[1], tok(3, 5), [2])]))
+    out.append(eng([(slots[0], tok(count, 1), [count - 1, 0] if count > 1 else [0])]))
+    out.append(eng([(slots[1], tok(1, 2), [0]), (slots[0], tok(min(7, 65 - count), 3), [])]))
+    out.append(eng([(slots[2], tok(9, 4), [8, 3]), (slots[1], tok(3, 5), [2])]))
     for i in range(3):
         dev = torch.tensor(tok(3, 10 + i), dtype=torch.int32, device=DEV) if i else None
-        out.append(eng.step([(s, [t], [0]) for s, t in zip(slots, tok(3, 10 + i))], device_tokens=dev))
-    borrowed = eng.step([(s, [1], [0]) for s in slots], borrow=True).clone()
-    out.append(borrowed)
-    for s in slots:
-        eng.close(s)
-    eng.cache.check()
+        out.append(eng([(s, [t], [0]) for s, t in zip(slots, tok(3, 10 + i))], device_tokens=dev))
+    out.append(eng([(s, [1], [0]) for s in slots], borrow=True).clone())
+    eng.done(slots)
     return out
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", list(SHAPES))
 def test_the_step_in_one_launch_equals_the_kernels_of_larger_models(name, dtype):
-    cfg = SHAPES[name]
+    cfg, most = SHAPES[name][0], SHAPES[name][1 + (dtype == "bfloat16")]
     model = Model.random(cfg, seed=3, dtype=dtype, device=DEV)
-    for count in [1, 2, 15, 16, 17, 31, 32, 33, 48, 61, 64]:
-        got = steps(Engine(model, max_tokens=1024), cfg["vocab_size"], count)
-        old = POLICY["small"]
-        POLICY["small"] = False
-        try:
-            want = steps(Engine(model, max_tokens=1024), cfg["vocab_size"], count)
-        finally:
-            POLICY["small"] = old
+    for count in [1, 2, 15, 16, 17, 31, 32, 33, 48, 58, 61, 64]:
+        with policy(small_always=True):
+            got = steps(Steps(model, cfg, dtype, most, True), cfg["vocab_size"], count)
+        with policy(small=False):
+            want = steps(Steps(model, cfg, dtype, most, False), cfg["vocab_size"], count)
         for i, (a, b) in enumerate(zip(got, want)):
-            close(a, b, dtype, "%s, prompt of %d, step %d" % (name, count, i))
+            assert torch.equal(a, b), "%s, prompt of %d, step %d: %g of the values differ, by up to %g" % (
+                name, count, i, (a != b).float().mean(), (a - b).abs().max())
+
+
+@pytest.mark.parametrize("use_graphs", [True, False])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("name", ["a", "b", "one head", "more tiles than waves", "more heads than a tile", "many layers"])
+def test_decoding_steps_of_many_sequences(name, dtype, use_graphs):
+    """1 to 40 sequences of 1 to 60 positions (a page that is filled to its last place among them), some of their logits wanted."""
+    cfg, most = SHAPES[name][0], SHAPES[name][1 + (dtype == "bfloat16")]
+    model = Model.random(cfg, seed=5, dtype=dtype, device=DEV)
+
+    def run(always):
+        out = []
+        for n in [1, 3, 15, 16, 17, 40]:
+            s = Steps(model, cfg, dtype, most, always)
+            s.eng = Engine(model, max_tokens=64 * 64, use_graphs=use_graphs)
+            slots = [s.eng.open() for _ in range(n)]
+            for i, slot in enumerate(slots):
+                s([(slot, helpers.random_tokens(60 - 7 * i % 53, cfg["vocab_size"], i), [])])
+            for k in range(4):
+                out.append(s([(slot, [(5 * i + k) % cfg["vocab_size"]], [0] if (i + k) % 3 or n == 1 else []) for i, slot in enumerate(slots)]))
+            s.done(slots)
+        return out
+
+    with policy(small_always=True):
+        got = run(True)
+    with policy(small=False):
+        want = run(False)
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert torch.equal(a, b), "%s, step %d: %g of the values differ, by up to %g" % (name, i, (a != b).float().mean(), (a - b).abs().max())
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-def test_several_pages_and_a_window_across_them(dtype):
-    cfg = SHAPES["more tiles than waves"]
+@pytest.mark.parametrize("head_dim", [64, 48, 32])
+def test_several_pages_and_a_window_across_them(head_dim, dtype):
+    cfg = shape(96, 96, 3, 1, head_dim, 2, vocab=700, window=70) if head_dim != 48 else shape(96, 96, 4, 2, head_dim, 2, vocab=700, window=70)
+    chunk = 32 if head_dim == 64 else 48                    # (what fits the unit's LDS)
     model = Model.random(cfg, seed=4, dtype=dtype, device=DEV)
     tokens = helpers.random_tokens(210, cfg["vocab_size"], 9)
 
-    def run():
-        eng = Engine(model, max_tokens=512)
-        s, out = eng.open(), []
-        for a in range(0, 192, 48):
-            out.append(eng.step([(s, tokens[a:a + 48], [47, 20, 0])]))
+    def run(always):
+        s = Steps(model, cfg, dtype, 64, always)
+        s.eng = Engine(model, max_tokens=512)
+        slot, out = s.eng.open(), []
+        for a in range(0, 192, chunk):
+            out.append(s([(slot, tokens[a:a + chunk], [chunk - 1, 20, 0])]))
         for t in tokens[192:]:
-            out.append(eng.step([(s, [t], [0])]))
+            out.append(s([(slot, [t], [0])]))
+        s.done([slot])
         return torch.cat(out)
 
-    got = run()
-    POLICY["small"] = False
-    try:
-        want = run()
-    finally:
-        POLICY["small"] = True
-    close(got, want, dtype, "several pages")
+    with policy(small_always=True):
+        got = run(True)
+    with policy(small=False):
+        want = run(False)
+    assert torch.equal(got, want)
+
+
+def test_the_estimate_picks_the_faster_way():
+    """Both sides of the rule's line, and a model that the kernel takes but that never pays."""
+    model = Model.random(helpers.TINY_A, seed=3, dtype="bfloat16", device=DEV)
+    for rows, small in ((1, 1), (64, 0)):
+        eng = Engine(model, max_tokens=256)
+        s = eng.open()
+        eng.step([(s, [1] * rows, [0])])
+        assert eng.n_small_steps == small
+    wide = Model.random(shape(256, 512, 4, 2, 64, 4), seed=3, dtype="float32", device=DEV)
+    eng = Engine(wide, max_tokens=256)
+    eng.step([(eng.open(), [1], [0])])
+    assert eng.n_small_steps == 0

@@ -733,6 +733,7 @@ const char* tqe_engine_describe(const tqe_engine_t* engine) {
         j.set("max_tokens", (long long)e->e->max_tokens);
         j.set("use_graphs", e->e->use_graphs);
         j.set("n_graphs", e->e->n_graphs());
+        j.set("n_small_steps", e->e->n_small_steps());
         j.set("vocab_size", (long long)e->model->spec.vocab_size);
         j.set("max_positions", (long long)e->model->spec.max_positions);
         e->text = j.dump();

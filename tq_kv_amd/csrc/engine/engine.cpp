@@ -88,12 +88,14 @@ const float* Engine::step(int n_seqs, const int32_t* slots, const int32_t* n_new
     long long n_tokens = 0;
     for (int i = 0; i < n_seqs; ++i) n_tokens += n_new[i];
     TqkSmallStep small;
+    // (the bits are the same either way; a trace shows the parts' ranges, which the one launch does not have)
     if (n_tokens <= Model::SMALL_ROWS && model->has_small_steps() && !trace_enabled() &&
-        (ctx.plan(cache->book, n_seqs, slots, starts.data(), n_new, tokens, want_counts, want_idx, 1), model->small_step(ctx, *cache, small))) {
+        (ctx.plan(cache->book, n_seqs, slots, starts.data(), n_new, tokens, want_counts, want_idx, 1), model->small_step(ctx, *cache, use_graphs && all_one ? GRAPH_WIDTH_STEP : 1, small))) {
         ws_.reset(stream);
         ctx.ws = &ws_;
         logits = (const float*)model->forward_small(ctx, small, device_tokens, logits_out).data;
         last_n_want_ = ctx.n_want;
+        ++n_small_steps_;
         if (use_graphs && all_one && single_.size() < (size_t)MAX_GRAPHS) single_.insert(ctx.shape());
     } else if (use_graphs && all_one && n_seqs <= mid_max_rows()) {
         logits = graphed_step(ctx, n_seqs, slots, starts.data(), n_new, tokens, want_counts, want_idx, device_tokens, logits_out, stream);

@@ -42,6 +42,7 @@ public:
                       const int32_t* want_idx, const int32_t* device_tokens, float* logits_out, hipStream_t stream);
     // shapes of one-token steps that are ready to be replayed: captured as graphs, or one launch as they are
     int n_graphs() const { return (int)(graphs_.size() + single_.size()); }
+    long long n_small_steps() const { return n_small_steps_; }          // steps that were one launch (small_step.hip)
     int last_n_want() const { return last_n_want_; }
 
     static const int GRAPH_WIDTH_STEP = 8;      // page-table widths of graphed steps grow in steps of 8 pages
@@ -64,6 +65,7 @@ private:
     Staging staging_;
     std::list<Graph> graphs_;            // least recently used first
     std::set<StepShape> single_;         // shapes of one-token steps that were one launch (MAX_GRAPHS of them at most)
+    long long n_small_steps_ = 0;
     hipStream_t capture_stream_ = nullptr;
     int last_n_want_ = 0;
 };

@@ -29,6 +29,7 @@ int* policy_field(const std::string& name) {
     if (name == "decode_mfma") return &p.decode_mfma;
     if (name == "prefill_mfma") return &p.prefill_mfma;
     if (name == "small") return &p.small;
+    if (name == "small_always") return &p.small_always;
     return nullptr;
 }
 

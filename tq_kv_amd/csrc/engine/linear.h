@@ -31,7 +31,7 @@ namespace tq {
 // prompts takes the packed copy itself.
 struct Policy {
     int skinny = 1, library = 1, fused = 1, prune_last = 1, packed = 1, mid = 1, keep_rows = 1, prompt = 1;
-    int decode_mfma = 1, prefill_mfma = 1, small = 1;
+    int decode_mfma = 1, prefill_mfma = 1, small = 1, small_always = 0;
     // whether a small model's steps may go through the one kernel for all of it: not while a routine is switched off that a test wants to see used or left out
     bool small_steps() const { return small && skinny && library && fused && prune_last && packed && mid && prompt && decode_mfma && prefill_mfma; }
 };

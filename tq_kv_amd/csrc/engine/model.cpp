@@ -107,7 +107,7 @@ void Model::find_small() {
     small_.reset();
     const ModelSpec& s = spec;
     if (!on_gpu || stream_position_ || s.has_embedding_scale || s.has_logit_scale || s.has_logit_cap || head_bias_) return;
-    if (embedding_->t.dtype != dtype || !head_.rows || head_.dtype != dtype || s.order.size() > TQK_SMALL_LAYERS || s.hidden_size > INT32_MAX || s.vocab_size > INT32_MAX) return;
+    if (embedding_->t.dtype != dtype || !head_.rows || head_.dtype != dtype || (dtype == BF16 && !head_.packed) || s.order.size() > TQK_SMALL_LAYERS || s.hidden_size > INT32_MAX || s.vocab_size > INT32_MAX) return;
     const Tensor* norm = final_norm_->plain_rms_weight();
     if (!norm || norm->dtype != dtype) return;
     std::unique_ptr<TqkSmallStep> m(new TqkSmallStep());
@@ -123,15 +123,20 @@ void Model::find_small() {
         const Run& run = s.order[(size_t)i];
         if (run.add_embedding || run.cache_of >= 0 || !blocks_[(size_t)run.layer]->small_layer(*m, m->layers[i])) return;
     }
-    m->n_rows = m->n_want = 1;
-    if (K::small_step_takes.raw(m.get()) && (K::small_step_pays.raw(m.get(), 0, 1) || K::small_step_pays.raw(m.get(), 1, 1))) small_ = std::move(m);
+    m->n_rows = m->n_want = m->n_seqs = m->max_end = 1;
+    m->n_last = -1;
+    if (K::small_step_takes.raw(m.get())) small_ = std::move(m);
 }
 
-bool Model::small_step(const StepContext& c, const CacheStore& cache, TqkSmallStep& step) const {
+bool Model::small_step(const StepContext& c, const CacheStore& cache, int graph_width, TqkSmallStep& step) const {
     if (!small_ || !policy().small_steps() || c.n_tokens > SMALL_ROWS || c.n_want > c.n_tokens) return false;
     step = *small_;
     step.n_rows = c.n_tokens;
     step.n_want = c.n_want;
+    step.n_seqs = c.n_seqs;
+    step.decode = c.all_decode ? 1 : 0;
+    step.max_end = c.max_end;
+    step.n_last = c.prune_last ? c.n_last : -1;
     int n = 0;
     auto put = [&](const int32_t* from, int count) {
         const int at = n;
@@ -144,6 +149,8 @@ bool Model::small_step(const StepContext& c, const CacheStore& cache, TqkSmallSt
     step.tok_seq = n <= TQK_SMALL_INTS ? put(c.host.tok_seq, c.n_tokens) : 0;
     step.tok_pos = n <= TQK_SMALL_INTS ? put(c.host.tok_pos, c.n_tokens) : 0;
     step.want = n <= TQK_SMALL_INTS ? put(c.host.want_rows, c.n_want) : 0;
+    step.seq_first = n <= TQK_SMALL_INTS ? put(c.host.cu, c.n_seqs + 1) : 0;
+    step.last_rows = c.prune_last && n <= TQK_SMALL_INTS ? put(c.host.last_rows, c.n_last) : 0;
     std::vector<int> tables;
     for (const StepContext::Table& t : c.tables) tables.push_back(n <= TQK_SMALL_INTS ? put(t.host, c.n_seqs * t.width) : 0);
     if (n > TQK_SMALL_INTS) return false;
@@ -155,8 +162,11 @@ bool Model::small_step(const StepContext& c, const CacheStore& cache, TqkSmallSt
         step.layers[i].values = e.values.data;
         step.layers[i].table = tables.at((size_t)e.group);
         step.layers[i].width = c.tables[(size_t)e.group].width;
+        const bool last = i + 1 == step.n_layers && c.prune_last;
+        const int width = (step.layers[i].width + graph_width - 1) / graph_width * graph_width;
+        step.layers[i].divided = blocks_[(size_t)spec.order[(size_t)i].layer]->row_partitions(last ? c.n_last : c.n_tokens, width) > 1;
     }
-    return K::small_step_takes.raw(&step) != 0 && K::small_step_pays.raw(&step, c.all_decode ? 1 : 0, c.max_end) != 0;
+    return K::small_step_takes.raw(&step) != 0 && (policy().small_always || K::small_step_pays.raw(&step, c.all_decode ? 1 : 0, c.max_end) != 0);
 }
 
 Tensor Model::forward_small(StepContext& c, TqkSmallStep& step, const int32_t* device_tokens, float* out) {

@@ -35,7 +35,8 @@ public:
     Tensor forward(StepContext& c, const CacheStore& cache, float* out = nullptr);
     // The step in one launch, for small models (small_step.hip): whether that is the way for the planned step, and the step itself.  Nothing
     // of the plan is uploaded: the step's arrays travel with the launch.  device_tokens: as Engine::step.
-    bool small_step(const StepContext& c, const CacheStore& cache, TqkSmallStep& step) const;
+    // graph_width: the step's tables would be filled up to a multiple of so many pages in a captured graph (1: it would not be captured).
+    bool small_step(const StepContext& c, const CacheStore& cache, int graph_width, TqkSmallStep& step) const;
     Tensor forward_small(StepContext& c, TqkSmallStep& step, const int32_t* device_tokens, float* out);
     bool has_small_steps() const { return small_ != nullptr; }
     static const int SMALL_ROWS = 64;           // (more rows are not asked about)
@@ -52,7 +53,7 @@ private:
     int stream_state_entry_ = -1;               // the cache entry of the stream position's state, if it keeps one
     OwnedPtr embedding_, head_bias_;
     Weight head_;
-    std::unique_ptr<TqkSmallStep> small_;       // the model as that kernel takes it, if it does
+    std::unique_ptr<TqkSmallStep> small_;       // the model as that kernel takes it, if it takes any step of it
     void find_small();
     Tensor head_logits(StepContext& c, Stream& stream, float* out);
 };

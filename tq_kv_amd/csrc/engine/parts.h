@@ -226,6 +226,8 @@ public:
     // Optional: the part as the kernel that runs a small model's whole step takes it.  model: sizes, types and angle tables, filled in by the first
     // part and the same for all; layer: what is this one's own.  False: not such a part.
     virtual bool small_layer(TqkSmallStep& model, TqkSmallLayer& layer) const { (void)model; (void)layer; return false; }
+    // into how many partitions its kernel for single rows deals a row's pages
+    virtual int row_partitions(int rows, int width) const { (void)rows; (void)width; return 1; }
 };
 
 class FeedForward : public Part {
@@ -248,6 +250,7 @@ public:
     virtual CacheNeed cache_need() const = 0;
     virtual Norm* first_norm() = 0;
     virtual Mixer* mixer() { return nullptr; }
+    virtual int row_partitions(int rows, int width) const { (void)rows; (void)width; return 1; }                                // (as a mixer's)
     virtual bool small_layer(TqkSmallStep& model, TqkSmallLayer& layer) const { (void)model; (void)layer; return false; }      // (as a mixer's)
     // next_norm: the norm that reads the stream after this block.  last: nothing but the head
     // reads the stream after it.  Returns the stream to go on with.

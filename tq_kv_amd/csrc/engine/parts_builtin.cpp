@@ -95,8 +95,8 @@ static OwnedPtr as_floats(const OwnedPtr& p, hipStream_t stream) {
     return out;
 }
 
-// whether a product's weight is rows of the run's own type
-static bool small_weight(const Weight& w, int dtype) { return w.rows && w.dtype == dtype; }
+// whether a product's weight is rows of the run's own type (in bfloat16 beside the packed copy, which the kernels whose order of sums the step keeps take)
+static bool small_weight(const Weight& w, int dtype) { return w.rows && w.dtype == dtype && (dtype != BF16 || w.packed); }
 
 // ---- RMSNorm -----------------------------------------------------------------------------------
 // As the reference computes it (src/models/turbo_generic.rs:41-51): x / sqrt(mean(x^2) + eps) *
@@ -574,6 +574,7 @@ public:
         l.window = window_;
         return true;
     }
+    int row_partitions(int rows, int width) const override { return decode_parts(rows, width); }
 
 private:
     // product, then biases, the heads' norm, rotation, value mixing and cache write in one kernel
@@ -1047,6 +1048,7 @@ public:
     CacheNeed cache_need() const override { return mixer_->cache_need(); }
     Norm* first_norm() override { return mixer_norm_.get(); }
     Mixer* mixer() override { return mixer_.get(); }
+    int row_partitions(int rows, int width) const override { return mixer_->row_partitions(rows, width); }
     bool small_layer(TqkSmallStep& m, TqkSmallLayer& l) const override {
         if (!feed_forward_ || post_mixer_norm_ || post_ff_norm_) return false;
         const Tensor *first = mixer_norm_->plain_rms_weight(), *second = ff_norm_->plain_rms_weight();

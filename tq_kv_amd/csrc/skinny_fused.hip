@@ -429,6 +429,11 @@ static int pick_waves(int blocks, int K, int tiles) {
     return waves;
 }
 
+extern "C" int tqk_fused_waves(int N, int K, int paired) {
+    const int rt = paired ? 1 : pick_tiles(N, K), n_out = paired ? N / 2 : N;
+    return pick_waves((n_out + 16 * rt - 1) / (16 * rt), K, paired ? 2 : rt);
+}
+
 template <bool NORM, int EPI, typename TY, bool GATHER = false, int RT = 1>
 static int launch_fused(const FusedArgs& a, int blocks, hipStream_t s) {
     const int tiles = (EPI == EPI_GATED || EPI == EPI_QKV) ? 2 : RT;

@@ -13,9 +13,11 @@
 // weights come straight from memory, those of its first tile before the barrier in front of the product, so that they travel while the work
 // before it is finished.
 //
-// Every sum has the order that the kernels of larger models give it (gemm_generic.hip, elementwise.hip, attention_walk.h), and every rounding its
-// place, so in float32 a position's result has the same bits whichever way its step went.  In bfloat16 the products' sums go by
-// increasing k and the probabilities stay in float32.
+// Every sum has the order that the kernels of larger models give it, and every rounding its place, so a position's result has the same bits whichever way
+// its step went.  In float32 that is gemm_generic.hip, elementwise.hip and attention_walk.h.  In bfloat16 the order goes by the kind of step
+// (SmallPlan): norms that are divided by behind their product in decoding steps of up to 16 rows (skinny_fused.hip), and the matrix cores' attention of
+// attention_decode.hip and attention_prefill.hip for heads of 32 and 64.  Steps with more than a page of positions for such heads, and products whose K
+// those kernels deal out to waves or cut into pieces, are left to them.
 //
 // (Eight or twelve waves in place of 16: more rows take 1.1 to 1.4 times as long.  The o product's first weights asked for before the attention: 3 us a step more, the
 // registers spill.  All heads of a kv head, or two queries, side by side in a wave's attention, so that keys are read once or chains overlap: slower,
@@ -27,7 +29,6 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
-static_assert(sizeof(TqkSmallStep) <= 4000, "a kernel's arguments");
 
 #define SS_WAVES 16
 #define SS_THREADS (SS_WAVES * TQK_WAVE)
@@ -58,6 +59,14 @@ template <typename T> __device__ __forceinline__ floatx4_t rounded(floatx4_t v) 
 // A barrier for what lies in LDS: loads from memory may stay under way across it (__syncthreads waits for them, and a product's first
 // weights are asked for in front of one).
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// What of a bfloat16 step's arithmetic goes by the kernels that it would run through otherwise.
+struct SmallPlan {
+    int behind, first_behind;               // norms are divided by behind their product: those in front of gate and up and of the head; those in front of q, k and v
+    int attention, last_attention;          // (last: the last layer's, where it runs for the last rows alone)
+};
+static_assert(sizeof(TqkSmallStep) + sizeof(SmallPlan) <= 4096, "a kernel's arguments");
+enum { SMALL_ROWS = 1, SMALL_TILES = 2 };          // attention_decode.hip, attention_prefill.hip (heads that they do not take: attention_walk.h)
 
 // y[rows, N] = x[rows, K] w[N, K]^T of rows in LDS, for P weights at once (gate and up rows of the same features).  A wave takes tiles of 16
 // features by 16 rows, the rows' tiles of some features one after the other.  `ask` loads the first steps of the wave's first tile; emit(row, first feature,
@@ -112,7 +121,7 @@ struct SmallProduct {
 // How a step's rows lie in LDS, in bytes: the step's arrays, the layers' arguments, the norms' weights and the biases of all layers, the rows' angles, the waves' probabilities, then
 // the stream and the two buffers.  Rows begin 16 bytes past a multiple of the banks' width, so that the 16 rows of an operand meet different ones.
 struct SmallLayout {
-    int ld_h, ld_a, ld_b, layers, norms, biases, angles, probs, a, b, h, bytes;       // ld_h in floats, ld_a in T, ld_b in bytes
+    int ld_h, ld_a, ld_b, layers, norms, biases, angles, probs, squares, a, b, h, bytes;       // ld_h in floats, ld_a in T, ld_b in bytes
 };
 static __device__ __host__ inline SmallLayout small_layout(const TqkSmallStep& p) {
     const int size = p.act_dtype == TQK_F32 ? 4 : 2, q = p.n_heads * p.head_dim, all = (p.n_heads + 2 * p.n_kv_heads) * p.head_dim;
@@ -127,7 +136,8 @@ static __device__ __host__ inline SmallLayout small_layout(const TqkSmallStep& p
     l.biases = l.norms + up((2 * p.n_layers + 1) * p.hidden * size);
     l.angles = l.biases + up(p.n_layers * all * size);
     l.probs = l.angles + up(p.n_rows * p.head_dim * 4);
-    l.h = l.probs + SS_WAVES * SS_QUERIES * TQK_PAGE * 4;
+    l.squares = l.probs + SS_WAVES * SS_QUERIES * TQK_PAGE * 4;             // (one root mean square of a row, then the squares' sums of 16 columns each, up to 16 rows)
+    l.h = l.squares + (size == 2 && p.decode && p.n_rows <= 16 ? 64 + p.hidden * 4 : 0);
     l.a = l.h + rows * l.ld_h * 4;
     l.b = l.a + up(rows * l.ld_a * size);
     l.bytes = l.b + rows * l.ld_b;
@@ -207,6 +217,184 @@ __device__ __forceinline__ float small_values(const T* base, const float* weight
     return sum;
 }
 
+// eight values in bfloat16 already, as an operand of the matrix cores
+__device__ __forceinline__ bf16x8_t operand8(const float* p) {
+    u32x4_t v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float2 two = *reinterpret_cast<const float2*>(p + 2 * i);
+        v[i] = __float_as_uint(two.x) >> 16 | (__float_as_uint(two.y) & 0xffff0000u);
+    }
+    return __builtin_bit_cast(bf16x8_t, v);
+}
+
+// The heads of a kv head (no more than 16) for one row whose keys lie in one page, as attention_decode.hip takes them: q its heads' values, positions lo .. pos of the page.
+// divided: what that kernel's partitions leave is divided by their sum, and not multiplied by its inverse.
+template <int D>
+__device__ __forceinline__ void attend_row(const float* q, int n_live, const bf16_t* keys, const bf16_t* values, int lo, int pos, float scale, bool divided,
+                                           bf16_t* out, int lane) {
+    constexpr int KB = D / 32, DB = D / 16;
+    const int col = lane % 16, g = lane / 16;
+    const bool live = col < n_live;
+    const float scale2 = scale * 1.4426950408889634f;
+    bf16x8_t bq[KB];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+        const bf16x8_t none = {0, 0, 0, 0, 0, 0, 0, 0};
+        bq[kb] = live ? operand8(q + col * D + kb * 32 + g * 8) : none;
+    }
+    floatx4_t s[4];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        s[t] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+            s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8_t*>(keys + (t * 16 + col) * D + kb * 32 + g * 8), bq[kb], s[t], 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int j = t * 16 + g * 4 + r;
+            s[t][r] = j >= lo && j <= pos ? s[t][r] * scale2 : -INFINITY;
+            mx = fmaxf(mx, s[t][r]);
+        }
+    }
+    float2 both = with_lane_16(mx);
+    mx = fmaxf(both.x, both.y);
+    both = with_lane_32(mx);
+    mx = fmaxf(both.x, both.y);
+    float l = 0.f;
+    u32x4_t pb[2];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; r += 2) {
+            const uint32_t a = float_to_bf16_bits(__builtin_amdgcn_exp2f(s[t][r] - mx)), b = float_to_bf16_bits(__builtin_amdgcn_exp2f(s[t][r + 1] - mx));
+            l += __uint_as_float(a << 16);
+            l += __uint_as_float(b << 16);
+            pb[t / 2][(t % 2) * 2 + r / 2] = a | b << 16;
+        }
+    both = with_lane_16(l);
+    l = both.x + both.y;
+    both = with_lane_32(l);
+    l = both.x + both.y;
+    uint32_t keep[2][4];                    // (whatever lies at places without a key must not count, not even with probability 0)
+#pragma unroll
+    for (int pr = 0; pr < 2; ++pr)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int j = (2 * pr + i / 2) * 16 + g * 4 + 2 * (i % 2);
+            keep[pr][i] = (j >= lo && j <= pos ? 0xffffu : 0u) | (j + 1 >= lo && j + 1 <= pos ? 0xffff0000u : 0u);
+        }
+    const float inv = 1.f / l;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+        floatx4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int pr = 0; pr < 2; ++pr) {
+            u32x4_t v = *reinterpret_cast<const u32x4_t*>(values + (db * 16 + col) * TQK_PAGE + pr * 32 + g * 8);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] &= keep[pr][i];
+            o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, v), __builtin_bit_cast(bf16x8_t, pb[pr]), o, 0, 0, 0);
+        }
+        if (!live) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = divided ? (0.f + o[r]) / l : o[r] * inv;
+        put4(out + col * D + db * 16 + g * 4, o);
+    }
+}
+
+// 32 columns (a query and a head each) of one sequence and kv head whose keys lie in one page, as attention_prefill.hip takes them: q and out the lane's query and head;
+// positions lo .. pos of the page (none: pos < 0), the sequence's end after the step, and how far any of the columns sees.
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16_t;
+template <int D>
+__device__ __forceinline__ void attend_columns(const float* q, const bf16_t* keys, const bf16_t* values, int lo, int pos, int end, int furthest, float scale, bf16_t* out, int lane) {
+    constexpr int KS = D / 16, DT = D / 32;
+    const int c32 = lane % 32, h = lane / 32;
+    const bool live = pos >= 0;
+    const float c2 = scale * 1.44269504088896340736f;
+    bf16x8_t bq[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        const bf16x8_t none = {0, 0, 0, 0, 0, 0, 0, 0};
+        bq[ks] = live ? operand8(q + ks * 16 + h * 8) : none;
+    }
+    float m = 0.f, pass = -INFINITY, l = 0.f;
+    floatx16_t o[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
+    const int key = 4 * (2 * (c32 >> 4) + (c32 >> 2 & 1)) + 16 * (c32 >> 3 & 1) + (c32 & 3);      // that row c32 of a tile holds
+#pragma unroll 1
+    for (int t = 0; t < 2; ++t) {
+        if (32 * t > furthest) break;
+        floatx16_t s;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8_t*>(keys + (32 * t + key) * D + ks * 16 + h * 8), bq[ks], s, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int a = i >> 2, j = 32 * t + 4 * (2 * (a >> 1) + h) + 16 * (a & 1) + (i & 3);
+            if (j < lo || j > pos) s[i] = -INFINITY;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = fmaf(s[i], c2, -m);
+        float mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
+        const float2 both = with_lane_32(mx);
+        mx = fmaxf(both.x, both.y);
+        const bool raise = mx > pass;
+        if (__any(raise)) {
+            const float up = raise ? mx : 0.f, alpha = __builtin_amdgcn_exp2f(-fmaxf(up, 0.f));
+            m += up;
+            if (raise) pass = 8.f;
+            l *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] -= up;
+        }
+        bf16x8_t pb[2];
+        float psum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const float pr = __builtin_amdgcn_exp2f(s[i]);
+            psum += pr;
+            pb[i >> 3][i & 7] = (__bf16)pr;
+        }
+        l += psum;
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            const int place = (4 * t + 2 * st + h) * 8;
+            uint32_t keep[4];                       // (values beyond the sequence are zeros)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                keep[i] = (value_position(place + 2 * i) < end ? 0xffffu : 0u) | (value_position(place + 2 * i + 1) < end ? 0xffff0000u : 0u);
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                u32x4_t v = *reinterpret_cast<const u32x4_t*>(values + (32 * dt + c32) * TQK_PAGE + place);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] &= keep[i];
+                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, v), pb[st], o[dt], 0, 0, 0);
+            }
+        }
+    }
+    const float2 both = with_lane_32(l);
+    l = both.x + both.y;
+    if (!live) return;
+    const float inv = 1.f / l;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+            put4(out + 32 * dt + 8 * a + 4 * h, floatx4_t{o[dt][4 * a] * inv, o[dt][4 * a + 1] * inv, o[dt][4 * a + 2] * inv, o[dt][4 * a + 3] * inv});
+}
+
 // The weights' way into the second-level cache of the die that runs the step: block 0 alone would wait for memory at every product.  Blocks are dealt to
 // the eight dies in turn, so those whose number is a multiple of 8 read a layer's weights each (where they run elsewhere, nothing is lost but
 // the time saved).
@@ -221,9 +409,10 @@ __device__ __forceinline__ void warm(const T* w, size_t n) {
     }
 }
 
-template <typename T>
+// D: the heads' size where the matrix cores take them (32 or 64), or 0.
+template <typename T, int D>
 __global__ __launch_bounds__(SS_THREADS)
-void small_step_kernel(const TqkSmallStep p) {
+void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int tid = threadIdx.x, lane = tid % TQK_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / TQK_WAVE);
     const int rows = p.n_rows, hidden = p.hidden, d = p.head_dim, half = d / 2, nh = p.n_heads, nkv = p.n_kv_heads, inter = p.inter;
@@ -250,6 +439,11 @@ void small_step_kernel(const TqkSmallStep p) {
     char* b = lds + at.b;
     auto round = [](float v) { return to_float(from_float<T>(v)); };
 
+    // (bfloat16, norms divided by behind their product: the rows' inverse root mean squares and the sums of the squares of 16 columns each, [columns / 16][row])
+    constexpr bool BF16 = sizeof(T) == 2;
+    const bool behind = BF16 && plan.behind;
+    float *inverse = reinterpret_cast<float*>(lds + at.squares), *square_sums = inverse + 16;
+
     auto product = [&](const void* w, int n, int k, int tiles) {
         SmallProduct<T, 1> one = {{(const char*)w}, n, k * (int)sizeof(T), tiles, lane, wave};
         one.ask();
@@ -274,6 +468,18 @@ void small_step_kernel(const TqkSmallStep p) {
         const bool ok = id >= 0 && id < p.vocab;
         const T* row = (const T*)p.embedding + (size_t)(ok ? id : 0) * hidden;
         for (int i = lane; i < hidden; i += TQK_WAVE) h[r * at.ld_h + i] = ok ? to_float(row[i]) : 0.f;
+        if (BF16 && plan.first_behind) {                // the first norm's squares: eight neighbouring values a lane
+            float sum = 0.f;
+            for (int i0 = 0; i0 < hidden / 8; i0 += TQK_WAVE) {
+                const int i = i0 + lane;
+                float ss = 0.f;
+                if (i < hidden / 8 && ok)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) { const float v = to_float(row[8 * i + j]); ss = fmaf(v, v, ss); }
+                sum += wave_sum(ss);
+            }
+            if (lane == 0) square_sums[r] = sum;
+        }
         for (int i = lane; i < d; i += TQK_WAVE) angles[r * d + i] = i < half ? p.cos_table[(size_t)pos * half + i] : p.sin_table[(size_t)pos * half + i - half];
     }
     lds_barrier();
@@ -300,9 +506,39 @@ void small_step_kernel(const TqkSmallStep p) {
             put4(a + to * at.ld_a + i, floatx4_t{(v[j][0] / rms) * w.x, (v[j][1] / rms) * w.y, (v[j][2] / rms) * w.z, (v[j][3] / rms) * w.w});
         }
     };
+    // A norm that is divided by behind its product: row `from` of the stream times the weight into row `to` of a, and the inverse of its root mean square.
+    // The sums of squares (of `sums` times 16 columns) are added as the product's kernel adds them.
+    auto norm_behind = [&](int from, int to, const T* weight, float eps, int sums) {
+        for (int i = lane * 4; i < hidden; i += 4 * TQK_WAVE) {
+            const floatx4_t v = *reinterpret_cast<const floatx4_t*>(h + from * at.ld_h + i);
+            const float4 w = load4(weight + i);
+            put4(a + to * at.ld_a + i, floatx4_t{v[0] * w.x, v[1] * w.y, v[2] * w.z, v[3] * w.w});
+        }
+        float ss = lane / 4 < sums ? square_sums[lane / 4 * 16 + from] : 0.f;
+        for (int s = 16 + lane / 4; s < sums; s += 16) ss += square_sums[s * 16 + from];
+        ss += lane_xor_4(ss);
+        ss += lane_xor_8(ss);
+        float2 both = with_lane_16(ss);
+        ss = both.x + both.y;
+        both = with_lane_32(ss);
+        ss = both.x + both.y;
+        if (lane == 0) inverse[to] = 1.f / sqrtf(ss / (float)hidden + eps);
+    };
+    auto divided = [&](floatx4_t v, int row, bool by) {
+        if (!BF16 || !by) return v;
+        const float f = inverse[row];
+        return floatx4_t{v[0] * f, v[1] * f, v[2] * f, v[3] * f};
+    };
     auto add_to_stream = [&](int row, int n, const floatx4_t* v) {
         floatx4_t* to = reinterpret_cast<floatx4_t*>(h + row * at.ld_h + n);
-        *to = *to + rounded<T>(v[0]);
+        const floatx4_t sum = *to + rounded<T>(v[0]);
+        *to = sum;
+        if (behind) {
+            // the squares of the tile's 16 columns: the four lanes of the row, in lane order
+            const float sq = fmaf(sum[3], sum[3], fmaf(sum[2], sum[2], fmaf(sum[1], sum[1], sum[0] * sum[0])));
+            const float s1 = with_lane_16(sq).y, s2 = with_lane_32(sq).y, s3 = with_lane_32(s1).y;
+            if (lane < 16) square_sums[n + row] = ((sq + s1) + s2) + s3;
+        }
     };
     // queries a wave takes together: their elements side by side in its lanes
     const int width = d <= 16 ? 16 : d <= 32 ? 32 : 64, n_queries = rows * nh;
@@ -317,12 +553,16 @@ void small_step_kernel(const TqkSmallStep p) {
         for (int i = 0; i < (int)(sizeof(l) / 4); ++i)
             reinterpret_cast<int32_t*>(&l)[i] = __builtin_amdgcn_readfirstlane(reinterpret_cast<const int32_t*>(layers + layer)[i]);
         const int32_t* table = ints + l.table;
+        const bool last = layer == p.n_layers - 1 && p.n_last >= 0;         // (what follows the cache's rows counts for the last rows alone)
         SmallProduct<T, 1> w_qkv = product(l.qkv, qkv, hidden, row_tiles);
-        for (int r = wave; r < rows; r += SS_WAVES) norm_row(r, r, norms + 2 * layer * hidden, l.eps1);
+        for (int r = wave; r < rows; r += SS_WAVES) {
+            if (BF16 && plan.first_behind) norm_behind(r, r, norms + 2 * layer * hidden, l.eps1, layer == 0 ? 1 : hidden / 16);
+            else norm_row(r, r, norms + 2 * layer * hidden, l.eps1);
+        }
         lds_barrier();
         float* bf = reinterpret_cast<float*>(b);
         const int ld_b = at.ld_b / 4;
-        w_qkv.run(a, at.ld_a, rows, [&](int row, int n, const floatx4_t* v) { put4(bf + row * ld_b + n, rounded<T>(v[0])); });
+        w_qkv.run(a, at.ld_a, rows, [&](int row, int n, const floatx4_t* v) { put4(bf + row * ld_b + n, rounded<T>(divided(v[0], row, plan.first_behind))); });
         lds_barrier();
         // biases, rotation of q and k, keys and values into the row's page: a wave a row's heads in turn, a lane a pair that rotates together
         const int per = half <= 16 ? 4 : half <= 32 ? 2 : 1, sub = TQK_WAVE / per;      // heads a wave takes at once
@@ -339,8 +579,11 @@ void small_step_kernel(const TqkSmallStep p) {
             }
             if (head < nh + nkv && pos < p.max_positions) {
                 const float co = angles[r * d + i], si = angles[r * d + i + half], x0 = lo, x1 = hi;
-                lo = fmaf(x0, co, -(x1 * si));
-                hi = fmaf(x1, co, x0 * si);
+                if (BF16) rotate_pair(lo, hi, co, si);
+                else {                                      // (which product is rounded is the kernels' of the type)
+                    lo = fmaf(x0, co, -(x1 * si));
+                    hi = fmaf(x1, co, x0 * si);
+                }
             }
             if (head < nh) {
                 src[i] = round(lo);
@@ -357,6 +600,44 @@ void small_step_kernel(const TqkSmallStep p) {
             dst[(size_t)(i + half) * stride] = from_float<T>(hi);
         }
         __syncthreads();                                    // (keys and values are read back out of memory)
+        if constexpr (D > 0) {
+            const int group = nh / nkv;
+            const size_t page_size = (size_t)TQK_PAGE * D;
+            if ((last ? plan.last_attention : plan.attention) == SMALL_ROWS) {
+                const int n = last ? p.n_last : rows;
+#pragma unroll 1
+                for (int e = wave; e < n * nkv; e += SS_WAVES) {
+                    const int kvh = __builtin_amdgcn_readfirstlane(e / n), which = __builtin_amdgcn_readfirstlane(e - kvh * n), head0 = kvh * group;
+                    const int r = __builtin_amdgcn_readfirstlane(last ? ints[p.last_rows + which] : which), pos = __builtin_amdgcn_readfirstlane(tok_pos[r]);
+                    const int page = __builtin_amdgcn_readfirstlane(table[tok_seq[r] * l.width]);
+                    if (page < 0) continue;                 // the host never lets this happen
+                    const size_t base = ((size_t)page * nkv + kvh) * page_size;
+                    const int lo = l.window > 0 ? max(0, pos - l.window + 1) : 0;
+                    attend_row<D>(bf + r * ld_b + head0 * D, group, (const bf16_t*)l.keys + base, (const bf16_t*)l.values + base, lo, pos, l.scale, l.divided != 0,
+                                  a + r * at.ld_a + head0 * D, lane);
+                }
+            } else {
+                int before = 0;                             // units of the sequences before
+#pragma unroll 1
+                for (int seq = 0; seq < p.n_seqs; ++seq) {
+                    const int r0 = __builtin_amdgcn_readfirstlane(ints[p.seq_first + seq]), n = __builtin_amdgcn_readfirstlane(ints[p.seq_first + seq + 1]) - r0;
+                    const int tiles = (n * group + 31) / 32, units = tiles * nkv;
+                    const int page = __builtin_amdgcn_readfirstlane(table[seq * l.width]), end = __builtin_amdgcn_readfirstlane(tok_pos[r0]) + n;
+#pragma unroll 1
+                    for (int e = (wave - before) & (SS_WAVES - 1); e < units; e += SS_WAVES) {
+                        if (page < 0) continue;             // the host never lets this happen
+                        const int kvh = __builtin_amdgcn_readfirstlane(e % nkv), col = e / nkv * 32 + lane % 32;
+                        const bool live = col < n * group;
+                        const int of_group_ = live ? col / n : 0, r = r0 + (live ? col - of_group_ * n : 0), head = kvh * group + of_group_;
+                        const int pos = live ? tok_pos[r] : -1, lo = l.window > 0 ? max(0, pos - l.window + 1) : 0;
+                        const size_t base = ((size_t)page * nkv + kvh) * page_size;
+                        attend_columns<D>(bf + r * ld_b + head * D, (const bf16_t*)l.keys + base, (const bf16_t*)l.values + base, lo, pos, end, end - 1, l.scale,
+                                          a + r * at.ld_a + head * D, lane);
+                    }
+                    before += units;
+                }
+            }
+        } else
 #pragma unroll 1
         for (int e0 = wave * together; e0 < n_queries; e0 += SS_WAVES * together) {
             SmallQuery mine;                                // the query whose elements this lane's are
@@ -417,12 +698,15 @@ void small_step_kernel(const TqkSmallStep p) {
         w_o.run(a, at.ld_a, rows, add_to_stream);
         w_gate_up.ask();
         lds_barrier();
-        for (int r = wave; r < rows; r += SS_WAVES) norm_row(r, r, norms + (2 * layer + 1) * hidden, l.eps2);
+        for (int r = wave; r < rows; r += SS_WAVES) {
+            if (behind) norm_behind(r, r, norms + (2 * layer + 1) * hidden, l.eps2, hidden / 16);
+            else norm_row(r, r, norms + (2 * layer + 1) * hidden, l.eps2);
+        }
         lds_barrier();
         T* act = reinterpret_cast<T*>(b);
         const int ld_act = at.ld_b / (int)sizeof(T);
         w_gate_up.run(a, at.ld_a, rows, [&](int row, int n, const floatx4_t* v) {
-            const floatx4_t g = rounded<T>(v[0]), u = rounded<T>(v[1]);
+            const floatx4_t g = rounded<T>(divided(v[0], row, behind)), u = rounded<T>(divided(v[1], row, behind));
             floatx4_t y;
 #pragma unroll
             for (int i = 0; i < 4; ++i) y[i] = gate_value(TQK_GATE_SILU, 0.f, 1.f, g[i], u[i]);
@@ -437,13 +721,29 @@ void small_step_kernel(const TqkSmallStep p) {
     if (p.n_want == 0) return;
     SmallProduct<T, 1> w_head = product(p.head, p.vocab, hidden, (p.n_want + 15) / 16);
     const int32_t* want = ints + p.want;
-    for (int r = wave; r < p.n_want; r += SS_WAVES) norm_row(want[r], r, norms + 2 * p.n_layers * hidden, p.final_eps);
+    for (int r = wave; r < p.n_want; r += SS_WAVES) {
+        if (behind) norm_behind(want[r], r, norms + 2 * p.n_layers * hidden, p.final_eps, hidden / 16);
+        else norm_row(want[r], r, norms + 2 * p.n_layers * hidden, p.final_eps);
+    }
     lds_barrier();
     w_head.run(a, at.ld_a, p.n_want, [&](int row, int n, const floatx4_t* v) {
+        const floatx4_t y = divided(v[0], row, behind);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            if (n + i < p.vocab) p.logits[(size_t)row * p.vocab + n + i] = v[0][i];
+            if (n + i < p.vocab) p.logits[(size_t)row * p.vocab + n + i] = y[i];
     });
+}
+
+// Whether the kernels that a bfloat16 step would run through add up its products by increasing k, as this one does.
+static bool in_order(const TqkSmallStep& p, int n_rows, int last, int n_want, bool decode) {
+    const int few = tqk_skinny_max_rows(), q = p.n_heads * p.head_dim, all = q + 2 * p.n_kv_heads * p.head_dim;
+    auto whole = [&](int rows, int n, int k, bool pairs, bool gated) { return (rows <= few ? tqk_fused_waves(n, k, pairs) : tqk_mid_splits(n, k, gated)) == 1; };
+    auto rest = [&](int rows) { return whole(rows, p.hidden, q, false, false) && whole(rows, 2 * p.inter, p.hidden, true, true) && whole(rows, p.hidden, p.inter, false, false); };
+    return whole(n_rows, all, p.hidden, decode && p.head_dim % 32 == 0, false) && rest(n_rows) && rest(last) && whole(n_want, p.vocab, p.hidden, false, false);
+}
+// Whether the matrix cores' attention of one page does for a bfloat16 step's heads.
+static bool heads_fit(const TqkSmallStep& p, int positions) {
+    return !tqk_attention_decode_supported(p.head_dim) || (positions <= TQK_PAGE && p.n_heads / p.n_kv_heads <= 16);
 }
 
 /* Whether the kernel takes a step: what of `step` describes the model and the step's size is filled in, pointers need not be. */
@@ -459,6 +759,7 @@ extern "C" int tqk_small_step_takes(const TqkSmallStep* step) {
     const int q = p.n_heads * p.head_dim, whole = 64 / size;
     if (p.hidden % whole || p.inter % whole || q % whole || (p.n_kv_heads * p.head_dim * 2) % 16) return 0;
     if (small_layout(p).bytes > 160 * 1024) return 0;
+    if (p.act_dtype == TQK_BF16 && !(heads_fit(p, p.max_end) && in_order(p, p.n_rows, p.n_last >= 0 ? p.n_last : p.n_rows, p.n_want, p.decode != 0))) return 0;
     // (larger products have another order of summation there)
     if (p.act_dtype == TQK_F32 && (tqk_gemm_takes_apart(p.vocab, p.hidden) || tqk_gemm_takes_apart(2 * p.inter, p.hidden) || tqk_gemm_takes_apart(q + 2 * p.n_kv_heads * p.head_dim, p.hidden))) return 0;
     return 1;
@@ -467,9 +768,11 @@ extern "C" int tqk_small_step_takes(const TqkSmallStep* step) {
 /* Whether that is the faster way, by an estimate in microseconds (decode: a step of one token a sequence, which the other kernels run as a replayed graph; positions: the
  * furthest one of the step).  One block: 5 a layer for its barriers and chains of short operations, its weights at 33 KB (27 in float32) a microsecond, and for every row what
  * its products, its other work and its heads' pages take; the head's weights at 39 KB.  The other kernels, ten launches a layer: 20 a layer in a graph (33 in float32) and 32 (45) one by one.
- * Measured, one block and the other kernels, two layers of 64 values with 160 in the feed-forward, bfloat16: 1 and 16 sequences 35 and 72, 63 and 68, 40 sequences 90 and 73, prompts of 8, 33
- * and 64 tokens 31 and 88, 61 and 88, 109 and 90; three of 96 with 224: 37 and 74, 77 and 77, 135 and 97, 40 and 120, 99 and 117, 165 and 118; four of 128 with 512: 88 and 83, 193 and 89, then 94
- * and 138, 263 and 141; four of 256 with 512: 171 and 98, 374 and 102, then 184 and 138.  float32: 36 and 81, 76 and 85, 38 and 91, 90 and 93, 149 and 99; three of 96: 64 and 108, 116 and 113, 71 and 117, 196 and 136. */
+ * Measured, one block and the other kernels, two layers of 64 values with 160 in the feed-forward, bfloat16: 1, 16 and 40 sequences 31 and 72, 65 and 79, 92 and 88, prompts of 8, 33
+ * and 64 tokens 31 and 96, 61 and 96, 109 and 97; three of 96 with 224 and heads of 32: 47 and 73, 75 and 82, 108 and 97, then 35 and 132, 70 and 134, 95 and 135; with heads of 64: 66 and 78, 87
+ * and 83, 156 and 106, then 43 and 132, 87 and 137, 133 and 137; four of 128 with 224: 69 and 83, 94 and 88, 207 and 122, then 55 and 175, 126 and 179, 175 and 179.  float32, two of 64: 35 and 81, 74 and
+ * 85, 125 and 111, then 36 and 100, 88 and 102, 145 and 103; three of 96: 62 and 108, 113 and 113, 249 and 152, then 69 and 132, 192 and 138, 306 and 147; four of 128 with 512: 159 and 146, 313 and 154,
+ * then 171 and 173. */
 extern "C" int tqk_small_step_pays(const TqkSmallStep* step, int decode, int positions) {
     const TqkSmallStep& p = *step;
     const bool f32 = p.act_dtype == TQK_F32;
@@ -481,11 +784,25 @@ extern "C" int tqk_small_step_pays(const TqkSmallStep* step, int decode, int pos
     return here < there;
 }
 
-template <typename T>
+// Which kernels a step in bfloat16 would run through: decoding steps of up to 16 rows with their norms behind the products (heads by 32: the
+// first ones too), and the attention of heads that the matrix cores take, the last layer for the last rows alone.
+static SmallPlan small_plan(const TqkSmallStep& p) {
+    SmallPlan plan = {};
+    if (p.act_dtype != TQK_BF16) return plan;
+    plan.behind = p.decode && p.n_rows <= tqk_skinny_max_rows();
+    plan.first_behind = plan.behind && p.head_dim % 32 == 0;
+    if (tqk_attention_decode_supported(p.head_dim)) {
+        plan.attention = p.decode ? SMALL_ROWS : SMALL_TILES;
+        plan.last_attention = p.decode || (p.n_last >= 0 && p.n_last <= TQK_SMALL_LAST_ROWS) ? SMALL_ROWS : SMALL_TILES;
+    }
+    return plan;
+}
+
+template <typename T, int D>
 static int launch_small(const TqkSmallStep& p, hipStream_t s) {
-    static const hipError_t grown = hipFuncSetAttribute((const void*)small_step_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    static const hipError_t grown = hipFuncSetAttribute((const void*)small_step_kernel<T, D>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (grown != hipSuccess) return tqk_fail("tqk_small_step: %s", hipGetErrorString(grown));
-    small_step_kernel<T><<<1 + 8 * (p.n_layers + 1), SS_THREADS, small_layout(p).bytes, s>>>(p);
+    small_step_kernel<T, D><<<1 + 8 * (p.n_layers + 1), SS_THREADS, small_layout(p).bytes, s>>>(p, small_plan(p));
     return tqk_check_launch("tqk_small_step");
 }
 
@@ -501,8 +818,10 @@ extern "C" int tqk_small_step(const TqkSmallStep* step, void* stream) {
         TQK_REQUIRE(l.width > 0 && l.window >= 0 && l.table >= 0 && l.table + l.width <= p.n_ints, "tqk_small_step: layer %d: no page table", i);
     }
     TQK_REQUIRE((((uintptr_t)p.head) & 15) == 0, "tqk_small_step: the head must be 16-byte aligned");
-    TQK_REQUIRE(p.tok_seq >= 0 && p.tok_pos >= 0 && p.want >= 0 && p.tok_seq + p.n_rows <= p.n_ints && p.tok_pos + p.n_rows <= p.n_ints && p.want + p.n_want <= p.n_ints &&
+    TQK_REQUIRE(p.tok_seq >= 0 && p.tok_pos >= 0 && p.want >= 0 && p.tok_seq + p.n_rows <= p.n_ints && p.tok_pos + p.n_rows <= p.n_ints && p.want + p.n_want <= p.n_ints && p.seq_first >= 0 && p.n_seqs > 0 &&
+                    p.seq_first + p.n_seqs + 1 <= p.n_ints && (p.n_last < 0 || (p.last_rows >= 0 && p.last_rows + p.n_last <= p.n_ints)) &&
                     (p.device_tokens || (p.tokens >= 0 && p.tokens + p.n_rows <= p.n_ints)), "tqk_small_step: the step's arrays do not lie in what was given");
     hipStream_t s = (hipStream_t)stream;
-    return p.act_dtype == TQK_F32 ? launch_small<float>(p, s) : launch_small<bf16_t>(p, s);
+    if (p.act_dtype == TQK_F32) return launch_small<float, 0>(p, s);
+    return p.head_dim == 32 ? launch_small<bf16_t, 32>(p, s) : p.head_dim == 64 ? launch_small<bf16_t, 64>(p, s) : launch_small<bf16_t, 0>(p, s);
 }

@@ -95,6 +95,7 @@ int tqk_fused_gated(const void* x, const float* ss_parts, int n_ss_parts, float 
                     int M, int N, int K, void* stream);
 /* h[M,N] += bfloat16(x w^T) in float32; xw_out = bfloat16(h * next_norm_w) or bfloat16(h);
  * ss_out (optional) [tqk_fused_residual_parts(N, K), 16] */
+int tqk_fused_waves(int N, int K, int paired);        /* how many waves share K (paired: gated and q/k/v products, of pairs of tiles) */
 int tqk_fused_residual_parts(int N, int K);
 int tqk_fused_residual_wf32(const void* x, const void* w, int w_packed, float* h, const float* next_norm_w, void* xw_out,
                             float* ss_out, int M, int N, int K, void* stream);        /* the same, the norm's weight in float32 */
@@ -626,14 +627,17 @@ int tqk_normed_pair_sum(const void* x, const void* y, int dtype, const float* wx
 
 /* A whole step of a small pre-norm decoder (grouped-query attention with rotary positions in halves, gated SiLU) in one launch (small_step.hip).
  * Weights are rows as the checkpoint has them, all of the activation type; gate's rows in front of up's; q's, k's and v's one after the other.  The step's
- * arrays (tokens, the rows' sequences and positions, the wanted rows, the page tables [sequences][width]) travel with the launch, in `ints` at the
- * places named; device_tokens: the rows' tokens, on the device instead.  logits [n_want, vocab] float32. */
-enum { TQK_SMALL_LAYERS = 16, TQK_SMALL_INTS = 416 };
+ * arrays (tokens, the rows' sequences and positions, the wanted rows, the sequences' first rows and the end, the last rows, the page tables [sequences][width]) travel with the
+ * launch, in `ints` at the places named; device_tokens: the rows' tokens, on the device instead.  logits [n_want, vocab] float32.
+ * decode: a step of one token a sequence; max_end: the furthest sequence's positions after it; n_last: how many rows the last layer needs to go on with
+ * (-1: it runs for all of them).  bfloat16 results go by these, as those of the kernels of larger models do. */
+enum { TQK_SMALL_LAYERS = 16, TQK_SMALL_INTS = 400, TQK_SMALL_LAST_ROWS = 32 };
 typedef struct {
     const void *norm1, *qkv, *qkv_bias, *o, *norm2, *gate_up, *down;
     void *keys, *values;
     float eps1, eps2, scale;
     int window, table, width;
+    int divided;        /* bfloat16, heads of 32 and 64: attention_decode.hip would have a row's pages in partitions */
 } TqkSmallLayer;
 typedef struct {
     const void *embedding, *final_norm, *head;
@@ -642,7 +646,8 @@ typedef struct {
     float* logits;
     float final_eps;
     int act_dtype, max_positions, n_layers, hidden, n_heads, n_kv_heads, head_dim, inter, vocab, n_rows, n_want, n_ints;
-    int tokens, tok_seq, tok_pos, want;
+    int tokens, tok_seq, tok_pos, want, seq_first, last_rows;
+    int n_seqs, decode, max_end, n_last;
     TqkSmallLayer layers[TQK_SMALL_LAYERS];
     int32_t ints[TQK_SMALL_INTS];
 } TqkSmallStep;

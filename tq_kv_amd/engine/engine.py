@@ -50,6 +50,11 @@ class Engine:
         """The steps captured as graphs so far (their number is what len() gives)."""
         return range(int(self._describe()["n_graphs"]))
 
+    @property
+    def n_small_steps(self):
+        """How many steps went through the one launch that small models have (csrc/small_step.hip)."""
+        return int(self._describe()["n_small_steps"])
+
     def _stream(self):
         return native.current_stream() if self.model.on_gpu else None
 

@@ -11,10 +11,11 @@ another; nothing else reads these.  They live in the engine library (tqe_policy_
                          prompts does not take gets the rows back from the packed copy for its own length
   decode_mfma, prefill_mfma   the two matrix-core attention kernels (off: the plain kernel)
   small                  steps of small models in one launch (they are not while any of the routines above is off)
+  small_always           (off) also where the estimate says that the other kernels are faster
 """
 from . import native
 
-NAMES = ("skinny", "library", "fused", "prune_last", "packed", "mid", "keep_rows", "decode_mfma", "prefill_mfma", "prompt", "small")
+NAMES = ("skinny", "library", "fused", "prune_last", "packed", "mid", "keep_rows", "decode_mfma", "prefill_mfma", "prompt", "small", "small_always")
 
 
 class _Policy:
