@@ -21,10 +21,28 @@ CASES = [("A", False), ("A", True), ("B", False), ("B", True), ("C", False), ("C
 LENS = {"A": [5, 11, 17, 64, 65, 100], "B": [1, 7, 20, 33, 64, 90], "C": [70, 129, 333, 600]}
 
 
+@pytest.fixture(params=["one launch", "kernels"])
+def either_way(request):
+    """Steps of the small configurations in one launch where that is the faster way (the default), and through the kernels of larger models alone."""
+    from tq_kv_amd import POLICY
+    POLICY["small"] = request.param == "one launch"
+    yield
+    POLICY["small"] = True
+
+
+@pytest.fixture
+def without_small_steps():
+    from tq_kv_amd import POLICY
+    POLICY["small"] = False
+    yield
+    POLICY["small"] = True
+
+
 def all_places(p):
     return list(range(len(p)))
 
 
+@pytest.mark.usefixtures("either_way")
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name,sharp", CASES)
 def test_each_request_alone_and_whole(name, sharp, dtype):
@@ -37,6 +55,7 @@ def test_each_request_alone_and_whole(name, sharp, dtype):
     eng.cache.check()
 
 
+@pytest.mark.usefixtures("either_way")
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name,sharp", CASES)
 def test_last_32_tokens_one_by_one(name, sharp, dtype):
@@ -81,6 +100,7 @@ def run_batch(eng, reqs, tails):
     return [torch.cat(g) for g in got], slots
 
 
+@pytest.mark.usefixtures("either_way")
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name,sharp", CASES)
 def test_unequal_batches_one_after_another(name, sharp, dtype):
@@ -100,6 +120,7 @@ def test_unequal_batches_one_after_another(name, sharp, dtype):
     assert used[0] == used[1] == used[2]                 # the same slots, again and again
 
 
+@pytest.mark.usefixtures("either_way")
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name,seed", [("A", 1), ("B", 2), ("B", 3), ("C", 4)])
 def test_batches_of_random_sizes_shrink_through_every_kind_of_step(name, seed, dtype):
@@ -128,6 +149,7 @@ def test_batches_of_random_sizes_shrink_through_every_kind_of_step(name, seed, d
 PIECES = {"B": [2, 7, 31, 33], "C": [2, 7, 63, 64, 65, 129]}
 
 
+@pytest.mark.usefixtures("either_way")
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", ["B", "C"])
 def test_prompts_fed_in_pieces(name, dtype):
@@ -205,6 +227,7 @@ def test_a_foreign_page_in_the_cache_is_noticed(name, sharp, mode):
             G.close(got, ref[k:], "bfloat16", "the clean run")
 
 
+@pytest.mark.usefixtures("either_way")
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_long_decoding(dtype):
     # 70 prompt tokens, then 400 single steps: across pages and far beyond the window
@@ -221,6 +244,7 @@ def test_long_decoding(dtype):
     G.close(torch.cat(outs), ref, dtype, "long decode")
 
 
+@pytest.mark.usefixtures("either_way")
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", ["A", "B"])
 def test_first_tokens_of_a_sequence(name, dtype):
@@ -250,6 +274,7 @@ def test_wanted_places_and_their_order():
     eng.close(sa), eng.close(sb)
 
 
+@pytest.mark.usefixtures("either_way")
 @pytest.mark.parametrize("name,dtype", [("B", "float32"), ("B", "bfloat16"), ("C", "float32"), ("C", "bfloat16")])
 def test_few_wanted_places_in_any_order_equal_all_places(name, dtype):
     # where a step wants fewer places than it has tokens, the last layer computes only those
@@ -280,6 +305,7 @@ def test_few_wanted_places_in_any_order_equal_all_places(name, dtype):
     eng.cache.check()
 
 
+@pytest.mark.usefixtures("either_way")
 def test_float32_results_do_not_depend_on_the_cut_at_all():
     # in float32 every kernel sums in an order that depends on the position only
     eng = G.engine("C", "float32", True)
@@ -324,6 +350,7 @@ def test_step_refuses_what_it_cannot_run():
     small.cache.check()
 
 
+@pytest.mark.usefixtures("either_way")
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_tokens_given_on_the_device_equal_tokens_given_by_the_host(dtype):
     from tq_kv_amd import StepError
@@ -359,6 +386,7 @@ def test_tokens_given_on_the_device_equal_tokens_given_by_the_host(dtype):
 
 
 # ---- generation through the entry point -------------------------------------------------------
+@pytest.mark.usefixtures("either_way")
 @pytest.mark.parametrize("name", ["A", "B"])
 def test_greedy_generation_float32_equals_plain(name):
     from tq_kv_amd import GenerationParams, generate
@@ -381,6 +409,7 @@ def test_greedy_generation_float32_equals_plain(name):
     assert eng.cache.slots.n_held == 0
 
 
+@pytest.mark.usefixtures("either_way")
 @pytest.mark.parametrize("name", ["A", "B"])
 def test_greedy_generation_bfloat16_picks_a_best_token_each_time(name):
     # bfloat16 logits differ a little from the plain ones, so a near-tie may go the other
@@ -436,7 +465,7 @@ def products_of_17_to_128_rows(request):
 
 @pytest.mark.parametrize("n_seqs", [40, 100])
 @pytest.mark.parametrize("dtype", DTYPES)
-def test_many_sequences_decode_through_replayed_graphs(dtype, products_of_17_to_128_rows, n_seqs):
+def test_many_sequences_decode_through_replayed_graphs(dtype, products_of_17_to_128_rows, n_seqs, without_small_steps):
     # 40 or 100 sequences: more rows than the few-row products take, so the captured step holds the
     # products for 17 to 128 rows (4 and 8 groups of 16 rows); every replay is checked (with other
     # work between the replays)
@@ -474,7 +503,7 @@ def test_many_sequences_decode_through_replayed_graphs(dtype, products_of_17_to_
 @pytest.mark.parametrize("n_seqs", [128, 129, 200])
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name,sharp", [("B", True), ("D", False)])
-def test_decode_steps_of_a_hundred_and_more_sequences(name, sharp, dtype, n_seqs):
+def test_decode_steps_of_a_hundred_and_more_sequences(name, sharp, dtype, n_seqs, without_small_steps):
     """Steps of exactly 128 sequences (the last that is captured as a graph and runs the own products), of 129 and of
     200 (eager, the library's products, the decoding attention kernel with more than 128 rows), and on the way down
     the steps either side of every change of kernels: 128 and 127, 17 and 16.  Sequences of unequal lengths; every

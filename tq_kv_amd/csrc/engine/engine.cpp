@@ -96,7 +96,6 @@ const float* Engine::step(int n_seqs, const int32_t* slots, const int32_t* n_new
         logits = (const float*)model->forward_small(ctx, small, device_tokens, logits_out).data;
         last_n_want_ = ctx.n_want;
         ++n_small_steps_;
-        if (use_graphs && all_one && single_.size() < (size_t)MAX_GRAPHS) single_.insert(ctx.shape());
     } else if (use_graphs && all_one && n_seqs <= mid_max_rows()) {
         logits = graphed_step(ctx, n_seqs, slots, starts.data(), n_new, tokens, want_counts, want_idx, device_tokens, logits_out, stream);
     } else {

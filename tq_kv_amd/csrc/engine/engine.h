@@ -7,7 +7,6 @@
 // against what the cache holds, and returns the logits at the wanted places.
 #pragma once
 #include <list>
-#include <set>
 
 #include "model.h"
 
@@ -40,8 +39,7 @@ public:
     // the next step writes again.  Returns where they are.
     const float* step(int n_seqs, const int32_t* slots, const int32_t* n_new, const int32_t* tokens, const int32_t* want_counts,
                       const int32_t* want_idx, const int32_t* device_tokens, float* logits_out, hipStream_t stream);
-    // shapes of one-token steps that are ready to be replayed: captured as graphs, or one launch as they are
-    int n_graphs() const { return (int)(graphs_.size() + single_.size()); }
+    int n_graphs() const { return (int)graphs_.size(); }
     long long n_small_steps() const { return n_small_steps_; }          // steps that were one launch (small_step.hip)
     int last_n_want() const { return last_n_want_; }
 
@@ -64,7 +62,6 @@ private:
     Workspace ws_;
     Staging staging_;
     std::list<Graph> graphs_;            // least recently used first
-    std::set<StepShape> single_;         // shapes of one-token steps that were one launch (MAX_GRAPHS of them at most)
     long long n_small_steps_ = 0;
     hipStream_t capture_stream_ = nullptr;
     int last_n_want_ = 0;

@@ -324,8 +324,8 @@ void tqe_engine_free(tqe_engine_t* engine);
 int tqe_engine_open(tqe_engine_t* engine, int32_t* slot_out, void* stream);       /* a sequence starts: a slot with nothing in it */
 int tqe_engine_close(tqe_engine_t* engine, int slot);                              /* it ends: slot and pages will be used again */
 tqe_cache_t* tqe_engine_cache(tqe_engine_t* engine);
-/* JSON: the cache's groups (as tqe_store_describe), holds_pages, max_slots, max_tokens, use_graphs, n_graphs (shapes of step kept: captured
- * ones, and ones that a small model's single launch took), n_small_steps (steps that such a launch took), vocab_size, max_positions */
+/* JSON: the cache's groups (as tqe_store_describe), holds_pages, max_slots, max_tokens, use_graphs, n_graphs (shapes of step captured),
+ * n_small_steps (steps that a small model's single launch took), vocab_size, max_positions */
 const char* tqe_engine_describe(const tqe_engine_t* engine);
 /* One step: sequence i lives in slots[i] and brings n_new[i] tokens (tokens: all of them on the host, one sequence after the
  * other; or device_tokens: int32 [n_seqs] on the device for a step of one token each, tokens may then be NULL);
