@@ -86,10 +86,14 @@ const float* Engine::step(int n_seqs, const int32_t* slots, const int32_t* n_new
     ctx.staging = &staging_;
     ctx.act_dtype = model->dtype;
     long long n_tokens = 0;
-    for (int i = 0; i < n_seqs; ++i) n_tokens += n_new[i];
+    int max_end = 0;
+    for (int i = 0; i < n_seqs; ++i) {
+        n_tokens += n_new[i];
+        max_end = std::max(max_end, starts[(size_t)i] + n_new[i]);
+    }
     TqkSmallStep small;
     // (the bits are the same either way; a trace shows the parts' ranges, which the one launch does not have)
-    if (n_tokens <= Model::SMALL_ROWS && model->has_small_steps() && !trace_enabled() &&
+    if (!trace_enabled() && model->small_pays(n_tokens, all_one, max_end) &&
         (ctx.plan(cache->book, n_seqs, slots, starts.data(), n_new, tokens, want_counts, want_idx, 1), model->small_step(ctx, *cache, use_graphs && all_one ? GRAPH_WIDTH_STEP : 1, small))) {
         ws_.reset(stream);
         ctx.ws = &ws_;

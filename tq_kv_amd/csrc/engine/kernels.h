@@ -36,7 +36,7 @@ TQ_QUERY(int, mid_splits, int, int, int);
 TQ_KERNEL(mid_store, cptr, cptr, void*, int, int, int, int, void*, int, void*);
 TQ_KERNEL(mid_gated, cptr, cptr, void*, int, int, int, void*, void*);
 TQ_QUERY(int, small_step_takes, const TqkSmallStep*);
-TQ_QUERY(int, small_step_pays, const TqkSmallStep*, int, int);
+TQ_QUERY(int, small_step_pays, const TqkSmallStep*, int, int, int);
 TQ_KERNEL(small_step, const TqkSmallStep*, void*);
 TQ_QUERY(int, prompt_takes, int, int, int, int);
 TQ_QUERY(int, prompt_splits, int, int, int);

@@ -128,8 +128,13 @@ void Model::find_small() {
     if (K::small_step_takes.raw(m.get())) small_ = std::move(m);
 }
 
+bool Model::small_pays(long long n_tokens, bool decode, int max_end) const {
+    if (!small_ || n_tokens > SMALL_ROWS || !policy().small_steps()) return false;
+    return policy().small_always || K::small_step_pays.raw(small_.get(), (int)n_tokens, decode ? 1 : 0, max_end) != 0;
+}
+
 bool Model::small_step(const StepContext& c, const CacheStore& cache, int graph_width, TqkSmallStep& step) const {
-    if (!small_ || !policy().small_steps() || c.n_tokens > SMALL_ROWS || c.n_want > c.n_tokens) return false;
+    if (c.n_want > c.n_tokens) return false;
     step = *small_;
     step.n_rows = c.n_tokens;
     step.n_want = c.n_want;
@@ -166,7 +171,7 @@ bool Model::small_step(const StepContext& c, const CacheStore& cache, int graph_
         const int width = (step.layers[i].width + graph_width - 1) / graph_width * graph_width;
         step.layers[i].divided = blocks_[(size_t)spec.order[(size_t)i].layer]->row_partitions(last ? c.n_last : c.n_tokens, width) > 1;
     }
-    return K::small_step_takes.raw(&step) != 0 && (policy().small_always || K::small_step_pays.raw(&step, c.all_decode ? 1 : 0, c.max_end) != 0);
+    return K::small_step_takes.raw(&step) != 0;
 }
 
 Tensor Model::forward_small(StepContext& c, TqkSmallStep& step, const int32_t* device_tokens, float* out) {

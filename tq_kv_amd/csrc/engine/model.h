@@ -38,7 +38,8 @@ public:
     // graph_width: the step's tables would be filled up to a multiple of so many pages in a captured graph (1: it would not be captured).
     bool small_step(const StepContext& c, const CacheStore& cache, int graph_width, TqkSmallStep& step) const;
     Tensor forward_small(StepContext& c, TqkSmallStep& step, const int32_t* device_tokens, float* out);
-    bool has_small_steps() const { return small_ != nullptr; }
+    // Whether a step of that many tokens, decoding or not, up to the furthest position is to be asked about (before anything is planned).
+    bool small_pays(long long n_tokens, bool decode, int max_end) const;
     static const int SMALL_ROWS = 64;           // (more rows are not asked about)
     Json describe() const;
     // Lets the library try its kernels once for every product of the model at `rows` rows (more than the own kernels

@@ -765,21 +765,22 @@ extern "C" int tqk_small_step_takes(const TqkSmallStep* step) {
     return 1;
 }
 
-/* Whether that is the faster way, by an estimate in microseconds (decode: a step of one token a sequence, which the other kernels run as a replayed graph; positions: the
- * furthest one of the step).  One block: 5 a layer for its barriers and chains of short operations, its weights at 33 KB (27 in float32) a microsecond, and for every row what
+/* Whether that is the faster way, by an estimate in microseconds (n_rows: of the step; decode: one token a sequence, which the other kernels run as a replayed graph; positions: the
+ * furthest one).  One block: 5 a layer for its barriers and chains of short operations, its weights at 33 KB (27 in float32) a microsecond, and for every row what
  * its products, its other work and its heads' pages take; the head's weights at 39 KB.  The other kernels, ten launches a layer: 20 a layer in a graph (33 in float32) and 32 (45) one by one.
  * Measured, one block and the other kernels, two layers of 64 values with 160 in the feed-forward, bfloat16: 1, 16 and 40 sequences 31 and 72, 65 and 79, 92 and 88, prompts of 8, 33
  * and 64 tokens 31 and 96, 61 and 96, 109 and 97; three of 96 with 224 and heads of 32: 47 and 73, 75 and 82, 108 and 97, then 35 and 132, 70 and 134, 95 and 135; with heads of 64: 66 and 78, 87
  * and 83, 156 and 106, then 43 and 132, 87 and 137, 133 and 137; four of 128 with 224: 69 and 83, 94 and 88, 207 and 122, then 55 and 175, 126 and 179, 175 and 179.  float32, two of 64: 35 and 81, 74 and
  * 85, 125 and 111, then 36 and 100, 88 and 102, 145 and 103; three of 96: 62 and 108, 113 and 113, 249 and 152, then 69 and 132, 192 and 138, 306 and 147; four of 128 with 512: 159 and 146, 313 and 154,
  * then 171 and 173. */
-extern "C" int tqk_small_step_pays(const TqkSmallStep* step, int decode, int positions) {
+extern "C" int tqk_small_step_pays(const TqkSmallStep* step, int n_rows, int decode, int positions) {
     const TqkSmallStep& p = *step;
     const bool f32 = p.act_dtype == TQK_F32;
+    if (!f32 && !(heads_fit(p, positions) && in_order(p, n_rows, n_rows, n_rows, decode != 0))) return 0;         // (what the kernel does not take)
     const double size = f32 ? 4 : 2, q = (double)p.n_heads * p.head_dim;
     const double thousands = 1e-3 * p.hidden * (2 * q + 2. * p.n_kv_heads * p.head_dim + 3. * p.inter);            // weights of a layer
     const double a_row = 0.15 + (f32 ? 0.0115 : 0.0043) * thousands + 0.08 * p.n_heads * ((positions + TQK_PAGE - 1) / TQK_PAGE);
-    const double here = 8 + p.n_layers * (5 + thousands * size / (f32 ? 27 : 33) + p.n_rows * a_row) + 1e-3 * p.vocab * p.hidden * size / 39;
+    const double here = 8 + p.n_layers * (5 + thousands * size / (f32 ? 27 : 33) + n_rows * a_row) + 1e-3 * p.vocab * p.hidden * size / 39;
     const double there = decode ? 15 + p.n_layers * (f32 ? 33 : 20) : 15 + p.n_layers * (f32 ? 45 : 32);
     return here < there;
 }
