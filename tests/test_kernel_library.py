@@ -114,3 +114,30 @@ def test_the_sizes_of_the_mid_products_tests_take_every_tile():
     (129, 37888, 3584 + 32, True, False), (129, 24, 256, False, False)])                                                           # not taken at all
 def test_which_products_pay_in_the_kernel_for_prompts(m, n, k, gated, pays):
     assert kernels.prompt_pays(m, n, k, gated) == pays
+
+
+def small_step(**sizes):
+    """What the kernel for small models' steps is asked about: a TqkSmallStep, its pointers left out."""
+    class Layer(ctypes.Structure):
+        _fields_ = [("pointers", ctypes.c_void_p * 9), ("eps1", ctypes.c_float), ("eps2", ctypes.c_float), ("scale", ctypes.c_float),
+                    ("window", ctypes.c_int), ("table", ctypes.c_int), ("width", ctypes.c_int), ("divided", ctypes.c_int)]
+
+    class Step(ctypes.Structure):
+        _fields_ = [("pointers", ctypes.c_void_p * 7), ("final_eps", ctypes.c_float)] + [(n, ctypes.c_int) for n in (
+            "act_dtype max_positions n_layers hidden n_heads n_kv_heads head_dim inter vocab n_rows n_want n_ints tokens tok_seq tok_pos want seq_first last_rows "
+            "n_seqs decode max_end n_last").split()] + [("layers", Layer * 16), ("ints", ctypes.c_int32 * 400)]
+    return Step(**dict(dict(act_dtype=1, max_positions=128, n_layers=2, hidden=64, n_heads=4, n_kv_heads=2, head_dim=16, inter=160, vocab=256, n_rows=1, n_want=1,
+                            n_seqs=1, decode=1, max_end=1, n_last=-1), **sizes))
+
+
+@pytest.mark.parametrize("sizes,takes", [
+    ({}, 1), ({"act_dtype": 0}, 1),
+    ({"vocab": 2 ** 24 - 1}, 1), ({"vocab": 2 ** 24}, 0), ({"vocab": 2 ** 31 - 1}, 0),                      # the head's bytes in 32 bits
+    ({"act_dtype": 0, "vocab": 2 ** 14}, 0),                                                               # another order of sums there
+    ({"head_dim": 32, "max_end": 64}, 1), ({"head_dim": 32, "max_end": 65}, 0), ({"max_end": 500}, 1),      # one page for the matrix cores' heads
+    ({"inter": 256}, 0), ({"inter": 256, "n_rows": 17, "n_want": 17, "n_seqs": 17}, 1), ({"inter": 224}, 1),       # K dealt out to waves
+    ({"n_heads": 17, "n_kv_heads": 1, "head_dim": 32, "n_rows": 17, "n_want": 17, "n_seqs": 17}, 0),        # more heads than a tile's columns
+    ({"n_rows": 65}, 0), ({"n_want": 2}, 0), ({"hidden": 72}, 0), ({"n_layers": 17}, 0)])
+def test_which_steps_the_kernel_for_small_models_takes(sizes, takes):
+    lib = ctypes.CDLL(kernels.library_path())
+    assert lib.tqk_small_step_takes(ctypes.byref(small_step(**sizes))) == takes
