@@ -24,6 +24,7 @@
 // 27 to 45 us for few rows, as lanes without a key then load, too.)
 #include "attention_walk.h"
 #include "tq_kernels.h"
+#include <atomic>
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
@@ -802,8 +803,16 @@ static SmallPlan small_plan(const TqkSmallStep& p) {
 
 template <typename T, int D>
 static int launch_small(const TqkSmallStep& p, hipStream_t s) {
-    static const hipError_t grown = hipFuncSetAttribute((const void*)small_step_kernel<T, D>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if (grown != hipSuccess) return tqk_fail("tqk_small_step: %s", hipGetErrorString(grown));
+    // (a limit of each device's own: raised once for it, or a few times by threads that meet here)
+    static std::atomic<uint64_t> grown{0};
+    int device = 0;
+    hipError_t e = hipGetDevice(&device);
+    const uint64_t bit = device < 64 ? 1ull << device : 0;
+    if (e == hipSuccess && !(grown.load(std::memory_order_acquire) & bit)) {
+        e = hipFuncSetAttribute((const void*)small_step_kernel<T, D>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e == hipSuccess) grown.fetch_or(bit, std::memory_order_release);
+    }
+    if (e != hipSuccess) return tqk_fail("tqk_small_step: %s", hipGetErrorString(e));
     small_step_kernel<T, D><<<1 + 8 * (p.n_layers + 1), SS_THREADS, small_layout(p).bytes, s>>>(p, small_plan(p));
     return tqk_check_launch("tqk_small_step");
 }
