@@ -451,8 +451,8 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
         return one;
     };
     for (int i = tid; i < p.n_ints; i += SS_THREADS) ints[i] = p.ints[i];
-    for (int i = tid; i < p.n_layers * (int)(sizeof(TqkSmallLayer) / 4); i += SS_THREADS)
-        reinterpret_cast<int32_t*>(lds + at.layers)[i] = reinterpret_cast<const int32_t*>(p.layers)[i];
+    for (int i = tid * 4; i < p.n_layers * (int)sizeof(TqkSmallLayer); i += SS_THREADS * 4)
+        __builtin_memcpy(__builtin_assume_aligned(lds + at.layers + i, 4), reinterpret_cast<const char*>(p.layers) + i, 4);
     for (int layer = wave; layer < p.n_layers; layer += SS_WAVES) {
         const TqkSmallLayer& l = p.layers[layer];
         for (int i = lane; i < hidden; i += TQK_WAVE) {
@@ -549,10 +549,12 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
 
 #pragma unroll 1
     for (int layer = 0; layer < p.n_layers; ++layer) {
-        TqkSmallLayer l;                                    // this layer's arguments, the same for all lanes
+        // this layer's arguments, the same for all lanes
+        struct Words { int32_t w[sizeof(TqkSmallLayer) / 4]; } words;
+        __builtin_memcpy(&words, layers + layer, sizeof(words));
 #pragma unroll
-        for (int i = 0; i < (int)(sizeof(l) / 4); ++i)
-            reinterpret_cast<int32_t*>(&l)[i] = __builtin_amdgcn_readfirstlane(reinterpret_cast<const int32_t*>(layers + layer)[i]);
+        for (int i = 0; i < (int)(sizeof(words) / 4); ++i) words.w[i] = __builtin_amdgcn_readfirstlane(words.w[i]);
+        const TqkSmallLayer l = __builtin_bit_cast(TqkSmallLayer, words);
         const int32_t* table = ints + l.table;
         const bool last = layer == p.n_layers - 1 && p.n_last >= 0;         // (what follows the cache's rows counts for the last rows alone)
         SmallProduct<T, 1> w_qkv = product(l.qkv, qkv, hidden, row_tiles);
