@@ -761,10 +761,10 @@ extern "C" int tqk_small_step_takes(const TqkSmallStep* step) {
     // whole steps of k, and whole tiles
     const int q = p.n_heads * p.head_dim, whole = 64 / size;
     if (p.hidden % whole || p.inter % whole || q % whole || (p.n_kv_heads * p.head_dim * 2) % 16) return 0;
+    if ((long long)p.vocab * p.hidden * size > 0x7fffffff) return 0;          // (a weight's bytes are counted in 32 bits)
     if (small_layout(p).bytes > 160 * 1024) return 0;
     if (p.act_dtype == TQK_BF16 && !(heads_fit(p, p.max_end) && in_order(p, p.n_rows, p.n_last >= 0 ? p.n_last : p.n_rows, p.n_want, p.decode != 0))) return 0;
     // (larger products have another order of summation there)
-    if ((long long)p.vocab * p.hidden * size > 0x7fffffff) return 0;          // (a weight's bytes are counted in 32 bits)
     if (p.act_dtype == TQK_F32 && (tqk_gemm_takes_apart(p.vocab, p.hidden) || tqk_gemm_takes_apart(2 * p.inter, p.hidden) || tqk_gemm_takes_apart(q + 2 * p.n_kv_heads * p.head_dim, p.hidden))) return 0;
     return 1;
 }
