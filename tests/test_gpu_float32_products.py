@@ -52,3 +52,30 @@ def test_infinities_nan_and_overflow(m, n, k):
     finite = torch.isfinite(want)
     assert torch.equal(torch.sign(y[~finite & ~torch.isnan(want)]), torch.sign(want[~finite & ~torch.isnan(want)]))
     torch.testing.assert_close(y[m - 1, 78], want[m - 1, 78])
+
+
+@pytest.mark.parametrize("n,k", [(2048, 1540), (1024, 3584), (4608, 2048)])
+def test_what_is_not_finite_changes_nothing_beside_it(n, k):
+    """One row of x and one of w hold what is not finite (in the first group of k, in the last, in both), and everything else keeps the bits that
+    it has without them, whatever the number of rows: the same tile's, the other groups' of the same sum, a row's alone."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, w = torch.randn((130, k), device="cuda", generator=g), torch.randn((n, k), device="cuda", generator=g)
+    clean = product(x, w, None)
+    for bad_row, bad_feature, places in ((0, 5, [7]), (3, n - 1, [k - 2]), (9, 17, [1, k - 1])):
+        xb, wb = x.clone(), w.clone()
+        for p in places:
+            xb[bad_row, p], wb[bad_feature, p] = float("inf"), float("nan")
+        alone = product(xb[bad_row:bad_row + 1].contiguous(), wb, None)[0]
+        for m in ROWS:
+            y, rows = product(xb[:m].contiguous(), wb, None), torch.arange(m, device="cuda") != bad_row
+            kept = torch.arange(n, device="cuda") != bad_feature
+            assert torch.equal(y[rows][:, kept], clean[:m][rows][:, kept]), m
+            assert not torch.isfinite(y[:, bad_feature]).any()
+            if m > bad_row:
+                assert torch.equal(y[bad_row].isnan(), alone.isnan()) and torch.equal(y[bad_row][~alone.isnan()], alone[~alone.isnan()]), m
+    # a sum that overflows in float32 in one group of k and the other groups finite: the same for every number of rows
+    x[1, :4], w[8, :4] = 2e19, 2e19
+    one = product(x[1:2].contiguous(), w, None)[0]
+    assert torch.isinf(one[8])
+    for m in ROWS[1:]:
+        assert torch.equal(product(x[:m].contiguous(), w, None)[1], one), m

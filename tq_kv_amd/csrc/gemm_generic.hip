@@ -117,7 +117,8 @@ __device__ __forceinline__ void multiply16(floatx4_t& acc, const floatx4_t& w, c
 // float32.  Six bfloat16 instructions stand for eight float32 ones of twice the time each, 2.7 times the rate, and their sums of 32 k at once round less often: error against 64 bits, 2-norm,
 // K of 3584 and 18944, operands N(0, 1) 1.73e-7 and 2.07e-7 (the float32 instructions 2.17e-7 and 2.28e-7), all of one sign 0.52e-7 and 0.64e-7 (0.55e-7 and 0.64e-7), spread over
 // twelve powers of ten 1.30e-7 and 1.65e-7 (1.79e-7 and 2.06e-7), N(0, 1e-33) as N(0, 1).  (With the five small products in a sum of their own 0.98e-7, and 32 registers more.)
-// Infinities have no parts (inf - inf): where a wave's sums are not finite it takes them again with the float32 instructions.
+// Infinities have no parts (inf - inf): a group's sum that is not finite is taken again with the float32 instructions, that one and no other, so that a result depends on
+// its own rows of x and w alone.
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 struct Parts { bf16x8_t p, q, t; };
 __device__ __forceinline__ uint32_t high_halves(float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); }
@@ -153,23 +154,19 @@ __device__ __forceinline__ void multiply32(floatx4_t& acc, const Parts& w, const
 __device__ __forceinline__ bool finite(floatx4_t v) {
     return __builtin_isfinite(v[0]) && __builtin_isfinite(v[1]) && __builtin_isfinite(v[2]) && __builtin_isfinite(v[3]);
 }
-// The sums of k_begin .. k_end (whole groups, or up to K) of 16 rows and 16 features by the float32 instructions, for a wave; xrow, wrow: the lane's rows.
-__device__ __forceinline__ floatx4_t plain_sums(const float* xrow, const float* wrow, int k_begin, int k_end, int k4) {
-    floatx4_t total = {0.f, 0.f, 0.f, 0.f};
-    for (int g0 = k_begin; g0 < k_end; g0 += G_GROUP) {
-        floatx4_t group = {0.f, 0.f, 0.f, 0.f};
-        for (int c0 = g0; c0 < min(g0 + G_GROUP, k_end); c0 += G_CHUNK) {
-            floatx4_t acc = {0.f, 0.f, 0.f, 0.f};
-            for (int k0 = c0; k0 < min(c0 + G_CHUNK, k_end); k0 += 16) {
-                const floatx4_t none = {0.f, 0.f, 0.f, 0.f};
-                const bool in = k0 + k4 < k_end;
-                multiply16(acc, in ? *reinterpret_cast<const floatx4_t*>(wrow + k0 + k4) : none, in ? *reinterpret_cast<const floatx4_t*>(xrow + k0 + k4) : none);
-            }
-            group += acc;
+// The sums of a group (k_begin .. k_end) of 16 rows and 16 features by the float32 instructions, for a wave; xrow, wrow: the lane's rows.
+__device__ __forceinline__ floatx4_t plain_group(const float* xrow, const float* wrow, int k_begin, int k_end, int k4) {
+    floatx4_t group = {0.f, 0.f, 0.f, 0.f};
+    for (int c0 = k_begin; c0 < k_end; c0 += G_CHUNK) {
+        floatx4_t acc = {0.f, 0.f, 0.f, 0.f};
+        for (int k0 = c0; k0 < min(c0 + G_CHUNK, k_end); k0 += 16) {
+            const floatx4_t none = {0.f, 0.f, 0.f, 0.f};
+            const bool in = k0 + k4 < k_end;
+            multiply16(acc, in ? *reinterpret_cast<const floatx4_t*>(wrow + k0 + k4) : none, in ? *reinterpret_cast<const floatx4_t*>(xrow + k0 + k4) : none);
         }
-        total += group;
+        group += acc;
     }
-    return total;
+    return group;
 }
 
 // Up to 16 rows of x: a wave per (16 output features, one group of k).  With one group the result is finished here.
@@ -372,7 +369,11 @@ void gemm_few_rows_apart_kernel(const float* __restrict__ x, const float* __rest
         s0 += NS;
     } while (s0 < n_stage);
     __builtin_amdgcn_s_waitcnt(0x0f70);                                 // nothing is on its way into LDS any more
-    if (__any(r16 < M && !finite(group))) group = plain_sums(x + (size_t)min(r16, M - 1) * K, w + (size_t)min(n0 + r16, N - 1) * K, k_begin, k_end, 4 * g);
+    if (__any(r16 < M && !finite(group))) {
+        const floatx4_t plain = plain_group(x + (size_t)min(r16, M - 1) * K, w + (size_t)min(n0 + r16, N - 1) * K, k_begin, k_end, 4 * g);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) group[i] = __builtin_isfinite(group[i]) ? group[i] : plain[i];
+    }
     if (r16 >= M) return;
     const bool whole = gridDim.y == 1;
     float* dst = out + ((size_t)blockIdx.y * M + r16) * N;
@@ -577,9 +578,8 @@ void gemm_split_kernel(const float* __restrict__ x, const float* __restrict__ w,
             acc[f][a] = group[f][a] = none;
             totals[f * RT + a][tid] = none;
         }
-    auto write = [&](float* y, int f, int a, floatx4_t v, bool with_bias, int k0, int k1) {
+    auto write = [&](float* y, int f, int a, floatx4_t v, bool with_bias) {
         const int m = m0 + 16 * a + r16;
-        if (__any(!finite(v))) v = plain_sums(x + (size_t)min(m, M - 1) * K, wrow[f], k0, k1, 4 * g);
         if (m >= M) return;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -645,23 +645,57 @@ void gemm_split_kernel(const float* __restrict__ x, const float* __restrict__ w,
         }
         const int done = c0 + G_CHUNK;
         const bool end = done % G_GROUP == 0 || done >= k_end;
+        bool all_finite = true;
 #pragma unroll
         for (int f = 0; f < FT; ++f)
 #pragma unroll
             for (int a = 0; a < RT; ++a) {
                 group[f][a] += acc[f][a];
                 acc[f][a] = none;
-                if (!end) continue;
-                if (shared_out) write(out + (size_t)(c0 / G_GROUP) * M * N, f, a, group[f][a], false, c0 / G_GROUP * G_GROUP, min(done, k_end));
+                all_finite = all_finite && finite(group[f][a]);
+            }
+        if (!end) continue;
+        uint32_t again = 0;                             // which of the lane's sums of the group are not finite
+        static_assert(FT * RT * 4 <= 32, "a bit each");
+        if (__any(!all_finite)) {
+#pragma unroll
+            for (int f = 0; f < FT; ++f)
+#pragma unroll
+                for (int a = 0; a < RT; ++a)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (!__builtin_isfinite(group[f][a][i])) { again |= 1u << (4 * (f * RT + a) + i); group[f][a][i] = 0.f; }
+        }
+#pragma unroll
+        for (int f = 0; f < FT; ++f)
+#pragma unroll
+            for (int a = 0; a < RT; ++a) {
+                if (shared_out) write(out + (size_t)(c0 / G_GROUP) * M * N, f, a, group[f][a], false);
                 else totals[f * RT + a][tid] += group[f][a];
                 group[f][a] = none;
             }
+        if (__any(again != 0)) {
+            const int g0 = c0 / G_GROUP * G_GROUP;
+#pragma unroll 1
+            for (int j = 0; j < FT * RT; ++j) {
+                const uint32_t which = again >> (4 * j) & 15;
+                if (!__any(which != 0)) continue;
+                const int m = m0 + 16 * (j % RT) + r16, n = n0 + 16 * (j / RT);
+                const floatx4_t plain = plain_group(x + (size_t)min(m, M - 1) * K, w + (size_t)min(n + r16, N - 1) * K, g0, min(done, k_end), 4 * g);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (!(which >> i & 1)) continue;
+                    if (!shared_out) totals[j][tid][i] += plain[i];
+                    else if (m < M && n + 4 * g + i < N) out[(size_t)(c0 / G_GROUP) * M * N + (size_t)m * N + n + 4 * g + i] = plain[i];
+                }
+            }
+        }
     }
     if (shared_out) return;
 #pragma unroll
     for (int f = 0; f < FT; ++f)
 #pragma unroll
-        for (int a = 0; a < RT; ++a) write(out, f, a, totals[f * RT + a][tid], bias != nullptr, k_begin, k_end);
+        for (int a = 0; a < RT; ++a) write(out, f, a, totals[f * RT + a][tid], bias != nullptr);
 }
 
 // The groups' sums in their order.  Eight loads under way together: one after the other they were most of the time (19 groups of one row of 3584 5.6 -> 4.7 us).
