@@ -1,6 +1,6 @@
 """float32 products with large weights, whose numbers go through the matrix cores as three bfloat16 ones each (csrc/gemm_generic.hip): the
-same bits whatever the number of rows (one kernel each for up to 4, 8 and 16 rows, four tiles for more), and no further from 64 bits than float32
-sums are; infinities, NaN and numbers that overflow come out as float32 arithmetic gives them."""
+same bits whatever the number of rows (one kernel each for up to 4, 8 and 16 rows, four tiles for more), and no further from 64 bits than the float32
+instructions are; infinities, NaN and numbers that overflow come out as float32 arithmetic gives them."""
 import pytest
 import torch
 
@@ -8,6 +8,38 @@ from tq_kv_amd import kernels as K
 
 pytestmark = pytest.mark.gpu
 ROWS = [1, 3, 4, 5, 8, 9, 16, 17, 32, 33, 64, 65, 130]
+
+
+def operands(kind, m, n, k):
+    """x and w of a kind: dense ones of several sizes, and rows that one value makes up, alone or by far."""
+    g = torch.Generator(device="cuda").manual_seed(len(kind) + k)
+    rand = lambda *s: torch.randn(s, device="cuda", generator=g)
+    x, w = rand(m, k), rand(n, k)
+    if kind == "one sign":
+        x, w = x.abs(), w.abs()
+    elif kind == "spread":
+        x = x * 10 ** (torch.rand((m, k), device="cuda", generator=g) * 12 - 6)
+    elif kind in ("one term", "one large term"):
+        at = torch.arange(m, device="cuda")
+        large = x[at, at * 7 % k]
+        x = torch.zeros_like(x) if kind == "one term" else x * 1e-4
+        x[at, at * 7 % k] = large if kind == "one term" else large * 1e4
+    return x, w
+
+
+@pytest.mark.parametrize("m", [8, 64])
+@pytest.mark.parametrize("k", [1024, 3584, 18944])
+@pytest.mark.parametrize("kind", ["normal", "one sign", "spread", "one term", "one large term"])
+def test_no_further_from_64_bits_than_the_float32_instructions(kind, k, m):
+    """The same rows and weights through the float32 instructions: slices of the weights that are too small to be taken apart.  Two ways to round the same sums differ by
+    chance as well: of 64 rows by more than a thousand features a hundredth."""
+    x, w = operands(kind, m, max(1024, (1 << 20) // k + 64), k)
+    step = ((1 << 20) - 1) // k
+    plain = torch.cat([product(x, w[a:a + step].contiguous(), None) for a in range(0, len(w), step)], 1)
+    y, want = product(x, w, None), x.double() @ w.double().t()
+    assert (y - want).norm() <= 1.01 * (plain - want).norm(), ((y - want).norm() / want.norm() * 2 ** 24, (plain - want).norm() / want.norm() * 2 ** 24)
+    if kind == "one term":          # a product rounded once, and what the smaller parts' sum is cut off by, 2^-7 of that
+        assert ((y - want).abs() / want.abs().clamp_min(1e-30)).max() <= (1 + 2 ** -5) * 2 ** -24
 
 
 def product(x, w, bias):
@@ -29,9 +61,9 @@ def test_rows_do_not_depend_on_the_batch_and_are_as_exact_as_float32_sums(n, k, 
         assert torch.equal(product(x[:m].contiguous(), w, b), whole[:m]), m
         assert torch.equal(product(x[-m:].contiguous(), w, b), whole[-m:]), m
     want = x.double() @ w.double().t() + (b.double() if bias else 0)
-    # A float32 sum by chunks: within a chunk each of four instructions' sums of 32 k and five small ones rounds once, 24 roundings of a sum that grows to the chunk's size, and one
-    # for each of the chunks, groups and the bias, 2^-24 of what is summed so far each and independent: no more than sqrt(24 / 3 + 2) 2^-24 of the result's spread, and the same
-    # again for terms that cancel.
+    # A float32 sum by chunks: within a chunk the sum of the largest products is cut off four times, 2^-23 of what is summed so far at most, and that of the others, a 128th of the
+    # size, 28 times; they round once where they meet, and once for each of the chunks, groups and the bias, 2^-24, all independent: variances of 4 / 3 and 1 / 3 of 2^-48,
+    # no more than sqrt(10) 2^-24 of the result's spread, and the same again for terms that cancel.
     spread = (x.double().norm(dim=1, keepdim=True) * w.double().norm(dim=1)) + (b.double().abs() if bias else 0)
     assert ((whole - want).abs() / spread).max() <= 8 * 2 ** -24
     assert (whole - want).norm() <= 2 * (10 ** 0.5) * 2 ** -24 * want.norm()

@@ -112,11 +112,13 @@ __device__ __forceinline__ void multiply16(floatx4_t& acc, const floatx4_t& w, c
 }
 
 // ---- large weights: a float32 number as three bfloat16 ones -----------------------------------------
-// 24 bits are 8 + 8 + 8: p the number cut off after 8 bits (so that nothing overflows), q what is left rounded to 8, t what is left then, exactly.
-// Of the nine products of two numbers' parts the three smallest (below 2^-22 of the whole, on average far less) are left out; the others are exact in
-// float32.  Six bfloat16 instructions stand for eight float32 ones of twice the time each, 2.7 times the rate, and their sums of 32 k at once round less often: error against 64 bits, 2-norm,
-// K of 3584 and 18944, operands N(0, 1) 1.73e-7 and 2.07e-7 (the float32 instructions 2.17e-7 and 2.28e-7), all of one sign 0.52e-7 and 0.64e-7 (0.55e-7 and 0.64e-7), spread over
-// twelve powers of ten 1.30e-7 and 1.65e-7 (1.79e-7 and 2.06e-7), N(0, 1e-33) as N(0, 1).  (With the five small products in a sum of their own 0.98e-7, and 32 registers more.)
+// 24 bits are 8 + 8 + 8: p the number cut off after 8 bits (so that nothing overflows), q what is left rounded to 8, t what is left then, exactly (from 2^-110 on: bfloat16
+// ends at 2^-133).  Of the nine products of two numbers' parts the smallest, t t, is left out (2^-32 of the whole); the others are exact in float32.  The matrix cores cut a sum off
+// where float32 instructions round it, so the largest products have a sum of their own, and the seven others, a 128th of it, another; the two are added at the end of a
+// chunk.  Eight bfloat16 instructions stand for eight float32 ones of twice the time each, and their sums of 32 k at once round less often: error against
+// 64 bits, 2-norm in 2^-24, K of 3584 and 18944, operands N(0, 1) 1.57 and 2.02 (the float32 instructions 3.61 and 3.82), all of one sign 0.83 and 1.18 (0.98 and 1.20), spread
+// over twelve powers of ten 1.90 and 2.49 (2.92 and 3.15), rows with one value alone 0.42 and 0.42 (0.42 and 0.42; the largest 1.0 both ways), with one 10^8 times the others 1.64 and 2.27 (1.69 and
+// 2.28).  Without q t and t q, and all in one sum, prompts took 0.87 of the time (300 rows of gate+up of the 7B shape 529 us and 601), but rows with one value had 0.67, the largest 3.9.
 // Infinities have no parts (inf - inf): a group's sum that is not finite is taken again with the float32 instructions, that one and no other, so that a result depends on
 // its own rows of x and w alone.
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
@@ -142,13 +144,15 @@ __device__ __forceinline__ Parts split8(floatx4_t a, floatx4_t b) {
     }
     return {__builtin_bit_cast(bf16x8_t, p), __builtin_bit_cast(bf16x8_t, q), __builtin_bit_cast(bf16x8_t, t)};
 }
-// 32 k more: a lane holds, of both operands, row lane % 16 and the eight k at 8 (lane / 16); the smallest products first.
-__device__ __forceinline__ void multiply32(floatx4_t& acc, const Parts& w, const Parts& x) {
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.t, x.p, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p, x.t, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.q, x.q, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.q, x.p, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p, x.q, acc, 0, 0, 0);
+// 32 k more: a lane holds, of both operands, row lane % 16 and the eight k at 8 (lane / 16); acc: the largest products, low: the others, the smallest first.
+__device__ __forceinline__ void multiply32(floatx4_t& acc, floatx4_t& low, const Parts& w, const Parts& x) {
+    low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.t, x.q, low, 0, 0, 0);
+    low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.q, x.t, low, 0, 0, 0);
+    low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.t, x.p, low, 0, 0, 0);
+    low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p, x.t, low, 0, 0, 0);
+    low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.q, x.q, low, 0, 0, 0);
+    low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.q, x.p, low, 0, 0, 0);
+    low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p, x.q, low, 0, 0, 0);
     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p, x.p, acc, 0, 0, 0);
 }
 __device__ __forceinline__ bool finite(floatx4_t v) {
@@ -294,7 +298,7 @@ void gemm_few_rows_apart_kernel(const float* __restrict__ x, const float* __rest
 #pragma unroll
         for (int u = 0; u < XU; ++u) xv[decltype(I)::value % NS][u] = *reinterpret_cast<const floatx4_t*>(xrow + min(k0 + x_place(u), K - 4));
     };
-    floatx4_t group = {0.f, 0.f, 0.f, 0.f}, acc = group;
+    floatx4_t group = {0.f, 0.f, 0.f, 0.f}, acc = group, low = group;
     // (no branch in a stage: every stage issues its loads and multiplies, past the end what is nothing)
     auto multiply = [&](auto I, int stage) {
         const float* src = buf(I);
@@ -343,7 +347,7 @@ void gemm_few_rows_apart_kernel(const float* __restrict__ x, const float* __rest
             xp[1] = turned(std::integral_constant<int, 0x128>{}, xp[0]);
         }
 #pragma unroll
-        for (int h = 0; h < 2; ++h) multiply32(acc, split8(wv[2 * h], wv[2 * h + 1]), xp[h]);
+        for (int h = 0; h < 2; ++h) multiply32(acc, low, split8(wv[2 * h], wv[2 * h + 1]), xp[h]);
     };
     // The waits below count LOADS loads a stage in the stages' order.  Barriers keep the scheduler to it, and there is no test in front
     // of the loop (n_stage is at least 1): behind one the compiler had put all loads of x after all those of the weights.
@@ -361,8 +365,8 @@ void gemm_few_rows_apart_kernel(const float* __restrict__ x, const float* __rest
             __builtin_amdgcn_sched_barrier(0);
             multiply(S, s0 + h);
             if constexpr (h % 2 == 1) {
-                group += acc;
-                acc = floatx4_t{0.f, 0.f, 0.f, 0.f};
+                group += acc + low;
+                acc = low = floatx4_t{0.f, 0.f, 0.f, 0.f};
             }
             __builtin_amdgcn_sched_barrier(0);
         });
@@ -570,12 +574,12 @@ void gemm_split_kernel(const float* __restrict__ x, const float* __restrict__ w,
             *reinterpret_cast<uint2*>(&lds[to][2][xdst[i]]) = t;
         }
     };
-    floatx4_t acc[FT][RT], group[FT][RT];
+    floatx4_t acc[FT][RT], low[FT][RT], group[FT][RT];
 #pragma unroll
     for (int f = 0; f < FT; ++f)
 #pragma unroll
         for (int a = 0; a < RT; ++a) {
-            acc[f][a] = group[f][a] = none;
+            acc[f][a] = low[f][a] = group[f][a] = none;
             totals[f * RT + a][tid] = none;
         }
     auto write = [&](float* y, int f, int a, floatx4_t v, bool with_bias) {
@@ -625,14 +629,14 @@ void gemm_split_kernel(const float* __restrict__ x, const float* __restrict__ w,
                     xp[a] = {*reinterpret_cast<const bf16x8_t*>(&lds[stage][0][at]), *reinterpret_cast<const bf16x8_t*>(&lds[stage][1][at]),
                              *reinterpret_cast<const bf16x8_t*>(&lds[stage][2][at])};
 #pragma unroll
-                    for (int f = 0; f < FT; ++f) multiply32(acc[f][a], wp[f], xp[a]);
+                    for (int f = 0; f < FT; ++f) multiply32(acc[f][a], low[f][a], wp[f], xp[a]);
                 }
                 // a product's instruction takes the matrix cores 16 cycles and the wave 4: three others beside each
                 __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
 #pragma unroll
                 for (int a = 0; a < RT; ++a) {
 #pragma unroll
-                    for (int i = 0; i < 6 * FT; ++i) {
+                    for (int i = 0; i < 8 * FT; ++i) {
                         __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
                         __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
                     }
@@ -650,8 +654,8 @@ void gemm_split_kernel(const float* __restrict__ x, const float* __restrict__ w,
         for (int f = 0; f < FT; ++f)
 #pragma unroll
             for (int a = 0; a < RT; ++a) {
-                group[f][a] += acc[f][a];
-                acc[f][a] = none;
+                group[f][a] += acc[f][a] + low[f][a];
+                acc[f][a] = low[f][a] = none;
                 all_finite = all_finite && finite(group[f][a]);
             }
         if (!end) continue;
