@@ -42,6 +42,24 @@ def test_no_further_from_64_bits_than_the_float32_instructions(kind, k, m):
         assert ((y - want).abs() / want.abs().clamp_min(1e-30)).max() <= (1 + 2 ** -5) * 2 ** -24
 
 
+# (the exponents of x and w: sums below 2^-64 of numbers that bfloat16's range ends in, of subnormal ones, of products that are subnormal, and sums above the line)
+@pytest.mark.parametrize("ex,ew", [(-100, 0), (-118, 0), (-118, 20), (-130, 0), (-70, -70), (-100, 34)])
+@pytest.mark.parametrize("n,k", [(1024, 1024), (2049, 1540)])
+def test_small_numbers(n, k, ex, ew):
+    """No further from 64 bits than the float32 instructions, the same rows in every batch, and where all sums are below the line the float32 instructions' bits."""
+    x, w = operands("normal", 130, n, k)
+    x, w = x * 2.0 ** ex, w * 2.0 ** ew
+    x[5], w[7] = 0.0, 0.0
+    step = ((1 << 20) - 1) // k
+    plain = torch.cat([product(x, w[a:a + step].contiguous(), None) for a in range(0, n, step)], 1)
+    y, want = product(x, w, None), x.double() @ w.double().t()
+    assert (y - want).norm() <= 1.01 * (plain - want).norm()
+    if -140 < ex + ew < -80:        # (below, where float32 keeps a few bits of a sum, what they are by parts may be 0, which stands)
+        assert torch.equal(y, plain)
+    for m in ROWS:
+        assert torch.equal(product(x[:m].contiguous(), w, None), y[:m]), m
+
+
 def product(x, w, bias):
     y = torch.empty((x.shape[0], w.shape[0]), dtype=torch.float32, device="cuda")
     return K.gemm(x, w, bias, y)

@@ -112,15 +112,16 @@ __device__ __forceinline__ void multiply16(floatx4_t& acc, const floatx4_t& w, c
 }
 
 // ---- large weights: a float32 number as three bfloat16 ones -----------------------------------------
-// 24 bits are 8 + 8 + 8: p the number cut off after 8 bits (so that nothing overflows), q what is left rounded to 8, t what is left then, exactly (from 2^-110 on: bfloat16
+// 24 bits are 8 + 8 + 8: p the number cut off after 8 bits (so that nothing overflows), q what is left rounded to 8, t what is left then, exactly from 2^-110 on (bfloat16
 // ends at 2^-133).  Of the nine products of two numbers' parts the smallest, t t, is left out (2^-32 of the whole); the others are exact in float32.  The matrix cores cut a sum off
 // where float32 instructions round it, so the largest products have a sum of their own, and the seven others, a 128th of it, another; the two are added at the end of a
 // chunk.  Eight bfloat16 instructions stand for eight float32 ones of twice the time each, and their sums of 32 k at once round less often: error against
 // 64 bits, 2-norm in 2^-24, K of 3584 and 18944, operands N(0, 1) 1.57 and 2.02 (the float32 instructions 3.61 and 3.82), all of one sign 0.83 and 1.18 (0.98 and 1.20), spread
 // over twelve powers of ten 1.90 and 2.49 (2.92 and 3.15), rows with one value alone 0.42 and 0.42 (0.42 and 0.42; the largest 1.0 both ways), with one 10^8 times the others 1.64 and 2.27 (1.69 and
 // 2.28).  Without q t and t q, and all in one sum, prompts took 0.87 of the time (300 rows of gate+up of the 7B shape 529 us and 601), but rows with one value had 0.67, the largest 3.9.
-// Infinities have no parts (inf - inf): a group's sum that is not finite is taken again with the float32 instructions, that one and no other, so that a result depends on
-// its own rows of x and w alone.
+// Infinities have no parts (inf - inf), and numbers below 2^-110 lose up to 2^-133 of theirs, which is less than 2^-24 of a sum from 2^-64 on unless what they meet is beyond
+// 2^30: a group's sum that is not finite, or smaller than that and not 0, is taken again with the float32 instructions, that one and no other, so that a
+// result depends on its own rows of x and w alone.  (Sums of 0 stand: rows of zeros are common.)
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 struct Parts { bf16x8_t p, q, t; };
 __device__ __forceinline__ uint32_t high_halves(float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); }
@@ -155,9 +156,11 @@ __device__ __forceinline__ void multiply32(floatx4_t& acc, floatx4_t& low, const
     low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p, x.q, low, 0, 0, 0);
     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p, x.p, acc, 0, 0, 0);
 }
-__device__ __forceinline__ bool finite(floatx4_t v) {
-    return __builtin_isfinite(v[0]) && __builtin_isfinite(v[1]) && __builtin_isfinite(v[2]) && __builtin_isfinite(v[3]);
+__device__ __forceinline__ bool stands(float v) {
+    const uint32_t twice = __float_as_uint(v) << 1;                     // (without its sign; 2^-64's exponent is 63, that of what is not finite 255)
+    return twice == 0 || twice - (63u << 24) < 192u << 24;
 }
+__device__ __forceinline__ bool stand(floatx4_t v) { return stands(v[0]) && stands(v[1]) && stands(v[2]) && stands(v[3]); }
 // The sums of a group (k_begin .. k_end) of 16 rows and 16 features by the float32 instructions, for a wave; xrow, wrow: the lane's rows.
 __device__ __forceinline__ floatx4_t plain_group(const float* xrow, const float* wrow, int k_begin, int k_end, int k4) {
     floatx4_t group = {0.f, 0.f, 0.f, 0.f};
@@ -373,10 +376,10 @@ void gemm_few_rows_apart_kernel(const float* __restrict__ x, const float* __rest
         s0 += NS;
     } while (s0 < n_stage);
     __builtin_amdgcn_s_waitcnt(0x0f70);                                 // nothing is on its way into LDS any more
-    if (__any(r16 < M && !finite(group))) {
+    if (__any(r16 < M && !stand(group))) {
         const floatx4_t plain = plain_group(x + (size_t)min(r16, M - 1) * K, w + (size_t)min(n0 + r16, N - 1) * K, k_begin, k_end, 4 * g);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) group[i] = __builtin_isfinite(group[i]) ? group[i] : plain[i];
+        for (int i = 0; i < 4; ++i) group[i] = stands(group[i]) ? group[i] : plain[i];
     }
     if (r16 >= M) return;
     const bool whole = gridDim.y == 1;
@@ -649,26 +652,29 @@ void gemm_split_kernel(const float* __restrict__ x, const float* __restrict__ w,
         }
         const int done = c0 + G_CHUNK;
         const bool end = done % G_GROUP == 0 || done >= k_end;
-        bool all_finite = true;
 #pragma unroll
         for (int f = 0; f < FT; ++f)
 #pragma unroll
             for (int a = 0; a < RT; ++a) {
                 group[f][a] += acc[f][a] + low[f][a];
                 acc[f][a] = low[f][a] = none;
-                all_finite = all_finite && finite(group[f][a]);
             }
         if (!end) continue;
-        uint32_t again = 0;                             // which of the lane's sums of the group are not finite
+        bool all_stand = true;
+#pragma unroll
+        for (int f = 0; f < FT; ++f)
+#pragma unroll
+            for (int a = 0; a < RT; ++a) all_stand = all_stand && stand(group[f][a]);
+        uint32_t again = 0;                             // which of the lane's sums of the group do not stand
         static_assert(FT * RT * 4 <= 32, "a bit each");
-        if (__any(!all_finite)) {
+        if (__any(!all_stand)) {
 #pragma unroll
             for (int f = 0; f < FT; ++f)
 #pragma unroll
                 for (int a = 0; a < RT; ++a)
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                        if (!__builtin_isfinite(group[f][a][i])) { again |= 1u << (4 * (f * RT + a) + i); group[f][a][i] = 0.f; }
+                        if (!stands(group[f][a][i])) { again |= 1u << (4 * (f * RT + a) + i); group[f][a][i] = 0.f; }
         }
 #pragma unroll
         for (int f = 0; f < FT; ++f)
