@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import helpers
-from tq_kv_amd import POLICY, Engine, Model
+from tq_kv_amd import POLICY, Engine, Model, tracing
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -149,6 +149,27 @@ def test_several_pages_and_a_window_across_them(head_dim, dtype):
     with policy(small=False):
         want = run(False)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_a_traced_step_gives_the_same_bits(dtype):
+    """With ranges on the parts run one by one, so that they show: one launch less and nothing else."""
+    model = Model.random(helpers.TINY_B, seed=3, dtype=dtype, device=DEV)
+    names, got = [], []
+    tracing.set_sink(lambda name: names.append(name.decode()), lambda: None)
+    try:
+        for on in (False, True):
+            tracing.enable(on)
+            eng = Engine(model, max_tokens=256)
+            s = eng.open()
+            got.append([eng.step([(s, helpers.random_tokens(12, helpers.TINY_B["vocab_size"], 1), [11, 0])]), eng.step([(s, [5], [0])])])
+            assert eng.n_small_steps == (0 if on else 2) and ("attn" in names) == on
+            eng.close(s)
+    finally:
+        tracing.enable(False)
+        tracing.set_sink(None, None)
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
 
 
 def test_the_estimate_picks_the_faster_way():

@@ -4,7 +4,8 @@ around the work at :43, :1957-1985).  The reference installs no subscriber, so i
 show; these show in a profiler's marker trace once switched on (`enable()`, `tq --trace`, or
 TQ_TRACE=1 in the environment) and cost one test of a flag otherwise.  A step replayed from a
 captured graph launches without passing through the parts, so only its outer range ("step")
-appears.  The ranges are the engine library's (csrc/engine/trace.cpp): they go to ROCm's ROCTx
+appears.  A small model's step in one launch would show as little: while the ranges are on it goes
+through the kernels of larger models, which give the same bits.  The ranges are the engine library's (csrc/engine/trace.cpp): they go to ROCm's ROCTx
 library, or to a pair of functions the caller installs."""
 from . import native
 
