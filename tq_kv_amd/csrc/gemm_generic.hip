@@ -118,10 +118,10 @@ __device__ __forceinline__ void multiply16(floatx4_t& acc, const floatx4_t& w, c
 // chunk.  Eight bfloat16 instructions stand for eight float32 ones of twice the time each, and their sums of 32 k at once round less often: error against
 // 64 bits, 2-norm in 2^-24, K of 3584 and 18944, operands N(0, 1) 1.57 and 2.02 (the float32 instructions 3.61 and 3.82), all of one sign 0.83 and 1.18 (0.98 and 1.20), spread
 // over twelve powers of ten 1.90 and 2.49 (2.92 and 3.15), rows with one value alone 0.42 and 0.42 (0.42 and 0.42; the largest 1.0 both ways), with one 10^8 times the others 1.64 and 2.27 (1.69 and
-// 2.28).  Without q t and t q, and all in one sum, prompts took 0.87 of the time (300 rows of gate+up of the 7B shape 529 us and 601), but rows with one value had 0.67, the largest 3.9.
+// 2.28).  Without q t and t q, and all in one sum, prompts took 0.88 of the time (300 rows of gate+up of the 7B shape 534 us and 607), but rows with one value had 0.67, the largest 3.9.
 // Infinities have no parts (inf - inf), and numbers below 2^-110 lose up to 2^-133 of theirs, which is less than 2^-24 of a sum from 2^-64 on unless what they meet is beyond
 // 2^30: a group's sum that is not finite, or smaller than that and not 0, is taken again with the float32 instructions, that one and no other, so that a
-// result depends on its own rows of x and w alone.  (Sums of 0 stand: rows of zeros are common.)
+// result depends on its own rows of x and w alone.  (Sums of 0 stand, as rows of zeros are common: where all that a row meets are numbers below 2^-133, the result is 0.)
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 struct Parts { bf16x8_t p, q, t; };
 __device__ __forceinline__ uint32_t high_halves(float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); }
@@ -179,7 +179,7 @@ __device__ __forceinline__ floatx4_t plain_group(const float* xrow, const float*
 // Up to 16 rows of x: a wave per (16 output features, one group of k).  With one group the result is finished here.
 // Bound by the weights.  They come in stages of 64 k, 256 contiguous bytes of each of the 16 rows, by loads that end in LDS, three
 // stages on their way while one is multiplied; a piece of 16 bytes lies at its number exclusive-or its row, so that the operands of 16
-// rows meet all banks.  gate+up of the 7B shape (543 MB), one row: 100 us (5.4 TB/s), eight rows 114; 131 and
+// rows meet all banks.  gate+up of the 7B shape (543 MB; products that large go by parts now, below), one row: 100 us (5.4 TB/s), eight rows 114; 131 and
 // 141 with the operands loaded as the lanes need them, 64 bytes out of 16 rows a load, eight of those under way.
 #define FEW_STAGES 4
 __global__ __launch_bounds__(TQK_WAVE)
@@ -261,8 +261,9 @@ void gemm_few_rows_kernel(const float* __restrict__ x, const float* __restrict__
 
 // The same by parts in bfloat16, for large weights.  What it spends beside its loads is taking numbers apart, 88 instructions for a stage's weights and as many for its x.
 // ROWS: up to 4, 8 or 16 rows of x.  Of the 16 lanes that hold x's rows four (two) stand for one row where there are few, each takes a quarter (half) of the row's values apart,
-// and the first gets the others' parts by turning the 16 lanes: 40 (56) instructions, and a quarter (half) of the loads.  One row, 4608, 3584 and 37888 features, K of 3584, 18944 and 3584:
-// 16.6, 61 and 102 us (17.2, 62 and 102 with the float32 instructions; 18.9, 66 and 104 without the turning).
+// and the first gets the others' parts by turning the 16 lanes: 40 (56) instructions, and a quarter (half) of the loads; without the turning it takes 1.14, 1.08 and 1.02 of the time of
+// one row, 4608, 3584 and 37888 features, K of 3584, 18944 and 3584.  Those and 152064 features, with the kernel that adds up the groups, against gemm_few_rows_kernel and one load of the groups' sums after the
+// other: 17.0, 55, 103 and 363 us (18.5, 59, 104 and 362), 8 rows 17.6, 59, 111 and 435 (19.0, 65, 113 and 446), 12 rows, the most by this kernel for some, 19.7 of 4608 (19.7).
 // TAIL: K is no multiple of 64.
 template <bool TAIL, int ROWS>
 __global__ __launch_bounds__(TQK_WAVE)
@@ -394,7 +395,7 @@ void gemm_few_rows_apart_kernel(const float* __restrict__ x, const float* __rest
 // More rows: 64 rows by 64 features a block, each of four waves 32 by 32.  Stages of 32 k go through registers into LDS, two in turn;
 // a row's 128 bytes lie 144 apart, so that the 16 rows of an operand meet all banks.  blockIdx.y: the block's share of the
 // groups; with more than one share every group's sums go to scratch on their own.  Bound by the matrix cores (157 TFLOP/s in
-// float32): gate+up of the 7B shape at 300 rows 750 us = 109 TFLOP/s (826 with the rows' tiles of some features far apart, 805 with loads one stage
+// float32): gate+up of the 7B shape at 300 rows (products that large go by parts now, below) 750 us = 109 TFLOP/s (826 with the rows' tiles of some features far apart, 805 with loads one stage
 // ahead, as a stage is hardly longer than a load takes, 855 with neither), and 2108 us through the FMA kernel above; down 465 us with the
 // groups' sums written and added (495 with neither), 40 rows 206 and 108 (229 and 111).  Blocks of 160 rows by 64 features took 967 us
 // for gate+up: fewer waves lose more than the bytes saved.
@@ -516,9 +517,9 @@ void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, c
 // memory to its own registers, which take them apart; x goes through LDS, taken apart once for the block (stages of 64 k, three parts a row of 128 bytes each, pieces of 16
 // bytes at their number exclusive-or half their row, so that the 16 rows of an operand meet all banks; two stages in turn, one barrier each).  Loads are issued
 // half a stage or a stage ahead of being taken apart, which happens beside the products of the half before.  Whole groups' sums wait in LDS too, a float4 of each thread's in turn, where
-// the registers would cost a wave per SIMD.  Bound by the matrix cores' power and by what LDS delivers of x (12 pieces a wave for 48 products: about half the time of those).  us, gate+up of the 7B
-// shape, down, q/k/v and o at 300 rows: 581, 381, 100 and 77 (820, 470, 115 and 97 with the float32 instructions); 2000 rows of o 350 (470).  Weights in whole lines in place of the
-// matrix cores' order: 4 % less, not without LDS between; waves of 48 or 64 features, one to a SIMD: 671 and 717; numbers taken apart in front of the products: 587.
+// the registers would cost a wave per SIMD.  Bound by the matrix cores' power and by what LDS delivers of x (12 pieces a wave for 64 products: two fifths of the time of those).  us, gate+up of the 7B
+// shape, down, q/k/v and o at 300 rows: 607, 406, 110 and 87 (744, 463, 114 and 98 with the float32 instructions); 2000 rows of o 380 (441).  With six products in place of eight gate+up took 581, and of that: weights in
+// whole lines in place of the matrix cores' order 0.96, not without LDS between; waves of 48 or 64 features, one to a SIMD, 1.15 and 1.23; numbers taken apart in front of the products 1.01.
 #define GS_WAVES 4
 template <int RT, int FT, bool TAIL>
 __global__ __launch_bounds__(GS_WAVES * TQK_WAVE, 2)
@@ -746,9 +747,9 @@ static bool f32_case(int x_dtype, int w_dtype, const void* bias, int bias_dtype,
 extern "C" int tqk_gemm_takes_apart(int N, int K) { return (long long)N * K >= 1 << 20; }
 
 // Tiles of 16 rows and of 16 features a wave of gemm_split_kernel takes, in blocks of four waves side by side: the largest that leaves every unit a block.  us with 64 rows by 128
-// features everywhere, and so: 300 rows of 1536 x 1536 39.0 and 25.1, 64 and 24 rows of 3584 x 3584 39.0 and 27.8, 33.5 and 25.2 (31.8, 32.1 and 31.3 with the float32 instructions).
+// features everywhere, and so: 300 rows of 1536 x 1536 43 and 27, 64 and 24 rows of 3584 x 3584 43 and 31, 40 and 26, 24 of 37888 x 3584 178 and 150 (32, 36, 35 and 185 with the float32 instructions).
 // 9 to 16 rows go there with one tile of each where that gives every unit two blocks (of whole groups): 16 rows of 37888 x 3584, 3584 x 18944, 152064 x 3584, 4608 x 3584 and 3584 x 3584
-// 124, 66, 512, 21.1 and 17.8, through the kernel for few rows 140, 77, 558, 19.7 and 16.8 (139, 76, 548, 18.8 and 16.3 with the float32 instructions).
+// 127, 62, 504, 23.3 and 21.0, through the kernel for few rows 143, 74, 538, 21.3 and 18.6 (138, 74, 538, 21.5 and 18.3 with the float32 instructions); 9 rows of the first and third 116 and 463, 119 and 461 (115 and 458).
 struct SplitTile { int rows, features; };
 static SplitTile split_tile(int M, int N, int K) {
     const int groups = (K + G_GROUP - 1) / G_GROUP;

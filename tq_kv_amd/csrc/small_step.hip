@@ -4,9 +4,9 @@
 // microsecond and costs two to four in a replayed graph, and about as much again on the host.  One block on one compute unit runs
 // the step with barriers in place of launches.  It pulls weights and does a row's work at a fraction of the chip's rate, so this is the better way only
 // while that takes no longer than the launches it stands for: tqk_small_step_pays says where that is.  Two layers of 64 values, 3 sequences after
-// 20 tokens: 22.2 us in bfloat16 and 30.2 in float32 for what a replayed graph of 21 kernels does in 65 and 81; three of 96: 34.3 and 62.5 for 76 and 110.
-// What a phase between two barriers takes (three of 96, bfloat16, us): norm 0.6 to 0.8, q/k/v 0.6, rotation 0.7, attention 2.6, o 1.2,
-// gate and up 1.5, down 1.3, none of it bytes or products but a wave's instructions one after the other, 4 and more cycles each.
+// 20 tokens, five steps asked for together: 31.6 us a step in bfloat16 and 37.6 in float32 for what a replayed graph of 21 kernels does in 75 and 87; three of 96: 38.0 and 67 for 79 and 115.
+// What a phase between two barriers takes (three of 96, bfloat16, attention by vector instructions, as other heads than those of 32 and 64 have it, us): norm 0.6 to 0.8, q/k/v 0.6, rotation 0.7,
+// attention 2.6, o 1.2, gate and up 1.5, down 1.3, none of it bytes or products but a wave's instructions one after the other, 4 and more cycles each.
 //
 // The step's rows stay in LDS: the stream h in float32, the operand of the next product (`a`: normed rows, then the attention's output),
 // and that product's result (`b`: q, k and v, then the gated values).  A wave takes tiles of 16 output features and all rows; its
