@@ -421,7 +421,7 @@ __global__ void rope_store_kernel(const TA* __restrict__ qkv, const TB* __restri
             const float y = to_float(src[partner]) + (b ? to_float(b[partner]) : 0.f);
             const float c = cos_table[(size_t)pos * half_rot + p];
             const float s = sin_table[(size_t)pos * half_rot + p];
-            x = fmaf(x, c, first ? -(y * s) : y * s);
+            x = fmaf(x, c, first ? -(y * s) : y * s);          // (fused by name, as small_step.hip has it: a plain expression's fusing changes with the code around it)
         }
         dst[(size_t)i * dst_stride] = from_float<TA>(x);
     }
