@@ -262,8 +262,11 @@ void gemm_few_rows_kernel(const float* __restrict__ x, const float* __restrict__
 // The same by parts in bfloat16, for large weights.  What it spends beside its loads is taking numbers apart, 88 instructions for a stage's weights and as many for its x.
 // ROWS: up to 4, 8 or 16 rows of x.  Of the 16 lanes that hold x's rows four (two) stand for one row where there are few, each takes a quarter (half) of the row's values apart,
 // and the first gets the others' parts by turning the 16 lanes: 40 (56) instructions, and a quarter (half) of the loads; without the turning it takes 1.14, 1.08 and 1.02 of the time of
-// one row, 4608, 3584 and 37888 features, K of 3584, 18944 and 3584.  Those and 152064 features, with the kernel that adds up the groups, against gemm_few_rows_kernel and one load of the groups' sums after the
-// other: 17.0, 55, 103 and 363 us (18.5, 59, 104 and 362), 8 rows 17.6, 59, 111 and 435 (19.0, 65, 113 and 446), 12 rows, the most by this kernel for some, 19.7 of 4608 (19.7).
+// one row, 4608, 3584 and 37888 features, K of 3584, 18944 and 3584.
+// The weights' loads say that they are read once (nt), as those of the bfloat16 kernels do: such weights are 4 MB and more, and a step reads each of them once.  Those sizes and 152064 features, with
+// the kernel that adds up the groups, weights that no cache holds, us with and without: one row 16.0, 51, 93 and 335 (17.3, 55, 100 and 376: 6.5 TB/s in place of 5.8), 8 rows
+// 17.9, 58, 105 and 428 (18.4, 62, 118 and 453); one weight of 51 to 66 MB alone over and over, which the memory-side cache holds, 13.4 and 15.0 (13.5 and 15.7), 8 rows 14.9 and 16.9 (14.2 and
+// 16.9).  gemm_few_rows_kernel's smaller weights may stay in a cache from step to step and keep plain loads (512 x 512: 6.1 us, 6.3 with the hint).
 // TAIL: K is no multiple of 64.
 template <bool TAIL, int ROWS>
 __global__ __launch_bounds__(TQK_WAVE)
@@ -298,7 +301,7 @@ void gemm_few_rows_apart_kernel(const float* __restrict__ x, const float* __rest
         const uint32_t nowhere = there ? 0u : 0x80000000u;              // (joined to the offsets, so that no branch lies here)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(w_mem, (lds_ptr_t)(buf(I) + j * 256), 16, (int)(w_at[j] | nowhere), k0 * 4, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(w_mem, (lds_ptr_t)(buf(I) + j * 256), 16, (int)(w_at[j] | nowhere), k0 * 4, 0, 2);
 #pragma unroll
         for (int u = 0; u < XU; ++u) xv[decltype(I)::value % NS][u] = *reinterpret_cast<const floatx4_t*>(xrow + min(k0 + x_place(u), K - 4));
     };
