@@ -765,15 +765,25 @@ static SplitTile split_tile(int M, int N, int K) {
 }
 
 // Into how many shares the groups are dealt for M rows: few rows, one a group; more, so that there are about four blocks a compute
-// unit (one: 280 blocks of 300 x 3584 leave most units idle while a few do a second block) and two of the larger ones that take numbers apart, no more than there are groups.
+// unit (one: 280 blocks of 300 x 3584 leave most units idle while a few do a second block), no more than there are groups.
+// Products that take numbers apart: a unit holds two blocks, and what sets the time is how many rounds of 512 there are, the last one 0.6 of a round where no unit has a second
+// block left.  Short blocks leave less of it over, so every group is a share of its own, unless blocks that walk all of K come out ahead of that with the sums that they need
+// not write and add up.  Tried with all numbers of shares, nine sizes at 17 to 1000 rows: this takes 1.005 of the best one's time (at most 1.05); two blocks a unit, which was the rule, 1.035 (us,
+// then and now: 300 and 1000 rows of 3584 x 18944 416 -> 358 and 1145 -> 991, 1000 of 1536 x 8960 282 -> 225, 500 of 4608 x 3584 178 -> 151, 64 of 37888 x 3584 207 -> 181).  768: bounds the scratch.
 static int f32_shares(int M, int N, int K) {
     const int groups = (K + G_GROUP - 1) / G_GROUP;
     if (M <= 16) return groups;
-    const bool apart = tqk_gemm_takes_apart(N, K);
-    const SplitTile t = split_tile(M, N, K);
-    const int rows = apart ? 16 * t.rows : GT, features = apart ? 64 * t.features : GT, blocks = apart ? 512 : 1024;
-    const long long tiles = (long long)((M + rows - 1) / rows) * ((N + features - 1) / features);
-    const int want = (int)(tiles >= blocks ? 1 : (blocks + tiles - 1) / tiles), per = (groups + want - 1) / want;
+    if (tqk_gemm_takes_apart(N, K)) {
+        const SplitTile t = split_tile(M, N, K);
+        const long long tiles = (long long)((M + 16 * t.rows - 1) / (16 * t.rows)) * ((N + 64 * t.features - 1) / (64 * t.features));
+        if (tiles < 400) return groups;
+        if (tiles >= 768) return 1;
+        auto rounds = [](long long blocks) { const int rest = (int)(blocks % 512); return (double)(blocks / 512) + (rest == 0 ? 0. : rest <= 256 ? 0.6 : 1.); };
+        const double us = 8 + 39. * t.rows * t.features / 8;             // of a round of single groups
+        return rounds(tiles) * (groups + 0.1) * us <= rounds(tiles * groups) * 1.1 * us + 5 + (double)groups * M * N * 8 / 4.0e6 ? 1 : groups;
+    }
+    const long long tiles = (long long)((M + GT - 1) / GT) * ((N + GT - 1) / GT);
+    const int want = (int)(tiles >= 1024 ? 1 : (1024 + tiles - 1) / tiles), per = (groups + want - 1) / want;
     return (groups + per - 1) / per;
 }
 
