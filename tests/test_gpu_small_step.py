@@ -184,3 +184,45 @@ def test_the_estimate_picks_the_faster_way():
     eng = Engine(wide, max_tokens=256)
     eng.step([(eng.open(), [1], [0])])
     assert eng.n_small_steps == 0
+
+
+# Weights through the ring in LDS: rows of an even and an odd number of 64 bytes, weights that end inside a unit of 1 KB, a ring that goes round inside a row and between layers, more and
+# fewer than 128 k, features that fill no tile; a head that does not fit (and steps that want no logits, for which it does not count).
+RING_SHAPES = {
+    "a": helpers.TINY_A, "b": helpers.TINY_B,
+    "long k": shape(144, 32, 2, 1, 16, 3, vocab=83),
+    "odd": shape(48, 80, 3, 1, 16, 3, vocab=97),
+    "small": shape(32, 32, 1, 1, 32, 5, vocab=33),
+    "heads of 64": shape(64, 96, 2, 1, 64, 2, vocab=161),
+    "no room for the head": shape(64, 160, 4, 2, 16, 2, vocab=600),
+}
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("name", list(RING_SHAPES))
+def test_decoding_steps_with_their_weights_brought_into_lds(name, dtype):
+    """1 to 13 sequences (4 and 12 are the most with a ring), some or none of their logits wanted."""
+    cfg = RING_SHAPES[name]
+    if dtype == "bfloat16" and cfg["hidden_size"] % 32:
+        pytest.skip("bfloat16 takes 32 k at a time")
+    model = Model.random(cfg, seed=7, dtype=dtype, device=DEV)
+
+    def run(always):
+        out = []
+        for n in [1, 2, 3, 4, 5, 12, 13]:
+            s = Steps(model, cfg, dtype, 64, always)
+            slots = [s.eng.open() for _ in range(n)]
+            for i, slot in enumerate(slots):
+                s([(slot, helpers.random_tokens(1 + 5 * i % 40, cfg["vocab_size"], i), [])])
+            for i in range(4):
+                tokens = helpers.random_tokens(n, cfg["vocab_size"], 50 + i)
+                out.append(s([(slot, [t], [0] if i == 3 or (i and j % 2 == 0) else []) for j, (slot, t) in enumerate(zip(slots, tokens))]))
+            s.done(slots)
+        return out
+
+    with policy(small_always=True):
+        got = run(True)
+    with policy(small=False):
+        want = run(False)
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert torch.equal(a, b), "%s, step %d" % (name, i)

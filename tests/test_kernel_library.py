@@ -141,3 +141,15 @@ def small_step(**sizes):
 def test_which_steps_the_kernel_for_small_models_takes(sizes, takes):
     lib = ctypes.CDLL(kernels.library_path())
     assert lib.tqk_small_step_takes(ctypes.byref(small_step(**sizes))) == takes
+
+
+@pytest.mark.parametrize("sizes,rings", [
+    ({"act_dtype": 0, "n_rows": 4, "n_want": 4, "n_seqs": 4}, 1), ({"act_dtype": 0, "n_rows": 5, "n_want": 5, "n_seqs": 5}, 0), ({"act_dtype": 0, "decode": 0}, 0),
+    ({"act_dtype": 0, "vocab": 256 + 64}, 1), ({"act_dtype": 0, "vocab": 512}, 0), ({"act_dtype": 0, "vocab": 512, "n_want": 0}, 1),      # the head beside down
+    ({}, 0), ({"n_heads": 3, "n_kv_heads": 1, "head_dim": 32, "hidden": 96, "inter": 224}, 1),                                        # the matrix cores' heads
+    ({"n_heads": 3, "n_kv_heads": 1, "head_dim": 32, "hidden": 96, "inter": 224, "n_rows": 12, "n_want": 12, "n_seqs": 12}, 1),
+    ({"n_heads": 3, "n_kv_heads": 1, "head_dim": 32, "hidden": 96, "inter": 224, "n_rows": 13, "n_want": 13, "n_seqs": 13}, 0)])
+def test_which_small_steps_have_their_weights_brought_into_lds(sizes, rings):
+    lib = ctypes.CDLL(kernels.library_path())
+    step = small_step(**sizes)
+    assert lib.tqk_small_step_takes(ctypes.byref(step)) and lib.tqk_small_step_rings(ctypes.byref(step)) == rings

@@ -4,14 +4,14 @@
 // microsecond and costs two to four in a replayed graph, and about as much again on the host.  One block on one compute unit runs
 // the step with barriers in place of launches.  It pulls weights and does a row's work at a fraction of the chip's rate, so this is the better way only
 // while that takes no longer than the launches it stands for: tqk_small_step_pays says where that is.  Two layers of 64 values, 3 sequences after
-// 20 tokens, five steps asked for together: 31.6 us a step in bfloat16 and 37.6 in float32 for what a replayed graph of 21 kernels does in 75 and 87; three of 96: 38.0 and 67 for 79 and 115.
+// 20 tokens, five steps asked for together: 31.6 us a step in bfloat16 and 34.1 in float32 for what a replayed graph of 21 kernels does in 75 and 87; three of 96: 36.8 and 67 for 79 and 115.
 // What a phase between two barriers takes (three of 96, bfloat16, attention by vector instructions, as other heads than those of 32 and 64 have it, us): norm 0.6 to 0.8, q/k/v 0.6, rotation 0.7,
 // attention 2.6, o 1.2, gate and up 1.5, down 1.3, none of it bytes or products but a wave's instructions one after the other, 4 and more cycles each.
 //
 // The step's rows stay in LDS: the stream h in float32, the operand of the next product (`a`: normed rows, then the attention's output),
 // and that product's result (`b`: q, k and v, then the gated values).  A wave takes tiles of 16 output features and all rows; its
 // weights come straight from memory, those of its first tile before the barrier in front of the product, so that they travel while the work
-// before it is finished.
+// before it is finished; in decoding steps of few rows out of LDS, where two waves bring them (SmallRing).
 //
 // Every sum has the order that the kernels of larger models give it, and every rounding its place, so a position's result has the same bits whichever way
 // its step went.  In float32 that is gemm_generic.hip, elementwise.hip and attention_walk.h.  In bfloat16 the order goes by the kind of step
@@ -29,10 +29,12 @@
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 #define SS_WAVES 16
 #define SS_THREADS (SS_WAVES * TQK_WAVE)
+#define SS_BRING 2              // waves that bring weights into the ring, where there is one
+#define SS_FEW 4                // rows that float32 steps with a ring have at most
 #define SS_QUERIES 4            // queries whose weights a wave keeps at a time
 #define SS_STEPS 4              // steps of k whose weights are under way together
 
@@ -119,12 +121,159 @@ struct SmallProduct {
     }
 };
 
+// Decoding steps of few rows: the weights' way into LDS.  Two waves of the block do nothing but bring them in, by loads that end there, ahead of the products.  A compute unit is served 12 to
+// 20 bytes a cycle by the second-level cache whoever asks, and where the computing waves asked, a product's barrier waited until the next one's loads had been taken.  The
+// weights lie in a ring: a layer's q/k/v, o, gate and up, down, and in the end the head, each in units of 1 KB, the ring as large as the most that is in use and on its way together.
+// Rows one after the other, their pieces of 16 bytes turned by the row (`turned`), so that the 16 rows of an operand meet different banks.
+// Cycles of one layer's phases before and now (two of 64 values, 3 rows, float32, stamps of the clock; with RingFewProduct): first norm 2160 and 1470, o 3700 and 2190, gate and up 5640 and
+// 3940, down 4370 and 3670 (what the waves that bring take then), the rest as before; the step 31.2 -> 28.3 us, three layers of 96 in bfloat16, 4 rows, 34.7 -> 32.8.
+struct SmallRing {
+    int qkv, o, gate_up, down, head, bytes;         // a weight's size in units' bytes, and the ring's
+};
+static __device__ __host__ inline SmallRing small_ring(const TqkSmallStep& p) {
+    const int size = p.act_dtype == TQK_F32 ? 4 : 2, q = p.n_heads * p.head_dim, all = (p.n_heads + 2 * p.n_kv_heads) * p.head_dim;
+    auto up = [&](long long n) { n = (n * size + 1023) / 1024 * 1024; return (int)(n < 1 << 20 ? n : 1 << 20); };
+    SmallRing r;
+    r.qkv = up((long long)all * p.hidden);
+    r.o = up((long long)p.hidden * q);
+    r.gate_up = up(2ll * p.inter * p.hidden);
+    r.down = up((long long)p.hidden * p.inter);
+    r.head = up((long long)p.vocab * p.hidden);
+    const int together[5] = {r.qkv + r.o, r.o + r.gate_up, r.gate_up + r.down, r.down + r.qkv, p.n_want > 0 ? r.down + r.head : 0};
+    r.bytes = 0;
+    for (int n : together) r.bytes = n > r.bytes ? n : r.bytes;
+    return r;
+}
+// by what a row's pieces of 16 bytes are turned (exclusive or): rows of an even number of 64 bytes by three bits
+__device__ __forceinline__ int turned(int row, int row_bytes) { return row & (row_bytes % 128 == 0 ? 7 : 3); }
+
+// a bringing wave's (number `which` of them): its units of a weight of `rows` rows into the ring from `at` on; returns the place behind the weight
+__device__ __forceinline__ int bring(const void* w, int rows, int row_bytes, char* ring, int ring_bytes, int at, int which, int lane) {
+    const int pieces = row_bytes / 16, all = rows * row_bytes;
+    const float of_pieces = 1.f / (float)pieces;
+    const __amdgpu_buffer_rsrc_t mem = __builtin_amdgcn_make_buffer_rsrc((void*)w, 0, all, 0x00020000);
+#pragma unroll 2
+    for (int unit = which * 1024; unit < all; unit += SS_BRING * 1024) {
+        const int piece = unit / 16 + lane, row = (int)(((float)piece + 0.5f) * of_pieces), from = piece ^ turned(row, row_bytes);       // (numbers this small: exact)
+        const int to = at + unit;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(mem, (lds_ptr_t)(ring + (to >= ring_bytes ? to - ring_bytes : to)), 16, from * 16, 0, 0, 0);
+    }
+    at += (all + 1023) / 1024 * 1024;
+    return at >= ring_bytes ? at - ring_bytes : at;
+}
+__device__ __forceinline__ void brought() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// SmallProduct with the weights in the ring from `at` on, by W waves; the second weight's rows N rows further on.
+template <typename T, int P, int W>
+struct RingProduct {
+    const char* ring;
+    int ring_bytes, at, N, bytes, row_tiles, lane, wave;
+
+    template <typename F>
+    __device__ __forceinline__ void run(const T* x, int ldx, int rows, F&& emit) const {
+#pragma unroll 1
+        for (int unit = wave;; unit += W) {
+            const int tile = row_tiles == 1 ? unit : unit / row_tiles, r0 = (unit - tile * row_tiles) * 16;
+            if (tile * 16 >= N) break;
+            uint32_t even[P], odd[P];
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                const int row = min(tile * 16 + lane % 16, N - 1) + p * N, turn = turned(row, bytes);
+                const uint32_t start = at + row * bytes + ((lane / 16) ^ (turn & 3)) * 16;
+                even[p] = start + (turn & 4) * 16;
+                odd[p] = start - (turn & 4) * 16;
+            }
+            floatx4_t acc[P], total[P];
+#pragma unroll
+            for (int p = 0; p < P; ++p) acc[p] = total[p] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+            const char* xr = (const char*)(x + (r0 + lane % 16) * ldx) + lane / 16 * 16;
+#pragma unroll 1
+            for (int b0 = 0; b0 < bytes; b0 += 64 * SS_STEPS) {
+                u32x4_t xv[SS_STEPS], wv[P][SS_STEPS];
+#pragma unroll
+                for (int u = 0; u < SS_STEPS; ++u) {
+                    if (b0 + 64 * u >= bytes) break;
+                    xv[u] = *reinterpret_cast<const u32x4_t*>(xr + b0 + 64 * u);
+#pragma unroll
+                    for (int p = 0; p < P; ++p) {
+                        const uint32_t to = (u % 2 ? odd[p] : even[p]) + b0 + 64 * u;
+                        wv[p][u] = *reinterpret_cast<const u32x4_t*>(ring + min(to, to - (uint32_t)ring_bytes));
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < SS_STEPS; ++u) {
+                    if (b0 + 64 * u >= bytes) break;
+#pragma unroll
+                    for (int p = 0; p < P; ++p) multiply(T(), acc[p], wv[p][u], xv[u]);
+                }
+                if (sizeof(T) == 4 && (b0 % (128 * SS_STEPS) != 0 || b0 + 64 * SS_STEPS >= bytes))
+#pragma unroll
+                    for (int p = 0; p < P; ++p) { total[p] += acc[p]; acc[p] = floatx4_t{0.f, 0.f, 0.f, 0.f}; }
+            }
+            if (r0 + lane % 16 < rows) emit(r0 + lane % 16, tile * 16 + lane / 16 * 4, sizeof(T) == 4 ? total : acc);
+        }
+    }
+};
+
+// The same for up to four rows in float32, 64 features a wave: 4 x 4 x 1 instructions, whose 16 blocks are 64 features by four rows (8 cycles a k), where 16 x 16 x 4 take
+// as long a k for 16 features.  That pays where the matrix cores are what a product waits for: gate and up (160 features of 64 k: 6100 -> 3900 cycles), the head, q/k/v; o and down have fewer tiles than
+// SIMDs and wait for a chain of sums, 12 cycles a k here and 8 there.
+// Each k enters its sum on its own, in the order that it has there: the same bits.  emit(feature, the four rows' sums[P]); x: rows that are not there may hold anything.
+template <int P, int W>
+struct RingFewProduct {
+    const char* ring;
+    int ring_bytes, at, N, bytes, lane, wave;
+
+    template <typename F>
+    __device__ __forceinline__ void run(const float* x, int ldx, F&& emit) const {
+#pragma unroll 1
+        for (int n0 = wave * 64; n0 < N; n0 += W * 64) {
+            uint32_t start[P], turn[P];
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                const int row = min(n0 + lane, N - 1) + p * N;
+                start[p] = at + row * bytes;
+                turn[p] = turned(row, bytes) * 16;
+            }
+            floatx4_t acc[P], total[P];
+#pragma unroll
+            for (int p = 0; p < P; ++p) acc[p] = total[p] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+            const float* xr = x + (lane % 4) * ldx + lane / 4;
+#pragma unroll 2
+            for (int b0 = 0; b0 < bytes; b0 += 64) {
+                const float xv = xr[b0 / 4];
+                floatx4_t wv[P][4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int p = 0; p < P; ++p) {
+                        const uint32_t to = start[p] + ((b0 + 16 * u) ^ turn[p]);
+                        wv[p][u] = *reinterpret_cast<const floatx4_t*>(ring + min(to, to - (uint32_t)ring_bytes));
+                    }
+#define FEW_K(k) _Pragma("unroll") for (int p = 0; p < P; ++p) acc[p] = __builtin_amdgcn_mfma_f32_4x4x1f32(xv, wv[p][(k) / 4][(k) % 4], acc[p], 4, k, 0);
+                FEW_K(0) FEW_K(4) FEW_K(8) FEW_K(12) FEW_K(1) FEW_K(5) FEW_K(9) FEW_K(13)
+                FEW_K(2) FEW_K(6) FEW_K(10) FEW_K(14) FEW_K(3) FEW_K(7) FEW_K(11) FEW_K(15)
+#undef FEW_K
+                if (b0 % 512 == 448 || b0 + 64 >= bytes)
+#pragma unroll
+                    for (int p = 0; p < P; ++p) { total[p] += acc[p]; acc[p] = floatx4_t{0.f, 0.f, 0.f, 0.f}; }
+            }
+            if (n0 + lane < N) emit(n0 + lane, total);
+        }
+    }
+};
+
 // How a step's rows lie in LDS, in bytes: the step's arrays, the layers' arguments, the norms' weights and the biases of all layers, the rows' angles, the waves' probabilities, then
 // the stream and the two buffers.  Rows begin 16 bytes past a multiple of the banks' width, so that the 16 rows of an operand meet different ones.
 struct SmallLayout {
     int ld_h, ld_a, ld_b, layers, norms, biases, angles, probs, squares, a, b, h, bytes;       // ld_h in floats, ld_a in T, ld_b in bytes
 };
-static __device__ __host__ inline SmallLayout small_layout(const TqkSmallStep& p) {
+// (waves: that compute, all 16 or one less beside the ring, which gets the room that few queries leave)
+static __device__ __host__ inline int queries_together(const TqkSmallStep& p, int waves) {
+    const int width = p.head_dim <= 16 ? 16 : p.head_dim <= 32 ? 32 : 64, each = (p.n_rows * p.n_heads + waves - 1) / waves;
+    return each < TQK_WAVE / width ? each : TQK_WAVE / width;
+}
+static __device__ __host__ inline SmallLayout small_layout(const TqkSmallStep& p, int waves) {
     const int size = p.act_dtype == TQK_F32 ? 4 : 2, q = p.n_heads * p.head_dim, all = (p.n_heads + 2 * p.n_kv_heads) * p.head_dim;
     const int rows = (p.n_rows + 15) / 16 * 16;
     SmallLayout l;
@@ -137,7 +286,7 @@ static __device__ __host__ inline SmallLayout small_layout(const TqkSmallStep& p
     l.biases = l.norms + up((2 * p.n_layers + 1) * p.hidden * size);
     l.angles = l.biases + up(p.n_layers * all * size);
     l.probs = l.angles + up(p.n_rows * p.head_dim * 4);
-    l.squares = l.probs + SS_WAVES * SS_QUERIES * TQK_PAGE * 4;             // (one root mean square of a row, then the squares' sums of 16 columns each, up to 16 rows)
+    l.squares = l.probs + waves * (waves == SS_WAVES ? SS_QUERIES : queries_together(p, waves)) * TQK_PAGE * 4;             // (one root mean square of a row, then the squares' sums of 16 columns each, up to 16 rows)
     l.h = l.squares + (size == 2 && p.decode && p.n_rows <= 16 ? 64 + p.hidden * 4 : 0);
     l.a = l.h + rows * l.ld_h * 4;
     l.b = l.a + up(rows * l.ld_a * size);
@@ -410,8 +559,8 @@ __device__ __forceinline__ void warm(const T* w, size_t n) {
     }
 }
 
-// D: the heads' size where the matrix cores take them (32 or 64), or 0.
-template <typename T, int D>
+// D: the heads' size where the matrix cores take them (32 or 64), or 0.  RING: one wave brings the weights into LDS (decoding steps of up to 16 rows).
+template <typename T, int D, bool RING>
 __global__ __launch_bounds__(SS_THREADS)
 void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -430,11 +579,46 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
         } else warm((const T*)p.head, (size_t)p.vocab * hidden);
         return;
     }
-    const SmallLayout at = small_layout(p);
+    constexpr int W = RING ? SS_WAVES - SS_BRING : SS_WAVES;           // waves that compute
+    const SmallLayout at = small_layout(p, W);
+    const SmallRing sizes = RING ? small_ring(p) : SmallRing{};
+    char* const ring = lds + at.bytes;
+    if (RING && wave >= W) {
+        // (the barriers are the others'.  A weight's place is asked for when what lay there is done with, in the phase before that is the longest, so that no barrier waits for a load to be asked for.)
+        int to = 0;
+        auto next = [&](const void* w, int n, int k) { to = bring(w, n, k * (int)sizeof(T), ring, sizes.bytes, to, wave - W, lane); };
+        next(p.layers[0].qkv, qkv, hidden);
+        lds_barrier();
+        lds_barrier();
+#pragma unroll 1
+        for (int layer = 0; layer < p.n_layers; ++layer) {
+            const TqkSmallLayer& l = p.layers[layer];
+            brought();
+            lds_barrier();                                      // q, k and v
+            next(l.o, hidden, qd);
+            lds_barrier();                                      // rotation
+            brought();
+            lds_barrier();                                      // attention
+            next(l.gate_up, 2 * inter, hidden);
+            lds_barrier();                                      // o
+            lds_barrier();                                      // norm
+            brought();
+            lds_barrier();                                      // gate and up
+            next(l.down, hidden, inter);
+            brought();
+            lds_barrier();                                      // down
+            if (layer + 1 < p.n_layers) next(p.layers[layer + 1].qkv, qkv, hidden);
+            else if (p.n_want > 0) next(p.head, p.vocab, hidden);
+            lds_barrier();
+        }
+        brought();
+        if (p.n_want > 0) lds_barrier();
+        return;
+    }
     int32_t* ints = reinterpret_cast<int32_t*>(lds);
     const TqkSmallLayer* layers = reinterpret_cast<const TqkSmallLayer*>(lds + at.layers);      // (the arguments lie far away)
     T *norms = reinterpret_cast<T*>(lds + at.norms), *biases = reinterpret_cast<T*>(lds + at.biases);
-    float *angles = reinterpret_cast<float*>(lds + at.angles), *probs = reinterpret_cast<float*>(lds + at.probs) + wave * SS_QUERIES * TQK_PAGE;
+    float *angles = reinterpret_cast<float*>(lds + at.angles), *probs = reinterpret_cast<float*>(lds + at.probs) + wave * (RING ? queries_together(p, W) : SS_QUERIES) * TQK_PAGE;
     float* h = reinterpret_cast<float*>(lds + at.h);
     T* a = reinterpret_cast<T*>(lds + at.a);
     char* b = lds + at.b;
@@ -442,18 +626,28 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
 
     // (bfloat16, norms divided by behind their product: the rows' inverse root mean squares and the sums of the squares of 16 columns each, [columns / 16][row])
     constexpr bool BF16 = sizeof(T) == 2;
+    constexpr bool FEW = RING && !BF16;             // (float32 has a ring for up to SS_FEW rows alone)
     const bool behind = BF16 && plan.behind;
     float *inverse = reinterpret_cast<float*>(lds + at.squares), *square_sums = inverse + 16;
 
-    auto product = [&](const void* w, int n, int k, int tiles) {
-        SmallProduct<T, 1> one = {{(const char*)w}, n, k * (int)sizeof(T), tiles, lane, wave};
-        one.ask();
-        return one;
+    // a product, its weights in the ring from `in_ring` on (which goes on behind them by `size`), or on their way to the wave from here on
+    int in_ring = 0;
+    auto product = [&](const void* w, int n, int k, int tiles, int size) {
+        if constexpr (RING) {
+            const RingProduct<T, 1, W> one = {ring, sizes.bytes, in_ring, n, k * (int)sizeof(T), tiles, lane, wave};
+            in_ring += size;
+            in_ring -= in_ring >= sizes.bytes ? sizes.bytes : 0;
+            return one;
+        } else {
+            SmallProduct<T, 1> one = {{(const char*)w}, n, k * (int)sizeof(T), tiles, lane, wave};
+            one.ask();
+            return one;
+        }
     };
-    for (int i = tid; i < p.n_ints; i += SS_THREADS) ints[i] = p.ints[i];
-    for (int i = tid * 4; i < p.n_layers * (int)sizeof(TqkSmallLayer); i += SS_THREADS * 4)
+    for (int i = tid; i < p.n_ints; i += W * TQK_WAVE) ints[i] = p.ints[i];
+    for (int i = tid * 4; i < p.n_layers * (int)sizeof(TqkSmallLayer); i += W * TQK_WAVE * 4)
         __builtin_memcpy(__builtin_assume_aligned(lds + at.layers + i, 4), reinterpret_cast<const char*>(p.layers) + i, 4);
-    for (int layer = wave; layer < p.n_layers; layer += SS_WAVES) {
+    for (int layer = wave; layer < p.n_layers; layer += W) {
         const TqkSmallLayer& l = p.layers[layer];
         for (int i = lane; i < hidden; i += TQK_WAVE) {
             norms[2 * layer * hidden + i] = ((const T*)l.norm1)[i];
@@ -461,10 +655,10 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
         }
         if (l.qkv_bias) for (int i = lane; i < qkv; i += TQK_WAVE) biases[layer * qkv + i] = ((const T*)l.qkv_bias)[i];
     }
-    for (int i = tid; i < hidden; i += SS_THREADS) norms[2 * p.n_layers * hidden + i] = ((const T*)p.final_norm)[i];
+    for (int i = tid; i < hidden; i += W * TQK_WAVE) norms[2 * p.n_layers * hidden + i] = ((const T*)p.final_norm)[i];
     lds_barrier();
     const int32_t *tokens = p.device_tokens ? p.device_tokens : ints + p.tokens, *tok_seq = ints + p.tok_seq, *tok_pos = ints + p.tok_pos;
-    for (int r = wave; r < rows; r += SS_WAVES) {
+    for (int r = wave; r < rows; r += W) {
         const int id = tokens[r], pos = min(tok_pos[r], p.max_positions - 1);
         const bool ok = id >= 0 && id < p.vocab;
         const T* row = (const T*)p.embedding + (size_t)(ok ? id : 0) * hidden;
@@ -543,7 +737,7 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
     };
     // queries a wave takes together: their elements side by side in its lanes
     const int width = d <= 16 ? 16 : d <= 32 ? 32 : 64, n_queries = rows * nh;
-    const int together = min(TQK_WAVE / width, (n_queries + SS_WAVES - 1) / SS_WAVES);
+    const int together = queries_together(p, W);
     const float of_rows = 1.f / (float)rows, of_group = 1.f / (float)(nh / nkv);
     auto quotient = [&](int n) { return __builtin_amdgcn_readfirstlane((int)(((float)n + 0.5f) * of_rows)); };         // n / rows (numbers this small: exact)
 
@@ -557,20 +751,26 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
         const TqkSmallLayer l = __builtin_bit_cast(TqkSmallLayer, words);
         const int32_t* table = ints + l.table;
         const bool last = layer == p.n_layers - 1 && p.n_last >= 0;         // (what follows the cache's rows counts for the last rows alone)
-        SmallProduct<T, 1> w_qkv = product(l.qkv, qkv, hidden, row_tiles);
-        for (int r = wave; r < rows; r += SS_WAVES) {
+        const RingFewProduct<1, W> few_qkv = {ring, sizes.bytes, in_ring, qkv, hidden * 4, lane, wave};
+        auto w_qkv = product(l.qkv, qkv, hidden, row_tiles, sizes.qkv);
+        for (int r = wave; r < rows; r += W) {
             if (BF16 && plan.first_behind) norm_behind(r, r, norms + 2 * layer * hidden, l.eps1, layer == 0 ? 1 : hidden / 16);
             else norm_row(r, r, norms + 2 * layer * hidden, l.eps1);
         }
         lds_barrier();
         float* bf = reinterpret_cast<float*>(b);
         const int ld_b = at.ld_b / 4;
-        w_qkv.run(a, at.ld_a, rows, [&](int row, int n, const floatx4_t* v) { put4(bf + row * ld_b + n, rounded<T>(divided(v[0], row, plan.first_behind))); });
+        if constexpr (FEW)
+            few_qkv.run((const float*)a, at.ld_a, [&](int n, const floatx4_t* v) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) if (r < rows) bf[r * ld_b + n] = v[0][r];
+            });
+        else w_qkv.run(a, at.ld_a, rows, [&](int row, int n, const floatx4_t* v) { put4(bf + row * ld_b + n, rounded<T>(divided(v[0], row, plan.first_behind))); });
         lds_barrier();
         // biases, rotation of q and k, keys and values into the row's page: a wave a row's heads in turn, a lane a pair that rotates together
         const int per = half <= 16 ? 4 : half <= 32 ? 2 : 1, sub = TQK_WAVE / per;      // heads a wave takes at once
 #pragma unroll 1
-        for (int e = wave; e < rows * ((nh + 2 * nkv + per - 1) / per); e += SS_WAVES) {
+        for (int e = wave; e < rows * ((nh + 2 * nkv + per - 1) / per); e += W) {
             const int heads0 = quotient(e), r = e - heads0 * rows, head = heads0 * per + lane / sub, i = lane % sub;
             if (i >= half || head >= nh + 2 * nkv) continue;
             const int pos = tok_pos[r];
@@ -606,10 +806,10 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
         if constexpr (D > 0) {
             const int group = nh / nkv;
             const size_t page_size = (size_t)TQK_PAGE * D;
-            if ((last ? plan.last_attention : plan.attention) == SMALL_ROWS) {
+            if (RING || (last ? plan.last_attention : plan.attention) == SMALL_ROWS) {          // (decoding steps: rows)
                 const int n = last ? p.n_last : rows;
 #pragma unroll 1
-                for (int e = wave; e < n * nkv; e += SS_WAVES) {
+                for (int e = wave; e < n * nkv; e += W) {
                     const int kvh = __builtin_amdgcn_readfirstlane(e / n), which = __builtin_amdgcn_readfirstlane(e - kvh * n), head0 = kvh * group;
                     const int r = __builtin_amdgcn_readfirstlane(last ? ints[p.last_rows + which] : which), pos = __builtin_amdgcn_readfirstlane(tok_pos[r]);
                     const int page = __builtin_amdgcn_readfirstlane(table[tok_seq[r] * l.width]);
@@ -627,7 +827,7 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
                     const int tiles = (n * group + 31) / 32, units = tiles * nkv;
                     const int page = __builtin_amdgcn_readfirstlane(table[seq * l.width]), end = __builtin_amdgcn_readfirstlane(tok_pos[r0]) + n;
 #pragma unroll 1
-                    for (int e = (wave - before) & (SS_WAVES - 1); e < units; e += SS_WAVES) {
+                    for (int e = (wave - before) & (SS_WAVES - 1); e < units; e += W) {
                         if (page < 0) continue;             // the host never lets this happen
                         const int kvh = __builtin_amdgcn_readfirstlane(e % nkv), col = e / nkv * 32 + lane % 32;
                         const bool live = col < n * group;
@@ -642,7 +842,7 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
             }
         } else
 #pragma unroll 1
-        for (int e0 = wave * together; e0 < n_queries; e0 += SS_WAVES * together) {
+        for (int e0 = wave * together; e0 < n_queries; e0 += W * together) {
             SmallQuery mine;                                // the query whose elements this lane's are
             float my_sum = 1.f;
             bool done = false;
@@ -695,41 +895,60 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
             }
             __builtin_amdgcn_wave_barrier();
         }
-        SmallProduct<T, 1> w_o = product(l.o, hidden, qd, row_tiles);
-        SmallProduct<T, 2> w_gate_up = {{(const char*)l.gate_up, (const char*)((const T*)l.gate_up + (size_t)inter * hidden)}, inter, hidden * (int)sizeof(T), row_tiles, lane, wave};
+        auto w_o = product(l.o, hidden, qd, row_tiles, sizes.o);
+        const RingFewProduct<2, W> few_gate_up = {ring, sizes.bytes, in_ring, inter, hidden * 4, lane, wave};
+        auto w_gate_up = [&]() {
+            if constexpr (RING) {
+                const RingProduct<T, 2, W> two = {ring, sizes.bytes, in_ring, inter, hidden * (int)sizeof(T), row_tiles, lane, wave};
+                in_ring += sizes.gate_up;
+                in_ring -= in_ring >= sizes.bytes ? sizes.bytes : 0;
+                return two;
+            } else return SmallProduct<T, 2>{{(const char*)l.gate_up, (const char*)((const T*)l.gate_up + (size_t)inter * hidden)}, inter, hidden * (int)sizeof(T), row_tiles, lane, wave};
+        }();
         lds_barrier();
         w_o.run(a, at.ld_a, rows, add_to_stream);
-        w_gate_up.ask();
+        if constexpr (!RING) w_gate_up.ask();
         lds_barrier();
-        for (int r = wave; r < rows; r += SS_WAVES) {
+        for (int r = wave; r < rows; r += W) {
             if (behind) norm_behind(r, r, norms + (2 * layer + 1) * hidden, l.eps2, hidden / 16);
             else norm_row(r, r, norms + (2 * layer + 1) * hidden, l.eps2);
         }
         lds_barrier();
         T* act = reinterpret_cast<T*>(b);
         const int ld_act = at.ld_b / (int)sizeof(T);
-        w_gate_up.run(a, at.ld_a, rows, [&](int row, int n, const floatx4_t* v) {
+        if constexpr (FEW)
+            few_gate_up.run((const float*)a, at.ld_a, [&](int n, const floatx4_t* v) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) if (r < rows) act[r * ld_act + n] = from_float<T>(gate_value(TQK_GATE_SILU, 0.f, 1.f, v[0][r], v[1][r]));
+            });
+        else w_gate_up.run(a, at.ld_a, rows, [&](int row, int n, const floatx4_t* v) {
             const floatx4_t g = rounded<T>(divided(v[0], row, behind)), u = rounded<T>(divided(v[1], row, behind));
             floatx4_t y;
 #pragma unroll
             for (int i = 0; i < 4; ++i) y[i] = gate_value(TQK_GATE_SILU, 0.f, 1.f, g[i], u[i]);
             put4(act + row * ld_act + n, y);
         });
-        SmallProduct<T, 1> w_down = product(l.down, hidden, inter, row_tiles);
+        auto w_down = product(l.down, hidden, inter, row_tiles, sizes.down);
         lds_barrier();
         w_down.run(act, ld_act, rows, add_to_stream);
         lds_barrier();
     }
 
     if (p.n_want == 0) return;
-    SmallProduct<T, 1> w_head = product(p.head, p.vocab, hidden, (p.n_want + 15) / 16);
+    const RingFewProduct<1, W> few_head = {ring, sizes.bytes, in_ring, p.vocab, hidden * 4, lane, wave};
+    auto w_head = product(p.head, p.vocab, hidden, (p.n_want + 15) / 16, sizes.head);
     const int32_t* want = ints + p.want;
-    for (int r = wave; r < p.n_want; r += SS_WAVES) {
+    for (int r = wave; r < p.n_want; r += W) {
         if (behind) norm_behind(want[r], r, norms + 2 * p.n_layers * hidden, p.final_eps, hidden / 16);
         else norm_row(want[r], r, norms + 2 * p.n_layers * hidden, p.final_eps);
     }
     lds_barrier();
-    w_head.run(a, at.ld_a, p.n_want, [&](int row, int n, const floatx4_t* v) {
+    if constexpr (FEW)
+        few_head.run((const float*)a, at.ld_a, [&](int n, const floatx4_t* v) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) if (r < p.n_want) p.logits[(size_t)r * p.vocab + n] = v[0][r];
+        });
+    else w_head.run(a, at.ld_a, p.n_want, [&](int row, int n, const floatx4_t* v) {
         const floatx4_t y = divided(v[0], row, behind);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -762,7 +981,7 @@ extern "C" int tqk_small_step_takes(const TqkSmallStep* step) {
     const int q = p.n_heads * p.head_dim, whole = 64 / size;
     if (p.hidden % whole || p.inter % whole || q % whole || (p.n_kv_heads * p.head_dim * 2) % 16) return 0;
     if ((long long)p.vocab * p.hidden * size > 0x7fffffff) return 0;          // (a weight's bytes are counted in 32 bits)
-    if (small_layout(p).bytes > 160 * 1024) return 0;
+    if (small_layout(p, SS_WAVES).bytes > 160 * 1024) return 0;
     if (p.act_dtype == TQK_BF16 && !(heads_fit(p, p.max_end) && in_order(p, p.n_rows, p.n_last >= 0 ? p.n_last : p.n_rows, p.n_want, p.decode != 0))) return 0;
     // (larger products have another order of summation there)
     if (p.act_dtype == TQK_F32 && (tqk_gemm_takes_apart(p.vocab, p.hidden) || tqk_gemm_takes_apart(2 * p.inter, p.hidden) || tqk_gemm_takes_apart(q + 2 * p.n_kv_heads * p.head_dim, p.hidden))) return 0;
@@ -803,20 +1022,38 @@ static SmallPlan small_plan(const TqkSmallStep& p) {
     return plan;
 }
 
-template <typename T, int D>
-static int launch_small(const TqkSmallStep& p, hipStream_t s) {
+template <typename T, int D, bool RING>
+static int launch_small(const TqkSmallStep& p, int lds, hipStream_t s) {
     // (a limit of each device's own: raised once for it, or a few times by threads that meet here)
     static std::atomic<uint64_t> grown{0};
     int device = 0;
     hipError_t e = hipGetDevice(&device);
     const uint64_t bit = device < 64 ? 1ull << device : 0;
     if (e == hipSuccess && !(grown.load(std::memory_order_acquire) & bit)) {
-        e = hipFuncSetAttribute((const void*)small_step_kernel<T, D>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        e = hipFuncSetAttribute((const void*)small_step_kernel<T, D, RING>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e == hipSuccess) grown.fetch_or(bit, std::memory_order_release);
     }
     if (e != hipSuccess) return tqk_fail("tqk_small_step: %s", hipGetErrorString(e));
-    small_step_kernel<T, D><<<1 + 8 * (p.n_layers + 1), SS_THREADS, small_layout(p).bytes, s>>>(p, small_plan(p));
+    small_step_kernel<T, D, RING><<<1 + 8 * (p.n_layers + 1), SS_THREADS, lds, s>>>(p, small_plan(p));
     return tqk_check_launch("tqk_small_step");
+}
+
+/* Whether a step's weights come into LDS by waves of their own: decoding steps of few rows, where the ring fits beside the rows.  us a step without and with it, steps asked
+ * for one by one: float32, two layers of 64, 1, 3, 4, 5 and 16 rows 36.5, 37.8, 37.5, 39.4, 54.0 and 33.3, 34.1, 35.8, 40.1, 57.3; bfloat16, heads of 32, three layers of 96, 1, 5, 8, 12 and 16 rows
+ * 38.2, 40.9, 42.0, 46.3, 81.5 and 36.0, 38.5, 41.3, 45.4, 81.8.  bfloat16 with other heads, whose attention every wave has a part in, loses: two layers of 64, 1, 4, 8 and 16 rows
+ * 28.1, 29.5, 33.0, 42.1 and 28.3, 29.8, 34.0, 48.1. */
+extern "C" int tqk_small_step_rings(const TqkSmallStep* step) {
+    const TqkSmallStep& p = *step;
+    const bool few = p.act_dtype == TQK_F32 ? p.n_rows <= SS_FEW : p.n_rows <= 12 && (p.head_dim == 32 || p.head_dim == 64);
+    return p.decode && few && small_layout(p, SS_WAVES - SS_BRING).bytes + small_ring(p).bytes <= 160 * 1024;
+}
+
+template <typename T, int D>
+static int launch_small(const TqkSmallStep& p, hipStream_t s) {
+    if constexpr (D > 0 || sizeof(T) == 4) {
+        if (tqk_small_step_rings(&p)) return launch_small<T, D, true>(p, small_layout(p, SS_WAVES - SS_BRING).bytes + small_ring(p).bytes, s);
+    }
+    return launch_small<T, D, false>(p, small_layout(p, SS_WAVES).bytes, s);
 }
 
 extern "C" int tqk_small_step(const TqkSmallStep* step, void* stream) {
