@@ -226,3 +226,82 @@ def test_decoding_steps_with_their_weights_brought_into_lds(name, dtype):
         want = run(False)
     for i, (a, b) in enumerate(zip(got, want)):
         assert torch.equal(a, b), "%s, step %d" % (name, i)
+
+
+PAGE_SHAPES = {
+    "heads of 4": shape(32, 32, 8, 8, 4, 2), "heads of 20": shape(48, 80, 4, 2, 20, 2, window=5), "heads of 16": shape(32, 32, 4, 2, 16, 2, window=33),
+    "heads of 48": shape(96, 96, 2, 1, 48, 2), "heads of 64": shape(64, 64, 3, 1, 64, 2, window=17), "many heads on one": shape(32, 32, 20, 1, 16, 2),
+}
+
+
+@pytest.mark.parametrize("name", list(PAGE_SHAPES))
+def test_float32_attention_within_a_page(name):
+    """Several sequences of one step, up to the page's last place and one past it; columns that fill no tile and more than one; windows."""
+    cfg = PAGE_SHAPES[name]
+    model = Model.random(cfg, seed=11, dtype="float32", device=DEV)
+
+    def run(always):
+        out = []
+        for lens in [(1,), (1, 16, 17), (33, 2), (20, 20, 24), (63,), (64,)]:
+            eng = Engine(model, max_tokens=1024)
+            slots = [eng.open() for _ in lens]
+            tok = lambda n, seed: helpers.random_tokens(n, cfg["vocab_size"], seed)
+            if sum(lens) <= 48 or cfg["head_dim"] < 64:             # (what fits the unit's LDS, which the count shows)
+                out.append(eng.step([(s, tok(n, n), list(range(n))) for s, n in zip(slots, lens)]))
+            else:
+                for s, n in zip(slots, lens):
+                    for a in range(0, n, 32):
+                        out.append(eng.step([(s, tok(n, n)[a:a + 32], [0])]))
+            for i in range(2):                                      # a chunk, then single tokens, one of them past the page
+                out.append(eng.step([(s, tok(1 + 4 * (i == 0 and n < 60), i), [0]) for s, n in zip(slots, lens)]))
+            assert (eng.n_small_steps == 0) == (not always)
+        return out
+
+    with policy(small_always=True):
+        got = run(True)
+    with policy(small=False):
+        want = run(False)
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert torch.equal(a, b), "%s, step %d: %g of the values differ, by up to %g" % (name, i, (a != b).float().mean(), (a - b).abs().max())
+
+
+@pytest.mark.parametrize("window", [None, 3])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_float32_attention_within_a_page_keeps_what_is_not_finite_to_the_columns_that_see_it(value, window):
+    """One token's embedding is not finite: every position before it, and every one whose window is past it in all layers, has the bits that it has in the other kernels."""
+    cfg = shape(32, 32, 4, 2, 16, 2, window=window)
+    if window:
+        cfg["max_window_layers"] = 0
+    weights = model_weights(cfg)
+    weights["model.embed_tokens.weight"][5] = value
+    model = Model.from_config_dict(cfg, "float32", DEV).load(weights)
+    tokens = [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17]
+
+    def run():
+        eng = Engine(model, max_tokens=256)
+        a, b = eng.open(), eng.open()
+        return eng.step([(a, tokens, list(range(17))), (b, tokens[:4], [3])])
+
+    with policy(small_always=True):
+        got = run()
+    with policy(small=False):
+        want = run()
+    assert torch.isfinite(want[:4]).all() and torch.isfinite(want[17]).all() and not torch.isfinite(want[4]).any()
+    assert torch.isfinite(want[16]).all() == bool(window)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.nan_to_num(got), torch.nan_to_num(want))
+
+
+def model_weights(cfg, seed=13):
+    """A whole model's tensors, N(0, 0.05), norms 1."""
+    g = torch.Generator().manual_seed(seed)
+    made = lambda *sizes: torch.randn(sizes, generator=g).mul_(0.05).to(DEV)
+    h, q, kv, inter = cfg["hidden_size"], cfg["num_attention_heads"] * cfg["head_dim"], cfg["num_key_value_heads"] * cfg["head_dim"], cfg["intermediate_size"]
+    out = {"model.embed_tokens.weight": made(cfg["vocab_size"], h), "model.norm.weight": torch.ones(h, device=DEV), "lm_head.weight": made(cfg["vocab_size"], h)}
+    for i in range(cfg["num_hidden_layers"]):
+        p = "model.layers.%d." % i
+        out.update({p + "input_layernorm.weight": torch.ones(h, device=DEV), p + "post_attention_layernorm.weight": torch.ones(h, device=DEV),
+                    p + "self_attn.o_proj.weight": made(h, q), p + "mlp.gate_proj.weight": made(inter, h), p + "mlp.up_proj.weight": made(inter, h), p + "mlp.down_proj.weight": made(h, inter)})
+        for name, n in (("q", q), ("k", kv), ("v", kv)):
+            out[p + "self_attn.%s_proj.weight" % name] = made(n, h)
+            out[p + "self_attn.%s_proj.bias" % name] = made(n)
+    return out

@@ -14,7 +14,7 @@
 // before it is finished; in decoding steps of few rows out of LDS, where two waves bring them (SmallRing).
 //
 // Every sum has the order that the kernels of larger models give it, and every rounding its place, so a position's result has the same bits whichever way
-// its step went.  In float32 that is gemm_generic.hip, elementwise.hip and attention_walk.h.  In bfloat16 the order goes by the kind of step
+// its step went.  In float32 that is gemm_generic.hip, elementwise.hip and attention_walk.h (within a page by the matrix cores, attend_page).  In bfloat16 the order goes by the kind of step
 // (SmallPlan): norms that are divided by behind their product in decoding steps of up to 16 rows (skinny_fused.hip), and the matrix cores' attention of
 // attention_decode.hip and attention_prefill.hip for heads of 32 and 64.  Steps with more than a page of positions for such heads, and products whose K
 // those kernels deal out to waves or cut into pieces, are left to them.
@@ -25,6 +25,7 @@
 #include "attention_walk.h"
 #include "tq_kernels.h"
 #include <atomic>
+#include <type_traits>
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
@@ -34,6 +35,7 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 #define SS_WAVES 16
 #define SS_THREADS (SS_WAVES * TQK_WAVE)
 #define SS_BRING 2              // waves that bring weights into the ring, where there is one
+#define SS_AHEAD 4              // units of 1 KB that each of them has under way besides one
 #define SS_FEW 4                // rows that float32 steps with a ring have at most
 #define SS_QUERIES 4            // queries whose weights a wave keeps at a time
 #define SS_STEPS 4              // steps of k whose weights are under way together
@@ -125,8 +127,9 @@ struct SmallProduct {
 // 20 bytes a cycle by the second-level cache whoever asks, and where the computing waves asked, a product's barrier waited until the next one's loads had been taken.  The
 // weights lie in a ring: a layer's q/k/v, o, gate and up, down, and in the end the head, each in units of 1 KB, the ring as large as the most that is in use and on its way together.
 // Rows one after the other, their pieces of 16 bytes turned by the row (`turned`), so that the 16 rows of an operand meet different banks.
-// Cycles of one layer's phases before and now (two of 64 values, 3 rows, float32, stamps of the clock; with RingFewProduct): first norm 2160 and 1470, o 3700 and 2190, gate and up 5640 and
-// 3940, down 4370 and 3670 (what the waves that bring take then), the rest as before; the step 31.2 -> 28.3 us, three layers of 96 in bfloat16, 4 rows, 34.7 -> 32.8.
+// Cycles of one layer's phases before and now (two of 64 values, 3 rows, float32, stamps of the clock; with RingFewProduct): first norm 2160 and 1390, o 3700 and 1630, gate and up 5640 and
+// 3460, down 4370 and 3200; the step 31.2 -> 28.3 us, three layers of 96 in bfloat16, 4 rows, 34.7 -> 32.8.  Each of the two has few units under way (SS_AHEAD), since what the other waves ask for waits
+// behind them (attention 9000 -> 8400 cycles), and a weight is brought in the phases that leave time for it (down's and the next q/k/v's in thirds: gate and up 3900 -> 3460, down 3670 -> 3200).
 struct SmallRing {
     int qkv, o, gate_up, down, head, bytes;         // a weight's size in units' bytes, and the ring's
 };
@@ -147,18 +150,20 @@ static __device__ __host__ inline SmallRing small_ring(const TqkSmallStep& p) {
 // by what a row's pieces of 16 bytes are turned (exclusive or): rows of an even number of 64 bytes by three bits
 __device__ __forceinline__ int turned(int row, int row_bytes) { return row & (row_bytes % 128 == 0 ? 7 : 3); }
 
-// a bringing wave's (number `which` of them): its units of a weight of `rows` rows into the ring from `at` on; returns the place behind the weight
-__device__ __forceinline__ int bring(const void* w, int rows, int row_bytes, char* ring, int ring_bytes, int at, int which, int lane) {
-    const int pieces = row_bytes / 16, all = rows * row_bytes;
+// a bringing wave's (number `which` of them): its units of a weight of `rows` rows into the ring, where the weight lies from `at` on; those of the thirds
+// from .. to - 1 of it.  Returns the place behind the weight, once it is whole.
+__device__ __forceinline__ int bring(const void* w, int rows, int row_bytes, char* ring, int ring_bytes, int at, int from, int to, int which, int lane) {
+    const int pieces = row_bytes / 16, all = rows * row_bytes, third = all / (3 * SS_BRING * 1024) * SS_BRING * 1024;
     const float of_pieces = 1.f / (float)pieces;
     const __amdgpu_buffer_rsrc_t mem = __builtin_amdgcn_make_buffer_rsrc((void*)w, 0, all, 0x00020000);
 #pragma unroll 2
-    for (int unit = which * 1024; unit < all; unit += SS_BRING * 1024) {
-        const int piece = unit / 16 + lane, row = (int)(((float)piece + 0.5f) * of_pieces), from = piece ^ turned(row, row_bytes);       // (numbers this small: exact)
-        const int to = at + unit;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(mem, (lds_ptr_t)(ring + (to >= ring_bytes ? to - ring_bytes : to)), 16, from * 16, 0, 0, 0);
+    for (int unit = from * third + which * 1024; unit < (to == 3 ? all : to * third); unit += SS_BRING * 1024) {
+        const int piece = unit / 16 + lane, row = (int)(((float)piece + 0.5f) * of_pieces), source = piece ^ turned(row, row_bytes);       // (numbers this small: exact)
+        const int place = at + unit;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(mem, (lds_ptr_t)(ring + (place >= ring_bytes ? place - ring_bytes : place)), 16, source * 16, 0, 0, 0);
+        __builtin_amdgcn_s_waitcnt(0x0f70 | SS_AHEAD);          // (no more under way: what the others ask for waits behind them)
     }
-    at += (all + 1023) / 1024 * 1024;
+    at += to == 3 ? (all + 1023) / 1024 * 1024 : 0;
     return at >= ring_bytes ? at - ring_bytes : at;
 }
 __device__ __forceinline__ void brought() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
@@ -216,7 +221,7 @@ struct RingProduct {
 };
 
 // The same for up to four rows in float32, 64 features a wave: 4 x 4 x 1 instructions, whose 16 blocks are 64 features by four rows (8 cycles a k), where 16 x 16 x 4 take
-// as long a k for 16 features.  That pays where the matrix cores are what a product waits for: gate and up (160 features of 64 k: 6100 -> 3900 cycles), the head, q/k/v; o and down have fewer tiles than
+// as long a k for 16 features.  That pays where the matrix cores are what a product waits for: gate and up (160 features of 64 k: 6100 -> 3500 cycles), the head, q/k/v; o and down have fewer tiles than
 // SIMDs and wait for a chain of sums, 12 cycles a k here and 8 there.
 // Each k enters its sum on its own, in the order that it has there: the same bits.  emit(feature, the four rows' sums[P]); x: rows that are not there may hold anything.
 template <int P, int W>
@@ -545,6 +550,117 @@ __device__ __forceinline__ void attend_columns(const float* q, const bf16_t* key
             put4(out + 32 * dt + 8 * a + 4 * h, floatx4_t{o[dt][4 * a] * inv, o[dt][4 * a + 1] * inv, o[dt][4 * a + 2] * inv, o[dt][4 * a + 3] * inv});
 }
 
+// float32, up to 16 columns (a query and a head each) of one sequence and kv head whose keys lie in one page, by the matrix cores: the sums of attention_walk.h in their order, element after
+// element in the scores and position after position in the output, which is what the instruction does with its four k (an instruction's sums are those of four fmaf).  Row i of a tile of 16 keys
+// is key 4 (i % 4) + i / 4, so that what a lane holds of the weights is its operand of the output's product.  q and out: the lane's column; lo .. pos its positions of the page; first:
+// the first position that any column sees; end: the sequence's after the step.  M: heads of up to 16 M.
+// A value that is not finite would reach columns that do not see it, by 0 times it; where there is one, the columns' outputs are worked out one by one.
+// Bound by a wave's instructions one after the other: a few hundred cycles each to look the unit up, ask for keys, multiply, weigh, sum, multiply and divide.  Cycles of the phase where every query's keys and
+// values went by vector instructions, and now (two layers of 64, 4 heads on 2 of 16): 12 queries of up to 25 positions 7900 and 6900, a prompt's 132 of up to 17 39500 and 9400; us a step with
+// queries by vector instructions and now, prompts of 8, 33 and 64 tokens 41, 93, 150 and 35, 69, 93; three layers of 96, one head of keys of 64: 94, 286 and 79, 189.
+__device__ __forceinline__ void turn_4x4(floatx4_t& v) {       // register m of lanes 16 g .. + 15 <-> register g of lanes 16 m .. + 15
+    auto swap32 = [&](int a, int b) { const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[a]), __float_as_uint(v[b]), false, false); v[a] = __uint_as_float(r[0]); v[b] = __uint_as_float(r[1]); };
+    auto swap16 = [&](int a, int b) { const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[a]), __float_as_uint(v[b]), false, false); v[a] = __uint_as_float(r[0]); v[b] = __uint_as_float(r[1]); };
+    swap32(0, 2); swap32(1, 3); swap16(0, 1); swap16(2, 3);
+}
+template <int M>
+__device__ __forceinline__ void attend_page(const float* q, const float* keys, const float* values, int d, int lo, int pos, int first, int end, float scale, float* out, bool live, int lane) {
+    const int i = lane % 16, g = lane / 16, furthest = end - 1;
+    constexpr bool AHEAD = M == 1;          // (all loads together, where the registers hold them)
+    floatx4_t k[AHEAD ? 4 : 1][M], v[4];
+    auto ask_values = [&](int row) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)             // positions 16 t + 4 g .. + 3 (value_place)
+            if (16 * t <= furthest) v[t] = *reinterpret_cast<const floatx4_t*>(values + row * TQK_PAGE + t / 2 * 32 + 8 * g + t % 2 * 4);
+    };
+    auto ask_keys = [&](int t) {
+#pragma unroll
+        for (int m = 0; m < M; ++m) k[AHEAD ? t : 0][m] = *reinterpret_cast<const floatx4_t*>(keys + (16 * t + 4 * (i % 4) + i / 4) * d + min(16 * m + 4 * g, d - 4));
+    };
+    if (AHEAD) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) if (16 * t <= furthest) ask_keys(t);
+        ask_values(min(i, d - 1));
+    }
+    float qv[4 * M];
+#pragma unroll
+    for (int m = 0; m < 4 * M; ++m) qv[m] = q[min(4 * m + g, d - 1)];
+    floatx4_t s[4];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        s[t] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+        if (16 * t <= furthest) {
+            if (!AHEAD) ask_keys(t);
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                if (16 * m >= d) break;
+                floatx4_t& of = k[AHEAD ? t : 0][m];
+                turn_4x4(of);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (16 * m + 4 * e < d) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(of[e], qv[4 * m + e], s[t], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        if (16 * t > furthest) break;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int j = 16 * t + 4 * r + g;
+            s[t][r] = j >= lo && j <= pos ? s[t][r] * scale : -INFINITY;
+            mx = fmaxf(mx, s[t][r]);
+        }
+    }
+    float2 both = with_lane_32(mx);
+    mx = fmaxf(both.x, both.y);
+    both = with_lane_16(mx);
+    mx = fmaxf(both.x, both.y);
+    const float from = from_max(mx);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        if (16 * t > furthest) break;               // (nothing there: they are 0)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[t][r] = expf(s[t][r] - from);         // (a position that is not seen: exp(-inf) = 0)
+    }
+    // their sum as wave_sum has it: positions 32 apart first, then 16, 8, 4, 2 and 1
+    const floatx4_t sums = (s[0] + s[2]) + (s[1] + s[3]);
+    float sum = (sums[0] + sums[2]) + (sums[1] + sums[3]);
+    both = with_lane_32(sum);
+    sum = both.x + both.y;
+    both = with_lane_16(sum);
+    sum = both.x + both.y;
+#pragma unroll 1
+    for (int e0 = 0; e0 < d; e0 += 16) {
+        if (!AHEAD || e0 > 0) ask_values(min(e0 + i, d - 1));
+        // (one: the column whose output is worked out alone; -1, all of them)
+#pragma unroll 1
+        for (int one = -1; one < 16; ++one) {
+            const int from_j = one < 0 ? first : __builtin_amdgcn_readlane(lo, one), to_j = one < 0 ? end : __builtin_amdgcn_readlane(pos, one) + 1;
+            floatx4_t o = {0.f, 0.f, 0.f, 0.f};
+            uint32_t largest = 0;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                if (16 * t > furthest) break;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int j = 16 * t + 4 * g + e;
+                    v[t][e] = j >= from_j && j < to_j ? v[t][e] : 0.f;
+                    largest = max(largest, __float_as_uint(v[t][e]) & 0x7fffffffu);
+                }
+                turn_4x4(v[t]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][r], s[t][r], o, 0, 0, 0);
+            }
+            const bool again = one < 0 && __any(largest >= 0x7f800000u);
+            if (live && !again && (one < 0 || one == i) && e0 + 4 * g < d) put4(out + e0 + 4 * g, floatx4_t{o[0] / sum, o[1] / sum, o[2] / sum, o[3] / sum});
+            if (one < 0 && !again) break;
+            ask_values(min(e0 + i, d - 1));
+        }
+    }
+}
+
 // The weights' way into the second-level cache of the die that runs the step: block 0 alone would wait for memory at every product.  Blocks are dealt to
 // the eight dies in turn, so those whose number is a multiple of 8 read a layer's weights each (where they run elsewhere, nothing is lost but
 // the time saved).
@@ -559,7 +675,7 @@ __device__ __forceinline__ void warm(const T* w, size_t n) {
     }
 }
 
-// D: the heads' size where the matrix cores take them (32 or 64), or 0.  RING: one wave brings the weights into LDS (decoding steps of up to 16 rows).
+// D: the heads' size where the matrix cores take them (bfloat16: 32 or 64; float32, where the step lies in one page: up to 16, 32 or 64), or 0.  RING: one wave brings the weights into LDS (decoding steps of up to 16 rows).
 template <typename T, int D, bool RING>
 __global__ __launch_bounds__(SS_THREADS)
 void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
@@ -584,35 +700,39 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
     const SmallRing sizes = RING ? small_ring(p) : SmallRing{};
     char* const ring = lds + at.bytes;
     if (RING && wave >= W) {
-        // (the barriers are the others'.  A weight's place is asked for when what lay there is done with, in the phase before that is the longest, so that no barrier waits for a load to be asked for.)
+        // (the barriers are the others'.  A weight's place is free once what lay there is done with, and its units are dealt to the phases so that no barrier waits for loads to be asked for.)
         int to = 0;
-        auto next = [&](const void* w, int n, int k) { to = bring(w, n, k * (int)sizeof(T), ring, sizes.bytes, to, wave - W, lane); };
-        next(p.layers[0].qkv, qkv, hidden);
+        auto next = [&](const void* w, int n, int k, int from_third, int to_third) { to = bring(w, n, k * (int)sizeof(T), ring, sizes.bytes, to, from_third, to_third, wave - W, lane); };
+        next(p.layers[0].qkv, qkv, hidden, 0, 3);
         lds_barrier();
         lds_barrier();
 #pragma unroll 1
         for (int layer = 0; layer < p.n_layers; ++layer) {
             const TqkSmallLayer& l = p.layers[layer];
+            if (layer > 0) next(l.qkv, qkv, hidden, 2, 3);
             brought();
             lds_barrier();                                      // q, k and v
-            next(l.o, hidden, qd);
+            next(l.o, hidden, qd, 0, 3);
             lds_barrier();                                      // rotation
             brought();
             lds_barrier();                                      // attention
-            next(l.gate_up, 2 * inter, hidden);
+            next(l.gate_up, 2 * inter, hidden, 0, 3);
             lds_barrier();                                      // o
             lds_barrier();                                      // norm
+            next(l.down, hidden, inter, 0, 1);
             brought();
             lds_barrier();                                      // gate and up
-            next(l.down, hidden, inter);
+            next(l.down, hidden, inter, 1, 3);
             brought();
             lds_barrier();                                      // down
-            if (layer + 1 < p.n_layers) next(p.layers[layer + 1].qkv, qkv, hidden);
-            else if (p.n_want > 0) next(p.head, p.vocab, hidden);
+            if (layer + 1 < p.n_layers) next(p.layers[layer + 1].qkv, qkv, hidden, 0, 2);
+            else if (p.n_want > 0) next(p.head, p.vocab, hidden, 0, 2);
             lds_barrier();
         }
+        if (p.n_want == 0) return;
+        next(p.head, p.vocab, hidden, 2, 3);
         brought();
-        if (p.n_want > 0) lds_barrier();
+        lds_barrier();
         return;
     }
     int32_t* ints = reinterpret_cast<int32_t*>(lds);
@@ -741,6 +861,25 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
     const float of_rows = 1.f / (float)rows, of_group = 1.f / (float)(nh / nkv);
     auto quotient = [&](int n) { return __builtin_amdgcn_readfirstlane((int)(((float)n + 0.5f) * of_rows)); };         // n / rows (numbers this small: exact)
 
+    // float32, steps of one page: units of up to 16 columns of a sequence and kv head, a wave each; a lane knows a sequence's first row, rows, first position and the units up to its end
+    int my_r0 = 0, my_n = 0, my_start = 0, units_to = 0, n_units = 0;
+    if constexpr (!BF16 && D > 0) {
+        if (lane < p.n_seqs) {
+            my_r0 = ints[p.seq_first + lane];
+            my_n = ints[p.seq_first + lane + 1] - my_r0;
+            my_start = tok_pos[my_r0];
+            units_to = (my_n * (nh / nkv) + 15) / 16 * nkv;
+        }
+        auto add = [&](auto ctrl, auto rows_of) { units_to += __builtin_amdgcn_update_dpp(0, units_to, decltype(ctrl)::value, decltype(rows_of)::value, 0xf, true); };
+        add(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});          // 1, 2, 4 and 8 lanes before, then the last lanes of 16 and of 32
+        add(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+        add(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+        add(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+        add(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});
+        add(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+        n_units = __builtin_amdgcn_readlane(units_to, 63);
+    }
+
 #pragma unroll 1
     for (int layer = 0; layer < p.n_layers; ++layer) {
         // this layer's arguments, the same for all lanes
@@ -803,7 +942,7 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
             dst[(size_t)(i + half) * stride] = from_float<T>(hi);
         }
         __syncthreads();                                    // (keys and values are read back out of memory)
-        if constexpr (D > 0) {
+        if constexpr (D > 0 && BF16) {
             const int group = nh / nkv;
             const size_t page_size = (size_t)TQK_PAGE * D;
             if (RING || (last ? plan.last_attention : plan.attention) == SMALL_ROWS) {          // (decoding steps: rows)
@@ -839,6 +978,23 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
                     }
                     before += units;
                 }
+            }
+        } else if constexpr (D > 0) {
+            int at_lane = lane;
+            asm volatile("" : "+v"(at_lane));               // (what follows from it is not held in registers across the layers)
+            const int group = nh / nkv;
+#pragma unroll 1
+            for (int e = wave; e < n_units; e += W) {
+                const int seq = __builtin_popcountll(__ballot(units_to <= e)), before = seq > 0 ? __builtin_amdgcn_readlane(units_to, seq - 1) : 0;
+                const int r0 = __builtin_amdgcn_readlane(my_r0, seq), n = __builtin_amdgcn_readlane(my_n, seq), tiles = (n * group + 15) / 16;
+                const int kvh = __builtin_amdgcn_readfirstlane((int)(((float)(e - before) + 0.5f) / (float)tiles)), c = (e - before - kvh * tiles) * 16 + at_lane % 16, col = min(c, n * group - 1);
+                const int of_group_ = (int)(((float)col + 0.5f) / (float)n), r = r0 + col - of_group_ * n, head = kvh * group + of_group_;
+                const int page = __builtin_amdgcn_readfirstlane(table[seq * l.width]), start = __builtin_amdgcn_readlane(my_start, seq);
+                if (page < 0) continue;                     // the host never lets this happen
+                const int pos = start + r - r0, lo = l.window > 0 ? max(0, pos - l.window + 1) : 0, first = l.window > 0 ? max(0, start - l.window + 1) : 0;
+                const size_t base = ((size_t)page * nkv + kvh) * TQK_PAGE * d;
+                attend_page<D / 16>(bf + r * ld_b + head * d, (const float*)l.keys + base, (const float*)l.values + base, d, lo, pos, first, start + n, l.scale, (float*)a + r * at.ld_a + head * d,
+                                    c < n * group, at_lane);
             }
         } else
 #pragma unroll 1
@@ -993,16 +1149,18 @@ extern "C" int tqk_small_step_takes(const TqkSmallStep* step) {
  * its products, its other work and its heads' pages take; the head's weights at 39 KB.  The other kernels, ten launches a layer: 20 a layer in a graph (33 in float32) and 32 (45) one by one.
  * Measured, one block and the other kernels, two layers of 64 values with 160 in the feed-forward, bfloat16: 1, 16 and 40 sequences 31 and 72, 65 and 79, 92 and 88, prompts of 8, 33
  * and 64 tokens 31 and 96, 61 and 96, 109 and 97; three of 96 with 224 and heads of 32: 47 and 73, 75 and 82, 108 and 97, then 35 and 132, 70 and 134, 95 and 135; with heads of 64: 66 and 78, 87
- * and 83, 156 and 106, then 43 and 132, 87 and 137, 133 and 137; four of 128 with 224: 69 and 83, 94 and 88, 207 and 122, then 55 and 175, 126 and 179, 175 and 179.  float32, two of 64: 35 and 81, 74 and
- * 85, 125 and 111, then 36 and 100, 88 and 102, 145 and 103; three of 96: 62 and 108, 113 and 113, 249 and 152, then 69 and 132, 192 and 138, 306 and 147; four of 128 with 512: 159 and 146, 313 and 154,
- * then 171 and 173. */
+ * and 83, 156 and 106, then 43 and 132, 87 and 137, 133 and 137; four of 128 with 224: 69 and 83, 94 and 88, 207 and 122, then 55 and 175, 126 and 179, 175 and 179.  float32, two of 64: 1, 4, 16 and 40 sequences 32 and 83, 33 and 86, 55 and 88, 115 and 114, prompts of 8, 33 and 64 tokens 35 and 92, 69 and 99, 93 and 106; three of 96 67 and 111, 67 and 113,
+ * 87 and 116, 195 and 156, then 65 and 118, 147 and 142, 199 and 150; with heads of 64 82 and 112, 83 and 114, 111 and 117, 257 and 166, then 79 and 118, 189 and 149; four of 128 with 512: 156 and 147,
+ * 161 and 150, 210 and 153, then 154 and 154. */
 extern "C" int tqk_small_step_pays(const TqkSmallStep* step, int n_rows, int decode, int positions) {
     const TqkSmallStep& p = *step;
     const bool f32 = p.act_dtype == TQK_F32;
     if (!f32 && !(heads_fit(p, positions) && in_order(p, n_rows, n_rows, n_rows, decode != 0))) return 0;         // (what the kernel does not take)
     const double size = f32 ? 4 : 2, q = (double)p.n_heads * p.head_dim;
     const double thousands = 1e-3 * p.hidden * (2 * q + 2. * p.n_kv_heads * p.head_dim + 3. * p.inter);            // weights of a layer
-    const double a_row = 0.15 + (f32 ? 0.0115 : 0.0043) * thousands + 0.08 * p.n_heads * ((positions + TQK_PAGE - 1) / TQK_PAGE);
+    const double heads = 0.08 * p.n_heads * ((positions + TQK_PAGE - 1) / TQK_PAGE);
+    // (float32 within a page: columns of a sequence share an instruction in prompts)
+    const double a_row = f32 && positions <= TQK_PAGE ? 0.15 + 0.0085 * thousands + (decode ? heads : 0) : 0.15 + (f32 ? 0.0115 : 0.0043) * thousands + heads;
     const double here = 8 + p.n_layers * (5 + thousands * size / (f32 ? 27 : 33) + n_rows * a_row) + 1e-3 * p.vocab * p.hidden * size / 39;
     const double there = decode ? 15 + p.n_layers * (f32 ? 33 : 20) : 15 + p.n_layers * (f32 ? 45 : 32);
     return here < there;
@@ -1072,6 +1230,11 @@ extern "C" int tqk_small_step(const TqkSmallStep* step, void* stream) {
                     p.seq_first + p.n_seqs + 1 <= p.n_ints && (p.n_last < 0 || (p.last_rows >= 0 && p.last_rows + p.n_last <= p.n_ints)) &&
                     (p.device_tokens || (p.tokens >= 0 && p.tokens + p.n_rows <= p.n_ints)), "tqk_small_step: the step's arrays do not lie in what was given");
     hipStream_t s = (hipStream_t)stream;
-    if (p.act_dtype == TQK_F32) return launch_small<float, 0>(p, s);
+    if (p.act_dtype == TQK_F32) {
+        // (one or two rows of large heads: a query a wave is faster, since loads of up to 16 elements of a head alone are asked for together here; us a step, three layers of 96, three heads of
+        // 32 and of 64, one row 64 and 76, 67 and 82 here, four rows 68 and 86, 67 and 83 here)
+        if (p.max_end > TQK_PAGE || (p.head_dim > 16 && p.n_rows * p.n_heads <= 6)) return launch_small<float, 0>(p, s);
+        return p.head_dim <= 16 ? launch_small<float, 16>(p, s) : p.head_dim <= 32 ? launch_small<float, 32>(p, s) : launch_small<float, 64>(p, s);
+    }
     return p.head_dim == 32 ? launch_small<bf16_t, 32>(p, s) : p.head_dim == 64 ? launch_small<bf16_t, 64>(p, s) : launch_small<bf16_t, 0>(p, s);
 }
