@@ -7,6 +7,7 @@ logits (src/models/turbo_generic.rs:1950-1987) and its per-request state is one 
 tokens (whole prompts, or one token each, or anything between), runs exactly those tokens against
 what the cache holds, and returns the logits at the wanted places.
 """
+import array
 import ctypes
 
 import numpy as np
@@ -17,13 +18,17 @@ from ..cache.store import Cache
 from ..native import StepError
 
 
+_PLAIN = {int, np.int32, np.int64}
+
+
 def _int32(values):
-    """What does not fit 32 bits becomes the ends of what does, which no step accepts either."""
-    try:
-        out = np.asarray(values, dtype=np.int32)        # (a fifth of the time of the way by 64 bits)
-    except OverflowError:
-        out = np.asarray(values, dtype=np.int64).clip(-1, 2 ** 31 - 1).astype(np.int32)
-    return np.maximum(out, -1, out=out)
+    """A list in the library's 32 bits.  What does not fit becomes the ends of what does, which no step accepts either."""
+    if _PLAIN.issuperset(map(type, values)):
+        try:                    # (two fifths of the time of the way by 64 bits; array refuses what does not fit, as casts of arrays and tensors do not)
+            return np.maximum(np.array(array.array("i", values), dtype=np.int32), -1)
+        except OverflowError:
+            pass
+    return np.asarray(values, dtype=np.int64).clip(-1, 2 ** 31 - 1).astype(np.int32)
 
 
 class Engine:
