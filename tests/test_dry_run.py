@@ -12,6 +12,15 @@ from tq_kv_amd import Engine, GenerationParams, Model, generate
 from tq_kv_amd.cache import PAGE, CacheFull
 
 
+@pytest.mark.parametrize("want", [[0, 2], [[0], [2]], [[0, 1], [2, 0]], torch.tensor([[0, 1], [2, 0]])])
+def test_a_step_returns_a_row_for_each_wanted_entry(want):
+    """Two entries each; the library writes two rows, however many numbers an entry has."""
+    cfg, seed = helpers.CONFIGS["A"]
+    engine = Engine(Model.random(cfg, seed=seed, dtype="float32", device="cpu"), max_tokens=4 * PAGE)
+    for borrow in (False, True):
+        assert tuple(engine.step([(engine.open(), [1, 2, 3], want)], borrow=borrow).shape) == (2, cfg["vocab_size"])
+
+
 @pytest.mark.parametrize("name", sorted(helpers.CONFIGS))
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_steps_and_generation_on_the_null_device(name, dtype):

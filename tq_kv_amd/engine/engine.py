@@ -110,7 +110,7 @@ class Engine:
             dev_ptr = ctypes.c_void_p(device_tokens.data_ptr())
         else:                       # ids too large for the library's int32 stay too large for any vocabulary
             flat = _int32([t for _, tokens, _ in items for t in tokens])
-        n_want = want_idx.size
+        n_want = sum(len(want) for _, _, want in items)            # (as many rows as the library writes)
         kept = ctypes.c_void_p(0)
         logits = None
         if not borrow:
