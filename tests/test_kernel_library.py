@@ -153,3 +153,21 @@ def test_which_small_steps_have_their_weights_brought_into_lds(sizes, rings):
     lib = ctypes.CDLL(kernels.library_path())
     step = small_step(**sizes)
     assert lib.tqk_small_step_takes(ctypes.byref(step)) and lib.tqk_small_step_rings(ctypes.byref(step)) == rings
+
+
+# heads, kv heads, head_dim; the sequences' new tokens; whether they are single tokens
+@pytest.mark.parametrize("heads,rows,decode,pages", [
+    ((4, 2, 16), [1] * 3, 1, 1), ((4, 2, 16), [1] * 16, 1, 0), ((4, 2, 16), [33], 0, 1), ((4, 4, 16), [1] * 4, 1, 0), ((4, 1, 16), [1] * 40, 1, 1),
+    ((8, 8, 4), [1] * 2, 1, 0), ((8, 8, 4), [1] * 16, 1, 0), ((8, 8, 4), [2] * 16, 0, 0), ((8, 8, 4), [15, 15, 15], 0, 1),
+    ((2, 1, 32), [1], 1, 0), ((2, 1, 32), [8], 0, 1), ((4, 2, 32), [1], 1, 0), ((4, 2, 20), [1] * 16, 1, 0), ((8, 2, 32), [1] * 4, 1, 1),
+    ((1, 1, 64), [1] * 40, 1, 0), ((1, 1, 64), [5], 0, 0), ((1, 1, 64), [16], 0, 1), ((4, 2, 64), [1], 1, 0), ((4, 2, 64), [1] * 4, 1, 1), ((3, 3, 64), [1] * 8, 1, 0)])
+def test_which_float32_small_steps_have_their_attention_by_units_of_columns(heads, rows, decode, pages):
+    """Steps within a page: by units where these are few beside the queries (the same bits either way, tests/test_gpu_small_step.py)."""
+    lib = ctypes.CDLL(kernels.library_path())
+    n_heads, n_kv, d = heads
+    step = small_step(act_dtype=0, n_heads=n_heads, n_kv_heads=n_kv, head_dim=d, n_rows=sum(rows), n_want=1, n_seqs=len(rows), decode=decode, max_end=64, seq_first=10)
+    for i in range(len(rows) + 1):
+        step.ints[10 + i] = sum(rows[:i])
+    assert lib.tqk_small_step_takes(ctypes.byref(step)) and lib.tqk_small_step_pages(ctypes.byref(step)) == pages
+    step.max_end = 65
+    assert lib.tqk_small_step_pages(ctypes.byref(step)) == 0

@@ -1206,6 +1206,28 @@ extern "C" int tqk_small_step_rings(const TqkSmallStep* step) {
     return p.decode && few && small_layout(p, SS_WAVES - SS_BRING).bytes + small_ring(p).bytes <= 160 * 1024;
 }
 
+/* Whether a float32 step within a page has its attention by the matrix cores, in units of up to 16 columns of a sequence and kv head (attend_page), and not a query a
+ * wave: where the waves' units are few beside their queries.  Heads of up to 16: a wave's turn of units takes as long as one and a half of four queries.  Larger heads: 16 lanes of a
+ * unit's loads read one row of 16 elements each, a query's read whole rows, so that a query of d elements costs a wave d and the unit's served bytes set the rest: a turn 9 d and each unit 50.  us a
+ * step, queries and units, two layers; three, 16 and 40 sequences, four heads of 16 on two 32.3 and 30.9 (units), 54 and 56, 109 and 117 (queries), on four 32.7 and 32.9, 56 and 76, 112 and 168
+ * (queries but for the first), on one 32.2 and 29.1, 54 and 46, 107 and 89 (units); 16 sequences, eight heads of 4 57 and 102 (queries); one, four and 16 sequences, four heads of 32 on two 32.5 and
+ * 33.3, 39.4 and 38.0, 71 and 69 (queries), eight on two 40.0 and 40.7 (queries), 51.6 and 44.3, 102 and 70 (units), one head of 64 30.4 and 35.7, 34.4 and 38.2, 52 and 60 (queries), four on two
+ * 58 and 64 (queries), 71.5 and 69.7, 122 and 109 (units); prompts of 16 and 63 tokens, four heads of 16 on two 48 and 37, 149 and 92, one head of 64 45 and 39, 150 and 92 (units).  Of
+ * 649 steps of 20 shapes with heads of 4 to 64 the chosen way takes 1.003 of the faster one's time, 1.14 at most. */
+extern "C" int tqk_small_step_pages(const TqkSmallStep* step) {
+    const TqkSmallStep& p = *step;
+    if (p.act_dtype != TQK_F32 || p.max_end > TQK_PAGE || p.seq_first < 0 || p.n_seqs < 1 || p.seq_first + p.n_seqs + 1 > TQK_SMALL_INTS) return 0;
+    const int waves = tqk_small_step_rings(&p) ? SS_WAVES - SS_BRING : SS_WAVES, group = p.n_heads / p.n_kv_heads, queries = p.n_rows * p.n_heads;
+    int units = 0;
+    for (const int32_t* first = p.ints + p.seq_first, *end = first + p.n_seqs; first < end; ++first) units += ((first[1] - first[0]) * group + 15) / 16 * p.n_kv_heads;
+    const int turns = (units + waves - 1) / waves;
+    if (p.head_dim <= 16) {
+        const int together = waves * queries_together(p, waves);
+        return 2 * turns < 3 * ((queries + together - 1) / together);
+    }
+    return queries * p.head_dim >= 50 * units + 9 * turns * p.head_dim;
+}
+
 template <typename T, int D>
 static int launch_small(const TqkSmallStep& p, hipStream_t s) {
     if constexpr (D > 0 || sizeof(T) == 4) {
@@ -1231,9 +1253,7 @@ extern "C" int tqk_small_step(const TqkSmallStep* step, void* stream) {
                     (p.device_tokens || (p.tokens >= 0 && p.tokens + p.n_rows <= p.n_ints)), "tqk_small_step: the step's arrays do not lie in what was given");
     hipStream_t s = (hipStream_t)stream;
     if (p.act_dtype == TQK_F32) {
-        // (one or two rows of large heads: a query a wave is faster, since loads of up to 16 elements of a head alone are asked for together here; us a step, three layers of 96, three heads of
-        // 32 and of 64, one row 64 and 76, 67 and 82 here, four rows 68 and 86, 67 and 83 here)
-        if (p.max_end > TQK_PAGE || (p.head_dim > 16 && p.n_rows * p.n_heads <= 6)) return launch_small<float, 0>(p, s);
+        if (!tqk_small_step_pages(&p)) return launch_small<float, 0>(p, s);
         return p.head_dim <= 16 ? launch_small<float, 16>(p, s) : p.head_dim <= 32 ? launch_small<float, 32>(p, s) : launch_small<float, 64>(p, s);
     }
     return p.head_dim == 32 ? launch_small<bf16_t, 32>(p, s) : p.head_dim == 64 ? launch_small<bf16_t, 64>(p, s) : launch_small<bf16_t, 0>(p, s);

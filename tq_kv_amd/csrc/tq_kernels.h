@@ -654,6 +654,7 @@ typedef struct {
 int tqk_small_step_takes(const TqkSmallStep* step);
 int tqk_small_step_pays(const TqkSmallStep* step, int n_rows, int decode, int positions);
 int tqk_small_step_rings(const TqkSmallStep* step);
+int tqk_small_step_pages(const TqkSmallStep* step);
 int tqk_small_step(const TqkSmallStep* step, void* stream);
 
 #ifdef __cplusplus
