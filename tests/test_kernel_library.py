@@ -157,7 +157,7 @@ def test_which_small_steps_have_their_weights_brought_into_lds(sizes, rings):
 
 # heads, kv heads, head_dim; the sequences' new tokens; whether they are single tokens
 @pytest.mark.parametrize("heads,rows,decode,pages", [
-    ((4, 2, 16), [1] * 3, 1, 1), ((4, 2, 16), [1] * 16, 1, 0), ((4, 2, 16), [33], 0, 1), ((4, 4, 16), [1] * 4, 1, 0), ((4, 1, 16), [1] * 40, 1, 1),
+    ((4, 2, 16), [1] * 2, 1, 1), ((4, 2, 16), [1] * 16, 1, 0), ((4, 2, 16), [33], 0, 1), ((4, 4, 16), [1] * 4, 1, 0), ((5, 5, 16), [1] * 2, 1, 0), ((4, 1, 16), [1] * 40, 1, 1),
     ((8, 8, 4), [1] * 2, 1, 0), ((8, 8, 4), [1] * 16, 1, 0), ((8, 8, 4), [2] * 16, 0, 0), ((8, 8, 4), [15, 15, 15], 0, 1),
     ((2, 1, 32), [1], 1, 0), ((2, 1, 32), [8], 0, 1), ((4, 2, 32), [1], 1, 0), ((4, 2, 20), [1] * 16, 1, 0), ((8, 2, 32), [1] * 4, 1, 1),
     ((1, 1, 64), [1] * 40, 1, 0), ((1, 1, 64), [5], 0, 0), ((1, 1, 64), [16], 0, 1), ((4, 2, 64), [1], 1, 0), ((4, 2, 64), [1] * 4, 1, 1), ((3, 3, 64), [1] * 8, 1, 0)])

@@ -1196,36 +1196,35 @@ static int launch_small(const TqkSmallStep& p, int lds, hipStream_t s) {
     return tqk_check_launch("tqk_small_step");
 }
 
-/* Whether a step's weights come into LDS by waves of their own: decoding steps of few rows, where the ring fits beside the rows.  us a step without and with it, steps asked
- * for one by one: float32, two layers of 64, 1, 3, 4, 5 and 16 rows 36.5, 37.8, 37.5, 39.4, 54.0 and 33.3, 34.1, 35.8, 40.1, 57.3; bfloat16, heads of 32, three layers of 96, 1, 5, 8, 12 and 16 rows
- * 38.2, 40.9, 42.0, 46.3, 81.5 and 36.0, 38.5, 41.3, 45.4, 81.8.  bfloat16 with other heads, whose attention every wave has a part in, loses: two layers of 64, 1, 4, 8 and 16 rows
- * 28.1, 29.5, 33.0, 42.1 and 28.3, 29.8, 34.0, 48.1. */
-extern "C" int tqk_small_step_rings(const TqkSmallStep* step) {
-    const TqkSmallStep& p = *step;
-    const bool few = p.act_dtype == TQK_F32 ? p.n_rows <= SS_FEW : p.n_rows <= 12 && (p.head_dim == 32 || p.head_dim == 64);
-    return p.decode && few && small_layout(p, SS_WAVES - SS_BRING).bytes + small_ring(p).bytes <= 160 * 1024;
+// Units of a float32 step's attention: up to 16 columns (a query and a head each) of a sequence and kv head.
+static int attention_units(const TqkSmallStep& p) {
+    int units = 0;
+    for (const int32_t *first = p.ints + p.seq_first, *end = first + p.n_seqs; first < end; ++first)
+        units += ((first[1] - first[0]) * (p.n_heads / p.n_kv_heads) + 15) / 16 * p.n_kv_heads;
+    return units;
 }
-
-/* Whether a float32 step within a page has its attention by the matrix cores, in units of up to 16 columns of a sequence and kv head (attend_page), and not a query a
- * wave: where the waves' units are few beside their queries.  Heads of up to 16: a wave's turn of units takes as long as one and a half of four queries.  Larger heads: 16 lanes of a
- * unit's loads read one row of 16 elements each, a query's read whole rows, so that a query of d elements costs a wave d and the unit's served bytes set the rest: a turn 9 d and each unit 50.  us a
- * step, queries and units, two layers; three, 16 and 40 sequences, four heads of 16 on two 32.3 and 30.9 (units), 54 and 56, 109 and 117 (queries), on four 32.7 and 32.9, 56 and 76, 112 and 168
- * (queries but for the first), on one 32.2 and 29.1, 54 and 46, 107 and 89 (units); 16 sequences, eight heads of 4 57 and 102 (queries); one, four and 16 sequences, four heads of 32 on two 32.5 and
- * 33.3, 39.4 and 38.0, 71 and 69 (queries), eight on two 40.0 and 40.7 (queries), 51.6 and 44.3, 102 and 70 (units), one head of 64 30.4 and 35.7, 34.4 and 38.2, 52 and 60 (queries), four on two
- * 58 and 64 (queries), 71.5 and 69.7, 122 and 109 (units); prompts of 16 and 63 tokens, four heads of 16 on two 48 and 37, 149 and 92, one head of 64 45 and 39, 150 and 92 (units).  Of
- * 649 steps of 20 shapes with heads of 4 to 64 the chosen way takes 1.003 of the faster one's time, 1.14 at most. */
+/* Whether a float32 step within a page has its attention by the matrix cores, a wave a unit (attend_page), and not a query a wave: where units are few beside the queries.  Heads of up to 16:
+ * a unit costs four queries for every 16 positions, and what a step saves beside them pays for ten.  Larger heads: a query of d elements costs d, a wave's turn of units, whose loads take 16 elements of a row at a
+ * time, 9 d, and each unit 50 for what it is served.  us a step by queries and by units, two layers: 3, 16 and 40 sequences, four heads of 16 on two 32.3 and 30.9 (units), 54 and 56, 109 and 117
+ * (queries), on four 32.7 and 32.9, 56 and 76, 112 and 168 (queries), on one 32.2 and 29.1, 54 and 46, 107 and 89 (units); 16 sequences, eight heads of 4 57 and 102
+ * (queries); one, four and 16 sequences, four heads of 32 on two 32.5 and 33.3, 39.4 and 38.0, 71 and 69 (queries), eight on two 40.0 and 40.7 (queries), 51.6 and 44.3, 102 and 70 (units), one head of
+ * 64 30.4 and 35.7, 34.4 and 38.2, 52 and 60 (queries), four on two 58 and 64 (queries), 71.5 and 69.7, 122 and 109 (units); prompts of 16 and 63 tokens, four heads of 16 on two 48
+ * and 37, 149 and 92, one head of 64 45 and 39, 150 and 92 (units).  925 steps of 37 shapes with heads of 4 to 64: 1.003 of the faster way's time (at most 1.14), and at most 1.045 of that by queries. */
 extern "C" int tqk_small_step_pages(const TqkSmallStep* step) {
     const TqkSmallStep& p = *step;
     if (p.act_dtype != TQK_F32 || p.max_end > TQK_PAGE || p.seq_first < 0 || p.n_seqs < 1 || p.seq_first + p.n_seqs + 1 > TQK_SMALL_INTS) return 0;
-    const int waves = tqk_small_step_rings(&p) ? SS_WAVES - SS_BRING : SS_WAVES, group = p.n_heads / p.n_kv_heads, queries = p.n_rows * p.n_heads;
-    int units = 0;
-    for (const int32_t* first = p.ints + p.seq_first, *end = first + p.n_seqs; first < end; ++first) units += ((first[1] - first[0]) * group + 15) / 16 * p.n_kv_heads;
-    const int turns = (units + waves - 1) / waves;
-    if (p.head_dim <= 16) {
-        const int together = waves * queries_together(p, waves);
-        return 2 * turns < 3 * ((queries + together - 1) / together);
-    }
-    return queries * p.head_dim >= 50 * units + 9 * turns * p.head_dim;
+    const int queries = p.n_rows * p.n_heads, units = attention_units(p);
+    if (p.head_dim <= 16) return (4 * units - queries) * ((p.max_end + 15) / 16) < 40;
+    return queries * p.head_dim >= 50 * units + 9 * ((units + SS_WAVES - 1) / SS_WAVES) * p.head_dim;
+}
+
+/* Whether a step's weights come into LDS by waves of their own: decoding steps of few rows, where the ring fits beside the rows.  us a step without and with it, steps asked for one by one: float32, two layers of 64, 1, 3, 4, 5 and 16 rows 36.5, 37.8, 37.5, 39.4, 54.0 and 33.3, 34.1, 35.8, 40.1, 57.3;
+ * bfloat16, heads of 32, three layers of 96, 1, 5, 8, 12 and 16 rows 38.2, 40.9, 42.0, 46.3, 81.5 and 36.0, 38.5, 41.3, 45.4, 81.8.  bfloat16 with other heads, whose attention every wave has a part
+ * in, loses: two layers of 64, 1, 4, 8 and 16 rows 28.1, 29.5, 33.0, 42.1 and 28.3, 29.8, 34.0, 48.1. */
+extern "C" int tqk_small_step_rings(const TqkSmallStep* step) {
+    const TqkSmallStep& p = *step;
+    const bool f32 = p.act_dtype == TQK_F32, few = f32 ? p.n_rows <= SS_FEW : p.n_rows <= 12 && (p.head_dim == 32 || p.head_dim == 64);
+    return p.decode && few && small_layout(p, SS_WAVES - SS_BRING).bytes + small_ring(p).bytes <= 160 * 1024;
 }
 
 template <typename T, int D>
