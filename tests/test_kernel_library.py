@@ -148,7 +148,11 @@ def test_which_steps_the_kernel_for_small_models_takes(sizes, takes):
     ({"act_dtype": 0, "vocab": 256 + 64}, 1), ({"act_dtype": 0, "vocab": 512}, 0), ({"act_dtype": 0, "vocab": 512, "n_want": 0}, 1),      # the head beside down
     ({}, 0), ({"n_heads": 3, "n_kv_heads": 1, "head_dim": 32, "hidden": 96, "inter": 224}, 1),                                        # the matrix cores' heads
     ({"n_heads": 3, "n_kv_heads": 1, "head_dim": 32, "hidden": 96, "inter": 224, "n_rows": 12, "n_want": 12, "n_seqs": 12}, 1),
-    ({"n_heads": 3, "n_kv_heads": 1, "head_dim": 32, "hidden": 96, "inter": 224, "n_rows": 13, "n_want": 13, "n_seqs": 13}, 0)])
+    ({"n_heads": 3, "n_kv_heads": 1, "head_dim": 32, "hidden": 96, "inter": 224, "n_rows": 13, "n_want": 13, "n_seqs": 13}, 0),
+    ({"head_dim": 32, "n_rows": 7, "n_want": 7, "n_seqs": 7}, 1), ({"head_dim": 32, "n_rows": 8, "n_want": 8, "n_seqs": 8}, 0),          # 14 and 16 units of attention for 14 waves
+    ({"act_dtype": 0, "n_rows": 3, "n_want": 3, "n_seqs": 3, "max_end": 90}, 1), ({"act_dtype": 0, "n_rows": 4, "n_want": 4, "n_seqs": 4, "max_end": 90}, 0),
+    ({"act_dtype": 0, "n_heads": 8, "n_kv_heads": 8, "head_dim": 4, "hidden": 32, "n_rows": 3, "n_want": 3, "n_seqs": 3, "max_end": 90}, 1),
+    ({"act_dtype": 0, "n_heads": 8, "n_kv_heads": 8, "head_dim": 4, "hidden": 32, "n_rows": 4, "n_want": 4, "n_seqs": 4, "max_end": 90}, 0)])
 def test_which_small_steps_have_their_weights_brought_into_lds(sizes, rings):
     lib = ctypes.CDLL(kernels.library_path())
     step = small_step(**sizes)

@@ -1218,13 +1218,17 @@ extern "C" int tqk_small_step_pages(const TqkSmallStep* step) {
     return queries * p.head_dim >= 50 * units + 9 * ((units + SS_WAVES - 1) / SS_WAVES) * p.head_dim;
 }
 
-/* Whether a step's weights come into LDS by waves of their own: decoding steps of few rows, where the ring fits beside the rows.  us a step without and with it, steps asked for one by one: float32, two layers of 64, 1, 3, 4, 5 and 16 rows 36.5, 37.8, 37.5, 39.4, 54.0 and 33.3, 34.1, 35.8, 40.1, 57.3;
+/* Whether a step's weights come into LDS by waves of their own: decoding steps of few rows, where the ring fits beside the rows and two waves fewer take no more turns for the attention's
+ * queries or units.  us a step without and with it, steps asked for one by one: float32, two layers of 64, 1, 3, 4, 5 and 16 rows 36.5, 37.8, 37.5, 39.4, 54.0 and 33.3, 34.1, 35.8, 40.1, 57.3;
  * bfloat16, heads of 32, three layers of 96, 1, 5, 8, 12 and 16 rows 38.2, 40.9, 42.0, 46.3, 81.5 and 36.0, 38.5, 41.3, 45.4, 81.8.  bfloat16 with other heads, whose attention every wave has a part
- * in, loses: two layers of 64, 1, 4, 8 and 16 rows 28.1, 29.5, 33.0, 42.1 and 28.3, 29.8, 34.0, 48.1. */
+ * in, loses: two layers of 64, 1, 4, 8 and 16 rows 28.1, 29.5, 33.0, 42.1 and 28.3, 29.8, 34.0, 48.1.  A turn more (six asked for together): float32, four heads of 16, 4 sequences after 240
+ * tokens 62.3 and 68.6, eight of 4, 2 after 90 and 240 34.1 and 38.8, 49.7 and 61.2; bfloat16, four heads of 32 on two, 8 sequences 30.2 and 32.0. */
 extern "C" int tqk_small_step_rings(const TqkSmallStep* step) {
     const TqkSmallStep& p = *step;
     const bool f32 = p.act_dtype == TQK_F32, few = f32 ? p.n_rows <= SS_FEW : p.n_rows <= 12 && (p.head_dim == 32 || p.head_dim == 64);
-    return p.decode && few && small_layout(p, SS_WAVES - SS_BRING).bytes + small_ring(p).bytes <= 160 * 1024;
+    if (!p.decode || !few || small_layout(p, SS_WAVES - SS_BRING).bytes + small_ring(p).bytes > 160 * 1024) return 0;
+    const int work = !f32 ? p.n_rows * p.n_kv_heads : tqk_small_step_pages(&p) ? attention_units(p) : p.n_rows * p.n_heads;
+    return (work + SS_WAVES - SS_BRING - 1) / (SS_WAVES - SS_BRING) == (work + SS_WAVES - 1) / SS_WAVES;
 }
 
 template <typename T, int D>
