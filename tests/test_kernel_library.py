@@ -159,6 +159,15 @@ def test_which_small_steps_have_their_weights_brought_into_lds(sizes, rings):
     assert lib.tqk_small_step_takes(ctypes.byref(step)) and lib.tqk_small_step_rings(ctypes.byref(step)) == rings
 
 
+@pytest.mark.parametrize("sizes,rows,decode,positions,pays", [
+    ({}, 33, 0, 33, 1), ({}, 40, 1, 60, 0), ({}, 24, 1, 60, 1), ({"hidden": 96, "inter": 224, "n_heads": 3, "n_kv_heads": 1, "head_dim": 32, "n_layers": 3}, 33, 0, 33, 0),
+    ({"hidden": 96, "inter": 224, "n_heads": 6, "n_kv_heads": 6, "n_layers": 3, "vocab": 300}, 24, 0, 3, 0),
+    ({"hidden": 96, "inter": 224, "n_heads": 6, "n_kv_heads": 1, "n_layers": 3, "vocab": 300}, 24, 0, 24, 1)])
+def test_which_float32_small_steps_pay_in_one_launch(sizes, rows, decode, positions, pays):
+    lib = ctypes.CDLL(kernels.library_path())
+    assert lib.tqk_small_step_pays(ctypes.byref(small_step(act_dtype=0, **sizes)), rows, decode, positions) == pays
+
+
 # heads, kv heads, head_dim; the sequences' new tokens; whether they are single tokens
 @pytest.mark.parametrize("heads,rows,decode,pages", [
     ((4, 2, 16), [1] * 2, 1, 1), ((4, 2, 16), [1] * 16, 1, 0), ((4, 2, 16), [33], 0, 1), ((4, 4, 16), [1] * 4, 1, 0), ((5, 5, 16), [1] * 2, 1, 0), ((4, 1, 16), [1] * 40, 1, 1),

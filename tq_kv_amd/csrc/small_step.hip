@@ -1149,9 +1149,9 @@ extern "C" int tqk_small_step_takes(const TqkSmallStep* step) {
  * its products, its other work and its heads' pages take; the head's weights at 39 KB.  The other kernels, ten launches a layer: 20 a layer in a graph (33 in float32) and 32 (45) one by one.
  * Measured, one block and the other kernels, two layers of 64 values with 160 in the feed-forward, bfloat16: 1, 16 and 40 sequences 31 and 72, 65 and 79, 92 and 88, prompts of 8, 33
  * and 64 tokens 31 and 96, 61 and 96, 109 and 97; three of 96 with 224 and heads of 32: 47 and 73, 75 and 82, 108 and 97, then 35 and 132, 70 and 134, 95 and 135; with heads of 64: 66 and 78, 87
- * and 83, 156 and 106, then 43 and 132, 87 and 137, 133 and 137; four of 128 with 224: 69 and 83, 94 and 88, 207 and 122, then 55 and 175, 126 and 179, 175 and 179.  float32, two of 64: 1, 4, 16 and 40 sequences 32 and 83, 33 and 86, 55 and 88, 115 and 114, prompts of 8, 33 and 64 tokens 35 and 92, 69 and 99, 93 and 106; three of 96 67 and 111, 67 and 113,
- * 87 and 116, 195 and 156, then 65 and 118, 147 and 142, 199 and 150; with heads of 64 82 and 112, 83 and 114, 111 and 117, 257 and 166, then 79 and 118, 189 and 149; four of 128 with 512: 156 and 147,
- * 161 and 150, 210 and 153, then 154 and 154. */
+ * and 83, 156 and 106, then 43 and 132, 87 and 137, 133 and 137; four of 128 with 224: 69 and 83, 94 and 88, 207 and 122, then 55 and 175, 126 and 179, 175 and 179.  float32, two of 64: 1, 4, 16
+ * and 40 sequences 29 and 82, 31 and 85, 52 and 87, 106 and 115, prompts of 8, 33 and 64 tokens 33 and 100, 67 and 102, 91 and 105; three of 96 62 and 111, 69 and 111, 85 and 116, 194 and 156, then 64 and 128,
+ * 147 and 145, 198 and 153; with heads of 64 74 and 109, 84 and 113, 109 and 117, 256 and 166, then 77 and 130, 188 and 154; four of 128 with 512: 152 and 145, 163 and 149, 219 and 155, then 153 and 159. */
 extern "C" int tqk_small_step_pays(const TqkSmallStep* step, int n_rows, int decode, int positions) {
     const TqkSmallStep& p = *step;
     const bool f32 = p.act_dtype == TQK_F32;
@@ -1159,8 +1159,9 @@ extern "C" int tqk_small_step_pays(const TqkSmallStep* step, int n_rows, int dec
     const double size = f32 ? 4 : 2, q = (double)p.n_heads * p.head_dim;
     const double thousands = 1e-3 * p.hidden * (2 * q + 2. * p.n_kv_heads * p.head_dim + 3. * p.inter);            // weights of a layer
     const double heads = 0.08 * p.n_heads * ((positions + TQK_PAGE - 1) / TQK_PAGE);
-    // (float32 within a page: columns of a sequence share an instruction in prompts)
-    const double a_row = f32 && positions <= TQK_PAGE ? 0.15 + 0.0085 * thousands + (decode ? heads : 0) : 0.15 + (f32 ? 0.0115 : 0.0043) * thousands + heads;
+    // (float32 within a page: columns of a sequence and kv head share an instruction in prompts.  Eight chunks of three tokens, three layers of 96, six heads of 16 on as many: 155 us here,
+    // 144 there)
+    const double a_row = f32 && positions <= TQK_PAGE ? 0.15 + 0.0085 * thousands + (decode ? heads : 0.03 * p.n_kv_heads) : 0.15 + (f32 ? 0.0115 : 0.0043) * thousands + heads;
     const double here = 8 + p.n_layers * (5 + thousands * size / (f32 ? 27 : 33) + n_rows * a_row) + 1e-3 * p.vocab * p.hidden * size / 39;
     const double there = decode ? 15 + p.n_layers * (f32 ? 33 : 20) : 15 + p.n_layers * (f32 ? 45 : 32);
     return here < there;
