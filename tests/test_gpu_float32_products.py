@@ -129,3 +129,29 @@ def test_what_is_not_finite_changes_nothing_beside_it(n, k):
     assert torch.isinf(one[8])
     for m in ROWS[1:]:
         assert torch.equal(product(x[:m].contiguous(), w, None)[1], one), m
+
+
+# m, n, k, and how many blocks share K: a group each, two groups and a last one alone, two and none left, one block for all of K (400 to 767 tiles and more)
+@pytest.mark.parametrize("m,n,k,shares", [(17, 3584, 18944, 19), (100, 3584, 18944, 10), (160, 4096, 11008, 6), (200, 7168, 5116, 3), (1000, 4608, 3584, 4),
+                                          (1000, 3584, 3584, 1), (1000, 3584, 3588, 1), (300, 37888, 2052, 1)])
+def test_the_bits_do_not_depend_on_how_groups_of_k_are_dealt_to_blocks(m, n, k, shares):
+    """A row alone has a block for each group.  With a bias, and then with what is not finite in the first, a middle and the last group of some sums."""
+    assert K.library().tqk_gemm_f32_shares(m, n, k) == shares
+    g = torch.Generator(device="cuda").manual_seed(m + k)
+    x, w = torch.randn((m, k), device="cuda", generator=g), torch.randn((n, k), device="cuda", generator=g) * 0.02
+    b = torch.randn((n,), device="cuda", generator=g)
+    rows = [0, 1, m // 2, m - 1]
+    clean = product(x, w, b)
+    for r in rows:
+        assert torch.equal(product(x[r:r + 1].contiguous(), w, b)[0], clean[r]), r
+    x[1, 5], x[m // 2, k // 2], x[m - 1, k - 1] = float("inf"), float("nan"), float("-inf")
+    w[7, 9], w[n - 1, k - 3] = float("nan"), float("inf")
+    x[3, :4], w[8, :4] = 2e19, 2e19                       # (a sum that overflows in the first group)
+    y = product(x, w, b)
+    for r in rows + [3]:
+        one = product(x[r:r + 1].contiguous(), w, b)[0]
+        assert torch.equal(one.isnan(), y[r].isnan()) and torch.equal(one.nan_to_num(), y[r].nan_to_num()), r
+    finite = torch.ones((m, n), dtype=torch.bool, device="cuda")
+    finite[:, [7, n - 1]], finite[[1, 3, m // 2, m - 1]] = False, False
+    finite[:, 8] = False
+    assert torch.equal(y[finite], clean[finite]) and torch.isinf(y[3, 8]) and not torch.isfinite(y[[1, m // 2, m - 1]]).any()

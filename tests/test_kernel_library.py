@@ -184,3 +184,15 @@ def test_which_float32_small_steps_have_their_attention_by_units_of_columns(head
     assert lib.tqk_small_step_takes(ctypes.byref(step)) and lib.tqk_small_step_pages(ctypes.byref(step)) == pages
     step.max_end = 65
     assert lib.tqk_small_step_pages(ctypes.byref(step)) == 0
+
+
+# up to 16 rows; few tiles with a group a share and with two (the last share of one, or none left over); 400 to 767 tiles either way; more
+SHARES = [(16, 3584, 18944, 19), (17, 3584, 18944, 19), (100, 3584, 18944, 10), (128, 3584, 18944, 10), (160, 4096, 11008, 6), (200, 7168, 5120, 3), (300, 3584, 3584, 4), (500, 4608, 3584, 4),
+          (64, 37888, 3584, 4), (128, 37888, 3584, 4), (1000, 4608, 3584, 4), (1000, 3584, 3584, 1), (1000, 3584, 18944, 1), (300, 37888, 3584, 1), (2000, 4608, 3584, 1), (40, 1024, 1024, 1)]
+
+
+@pytest.mark.parametrize("m,n,k,shares", SHARES)
+def test_how_many_blocks_share_a_float32_products_k(m, n, k, shares):
+    lib = kernels.library()
+    assert lib.tqk_gemm_f32_shares(m, n, k) == shares
+    assert lib.tqk_gemm_scratch_bytes(0, 0, 0, 0, m, n, k) == (0 if shares == 1 else -(-k // 1024) * m * n * 4)

@@ -764,23 +764,37 @@ static SplitTile split_tile(int M, int N, int K) {
     return {2, 1};
 }
 
+// How long blocks of `per` groups each (a last one of what is left) take for all tiles, in a single group's time: a unit holds two blocks, 512 are under way together, and 256 that are left
+// have a unit each and take 0.6 of the time.
+static double split_rounds(long long tiles, int groups, int per) {
+    auto busy = [](long long blocks) { return blocks == 0 ? 0. : blocks <= 256 ? 0.6 : 1.; };
+    const int rest = groups % per;
+    const long long whole = tiles * (groups / per) / 512, left = tiles * (groups / per) % 512;
+    if (rest == 0) return per * (whole + busy(left));
+    // (the last ones begin beside those that are left of the others, and behind them where these leave too few places)
+    if (tiles <= 512 - left) return per * whole + rest * busy(left + tiles) + (per - rest) * busy(left);
+    return per * (whole + 1) + rest * busy(tiles - (512 - left));
+}
+
 // Into how many shares the groups are dealt for M rows: few rows, one a group; more, so that there are about four blocks a compute
 // unit (one: 280 blocks of 300 x 3584 leave most units idle while a few do a second block), no more than there are groups.
-// Products that take numbers apart: a unit holds two blocks, and what sets the time is how many rounds of 512 there are, the last one 0.6 of a round where no unit has a second
-// block left.  Short blocks leave less of it over, so every group is a share of its own, unless blocks that walk all of K come out ahead of that with the sums that they need
-// not write and add up.  Tried with all numbers of shares, nine sizes at 17 to 1000 rows: this takes 1.005 of the best one's time (at most 1.05); two blocks a unit, which was the rule, 1.035 (us,
-// then and now: 300 and 1000 rows of 3584 x 18944 416 -> 358 and 1145 -> 991, 1000 of 1536 x 8960 282 -> 225, 500 of 4608 x 3584 178 -> 151, 64 of 37888 x 3584 207 -> 181).  768: bounds the scratch.
-static int f32_shares(int M, int N, int K) {
+// Products that take numbers apart: what sets the time is how many rounds of 512 blocks there are (split_rounds).  Short blocks leave less of a last round over, so every group is a share of its own,
+// unless blocks that walk all of K come out ahead of that with the sums that they need not write and add up, or two groups a block take no more rounds, which saves a start and
+// an end, where there is a full round of blocks without a tile's last group.  Below 400 tiles blocks of all of K leave a fifth of the places idle and were never the best.  From 768 on: no scratch.
+// us with two blocks a unit and so, weights that no cache holds: 300 and 1000 rows of 3584 x 18944 422 -> 354 and 1090 -> 985, 1000 of 1536 x 8960 276 -> 212, 500 of 4608 x 3584 178 -> 151, 64 of
+// 37888 x 3584 207 -> 181; a group a block and two: 100, 128 and 256 rows of 3584 x 18944 153 -> 145, 161 -> 152 and 279 -> 269, 160 of 4096 x 11008 155 -> 147, 200 of 7168 x 5120 161 -> 155 (28
+// tiles with 19 groups, 17 rows of 3584 x 18944, 70 -> 73: they keep one).  317 sizes of 19 weights, 17 to 2048 rows: 1.003 of the best number's time (at most 1.11, 80 rows of 7168 x 5120), two blocks a
+// unit 1.025 (at most 1.29).
+extern "C" int tqk_gemm_f32_shares(int M, int N, int K) {
     const int groups = (K + G_GROUP - 1) / G_GROUP;
     if (M <= 16) return groups;
     if (tqk_gemm_takes_apart(N, K)) {
         const SplitTile t = split_tile(M, N, K);
         const long long tiles = (long long)((M + 16 * t.rows - 1) / (16 * t.rows)) * ((N + 64 * t.features - 1) / (64 * t.features));
-        if (tiles < 400) return groups;
         if (tiles >= 768) return 1;
-        auto rounds = [](long long blocks) { const int rest = (int)(blocks % 512); return (double)(blocks / 512) + (rest == 0 ? 0. : rest <= 256 ? 0.6 : 1.); };
+        if (tiles < 400) return tiles * (groups - 1) >= 512 && split_rounds(tiles, groups, 2) <= split_rounds(tiles, groups, 1) ? (groups + 1) / 2 : groups;
         const double us = 8 + 39. * t.rows * t.features / 8;             // of a round of single groups
-        return rounds(tiles) * (groups + 0.1) * us <= rounds(tiles * groups) * 1.1 * us + 5 + (double)groups * M * N * 8 / 4.0e6 ? 1 : groups;
+        return split_rounds(tiles, 1, 1) * (groups + 0.1) * us <= split_rounds(tiles, groups, 1) * 1.1 * us + 5 + (double)groups * M * N * 8 / 4.0e6 ? 1 : groups;
     }
     const long long tiles = (long long)((M + GT - 1) / GT) * ((N + GT - 1) / GT);
     const int want = (int)(tiles >= 1024 ? 1 : (1024 + tiles - 1) / tiles), per = (groups + want - 1) / want;
@@ -789,7 +803,7 @@ static int f32_shares(int M, int N, int K) {
 
 /* Bytes of device scratch tqk_gemm wants for these sizes and dtypes (0: none). */
 extern "C" size_t tqk_gemm_scratch_bytes(int x_dtype, int w_dtype, int bias_dtype, int y_dtype, int M, int N, int K) {
-    if (M <= 0 || N <= 0 || K <= 0 || !f32_case(x_dtype, w_dtype, nullptr, bias_dtype, y_dtype, K, nullptr, nullptr) || f32_shares(M, N, K) == 1) return 0;
+    if (M <= 0 || N <= 0 || K <= 0 || !f32_case(x_dtype, w_dtype, nullptr, bias_dtype, y_dtype, K, nullptr, nullptr) || tqk_gemm_f32_shares(M, N, K) == 1) return 0;
     return (size_t)((K + G_GROUP - 1) / G_GROUP) * M * N * sizeof(float);
 }
 
@@ -814,7 +828,7 @@ extern "C" int tqk_gemm(const void* x, int x_dtype, const void* w, int w_dtype, 
     if (M == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
     if (f32_case(x_dtype, w_dtype, bias, bias_dtype, y_dtype, K, x, w)) {
-        const int groups = (K + G_GROUP - 1) / G_GROUP, shares = scratch ? f32_shares(M, N, K) : 1;       // (without scratch one block walks all of K)
+        const int groups = (K + G_GROUP - 1) / G_GROUP, shares = scratch ? tqk_gemm_f32_shares(M, N, K) : 1;       // (without scratch one block walks all of K)
         TQK_REQUIRE(groups <= 65535, "tqk_gemm: K=%d is more than the grid takes", K);
         const float *xf = (const float*)x, *wf = (const float*)w, *bf = (const float*)bias;
         float* out = shares > 1 ? (float*)scratch : (float*)y;

@@ -77,6 +77,7 @@ int tqk_add_rmsnorm_sums(float* h, const float* sums, int n_sums, int sum_rows, 
  * memory, 16-byte aligned (may be null: then, or where that is 0, the tiled kernel runs). */
 size_t tqk_gemm_scratch_bytes(int x_dtype, int w_dtype, int bias_dtype, int y_dtype, int M, int N, int K);
 int tqk_gemm_takes_apart(int N, int K);        /* whether a float32 product's numbers go through the matrix cores as three bfloat16 ones each */
+int tqk_gemm_f32_shares(int M, int N, int K);   /* how many blocks share the K of a float32 product's tile */
 int tqk_gemm(const void* x, int x_dtype, const void* w, int w_dtype, const void* bias,
              int bias_dtype, void* y, int y_dtype, int M, int N, int K, void* scratch, void* stream);
 
