@@ -196,3 +196,14 @@ def test_how_many_blocks_share_a_float32_products_k(m, n, k, shares):
     lib = kernels.library()
     assert lib.tqk_gemm_f32_shares(m, n, k) == shares
     assert lib.tqk_gemm_scratch_bytes(0, 0, 0, 0, m, n, k) == (0 if shares == 1 else -(-k // 1024) * m * n * 4)
+
+
+def test_the_scratch_of_float32_products_is_bounded():
+    """128 MB from 512 tiles of 64 rows by 128 features on, none from 768 on; fewer tiles bound it by their own size, 16 MB for each 1024 of K."""
+    lib = kernels.library()
+    for k in (1024, 2052, 3584, 11008, 18944, 65536):
+        for rows in range(64, 1601, 128):
+            for features in (2048, 3840, 5120, 37888):
+                got, tiles = lib.tqk_gemm_scratch_bytes(0, 0, 0, 0, rows, features, k), -(-rows // 64) * -(-features // 128)
+                if tiles * -(-k // 1024) >= 256 and rows > 32:         # (the largest tiles are taken)
+                    assert got <= (0 if tiles >= 768 else 128 << 20 if tiles >= 512 else tiles * 64 * 128 * 4 * -(-k // 1024)), (rows, features, k)

@@ -780,7 +780,8 @@ static double split_rounds(long long tiles, int groups, int per) {
 // unit (one: 280 blocks of 300 x 3584 leave most units idle while a few do a second block), no more than there are groups.
 // Products that take numbers apart: what sets the time is how many rounds of 512 blocks there are (split_rounds).  Short blocks leave less of a last round over, so every group is a share of its own,
 // unless blocks that walk all of K come out ahead of that with the sums that they need not write and add up, or two groups a block take no more rounds, which saves a start and
-// an end, where there is a full round of blocks without a tile's last group.  Below 400 tiles blocks of all of K leave a fifth of the places idle and were never the best.  From 768 on: no scratch.
+// an end, where there is a full round of blocks without a tile's last group.  Below 400 tiles blocks of all of K leave a fifth of the places idle and were never the best.  From 512 tiles on, where two blocks a unit need no
+// scratch, groups' sums take 128 MB of it at most (1000 rows of 4608 x 3584: 74 MB, 290 -> 265 us), and from 768 on none.
 // us with two blocks a unit and so, weights that no cache holds: 300 and 1000 rows of 3584 x 18944 422 -> 354 and 1090 -> 985, 1000 of 1536 x 8960 276 -> 212, 500 of 4608 x 3584 178 -> 151, 64 of
 // 37888 x 3584 207 -> 181; a group a block and two: 100, 128 and 256 rows of 3584 x 18944 153 -> 145, 161 -> 152 and 279 -> 269, 160 of 4096 x 11008 155 -> 147, 200 of 7168 x 5120 161 -> 155 (28
 // tiles with 19 groups, 17 rows of 3584 x 18944, 70 -> 73: they keep one).  317 sizes of 19 weights, 17 to 2048 rows: 1.003 of the best number's time (at most 1.11, 80 rows of 7168 x 5120), two blocks a
@@ -791,7 +792,7 @@ extern "C" int tqk_gemm_f32_shares(int M, int N, int K) {
     if (tqk_gemm_takes_apart(N, K)) {
         const SplitTile t = split_tile(M, N, K);
         const long long tiles = (long long)((M + 16 * t.rows - 1) / (16 * t.rows)) * ((N + 64 * t.features - 1) / (64 * t.features));
-        if (tiles >= 768) return 1;
+        if (tiles >= 768 || (tiles >= 512 && (long long)groups * M * N * 4 > 128 << 20)) return 1;
         if (tiles < 400) return tiles * (groups - 1) >= 512 && split_rounds(tiles, groups, 2) <= split_rounds(tiles, groups, 1) ? (groups + 1) / 2 : groups;
         const double us = 8 + 39. * t.rows * t.features / 8;             // of a round of single groups
         return split_rounds(tiles, 1, 1) * (groups + 0.1) * us <= split_rounds(tiles, groups, 1) * 1.1 * us + 5 + (double)groups * M * N * 8 / 4.0e6 ? 1 : groups;
