@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import helpers
+from tq_kv_amd import native
 from tq_kv_amd import Engine, GenerationParams, Model, generate
 from tq_kv_amd.cache import PAGE, CacheFull
 
@@ -19,6 +20,14 @@ def test_a_step_returns_a_row_for_each_wanted_entry(want):
     engine = Engine(Model.random(cfg, seed=seed, dtype="float32", device="cpu"), max_tokens=4 * PAGE)
     for borrow in (False, True):
         assert tuple(engine.step([(engine.open(), [1, 2, 3], want)], borrow=borrow).shape) == (2, cfg["vocab_size"])
+
+
+@pytest.mark.parametrize("tied,inter,once", [(False, 349400, False), (True, 349400, False), (True, 349500, True)])
+def test_weights_that_the_memory_side_cache_holds_are_not_said_to_be_read_once(tied, inter, once):
+    """256 MB of what steps read whole: beside the feed-forward's 768 bytes a unit 75008, 24576 of them the head's.  The embedding counts where it is the head too."""
+    cfg = dict(helpers.TINY_A, hidden_size=64, intermediate_size=inter, num_hidden_layers=1, tie_word_embeddings=tied, vocab_size=96)
+    model = Model.random(cfg, seed=1, dtype="float32", device="cpu")
+    assert native.parsed(model._lib.tqe_model_describe(model.handle))["weights_once"] == once
 
 
 @pytest.mark.parametrize("name", sorted(helpers.CONFIGS))

@@ -155,3 +155,17 @@ def test_the_bits_do_not_depend_on_how_groups_of_k_are_dealt_to_blocks(m, n, k, 
     finite[:, [7, n - 1]], finite[[1, 3, m // 2, m - 1]] = False, False
     finite[:, 8] = False
     assert torch.equal(y[finite], clean[finite]) and torch.isinf(y[3, 8]) and not torch.isfinite(y[[1, m // 2, m - 1]]).any()
+
+
+@pytest.mark.parametrize("n,k", [(1024, 1024), (1030, 1088), (2049, 516), (5003, 1028), (700, 18944)])
+def test_weights_read_once_give_the_same_bits(n, k):
+    """The other kind of loads: every kernel for few rows, whole stages of K and not, features that are no whole tiles; with what is not finite."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, w, b = torch.randn((17, k), device="cuda", generator=g), torch.randn((n, k), device="cuda", generator=g), torch.randn((n,), device="cuda", generator=g)
+    w[3, 7], x[2, k - 1] = float("inf"), float("nan")
+    for m in [1, 3, 4, 5, 8, 9, 12, 16, 17]:
+        for bias in (None, b):
+            y = torch.full((m + 1, n), float("nan"), device="cuda")
+            K.gemm(x[:m].contiguous(), w, bias, y[:m], once=True)
+            want = product(x[:m].contiguous(), w, bias)
+            assert y[m].isnan().all() and torch.equal(y[:m].isnan(), want.isnan()) and torch.equal(y[:m].nan_to_num(), want.nan_to_num()), m

@@ -25,6 +25,7 @@ TQ_KERNEL(add_rmsnorm, float*, cptr, int, cptr, int, float, ci32, int, int, void
 TQ_KERNEL(add_rmsnorm_sums, float*, cf32, int, int, int, cptr, int, float, ci32, int, int, void*, int, void*);
 TQ_QUERY(size_t, gemm_scratch_bytes, int, int, int, int, int, int, int);
 TQ_KERNEL(gemm, cptr, int, cptr, int, cptr, int, void*, int, int, int, int, void*, void*);
+TQ_KERNEL(gemm_once, cptr, int, cptr, int, cptr, int, void*, int, int, int, int, void*, void*);
 TQ_KERNEL(fused_store, cptr, ci32, cf32, int, float, cptr, int, void*, int, int, int, int, void*);
 TQ_KERNEL(fused_gated, cptr, cf32, int, float, cptr, int, void*, int, int, int, void*);
 TQ_QUERY(int, fused_residual_parts, int, int);

@@ -209,7 +209,7 @@ static void k_gemm(StepContext& c, const Tensor& x, const Tensor& w, const Tenso
     const int bias_dt = bias ? bias->dtype : 0;
     const size_t need = K::gemm_scratch_bytes.raw(x.dtype, w.dtype, bias_dt, out.dtype, m, n, k);
     void* scratch = need ? c.ws->alloc(need) : nullptr;
-    K::gemm(x.data, x.dtype, w.data, w.dtype, bias ? bias->data : nullptr, bias_dt, out.data, out.dtype, m, n, k, scratch, c.stream);
+    (c.weights_once ? K::gemm_once : K::gemm)(x.data, x.dtype, w.data, w.dtype, bias ? bias->data : nullptr, bias_dt, out.data, out.dtype, m, n, k, scratch, c.stream);
 }
 
 Product linear(StepContext& c, const Tensor& x, const Weight& w, const Tensor* bias, int out_dtype, bool leave_sums, Tensor* out) {

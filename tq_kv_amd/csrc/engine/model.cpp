@@ -72,6 +72,10 @@ static OwnedPtr need(Loaded& tensors, const std::string& name) {
 
 void Model::load(Loaded& tensors, hipStream_t stream) {
     embedding_ = need(tensors, spec.embedding_name);
+    size_t bytes = 0;                   // (of the embedding a step reads a few rows, unless it is the head too)
+    for (const auto& t : tensor_specs())
+        if (spec.head_name.empty() || t.first != spec.embedding_name) bytes += need(tensors, t.first)->t.bytes();
+    weights_once_ = bytes > ((size_t)256 << 20);
     for (size_t l = 0; l < blocks_.size(); ++l) {
         Loaded own;
         for (const auto& t : blocks_[l]->tensors()) own[t.first] = need(tensors, spec.layers[l].prefix + t.first);
@@ -215,6 +219,7 @@ Tensor Model::forward(StepContext& c, const CacheStore& cache, float* out) {
     Tensor h = c.alloc(F32, {c.n_tokens, s.hidden_size});
     // which kind of step this is for the products' folding is parts/linear's to say
     classify_step(c, s.hidden_size);
+    c.weights_once = weights_once_;
     // the norm that reads the stream first in every run, and after the last one
     std::vector<Norm*> firsts;
     for (const Run& run : s.order) firsts.push_back(blocks_[(size_t)run.layer]->first_norm());
@@ -325,6 +330,7 @@ Json Model::describe() const {
     j.set("on_gpu", on_gpu);
     j.set("graph_safe", graph_safe);
     j.set("loaded", loaded);
+    j.set("weights_once", weights_once_);
     Json stop = Json::array();
     for (int32_t t : stop_token_ids) stop.push(Json((int)t));
     j.set("stop_token_ids", stop);

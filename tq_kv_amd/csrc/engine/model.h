@@ -54,6 +54,7 @@ private:
     int stream_state_entry_ = -1;               // the cache entry of the stream position's state, if it keeps one
     OwnedPtr embedding_, head_bias_;
     Weight head_;
+    bool weights_once_ = false;                 // the weights that steps read whole are more than the memory-side cache holds (256 MB)
     std::unique_ptr<TqkSmallStep> small_;       // the model as that kernel takes it, if it takes any step of it
     void find_small();
     Tensor head_logits(StepContext& c, Stream& stream, float* out);

@@ -70,6 +70,7 @@ struct StepContext {
     bool all_decode = false, prune_last = false;
     bool capturing = false;                          // the step is being recorded into a graph: nothing may be uploaded
     bool fuse_small = false, fuse_mid = false;       // set by the model from what parts/linear says of the step
+    bool weights_once = false;                       // set by the model: its weights are more than the caches hold from one step to the next
     std::vector<int32_t> packed;                     // the host copy
     StepArrays host, dev;
     int32_t* flat = nullptr;                         // the device copy (workspace, or a captured graph's own buffer)

@@ -263,12 +263,13 @@ void gemm_few_rows_kernel(const float* __restrict__ x, const float* __restrict__
 // ROWS: up to 4, 8 or 16 rows of x.  Of the 16 lanes that hold x's rows four (two) stand for one row where there are few, each takes a quarter (half) of the row's values apart,
 // and the first gets the others' parts by turning the 16 lanes: 40 (56) instructions, and a quarter (half) of the loads; without the turning it takes 1.14, 1.08 and 1.02 of the time of
 // one row, 4608, 3584 and 37888 features, K of 3584, 18944 and 3584.
-// The weights' loads say that they are read once (nt), as those of the bfloat16 kernels do: such weights are 4 MB and more, and a step reads each of them once.  Those sizes and 152064 features, with
-// the kernel that adds up the groups, weights that no cache holds, us with and without: one row 16.0, 51, 93 and 335 (17.3, 55, 100 and 376: 6.5 TB/s in place of 5.8), 8 rows
-// 17.9, 58, 105 and 428 (18.4, 62, 118 and 453); one weight of 51 to 66 MB alone over and over, which the memory-side cache holds, 13.4 and 15.0 (13.5 and 15.7), 8 rows 14.9 and 16.9 (14.2 and
-// 16.9).  gemm_few_rows_kernel's smaller weights may stay in a cache from step to step and keep plain loads (512 x 512: 6.1 us, 6.3 with the hint).
+// ONCE: the weights' loads say that they are read once (nt), as those of the bfloat16 kernels do: for a caller whose weights together are more than the caches hold and who reads each once a step
+// (tqk_gemm_once).  Those sizes and 152064 features, with the kernel that adds up the groups, weights that no cache holds, us with and without: one row 16.0, 51, 93 and 335 (17.3, 55, 100 and
+// 376: 6.5 TB/s in place of 5.8), 8 rows 17.9, 58, 105 and 428 (18.4, 62, 118 and 453); 8192 features, K of 2048, and the other way about, and 17920, K of 1536, one row 17.5, 18.3 and 26.1 (19.1, 20.0 and 28.1).
+// Weights of 64 to 200 MB in all that the memory-side cache holds from one reading to the next lose by it: the first two of those sizes 16.5 and 18.2 (14.4 and 14.4), 16 rows 18.4 and 19.6 (16.2 and
+// 16.3), 37888 features, K of 1024, 33.5 (30.2); 4608 and 3584 features, K of 3584, 14.9 and 12.6 (15.2 and 13.0); those of 4 to 32 MB each 0 to 2 %.
 // TAIL: K is no multiple of 64.
-template <bool TAIL, int ROWS>
+template <bool TAIL, int ROWS, bool ONCE>
 __global__ __launch_bounds__(TQK_WAVE)
 void gemm_few_rows_apart_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ out,
                           int M, int N, int K) {
@@ -301,7 +302,7 @@ void gemm_few_rows_apart_kernel(const float* __restrict__ x, const float* __rest
         const uint32_t nowhere = there ? 0u : 0x80000000u;              // (joined to the offsets, so that no branch lies here)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(w_mem, (lds_ptr_t)(buf(I) + j * 256), 16, (int)(w_at[j] | nowhere), k0 * 4, 0, 2);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(w_mem, (lds_ptr_t)(buf(I) + j * 256), 16, (int)(w_at[j] | nowhere), k0 * 4, 0, ONCE ? 2 : 0);
 #pragma unroll
         for (int u = 0; u < XU; ++u) xv[decltype(I)::value % NS][u] = *reinterpret_cast<const floatx4_t*>(xrow + min(k0 + x_place(u), K - 4));
     };
@@ -821,8 +822,7 @@ static int launch_y(const void* x, const void* w, const void* bias, void* y, int
     return tqk_check_launch("tqk_gemm");
 }
 
-extern "C" int tqk_gemm(const void* x, int x_dtype, const void* w, int w_dtype, const void* bias,
-                        int bias_dtype, void* y, int y_dtype, int M, int N, int K, void* scratch, void* stream) {
+static int gemm(const void* x, int x_dtype, const void* w, int w_dtype, const void* bias, int bias_dtype, void* y, int y_dtype, int M, int N, int K, void* scratch, bool once, void* stream) {
     TQK_REQUIRE(x && w && y, "tqk_gemm: null pointer");
     TQK_REQUIRE(M >= 0 && N > 0 && K > 0, "tqk_gemm: bad sizes M=%d N=%d K=%d", M, N, K);
     TQK_REQUIRE((M + GT - 1) / GT <= 65535, "tqk_gemm: M=%d is more than the grid takes", M);
@@ -841,12 +841,14 @@ extern "C" int tqk_gemm(const void* x, int x_dtype, const void* w, int w_dtype, 
             const dim3 grid((N + 15) / 16, groups);
             if (!apart) gemm_few_rows_kernel<<<grid, TQK_WAVE, 0, s>>>(xf, wf, bf, out, M, N, K);
             else {
-#define LAUNCH(ROWS) do { if (K % 64) gemm_few_rows_apart_kernel<true, ROWS><<<grid, TQK_WAVE, 0, s>>>(xf, wf, bf, out, M, N, K); \
-        else gemm_few_rows_apart_kernel<false, ROWS><<<grid, TQK_WAVE, 0, s>>>(xf, wf, bf, out, M, N, K); } while (0)
+#define LAUNCH_ONCE(ROWS, ONCE) do { if (K % 64) gemm_few_rows_apart_kernel<true, ROWS, ONCE><<<grid, TQK_WAVE, 0, s>>>(xf, wf, bf, out, M, N, K); \
+        else gemm_few_rows_apart_kernel<false, ROWS, ONCE><<<grid, TQK_WAVE, 0, s>>>(xf, wf, bf, out, M, N, K); } while (0)
+#define LAUNCH(ROWS) do { if (once) LAUNCH_ONCE(ROWS, true); else LAUNCH_ONCE(ROWS, false); } while (0)
                 if (M <= 4) LAUNCH(4);
                 else if (M <= 8) LAUNCH(8);
                 else LAUNCH(16);
 #undef LAUNCH
+#undef LAUNCH_ONCE
             }
         } else if (apart) {
             const dim3 grid(((N + 64 * t.features - 1) / (64 * t.features)) * ((M + 16 * t.rows - 1) / (16 * t.rows)), shares);
@@ -877,4 +879,14 @@ extern "C" int tqk_gemm(const void* x, int x_dtype, const void* w, int w_dtype, 
         case 7: return launch_y<bf16_t, bf16_t, bf16_t>(x, w, bias, y, y_dtype, M, N, K, s);
     }
     return tqk_fail("tqk_gemm: unknown dtypes x=%d w=%d bias=%d", x_dtype, w_dtype, bias_dtype);
+}
+
+extern "C" int tqk_gemm(const void* x, int x_dtype, const void* w, int w_dtype, const void* bias,
+                        int bias_dtype, void* y, int y_dtype, int M, int N, int K, void* scratch, void* stream) {
+    return gemm(x, x_dtype, w, w_dtype, bias, bias_dtype, y, y_dtype, M, N, K, scratch, false, stream);
+}
+
+extern "C" int tqk_gemm_once(const void* x, int x_dtype, const void* w, int w_dtype, const void* bias,
+                             int bias_dtype, void* y, int y_dtype, int M, int N, int K, void* scratch, void* stream) {
+    return gemm(x, x_dtype, w, w_dtype, bias, bias_dtype, y, y_dtype, M, N, K, scratch, true, stream);
 }

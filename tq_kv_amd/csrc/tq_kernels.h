@@ -80,6 +80,9 @@ int tqk_gemm_takes_apart(int N, int K);        /* whether a float32 product's nu
 int tqk_gemm_f32_shares(int M, int N, int K);   /* how many blocks share the K of a float32 product's tile */
 int tqk_gemm(const void* x, int x_dtype, const void* w, int w_dtype, const void* bias,
              int bias_dtype, void* y, int y_dtype, int M, int N, int K, void* scratch, void* stream);
+/* the same, for a caller whose weights no cache holds from one reading to the next (the same bits) */
+int tqk_gemm_once(const void* x, int x_dtype, const void* w, int w_dtype, const void* bias,
+                  int bias_dtype, void* y, int y_dtype, int M, int N, int K, void* scratch, void* stream);
 
 /* Skinny products (up to 16 rows, bfloat16, K a multiple of 32) with the small operations
  * around them folded in.  A norm between two products is split over them: the one that adds

@@ -213,15 +213,16 @@ def add_rmsnorm(h, delta, weight, eps, out, rows=None, write_back=False):
     return out
 
 
-def gemm(x, w, bias, out):
-    """out[M,N] = x[M,K] w[N,K]^T (+ bias[N]), float32 accumulation, any dtype mix."""
+def gemm(x, w, bias, out, once=False):
+    """out[M,N] = x[M,K] w[N,K]^T (+ bias[N]), float32 accumulation, any dtype mix.  once: for weights that
+    no cache holds from one reading to the next."""
     m, k = x.shape
     n = w.shape[0]
     lib = library()
     bias_code = _code(bias.dtype) if bias is not None else 0
     need = int(lib.tqk_gemm_scratch_bytes(_code(x.dtype), _code(w.dtype), bias_code, _code(out.dtype), m, n, k))
     scratch = torch.empty((need,), dtype=torch.uint8, device=x.device) if need else None
-    _check(lib.tqk_gemm(
+    _check((lib.tqk_gemm_once if once else lib.tqk_gemm)(
         _dev(x, "x", None, (m, k)), _code(x.dtype), _dev(w, "w", None, (n, k)), _code(w.dtype),
         _opt(bias, "bias", None, (n,)), bias_code,
         _dev(out, "out", None, (m, n)), _code(out.dtype), m, n, k, _opt(scratch, "scratch"), _stream()), "gemm")
