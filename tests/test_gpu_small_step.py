@@ -1,11 +1,14 @@
 """Steps of small models in one launch (csrc/small_step.hip) against the same steps through the kernels of larger ones: the same bits.  Shapes with 16 to
 64 values a head, widths that are and are not whole steps of the matrix cores, more tiles than waves, K that other kernels deal out to
 waves or cut into pieces; steps of 1 to 64 rows on both sides of every change of the kernels that the step stands for.  Which way a step went is counted."""
+import ctypes
+
 import pytest
 import torch
 
 import helpers
-from tq_kv_amd import POLICY, Engine, Model, tracing
+import test_kernel_library
+from tq_kv_amd import POLICY, Engine, Model, kernels, tracing
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -234,61 +237,139 @@ PAGE_SHAPES = {
 }
 
 
+def goes_by_units(cfg, lens, end):
+    """Whether a float32 step of so many new tokens a sequence, up to `end` positions, has its attention by units of columns."""
+    step = test_kernel_library.small_step(act_dtype=0, n_layers=cfg["num_hidden_layers"], hidden=cfg["hidden_size"], n_heads=cfg["num_attention_heads"], n_kv_heads=cfg["num_key_value_heads"],
+                                          head_dim=cfg["head_dim"], inter=cfg["intermediate_size"], vocab=cfg["vocab_size"], n_rows=sum(lens), n_seqs=len(lens),
+                                          decode=int(max(lens) == 1), max_end=end)
+    for i in range(len(lens) + 1):
+        step.ints[i] = sum(lens[:i])
+    return bool(kernels.library().tqk_small_step_pages(ctypes.byref(step)))
+
+
 @pytest.mark.parametrize("name", list(PAGE_SHAPES))
 def test_float32_attention_within_a_page(name):
-    """Several sequences of one step, up to the page's last place and one past it; columns that fill no tile and more than one; windows."""
+    """Several sequences of one step, up to the page's last place and one past it; columns that fill no tile and more than one; windows; both ways to have the attention."""
     cfg = PAGE_SHAPES[name]
     model = Model.random(cfg, seed=11, dtype="float32", device=DEV)
+    ways = []
 
     def run(always):
         out = []
         for lens in [(1,), (1, 16, 17), (33, 2), (20, 20, 24), (63,), (64,)]:
-            eng = Engine(model, max_tokens=1024)
+            eng, n_steps = Engine(model, max_tokens=1024), 0
             slots = [eng.open() for _ in lens]
             tok = lambda n, seed: helpers.random_tokens(n, cfg["vocab_size"], seed)
-            if sum(lens) <= 48 or cfg["head_dim"] < 64:             # (what fits the unit's LDS, which the count shows)
-                out.append(eng.step([(s, tok(n, n), list(range(n))) for s, n in zip(slots, lens)]))
+
+            def step(items):
+                nonlocal n_steps
+                n_steps += 1
+                ways.append(goes_by_units(cfg, [len(t) for _, t, _ in items], max(eng.length(s) + len(t) for s, t, _ in items)))
+                out.append(eng.step(items))
+
+            if sum(lens) <= 48 or cfg["num_attention_heads"] * cfg["head_dim"] < 192:             # (what fits the unit's LDS)
+                step([(s, tok(n, n), list(range(n))) for s, n in zip(slots, lens)])
             else:
                 for s, n in zip(slots, lens):
                     for a in range(0, n, 32):
-                        out.append(eng.step([(s, tok(n, n)[a:a + 32], [0])]))
+                        step([(s, tok(n, n)[a:a + 32], [0])])
             for i in range(2):                                      # a chunk, then single tokens, one of them past the page
-                out.append(eng.step([(s, tok(1 + 4 * (i == 0 and n < 60), i), [0]) for s, n in zip(slots, lens)]))
-            assert (eng.n_small_steps == 0) == (not always)
+                step([(s, tok(1 + 4 * (i == 0 and n < 60), i), [0]) for s, n in zip(slots, lens)])
+            assert eng.n_small_steps == (n_steps if always else 0)
         return out
 
     with policy(small_always=True):
         got = run(True)
     with policy(small=False):
         want = run(False)
+    assert 8 <= sum(ways) // 2 <= len(ways) // 2 - 3, "%d of %d steps by units" % (sum(ways) // 2, len(ways) // 2)
     for i, (a, b) in enumerate(zip(got, want)):
         assert torch.equal(a, b), "%s, step %d: %g of the values differ, by up to %g" % (name, i, (a != b).float().mean(), (a - b).abs().max())
 
 
+def same_numbers(a, b):
+    return torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
+
+
+@pytest.mark.parametrize("head_dim", [16, 20, 32, 48, 64])
 @pytest.mark.parametrize("window", [None, 3])
-@pytest.mark.parametrize("value", [float("inf"), float("nan")])
-def test_float32_attention_within_a_page_keeps_what_is_not_finite_to_the_columns_that_see_it(value, window):
-    """One token's embedding is not finite: every position before it, and every one whose window is past it in all layers, has the bits that it has in the other kernels."""
-    cfg = shape(32, 32, 4, 2, 16, 2, window=window)
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), "one element"])
+def test_float32_attention_within_a_page_keeps_what_is_not_finite_to_the_columns_that_see_it(value, window, head_dim):
+    """One token's embedding is not finite, or one element of its value in the first layer: every position before it, and every one whose window is past it in all layers, has the bits
+    that it has in the other kernels."""
+    cfg = shape(32, 32, 4, 2, 16, 2, window=window) if head_dim == 16 else shape(64, 64, 4, 2, head_dim, 2, window=window)
     if window:
         cfg["max_window_layers"] = 0
     weights = model_weights(cfg)
-    weights["model.embed_tokens.weight"][5] = value
+    if value == "one element":
+        # (the token alone has something in its first place, eight in its normed row; that times 1e38 is beyond float32, in one of an element's neighbours only)
+        table = weights["model.embed_tokens.weight"]
+        table[:, 0], table[5] = 0.0, 0.0
+        table[5, 0] = 1.0
+        v = weights["model.layers.0.self_attn.v_proj.weight"]
+        v[head_dim + head_dim // 2 + 1, 0] = 1e38
+    else:
+        weights["model.embed_tokens.weight"][5] = value
     model = Model.from_config_dict(cfg, "float32", DEV).load(weights)
     tokens = [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17]
+    assert goes_by_units(cfg, [17, 4], 17)
 
-    def run():
+    def run(small):
         eng = Engine(model, max_tokens=256)
         a, b = eng.open(), eng.open()
-        return eng.step([(a, tokens, list(range(17))), (b, tokens[:4], [3])])
+        out = eng.step([(a, tokens, list(range(17))), (b, tokens[:4], [3])])
+        assert eng.n_small_steps == small
+        return out
 
     with policy(small_always=True):
-        got = run()
+        got = run(1)
     with policy(small=False):
-        want = run()
+        want = run(0)
     assert torch.isfinite(want[:4]).all() and torch.isfinite(want[17]).all() and not torch.isfinite(want[4]).any()
     assert torch.isfinite(want[16]).all() == bool(window)
-    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.nan_to_num(got), torch.nan_to_num(want))
+    assert same_numbers(got, want)
+
+
+@pytest.mark.parametrize("where", ["weights", "weights and values", "products"])
+@pytest.mark.parametrize("head_dim", [16, 20, 32, 64])
+def test_subnormal_numbers_in_float32_steps(where, head_dim):
+    """Values of 2^-130 and 2^-138 from subnormal weights, or of 2^-121 from ordinary ones, of which their products with the attention's weights are subnormal for some positions; the products behind
+    bring them back.  Decoding steps of one to five sequences (with a ring up to four), chunks, attention by units and by queries: the bits of the other kernels, and not those without values."""
+    cfg = shape(64, 96, 4, 2, head_dim, 2, vocab=97) if head_dim != 64 else shape(64, 96, 2, 1, 64, 2, vocab=97)
+
+    def made(values):
+        weights = model_weights(cfg)
+        for i in range(2):
+            p = "model.layers.%d." % i
+            down = {"weights": 2.0 ** -128, "weights and values": 2.0 ** -136, "products": 2.0 ** -120}[where]
+            weights[p + "self_attn.v_proj.weight"] *= down * values
+            weights[p + "self_attn.v_proj.bias"] *= down * values
+            weights[p + "self_attn.q_proj.weight"] *= 20.0                      # (weights of positions from 1 to 2^-20)
+            weights[p + "self_attn.k_proj.weight"] *= 20.0
+            weights[p + "self_attn.o_proj.weight"] *= 2.0 ** 125
+            weights[p + "mlp.up_proj.weight"][:40] *= 2.0 ** -126               # (and the second half of an MLP)
+            weights[p + "mlp.down_proj.weight"][:, :40] *= 2.0 ** 120
+        return Model.from_config_dict(cfg, "float32", DEV).load(weights)
+
+    def run(model):
+        out, ways = [], []
+        for n in (1, 2, 3, 4, 5):
+            eng = Engine(model, max_tokens=1024)
+            slots = [eng.open() for _ in range(n)]
+            for lens in ([33 - 4 * i for i in range(n)] if n < 3 else [12] * n, [1] * n, [1] * n, [3] * n, [1] * n):
+                ways.append(goes_by_units(cfg, lens, max(eng.length(s) + l for s, l in zip(slots, lens))))
+                out.append(eng.step([(s, helpers.random_tokens(l, 97, len(out) + i), [l - 1]) for i, (s, l) in enumerate(zip(slots, lens))]))
+            assert eng.n_small_steps == (5 if POLICY["small"] else 0)
+        return torch.cat(out), ways
+
+    model = made(1.0)
+    with policy(small_always=True):
+        got, ways = run(model)
+    with policy(small=False):
+        want, without = run(model)[0], run(made(0.0))[0]
+    assert torch.isfinite(want).all() and len(set(ways)) == 2
+    assert (want - without).abs().max() > 1e-4 * want.abs().max()
+    assert torch.equal(got, want)
 
 
 def model_weights(cfg, seed=13):
