@@ -522,7 +522,7 @@ void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, c
 // bytes at their number exclusive-or half their row, so that the 16 rows of an operand meet all banks; two stages in turn, one barrier each).  Loads are issued
 // half a stage or a stage ahead of being taken apart, which happens beside the products of the half before.  Whole groups' sums wait in LDS too, a float4 of each thread's in turn, where
 // the registers would cost a wave per SIMD.  Bound by the matrix cores' power and by what LDS delivers of x (12 pieces a wave for 64 products: two fifths of the time of those).  us, gate+up of the 7B
-// shape, down, q/k/v and o at 300 rows: 607, 406, 110 and 87 (744, 463, 114 and 98 with the float32 instructions); 2000 rows of o 380 (441).  With six products in place of eight gate+up took 581, and of that: weights in
+// shape, down, q/k/v and o at 300 rows: 607, 351, 103 and 86 (744, 463, 114 and 98 with the float32 instructions); 2000 rows of o 386 (441).  With six products in place of eight gate+up took 581, and of that: weights in
 // whole lines in place of the matrix cores' order 0.96, not without LDS between; waves of 48 or 64 features, one to a SIMD, 1.15 and 1.23; numbers taken apart in front of the products 1.01.
 #define GS_WAVES 4
 template <int RT, int FT, bool TAIL>
@@ -783,9 +783,9 @@ static double split_rounds(long long tiles, int groups, int per) {
 // unless blocks that walk all of K come out ahead of that with the sums that they need not write and add up, or two groups a block take no more rounds, which saves a start and
 // an end, where there is a full round of blocks without a tile's last group.  Below 400 tiles blocks of all of K leave a fifth of the places idle and were never the best.  From 512 tiles on, where two blocks a unit need no
 // scratch, groups' sums take 128 MB of it at most (1000 rows of 4608 x 3584: 74 MB, 290 -> 265 us), and from 768 on none.
-// us with two blocks a unit and so, weights that no cache holds: 300 and 1000 rows of 3584 x 18944 422 -> 354 and 1090 -> 985, 1000 of 1536 x 8960 276 -> 212, 500 of 4608 x 3584 178 -> 151, 64 of
-// 37888 x 3584 207 -> 181; a group a block and two: 100, 128 and 256 rows of 3584 x 18944 153 -> 145, 161 -> 152 and 279 -> 269, 160 of 4096 x 11008 155 -> 147, 200 of 7168 x 5120 161 -> 155 (28
-// tiles with 19 groups, 17 rows of 3584 x 18944, 70 -> 73: they keep one).  317 sizes of 19 weights, 17 to 2048 rows: 1.003 of the best number's time (at most 1.11, 80 rows of 7168 x 5120), two blocks a
+// us with two blocks a unit and so, weights that no cache holds, medians of ten turns: 300 and 1000 rows of 3584 x 18944 423 -> 351 and 1138 -> 993, 1000 of 1536 x 8960 284 -> 227, 500 of 4608 x 3584
+// 178 -> 152, 64 of 37888 x 3584 203 -> 178; a group a block and two: 100, 128 and 256 rows of 3584 x 18944 180 -> 160, 183 -> 167 and 302 -> 293, 160 of 4096 x 11008 172 -> 161, 200 of 7168 x 5120
+// 166 -> 161, 1000 of 1536 x 8960 234 -> 227.  317 sizes of 19 weights, 17 to 2048 rows: 1.003 of the best number's time (at most 1.11, 80 rows of 7168 x 5120), two blocks a
 // unit 1.025 (at most 1.29).
 extern "C" int tqk_gemm_f32_shares(int M, int N, int K) {
     const int groups = (K + G_GROUP - 1) / G_GROUP;

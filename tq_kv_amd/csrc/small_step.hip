@@ -4,7 +4,7 @@
 // microsecond and costs two to four in a replayed graph, and about as much again on the host.  One block on one compute unit runs
 // the step with barriers in place of launches.  It pulls weights and does a row's work at a fraction of the chip's rate, so this is the better way only
 // while that takes no longer than the launches it stands for: tqk_small_step_pays says where that is.  Two layers of 64 values, 3 sequences after
-// 20 tokens, five steps asked for together: 31.6 us a step in bfloat16 and 34.1 in float32 for what a replayed graph of 21 kernels does in 75 and 87; three of 96: 36.8 and 67 for 79 and 115.
+// 20 tokens, five steps asked for together: 27.1 us a step in bfloat16 and 30.7 in float32 for what a replayed graph of 21 kernels does in 75 and 87; three of 96: 35.5 and 64 for 79 and 115.
 // What a phase between two barriers takes (three of 96, bfloat16, attention by vector instructions, as other heads than those of 32 and 64 have it, us): norm 0.6 to 0.8, q/k/v 0.6, rotation 0.7,
 // attention 2.6, o 1.2, gate and up 1.5, down 1.3, none of it bytes or products but a wave's instructions one after the other, 4 and more cycles each.
 //
@@ -14,7 +14,7 @@
 // before it is finished; in decoding steps of few rows out of LDS, where two waves bring them (SmallRing).
 //
 // Every sum has the order that the kernels of larger models give it, and every rounding its place, so a position's result has the same bits whichever way
-// its step went.  In float32 that is gemm_generic.hip, elementwise.hip and attention_walk.h (within a page by the matrix cores, attend_page).  In bfloat16 the order goes by the kind of step
+// its step went.  In float32 that is gemm_generic.hip, elementwise.hip and attention_walk.h (within a page by the matrix cores where that is faster, attend_page).  In bfloat16 the order goes by the kind of step
 // (SmallPlan): norms that are divided by behind their product in decoding steps of up to 16 rows (skinny_fused.hip), and the matrix cores' attention of
 // attention_decode.hip and attention_prefill.hip for heads of 32 and 64.  Steps with more than a page of positions for such heads, and products whose K
 // those kernels deal out to waves or cut into pieces, are left to them.
@@ -273,7 +273,7 @@ struct RingFewProduct {
 struct SmallLayout {
     int ld_h, ld_a, ld_b, layers, norms, biases, angles, probs, squares, a, b, h, bytes;       // ld_h in floats, ld_a in T, ld_b in bytes
 };
-// (waves: that compute, all 16 or one less beside the ring, which gets the room that few queries leave)
+// (waves: that compute, all 16, or 14 beside the ring, which gets the room that few queries leave)
 static __device__ __host__ inline int queries_together(const TqkSmallStep& p, int waves) {
     const int width = p.head_dim <= 16 ? 16 : p.head_dim <= 32 ? 32 : 64, each = (p.n_rows * p.n_heads + waves - 1) / waves;
     return each < TQK_WAVE / width ? each : TQK_WAVE / width;
@@ -675,7 +675,8 @@ __device__ __forceinline__ void warm(const T* w, size_t n) {
     }
 }
 
-// D: the heads' size where the matrix cores take them (bfloat16: 32 or 64; float32, where the step lies in one page: up to 16, 32 or 64), or 0.  RING: one wave brings the weights into LDS (decoding steps of up to 16 rows).
+// D: the heads' size where the matrix cores take them (bfloat16: 32 or 64; float32, where tqk_small_step_pages has it so: up to 16, 32 or 64), or 0.  RING: two waves bring the
+// weights into LDS (tqk_small_step_rings: decoding steps of up to 4 rows in float32, 12 in bfloat16).
 template <typename T, int D, bool RING>
 __global__ __launch_bounds__(SS_THREADS)
 void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
@@ -861,7 +862,7 @@ void small_step_kernel(const TqkSmallStep p, const SmallPlan plan) {
     const float of_rows = 1.f / (float)rows, of_group = 1.f / (float)(nh / nkv);
     auto quotient = [&](int n) { return __builtin_amdgcn_readfirstlane((int)(((float)n + 0.5f) * of_rows)); };         // n / rows (numbers this small: exact)
 
-    // float32, steps of one page: units of up to 16 columns of a sequence and kv head, a wave each; a lane knows a sequence's first row, rows, first position and the units up to its end
+    // float32, steps that go by units: up to 16 columns of a sequence and kv head, a wave each; a lane knows a sequence's first row, rows, first position and the units up to its end
     int my_r0 = 0, my_n = 0, my_start = 0, units_to = 0, n_units = 0;
     if constexpr (!BF16 && D > 0) {
         if (lane < p.n_seqs) {
