@@ -162,7 +162,8 @@ def test_which_small_steps_have_their_weights_brought_into_lds(sizes, rings):
 @pytest.mark.parametrize("sizes,rows,decode,positions,pays", [
     ({}, 33, 0, 33, 1), ({}, 40, 1, 60, 0), ({}, 24, 1, 60, 1), ({"hidden": 96, "inter": 224, "n_heads": 3, "n_kv_heads": 1, "head_dim": 32, "n_layers": 3}, 33, 0, 33, 0),
     ({"hidden": 96, "inter": 224, "n_heads": 6, "n_kv_heads": 6, "n_layers": 3, "vocab": 300}, 24, 0, 3, 0),
-    ({"hidden": 96, "inter": 224, "n_heads": 6, "n_kv_heads": 1, "n_layers": 3, "vocab": 300}, 24, 0, 24, 1)])
+    ({"hidden": 96, "inter": 224, "n_heads": 6, "n_kv_heads": 1, "n_layers": 3, "vocab": 300}, 24, 0, 24, 1),
+    ({"inter": 32, "n_heads": 4, "n_kv_heads": 4, "head_dim": 48, "n_layers": 4, "vocab": 97}, 20, 1, 40, 0), ({"inter": 32, "n_heads": 4, "n_kv_heads": 1, "head_dim": 48, "n_layers": 4, "vocab": 97}, 20, 1, 40, 1)])
 def test_which_float32_small_steps_pay_in_one_launch(sizes, rows, decode, positions, pays):
     lib = ctypes.CDLL(kernels.library_path())
     assert lib.tqk_small_step_pays(ctypes.byref(small_step(act_dtype=0, **sizes)), rows, decode, positions) == pays

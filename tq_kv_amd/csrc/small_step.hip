@@ -1145,6 +1145,31 @@ extern "C" int tqk_small_step_takes(const TqkSmallStep* step) {
     return 1;
 }
 
+// Units of a float32 step's attention: up to 16 columns (a query and a head each) of a sequence and kv head.
+static int units_of(const TqkSmallStep& p, int rows) { return (rows * (p.n_heads / p.n_kv_heads) + 15) / 16 * p.n_kv_heads; }
+static int attention_units(const TqkSmallStep& p) {
+    int units = 0;
+    for (const int32_t *first = p.ints + p.seq_first, *end = first + p.n_seqs; first < end; ++first) units += units_of(p, first[1] - first[0]);
+    return units;
+}
+/* Whether a float32 step within a page has its attention by the matrix cores, a wave a unit (attend_page), and not a query a wave: where units are few beside the queries.  Heads of up to 16:
+ * a unit costs four queries for every 16 positions, and what a step saves beside them pays for ten.  Larger heads: a query of d elements costs d, a wave's turn of units, whose loads take 16 elements of a row at a
+ * time, 9 d, and each unit 50 for what it is served.  us a step by queries and by units, two layers: 3, 16 and 40 sequences, four heads of 16 on two 32.3 and 30.9 (units), 54 and 56, 109 and 117
+ * (queries), on four 32.7 and 32.9, 56 and 76, 112 and 168 (queries), on one 32.2 and 29.1, 54 and 46, 107 and 89 (units); 16 sequences, eight heads of 4 57 and 102
+ * (queries); one, four and 16 sequences, four heads of 32 on two 32.5 and 33.3, 39.4 and 38.0, 71 and 69 (queries), eight on two 40.0 and 40.7 (queries), 51.6 and 44.3, 102 and 70 (units), one head of
+ * 64 30.4 and 35.7, 34.4 and 38.2, 52 and 60 (queries), four on two 58 and 64 (queries), 71.5 and 69.7, 122 and 109 (units); prompts of 16 and 63 tokens, four heads of 16 on two 48
+ * and 37, 149 and 92, one head of 64 45 and 39, 150 and 92 (units).  925 steps of 37 shapes with heads of 4 to 64: 1.003 of the faster way's time (at most 1.14), and at most 1.045 of that by queries. */
+static bool by_units(const TqkSmallStep& p, int units, int n_rows, int positions) {
+    const int queries = n_rows * p.n_heads;
+    if (p.act_dtype != TQK_F32 || positions > TQK_PAGE) return false;
+    if (p.head_dim <= 16) return (4 * units - queries) * ((positions + 15) / 16) < 40;
+    return queries * p.head_dim >= 50 * units + 9 * ((units + SS_WAVES - 1) / SS_WAVES) * p.head_dim;
+}
+extern "C" int tqk_small_step_pages(const TqkSmallStep* step) {
+    const TqkSmallStep& p = *step;
+    return p.seq_first >= 0 && p.n_seqs > 0 && p.seq_first + p.n_seqs + 1 <= TQK_SMALL_INTS && by_units(p, attention_units(p), p.n_rows, p.max_end);
+}
+
 /* Whether that is the faster way, by an estimate in microseconds (n_rows: of the step; decode: one token a sequence, which the other kernels run as a replayed graph; positions: the
  * furthest one).  One block: 5 a layer for its barriers and chains of short operations, its weights at 33 KB (27 in float32) a microsecond, and for every row what
  * its products, its other work and its heads' pages take; the head's weights at 39 KB.  The other kernels, ten launches a layer: 20 a layer in a graph (33 in float32) and 32 (45) one by one.
@@ -1160,9 +1185,10 @@ extern "C" int tqk_small_step_pays(const TqkSmallStep* step, int n_rows, int dec
     const double size = f32 ? 4 : 2, q = (double)p.n_heads * p.head_dim;
     const double thousands = 1e-3 * p.hidden * (2 * q + 2. * p.n_kv_heads * p.head_dim + 3. * p.inter);            // weights of a layer
     const double heads = 0.08 * p.n_heads * ((positions + TQK_PAGE - 1) / TQK_PAGE);
-    // (float32 within a page: columns of a sequence and kv head share an instruction in prompts.  Eight chunks of three tokens, three layers of 96, six heads of 16 on as many: 155 us here,
-    // 144 there)
-    const double a_row = f32 && positions <= TQK_PAGE ? 0.15 + 0.0085 * thousands + (decode ? heads : 0.03 * p.n_kv_heads) : 0.15 + (f32 ? 0.0115 : 0.0043) * thousands + heads;
+    // (float32 by units: columns of a sequence and kv head share an instruction.  A prompt is taken for one sequence's; eight chunks of three tokens, three layers of 96, six heads of 16 on as many:
+    // 155 us here, 144 there; 20 sequences after 38 tokens, four layers of 64, four heads of 48 on as many, which go by queries: 329 and 194)
+    const bool units = by_units(p, decode ? n_rows * units_of(p, 1) : units_of(p, n_rows), n_rows, positions);
+    const double a_row = units ? 0.15 + 0.0085 * thousands + (decode ? heads : 0.03 * p.n_kv_heads) : 0.15 + (f32 ? 0.0115 : 0.0043) * thousands + heads;
     const double here = 8 + p.n_layers * (5 + thousands * size / (f32 ? 27 : 33) + n_rows * a_row) + 1e-3 * p.vocab * p.hidden * size / 39;
     const double there = decode ? 15 + p.n_layers * (f32 ? 33 : 20) : 15 + p.n_layers * (f32 ? 45 : 32);
     return here < there;
@@ -1196,28 +1222,6 @@ static int launch_small(const TqkSmallStep& p, int lds, hipStream_t s) {
     if (e != hipSuccess) return tqk_fail("tqk_small_step: %s", hipGetErrorString(e));
     small_step_kernel<T, D, RING><<<1 + 8 * (p.n_layers + 1), SS_THREADS, lds, s>>>(p, small_plan(p));
     return tqk_check_launch("tqk_small_step");
-}
-
-// Units of a float32 step's attention: up to 16 columns (a query and a head each) of a sequence and kv head.
-static int attention_units(const TqkSmallStep& p) {
-    int units = 0;
-    for (const int32_t *first = p.ints + p.seq_first, *end = first + p.n_seqs; first < end; ++first)
-        units += ((first[1] - first[0]) * (p.n_heads / p.n_kv_heads) + 15) / 16 * p.n_kv_heads;
-    return units;
-}
-/* Whether a float32 step within a page has its attention by the matrix cores, a wave a unit (attend_page), and not a query a wave: where units are few beside the queries.  Heads of up to 16:
- * a unit costs four queries for every 16 positions, and what a step saves beside them pays for ten.  Larger heads: a query of d elements costs d, a wave's turn of units, whose loads take 16 elements of a row at a
- * time, 9 d, and each unit 50 for what it is served.  us a step by queries and by units, two layers: 3, 16 and 40 sequences, four heads of 16 on two 32.3 and 30.9 (units), 54 and 56, 109 and 117
- * (queries), on four 32.7 and 32.9, 56 and 76, 112 and 168 (queries), on one 32.2 and 29.1, 54 and 46, 107 and 89 (units); 16 sequences, eight heads of 4 57 and 102
- * (queries); one, four and 16 sequences, four heads of 32 on two 32.5 and 33.3, 39.4 and 38.0, 71 and 69 (queries), eight on two 40.0 and 40.7 (queries), 51.6 and 44.3, 102 and 70 (units), one head of
- * 64 30.4 and 35.7, 34.4 and 38.2, 52 and 60 (queries), four on two 58 and 64 (queries), 71.5 and 69.7, 122 and 109 (units); prompts of 16 and 63 tokens, four heads of 16 on two 48
- * and 37, 149 and 92, one head of 64 45 and 39, 150 and 92 (units).  925 steps of 37 shapes with heads of 4 to 64: 1.003 of the faster way's time (at most 1.14), and at most 1.045 of that by queries. */
-extern "C" int tqk_small_step_pages(const TqkSmallStep* step) {
-    const TqkSmallStep& p = *step;
-    if (p.act_dtype != TQK_F32 || p.max_end > TQK_PAGE || p.seq_first < 0 || p.n_seqs < 1 || p.seq_first + p.n_seqs + 1 > TQK_SMALL_INTS) return 0;
-    const int queries = p.n_rows * p.n_heads, units = attention_units(p);
-    if (p.head_dim <= 16) return (4 * units - queries) * ((p.max_end + 15) / 16) < 40;
-    return queries * p.head_dim >= 50 * units + 9 * ((units + SS_WAVES - 1) / SS_WAVES) * p.head_dim;
 }
 
 /* Whether a step's weights come into LDS by waves of their own: decoding steps of few rows, where the ring fits beside the rows and two waves fewer take no more turns for the attention's
