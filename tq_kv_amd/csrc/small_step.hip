@@ -1158,7 +1158,7 @@ static int attention_units(const TqkSmallStep& p) {
  * (queries), on four 32.7 and 32.9, 56 and 76, 112 and 168 (queries), on one 32.2 and 29.1, 54 and 46, 107 and 89 (units); 16 sequences, eight heads of 4 57 and 102
  * (queries); one, four and 16 sequences, four heads of 32 on two 32.5 and 33.3, 39.4 and 38.0, 71 and 69 (queries), eight on two 40.0 and 40.7 (queries), 51.6 and 44.3, 102 and 70 (units), one head of
  * 64 30.4 and 35.7, 34.4 and 38.2, 52 and 60 (queries), four on two 58 and 64 (queries), 71.5 and 69.7, 122 and 109 (units); prompts of 16 and 63 tokens, four heads of 16 on two 48
- * and 37, 149 and 92, one head of 64 45 and 39, 150 and 92 (units).  925 steps of 37 shapes with heads of 4 to 64: 1.003 of the faster way's time (at most 1.14), and at most 1.045 of that by queries. */
+ * and 37, 149 and 92, one head of 64 45 and 39, 150 and 92 (units).  925 steps of 40 shapes with heads of 4 to 64: 1.004 of the faster way's time (at most 1.14), and at most 1.045 of that by queries. */
 static bool by_units(const TqkSmallStep& p, int units, int n_rows, int positions) {
     const int queries = n_rows * p.n_heads;
     if (p.act_dtype != TQK_F32 || positions > TQK_PAGE) return false;
